@@ -35,7 +35,6 @@ constexpr int kRounds = 16;                          // keys per lane
 constexpr int kTile = kThreads * kRounds;            // 4096 keys per tile
 constexpr int kWaveKeys = prim::kWave * kRounds;     // 1024 contiguous keys per wave
 constexpr int kDigits = 256;
-static_assert(kTile == kScanTile, "sort tiles match the chained-scan tiles");
 
 __device__ __forceinline__ unsigned digit_of(unsigned long long key, int shift)
 {
@@ -197,9 +196,7 @@ __global__ __launch_bounds__(kThreads) void unique_kernel(const unsigned long lo
 {
     __shared__ long long s_tile;
     __shared__ unsigned s_wave[kWaves], s_prefix;
-    if (threadIdx.x == 0) s_tile = (long long) (atomicAdd(c.tile_counter, 1ull) - c.tile_base);
-    __syncthreads();
-    const long long tile = s_tile;
+    const long long tile = prim::take_tile(c, &s_tile);
     const long long base = tile * kTile + (long long) threadIdx.x * kRounds;
     unsigned long long v[kRounds];
     unsigned long long prev = base > 0 && base - 1 < n ? in[base - 1] : 0ull;
@@ -213,23 +210,12 @@ __global__ __launch_bounds__(kThreads) void unique_kernel(const unsigned long lo
     }
     unsigned agg;
     const unsigned before = prim::block_exclusive_sum_u32<kThreads>((unsigned) __popc(keep), s_wave, &agg);
-    if (threadIdx.x < prim::kWave) {
-        unsigned prefix = 0;
-        if (tile == 0) {
-            if (threadIdx.x == 0) prim::publish(c.status, tile, c.epoch, prim::kStatePrefix, agg);
-        } else {
-            if (threadIdx.x == 0) prim::publish(c.status, tile, c.epoch, prim::kStateAggregate, agg);
-            prefix = prim::lookback_prefix(c.status, tile, c.epoch);
-            if (threadIdx.x == 0) prim::publish(c.status, tile, c.epoch, prim::kStatePrefix, prefix + agg);
-        }
-        if (threadIdx.x == 0) s_prefix = prefix;
-    }
-    __syncthreads();
-    unsigned at = s_prefix + before;
+    const unsigned prefix = prim::chain_prefix(c, tile, agg, &s_prefix);
+    unsigned at = prefix + before;
 #pragma unroll
     for (int k = 0; k < kRounds; k++)
         if ((keep >> k) & 1u) out[at++] = v[k];
-    if (tile == c.tiles - 1 && threadIdx.x == 0) *d_count = s_prefix + agg;
+    if (tile == c.tiles - 1 && threadIdx.x == 0) *d_count = prefix + agg;
 }
 
 // Columns and row offsets from E sorted keys: key i starts row u = key >> b,
@@ -348,7 +334,7 @@ struct Builder {
                                shift, counts, tiles);
             if (!ok(hipGetLastError())) return false;
             ChainArgs c;
-            if (!ok(chain.prepare(tiles * kDigits, kScanTile, &c, stream))) return false;
+            if (!ok(chain.prepare(tiles * kDigits, scan_tile_items(tiles * kDigits), &c, stream))) return false;
             if (!ok(launch_scan_u32(counts, counts, tiles * kDigits, true, c, nullptr, stream))) return false;
             hipLaunchKernelGGL(sort_downsweep_kernel, dim3((unsigned) tiles), dim3(kThreads), 0, stream, keys[cur],
                                keys[cur ^ 1], n, shift, counts, tiles);
@@ -368,7 +354,7 @@ struct Builder {
         long long m = n - loops;
         if (dedup && m > 0) {
             ChainArgs c;
-            if (!ok(chain.prepare(m, kScanTile, &c, stream))) return false;
+            if (!ok(chain.prepare(m, kTile, &c, stream))) return false;
             hipLaunchKernelGGL(unique_kernel, dim3((unsigned) c.tiles), dim3(kThreads), 0, stream, keys[0], keys[1],
                                m, c, chain.d_word);
             if (!ok(hipGetLastError())) return false;

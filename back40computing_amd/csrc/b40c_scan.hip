@@ -2,7 +2,7 @@
 // (C ABI in include/b40c_scan.h).
 //
 // One kernel per call.  A workgroup takes the next tile index from an atomic
-// counter, reduces its 4096 items, publishes the aggregate, looks back over
+// counter, reduces its items (4096 to 16384), publishes the aggregate, looks back over
 // the predecessors' status words for its exclusive prefix
 // (prim::lookback_prefix), publishes its inclusive prefix and writes its
 // outputs.  This replaces the reference's upsweep / spine / downsweep passes
@@ -23,26 +23,37 @@ namespace b40c_hip {
 namespace {
 
 constexpr int kThreads = kScanThreads;
-constexpr int kItems = kScanItems;
+constexpr int kWaves = kThreads / prim::kWave;
 
-// Items of one thread: kItems consecutive elements from `base` (blocked
-// arrangement), `fill` past the end.
-__device__ __forceinline__ void load_blocked(const uint32_t *in, long long n, long long base, bool vec,
-                                             uint32_t fill, uint32_t (&v)[kItems])
+// Wave-striped arrangement of a tile: wave w owns 64 * ITEMS consecutive
+// items and reads them in rounds of 256, lane l taking four consecutive
+// items at 4 l.  Each 16-byte load instruction of a wave then covers one
+// contiguous KiB (a blocked arrangement touched 64 lines per instruction),
+// and the items keep their order as (round, lane, item).  `fill` past the end.
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// Tiles of a large input stream through memory once: non-temporal (2^26
+// items 135.9 -> 127.7 us; small inputs keep the caches for their reader).
+template <int ROUNDS>
+__device__ __forceinline__ void load_striped(const uint32_t *in, long long n, long long base, bool vec, uint32_t fill,
+                                             uint4 (&v)[ROUNDS])
 {
-    if (vec && base + kItems <= n) {
-        const uint4 *p = reinterpret_cast<const uint4 *>(in + base);
 #pragma unroll
-        for (int k = 0; k < kItems / 4; k++) {
-            const uint4 q = p[k];
-            v[4 * k] = q.x;
-            v[4 * k + 1] = q.y;
-            v[4 * k + 2] = q.z;
-            v[4 * k + 3] = q.w;
+    for (int r = 0; r < ROUNDS; r++) {
+        const long long i = base + r * 256;
+        if (vec && i + 4 <= n) {
+            if constexpr (ROUNDS > 2) {
+                const u32x4 t = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(in + i));
+                v[r] = make_uint4(t.x, t.y, t.z, t.w);
+            } else {
+                v[r] = *reinterpret_cast<const uint4 *>(in + i);
+            }
+        } else {
+            v[r].x = i < n ? in[i] : fill;
+            v[r].y = i + 1 < n ? in[i + 1] : fill;
+            v[r].z = i + 2 < n ? in[i + 2] : fill;
+            v[r].w = i + 3 < n ? in[i + 3] : fill;
         }
-    } else {
-#pragma unroll
-        for (int k = 0; k < kItems; k++) v[k] = base + k < n ? in[base + k] : fill;
     }
 }
 
@@ -55,90 +66,137 @@ __device__ __forceinline__ bool selected(uint32_t key, int op, uint32_t comparan
     }
 }
 
-// Tile index from the launch-order counter, and the tile's exclusive prefix
-// given its aggregate (every thread calls it; the result is returned to all).
-__device__ __forceinline__ long long take_tile(const ChainArgs &c, long long *s_tile)
-{
-    if (threadIdx.x == 0)
-        *s_tile = (long long) (atomicAdd(c.tile_counter, 1ull) - c.tile_base);
-    __syncthreads();
-    return *s_tile;
-}
-
-__device__ __forceinline__ unsigned chain_prefix(const ChainArgs &c, long long tile, unsigned aggregate,
-                                                 unsigned *s_prefix)
-{
-    if (threadIdx.x < prim::kWave) {
-        unsigned prefix = 0;
-        if (tile == 0) {
-            if (threadIdx.x == 0) prim::publish(c.status, tile, c.epoch, prim::kStatePrefix, aggregate);
-        } else {
-            if (threadIdx.x == 0) prim::publish(c.status, tile, c.epoch, prim::kStateAggregate, aggregate);
-            prefix = prim::lookback_prefix(c.status, tile, c.epoch);
-            if (threadIdx.x == 0) prim::publish(c.status, tile, c.epoch, prim::kStatePrefix, prefix + aggregate);
-        }
-        if (threadIdx.x == 0) *s_prefix = prefix;
-    }
-    __syncthreads();
-    return *s_prefix;
-}
-
+// Bound: HBM, eight bytes per item.  The tile counter is one address whose
+// atomics serialise (about 15 ns each, so 16385 tiles of 4096 items alone
+// cost 245 us on 2^26 items): large inputs take tiles of 16384 items
+// (ROUNDS = 8), small ones tiles of 4096 (ROUNDS = 2), which spread a short
+// input over more workgroups (see scan_tile_items).
+template <int ROUNDS>
 __global__ __launch_bounds__(kThreads) void scan_kernel(const uint32_t *in, uint32_t *out, long long n, int exclusive,
                                                         int vec, ChainArgs c, uint32_t *d_total)
 {
     __shared__ long long s_tile;
-    __shared__ unsigned s_wave[kThreads / prim::kWave], s_prefix;
-    const long long tile = take_tile(c, &s_tile);
-    const long long base = tile * kScanTile + (long long) threadIdx.x * kItems;
-    uint32_t v[kItems];
-    load_blocked(in, n, base, vec != 0, 0u, v);
-    unsigned sum = 0;
+    __shared__ unsigned s_wave[kWaves], s_prefix;
+    const long long tile = prim::take_tile(c, &s_tile);
+    const int lane = prim::lane(), wave = threadIdx.x / prim::kWave;
+    const long long base = tile * (kThreads * 4LL * ROUNDS) + (long long) wave * (256 * ROUNDS) + 4 * lane;
+    uint4 v[ROUNDS];
+    load_striped<ROUNDS>(in, n, base, vec != 0, 0u, v);
+    unsigned off[ROUNDS], run = 0;  // sum of the wave's items before the lane's four of each round
 #pragma unroll
-    for (int k = 0; k < kItems; k++) sum += v[k];
-    unsigned agg;
-    const unsigned before = prim::block_exclusive_sum_u32<kThreads>(sum, s_wave, &agg);
-    const unsigned prefix = chain_prefix(c, tile, agg, &s_prefix);
-    unsigned run = prefix + before;
-#pragma unroll
-    for (int k = 0; k < kItems; k++) {
-        const unsigned x = v[k];
-        v[k] = exclusive ? run : run + x;
-        run += x;
+    for (int r = 0; r < ROUNDS; r++) {
+        const unsigned sum = v[r].x + v[r].y + v[r].z + v[r].w;
+        const unsigned incl = prim::wave_inclusive_sum_u32(sum);
+        off[r] = run + incl - sum;
+        run += (unsigned) __builtin_amdgcn_readlane((int) incl, prim::kWave - 1);
     }
-    if (vec && base + kItems <= n) {
-        uint4 *p = reinterpret_cast<uint4 *>(out + base);
+    if (lane == 0) s_wave[wave] = run;
+    __syncthreads();
+    unsigned before = 0, agg = 0;
 #pragma unroll
-        for (int k = 0; k < kItems / 4; k++) p[k] = make_uint4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
-    } else {
-#pragma unroll
-        for (int k = 0; k < kItems; k++)
-            if (base + k < n) out[base + k] = v[k];
+    for (int w = 0; w < kWaves; w++) {
+        const unsigned t = s_wave[w];
+        if (w < wave) before += t;
+        agg += t;
     }
-    if (d_total && tile == c.tiles - 1 && threadIdx.x == 0) *d_total = prefix + agg;
+    const unsigned prefix = prim::chain_prefix(c, tile, agg, &s_prefix);
+    const unsigned shift = prefix + before;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        const long long i = base + r * 256;
+        const unsigned x = shift + off[r];
+        uint4 o;
+        if (exclusive) {
+            o.x = x;
+            o.y = o.x + v[r].x;
+            o.z = o.y + v[r].y;
+            o.w = o.z + v[r].z;
+        } else {
+            o.x = x + v[r].x;
+            o.y = o.x + v[r].y;
+            o.z = o.y + v[r].z;
+            o.w = o.z + v[r].w;
+        }
+        if (vec && i + 4 <= n) {
+            if constexpr (ROUNDS > 2)
+                __builtin_nontemporal_store(u32x4{o.x, o.y, o.z, o.w}, reinterpret_cast<u32x4 *>(out + i));
+            else
+                *reinterpret_cast<uint4 *>(out + i) = o;
+        } else {
+            if (i < n) out[i] = o.x;
+            if (i + 1 < n) out[i + 1] = o.y;
+            if (i + 2 < n) out[i + 2] = o.z;
+            if (i + 3 < n) out[i + 3] = o.w;
+        }
+    }
+    if (d_total && tile == c.tiles - 1 && threadIdx.x == 0) {
+        *d_total = prefix + agg;
+        __threadfence_system();  // (may be pinned host memory)
+    }
 }
 
+// Kept items are staged in LDS at their rank in the tile and leave it as
+// consecutive words per wave (one contiguous run a tile), whatever the
+// share that is kept.  Bound: HBM.
+template <int ROUNDS>
 __global__ __launch_bounds__(kThreads) void copy_if_kernel(const uint32_t *in, uint32_t *out, long long n, int op,
                                                            uint32_t comparand, int vec, ChainArgs c,
-                                                           uint32_t *d_count)
+                                                           uint32_t *d_count, uint32_t *h_count)
 {
+    constexpr int kTileItems = kThreads * 4 * ROUNDS;
     __shared__ long long s_tile;
-    __shared__ unsigned s_wave[kThreads / prim::kWave], s_prefix;
-    const long long tile = take_tile(c, &s_tile);
-    const long long base = tile * kScanTile + (long long) threadIdx.x * kItems;
-    uint32_t v[kItems];
-    load_blocked(in, n, base, vec != 0, 0u, v);
-    unsigned keep = 0;
+    __shared__ unsigned s_wave[kWaves], s_prefix;
+    __shared__ uint32_t stage[kTileItems];
+    const long long tile = prim::take_tile(c, &s_tile);
+    const int lane = prim::lane(), wave = threadIdx.x / prim::kWave;
+    const long long base = tile * (long long) kTileItems + (long long) wave * (256 * ROUNDS) + 4 * lane;
+    uint4 v[ROUNDS];
+    load_striped<ROUNDS>(in, n, base, vec != 0, 0u, v);
+    unsigned keep = 0, run = 0, off[ROUNDS];
 #pragma unroll
-    for (int k = 0; k < kItems; k++)
-        if (base + k < n && selected(v[k], op, comparand)) keep |= 1u << k;
-    unsigned agg;
-    const unsigned before = prim::block_exclusive_sum_u32<kThreads>((unsigned) __popc(keep), s_wave, &agg);
-    const unsigned prefix = chain_prefix(c, tile, agg, &s_prefix);
-    unsigned at = prefix + before;
+    for (int r = 0; r < ROUNDS; r++) {
+        const long long i = base + r * 256;
+        unsigned m = 0;
+        if (i < n && selected(v[r].x, op, comparand)) m |= 1u;
+        if (i + 1 < n && selected(v[r].y, op, comparand)) m |= 2u;
+        if (i + 2 < n && selected(v[r].z, op, comparand)) m |= 4u;
+        if (i + 3 < n && selected(v[r].w, op, comparand)) m |= 8u;
+        keep |= m << (4 * r);
+        const unsigned cnt = (unsigned) __popc(m);
+        const unsigned incl = prim::wave_inclusive_sum_u32(cnt);
+        off[r] = run + incl - cnt;
+        run += (unsigned) __builtin_amdgcn_readlane((int) incl, prim::kWave - 1);
+    }
+    static_assert(4 * ROUNDS <= 32, "one keep bit per item");
+    if (lane == 0) s_wave[wave] = run;
+    __syncthreads();
+    unsigned before = 0, agg = 0;
 #pragma unroll
-    for (int k = 0; k < kItems; k++)
-        if ((keep >> k) & 1u) out[at++] = v[k];
-    if (d_count && tile == c.tiles - 1 && threadIdx.x == 0) *d_count = prefix + agg;
+    for (int w = 0; w < kWaves; w++) {
+        const unsigned t = s_wave[w];
+        if (w < wave) before += t;
+        agg += t;
+    }
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        unsigned at = before + off[r];
+        const unsigned m = keep >> (4 * r);
+        if (m & 1u) stage[at++] = v[r].x;
+        if (m & 2u) stage[at++] = v[r].y;
+        if (m & 4u) stage[at++] = v[r].z;
+        if (m & 8u) stage[at++] = v[r].w;
+    }
+    // (chain_prefix's workgroup barrier orders the staging before its reads)
+    const unsigned prefix = prim::chain_prefix(c, tile, agg, &s_prefix);
+    for (unsigned i = threadIdx.x; i < agg; i += kThreads) {
+        if constexpr (ROUNDS > 2) __builtin_nontemporal_store(stage[i], out + prefix + i);
+        else out[prefix + i] = stage[i];
+    }
+    if (tile == c.tiles - 1 && threadIdx.x == 0) {
+        if (d_count) *d_count = prefix + agg;
+        if (h_count) *h_count = prefix + agg;
+        __threadfence_system();
+    }
 }
 
 __global__ void fill_u32_kernel(uint32_t *p, long long n, uint32_t value)
@@ -149,21 +207,41 @@ __global__ void fill_u32_kernel(uint32_t *p, long long n, uint32_t value)
 
 }  // namespace
 
+// Inputs past 2^20 items take 16384-item tiles (see scan_kernel): there the
+// tile counter, not the workgroups in flight, sets the pace (2^22 items:
+// 26.8 us in tiles of 4096, 14.4 in tiles of 16384; 2^20 items, which are
+// 256 of the small tiles: 10.4 us either way).  2^26 items: 249 us in tiles
+// of 4096 read in a blocked arrangement, 130 us now (4.1 TB/s; a copy of
+// the same size reaches 5.1).
+int scan_tile_items(long long n) { return n > (1LL << 20) ? 16384 : 4096; }
+
 hipError_t launch_scan_u32(const uint32_t *in, uint32_t *out, long long n, bool exclusive, const ChainArgs &c,
                            uint32_t *d_total, hipStream_t st)
 {
     const int vec = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-    hipLaunchKernelGGL(scan_kernel, dim3((unsigned) c.tiles), dim3(kThreads), 0, st, in, out, n, exclusive ? 1 : 0,
-                       vec, c, d_total);
+    if (scan_tile_items(n) == 16384)
+        hipLaunchKernelGGL(scan_kernel<8>, dim3((unsigned) c.tiles), dim3(kThreads), 0, st, in, out, n,
+                           exclusive ? 1 : 0, vec, c, d_total);
+    else
+        hipLaunchKernelGGL(scan_kernel<2>, dim3((unsigned) c.tiles), dim3(kThreads), 0, st, in, out, n,
+                           exclusive ? 1 : 0, vec, c, d_total);
     return hipGetLastError();
 }
 
+// (8192: a 16384-item stage takes 64 KiB of LDS and leaves two workgroups
+// per CU, 2^26 items keeping nearly all 169 us instead of 160)
+int copy_if_tile_items(long long n) { return n > (1LL << 20) ? 8192 : 4096; }
+
 hipError_t launch_copy_if_u32(const uint32_t *in, uint32_t *out, long long n, int op, uint32_t comparand,
-                              const ChainArgs &c, uint32_t *d_count, hipStream_t st)
+                              const ChainArgs &c, uint32_t *d_count, uint32_t *h_count, hipStream_t st)
 {
     const int vec = (reinterpret_cast<uintptr_t>(in) & 15) == 0;
-    hipLaunchKernelGGL(copy_if_kernel, dim3((unsigned) c.tiles), dim3(kThreads), 0, st, in, out, n, op, comparand,
-                       vec, c, d_count);
+    if (copy_if_tile_items(n) == 8192)
+        hipLaunchKernelGGL(copy_if_kernel<4>, dim3((unsigned) c.tiles), dim3(kThreads), 0, st, in, out, n, op,
+                           comparand, vec, c, d_count, h_count);
+    else
+        hipLaunchKernelGGL(copy_if_kernel<2>, dim3((unsigned) c.tiles), dim3(kThreads), 0, st, in, out, n, op,
+                           comparand, vec, c, d_count, h_count);
     return hipGetLastError();
 }
 
@@ -176,7 +254,8 @@ hipError_t launch_copy_if_u32(const uint32_t *in, uint32_t *out, long long n, in
 // ---------------------------------------------------------------------------
 namespace {
 
-constexpr long long kNoAllocMaxTiles = 16384;  // 2^26 items
+constexpr long long kNoAllocMaxItems = 1LL << 26;
+constexpr long long kNoAllocMaxTiles = 16384;  // (of at least 4096 items)
 constexpr int kNoAllocStatus = 32;
 constexpr int kNoAllocDevices = 64;
 
@@ -250,10 +329,9 @@ hipError_t ChainState::prepare(long long items, int tile_items, ChainArgs *c, hi
     }
     c->status = d_status;
     c->tile_counter = d_counter;
-    c->tile_base = 0;
     c->epoch = epoch;
     c->tiles = tiles;
-    return hipMemsetAsync(d_counter, 0, sizeof(unsigned long long), st);
+    return hipSuccess;
 }
 
 void ChainState::release()
@@ -272,6 +350,10 @@ struct b40c_scan_enactor {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     ChainState chain;
+    // Pinned host word the last tile of a launch writes its total to: the
+    // host reads it once the launch's stop event has passed, with no copy
+    // of its own (about 25 us of a call).
+    uint32_t *h_word = nullptr, *h_word_dev = nullptr;
     float last_ms = 0.f;
 };
 
@@ -303,7 +385,9 @@ bfs_status b40c_scan_enactor_create(int32_t device, b40c_scan_enactor **out)
     en->device = device;
     if ((e = hipStreamCreateWithFlags(&en->stream, hipStreamNonBlocking)) != hipSuccess ||
         (e = hipEventCreate(&en->ev0)) != hipSuccess || (e = hipEventCreate(&en->ev1)) != hipSuccess ||
-        (e = en->chain.init(device)) != hipSuccess) {
+        (e = en->chain.init(device)) != hipSuccess ||
+        (e = hipHostMalloc(&en->h_word, sizeof(uint32_t), hipHostMallocDefault)) != hipSuccess ||
+        (e = hipHostGetDevicePointer(reinterpret_cast<void **>(&en->h_word_dev), en->h_word, 0)) != hipSuccess) {
         b40c_scan_enactor_destroy(en);
         return host_hip_fail(e, "create scan enactor");
     }
@@ -317,6 +401,7 @@ void b40c_scan_enactor_destroy(b40c_scan_enactor *e)
     (void) hipSetDevice(e->device);
     if (e->stream) (void) hipStreamSynchronize(e->stream);
     e->chain.release();
+    if (e->h_word) (void) hipHostFree(e->h_word);
     if (e->ev0) (void) hipEventDestroy(e->ev0);
     if (e->ev1) (void) hipEventDestroy(e->ev1);
     if (e->stream) (void) hipStreamDestroy(e->stream);
@@ -336,14 +421,15 @@ bfs_status b40c_scan(b40c_scan_enactor *e, const uint32_t *d_in, uint32_t *d_out
         return BFS_OK;
     }
     ChainArgs c;
-    if ((r = e->chain.prepare(n, kScanTile, &c, e->stream)) != hipSuccess) return host_hip_fail(r, "scan status storage");
+    if ((r = e->chain.prepare(n, scan_tile_items(n), &c, e->stream)) != hipSuccess)
+        return host_hip_fail(r, "scan status storage");
     if ((r = hipEventRecord(e->ev0, e->stream)) != hipSuccess) return host_hip_fail(r, "record");
-    if ((r = launch_scan_u32(d_in, d_out, n, exclusive != 0, c, e->chain.d_word, e->stream)) != hipSuccess)
+    if ((r = launch_scan_u32(d_in, d_out, n, exclusive != 0, c, h_total ? e->h_word_dev : nullptr, e->stream)) !=
+        hipSuccess)
         return host_hip_fail(r, "launch scan");
     bfs_status st = timed_sync(e);
     if (st != BFS_OK) return st;
-    if (h_total && (r = hipMemcpy(h_total, e->chain.d_word, sizeof(uint32_t), hipMemcpyDeviceToHost)) != hipSuccess)
-        return host_hip_fail(r, "read scan total");
+    if (h_total) *h_total = *static_cast<volatile uint32_t *>(e->h_word);
     return BFS_OK;
 }
 
@@ -364,19 +450,15 @@ bfs_status b40c_copy_if(b40c_scan_enactor *e, const uint32_t *d_in, uint32_t *d_
         return BFS_OK;
     }
     ChainArgs c;
-    if ((r = e->chain.prepare(n, kScanTile, &c, e->stream)) != hipSuccess) return host_hip_fail(r, "copy-if status storage");
-    uint32_t *count = d_num_compacted ? d_num_compacted : e->chain.d_word;
+    if ((r = e->chain.prepare(n, copy_if_tile_items(n), &c, e->stream)) != hipSuccess)
+        return host_hip_fail(r, "copy-if status storage");
     if ((r = hipEventRecord(e->ev0, e->stream)) != hipSuccess) return host_hip_fail(r, "record");
-    if ((r = launch_copy_if_u32(d_in, d_out, n, (int) op, comparand, c, count, e->stream)) != hipSuccess)
+    if ((r = launch_copy_if_u32(d_in, d_out, n, (int) op, comparand, c, d_num_compacted,
+                                h_num_compacted ? e->h_word_dev : nullptr, e->stream)) != hipSuccess)
         return host_hip_fail(r, "launch copy-if");
     bfs_status st = timed_sync(e);
     if (st != BFS_OK) return st;
-    if (h_num_compacted) {
-        uint32_t k = 0;
-        if ((r = hipMemcpy(&k, count, sizeof(uint32_t), hipMemcpyDeviceToHost)) != hipSuccess)
-            return host_hip_fail(r, "read compacted count");
-        *h_num_compacted = k;
-    }
+    if (h_num_compacted) *h_num_compacted = *static_cast<volatile uint32_t *>(e->h_word);
     return BFS_OK;
 }
 
@@ -384,7 +466,7 @@ bfs_status b40c_scan_noalloc(int32_t device, const uint32_t *d_in, uint32_t *d_o
                              uint32_t *d_total, void *stream)
 {
     if (n < 0 || (n > 0 && (!d_in || !d_out))) return host_fail(BFS_ERR_INVALID_ARG, "invalid scan arguments");
-    if (n > kNoAllocMaxTiles * kScanTile)
+    if (n > kNoAllocMaxItems)
         return host_fail(BFS_ERR_INVALID_ARG, "scan longer than the allocation-free limit of 2^26 items");
     int count = 0;
     if (hipGetDeviceCount(&count) != hipSuccess || count == 0) return host_fail(BFS_ERR_NO_DEVICE, "no HIP device");
@@ -403,10 +485,10 @@ bfs_status b40c_scan_noalloc(int32_t device, const uint32_t *d_in, uint32_t *d_o
     unsigned long long *words = nullptr;
     if ((r = noalloc_scratch(device, &words)) != hipSuccess) return host_hip_fail(r, "scan scratch address");
     ChainArgs c;
-    c.tiles = (n + kScanTile - 1) / kScanTile;
+    const int tile_items = scan_tile_items(n);
+    c.tiles = (n + tile_items - 1) / tile_items;
     c.status = words + kNoAllocStatus;
     c.tile_counter = words;
-    c.tile_base = 0;
     c.epoch = 0;
     const unsigned clear_blocks = (unsigned) std::min<long long>((c.tiles + kThreads - 1) / kThreads, 64);
     hipLaunchKernelGGL(noalloc_clear_kernel, dim3(clear_blocks), dim3(kThreads), 0, st, words, c.tiles);
