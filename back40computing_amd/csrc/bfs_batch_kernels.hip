@@ -189,6 +189,7 @@ __device__ __forceinline__ void out_open(SlotOut &o, const BatchArgs &a, BatchLd
     o.wq.buf = L.base.wq[threadIdx.x / kWave];
     o.wq.pbuf = nullptr;
     o.wq.count = 0;
+    o.wq.through = false;
     o.wq.out = sl.q[(step + 1) & 1];
     o.wq.pout = nullptr;
     o.wq.out_len = &sl.qlen[(step + 1) % 3];
@@ -243,7 +244,7 @@ __device__ void batch_td_tile(const BatchArgs &a, BatchLds &L, int q, unsigned l
     const BatchGraph g = a.graphs[sl.graph];
     const int step = L.step[q];
     const unsigned n = (unsigned) L.n[q];
-    HubList hub{a.hubs[level & 1], a.hub_cap, &a.ctl->hub_alloc[level & 1], L.grid_t, q, L.chunk};
+    HubList hub{a.hubs[level & 1], a.hub_cap, &a.ctl->hub_alloc[level & 1], L.grid_t, q, L.chunk, nullptr};
     unsigned i = local * kBlock + threadIdx.x;
     int v = -1, beg = 0, end = 0;
     if (i < n) {
@@ -373,9 +374,9 @@ __device__ void batch_bu_tile(const BatchArgs &a, BatchLds &L, int q, unsigned l
     const unsigned last = min(nblocks, first + (unsigned) L.bu_tile);
     int *qv = L.base.hist + wave * 256;  // [128] vertices
     int *qb = qv + 128;                  // [128] row starts
-    int *qe0 = L.base.sc_excl[wave];     // row ends, entries 0..63
-    int *qe1 = L.base.sc_beg[wave];      // row ends, entries 64..127
-    unsigned *fb = reinterpret_cast<unsigned *>(L.base.sc_par[wave]);  // found bits of the window
+    int *qe0 = L.base.rt.excl[wave];     // row ends, entries 0..63
+    int *qe1 = L.base.rt.beg[wave];      // row ends, entries 64..127
+    unsigned *fb = reinterpret_cast<unsigned *>(L.base.rt.par[wave]);  // found bits of the window
 
     auto in_frontier = [&](int u) {
         if (use_bitmap) return ((cur[u >> 5] >> (u & 31)) & 1u) != 0;

@@ -84,6 +84,7 @@ struct bfs_problem {
     int *d_rrow = nullptr;       // reverse CSR (aliases d_row / d_col when symmetric)
     int *d_rcol = nullptr;
     bool symmetric = true;
+    int max_degree = 0;
     int *d_depth = nullptr;
     int *d_pred = nullptr;
     unsigned *d_visited = nullptr;
@@ -151,6 +152,7 @@ SearchArgs search_args(const bfs_problem *p, int grid)
     s.tile_status = p->cfg.compaction == 2 ? p->d_tile_status : nullptr;
     s.scan_epoch = p->scan_epoch;
     s.nodes = p->nodes;
+    s.max_degree = p->max_degree;
     s.total_edges = (unsigned long long) p->edges;
     return s;
 }
@@ -270,7 +272,8 @@ bfs_status enact_direction_iterative(bfs_problem *p, const GraphArgs &g, const S
         unsigned n = h.qlen[c.step % 3];
         if (h.overflow || n == 0) return BFS_OK;
         unsigned long long mf = h.fedges[c.step % 3];
-        unsigned long long mu = s.total_edges > h.visited_edges ? s.total_edges - h.visited_edges : 0ull;
+        const unsigned long long ve = h.visited_edges + mf;
+        unsigned long long mu = s.total_edges > ve ? s.total_edges - ve : 0ull;
         // the persistent loop's rule (bottom-up only while the frontier grows)
         int dir = c.phase;
         if (c.phase == kPhaseExpandContract) {
@@ -427,6 +430,8 @@ bfs_status bfs_problem_create(const int32_t *h_row_offsets, const int32_t *h_col
     p->nodes = nodes;
     p->edges = edges;
     p->mark_pred = mark_predecessors != 0;
+    for (int32_t v = 0; v < nodes; v++)
+        p->max_degree = std::max(p->max_degree, h_row_offsets[v + 1] - h_row_offsets[v]);
     auto cleanup = [&](bfs_status s) {
         bfs_problem_destroy(p);
         return s;
@@ -909,6 +914,7 @@ void apply_search_config(SearchArgs &s, const bfs_config &cfg, int grid)
               : (cfg.saturation_threshold < 0 ? -1 : grid * kBlock * 4);
     s.hybrid_steps = 0;
     s.instrument = cfg.instrument;
+    s.max_degree = 0x7fffffff;
     s.tile_status = nullptr;
     s.scan_epoch = 0;
     s.track_edges = 1;

@@ -18,7 +18,6 @@ namespace b40c_hip {
 constexpr int kWave = 64;
 constexpr int kHistory = 1024;                 // LDS history-hash entries per workgroup
 constexpr int kBarrierFanIn = 16;              // first-level barrier counters
-constexpr int kMaxXcdGrid = 1024;              // largest grid whose barriers may use XCD leaves
 constexpr int kHubChunk = 2048;                // edges per grid-tier chunk
 constexpr int kLevelLog = 64;                  // steps with recorded length/clock
 
@@ -51,7 +50,7 @@ struct alignas(256) Control {
     unsigned pad1[3];
     // Direction-optimizing bookkeeping (second 128-byte line).
     unsigned long long fedges[3];     // sum of degrees of each frontier, by step % 3
-    unsigned long long visited_edges; // sum of degrees of all vertices labelled so far
+    unsigned long long visited_edges; // launches per step: sum of fedges over the steps before the current one
     unsigned long long fast_vsum;     // fast-path hand-off of the per-workgroup visited-edge sum
     unsigned ovf[4];                  // per-step overflow of the output queue, by step % 3
     unsigned long long fast_prev_fe;  // fast-path hand-off: frontier edges of the level before the next step's
@@ -64,7 +63,6 @@ struct alignas(256) Control {
     unsigned bar_release[kBarrierFanIn * 32];  // one 128-byte line per leaf release word
     unsigned level_len[kLevelLog];             // input length of each step
     unsigned long long level_clock[kLevelLog]; // wall clock at the start of each step
-    unsigned xcd_of[kMaxXcdGrid];              // XCD of each workgroup of a persistent launch
 };
 
 // Bytes of the control block's status head (counters, flags, statistics):
@@ -78,7 +76,7 @@ static_assert(offsetof(Control, bar_root) == kControlHead, "status head ends whe
 struct HubEntry {
     int beg, end, par;
     unsigned first_chunk;
-    int tag;   // owner of the row (the query, in batched searches)
+    int tag;   // batched searches: the query; expansions: the row's place in the output queue
 };
 
 enum ExitReason { kExitDone = 0, kExitSaturated = 1, kExitOverflow = 2 };
@@ -268,15 +266,23 @@ struct PredStore<false> {
     int buf[1][1];
 };
 
+// Row table of gather_tile (and the scan tier's staging of gather_rows).
+struct RowTable {
+    int excl[kWaves][kWave];             // edge offset (scan tier: exclusive rank per lane)
+    int beg[kWaves][kWave];              // row begin (gather_tile: less the edge offset)
+    int par[kWaves][kWave];              // row owner
+    int scan[kWaves], scan2[kWaves];
+    int end;                             // end of the table's edges
+};
+
 template <bool PRED>
 struct Lds {
     int wq[kWaves][kWaveQueueCap];       // per-wave frontier staging
     PredStore<PRED> wqp;                 // per-wave predecessor staging
-    int sc_excl[kWaves][kWave];          // scan tier: exclusive rank per lane
-    int sc_beg[kWaves][kWave];           // scan tier: row begin per lane
-    int sc_par[kWaves][kWave];           // scan tier: row owner per lane
+    RowTable rt;
     int hist[kHistory];                  // history hash (contract / filter)
     int cta_owner, cta_beg, cta_end, cta_par;
+    unsigned cta_out;                    // expansions: the chunk's place in the output queue
     unsigned tile;
     unsigned nb;                         // broadcast frontier length
     int step, iteration;
@@ -309,6 +315,18 @@ struct WaveQueue {
     unsigned cap;
     unsigned *overflow;
     unsigned *overflow_step;   // per-step flag the level loop decides on (may alias overflow)
+    bool through;              // a light barrier follows: entries go past the L2 (agent-scope stores)
+
+    __device__ __forceinline__ void store(unsigned at, int u, int p)
+    {
+        if (through) {
+            st_agent(out + at, u);
+            if (PRED) st_agent(pout + at, p);
+        } else {
+            out[at] = u;
+            if (PRED) pout[at] = p;
+        }
+    }
 
     __device__ __forceinline__ void flush()
     {
@@ -325,10 +343,7 @@ struct WaveQueue {
             st_agent(overflow, 1u);
             st_agent(overflow_step, 1u);
         }
-        for (unsigned i = lane; i < lim; i += kWave) {
-            out[base + i] = buf[i];
-            if (PRED) pout[base + i] = pbuf[i];
-        }
+        for (unsigned i = lane; i < lim; i += kWave) store(base + i, buf[i], PRED ? pbuf[i] : -1);
         count = 0;
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -370,6 +385,7 @@ struct HubList {
     int grid_t;        // rows at least this long go to the grid tier
     int tag;           // stored with every published row
     int chunk;         // edges per chunk
+    unsigned *out_len; // expansions: length of the output queue (null: none reserved)
 };
 
 // Index of the last grid-tier entry whose first chunk is <= ch (entries are
@@ -401,6 +417,9 @@ __device__ __forceinline__ unsigned hub_entry_of(const HubEntry *list, unsigned 
 // wave-converged; true when this lane's row was published).  The wave
 // reserves list entries and chunk numbers for all its long rows with one
 // atomic; entries keep lane order, so the list stays sorted by first chunk.
+// With hub.out_len set, the wave also reserves that many elements of the
+// output queue for its published rows (one more atomic), and an entry's tag
+// is its row's place there: the grid tier then writes without reserving.
 __device__ __forceinline__ bool publish_hub_row(int beg, int end, int par, const HubList &hub)
 {
     const int lane = lane_id();
@@ -421,11 +440,24 @@ __device__ __forceinline__ bool publish_hub_row(int beg, int end, int par, const
     lo = (unsigned) uniform((int) lo);
     hi = (unsigned) uniform((int) hi);
     const unsigned slot = hi + (unsigned) lanes_below(pm);
-    if (pub && slot < hub.cap) {
-        hub.entries[slot] = HubEntry{beg, end, par, lo + (unsigned) (incl - nch), hub.tag};
-        return true;
+    const bool done = pub && slot < hub.cap;
+    int tag = hub.tag;
+    if (hub.out_len) {
+        const int lens = wave_inclusive_sum(done ? len : 0);
+        unsigned at = 0;
+        if (lane == kWave - 1) at = add_agent(hub.out_len, (unsigned) lens);
+        tag = (int) ((unsigned) readlane((int) at, kWave - 1) + (unsigned) (lens - len));
     }
-    return false;
+    if (done) {
+        // (past the L2: a light barrier may follow)
+        HubEntry *h = hub.entries + slot;
+        st_agent(&h->beg, beg);
+        st_agent(&h->end, end);
+        st_agent(&h->par, par);
+        st_agent(&h->first_chunk, lo + (unsigned) (incl - nch));
+        st_agent(&h->tag, tag);
+    }
+    return done;
 }
 
 template <bool PRED, typename Fn>
@@ -486,9 +518,9 @@ __device__ __forceinline__ void gather_rows(int beg, int end, int par, const int
     int incl = wave_inclusive_sum(len);
     int total = readlane(incl, kWave - 1);
     if (total == 0) return;
-    int *excl = lds.sc_excl[wave];
-    int *rb = lds.sc_beg[wave];
-    int *rp = lds.sc_par[wave];
+    int *excl = lds.rt.excl[wave];
+    int *rb = lds.rt.beg[wave];
+    int *rp = lds.rt.par[wave];
     excl[lane] = incl - len;
     rb[lane] = beg;
     rp[lane] = par;
@@ -513,6 +545,121 @@ __device__ __forceinline__ void gather_rows(int beg, int end, int par, const int
 }
 
 // ---------------------------------------------------------------------------
+// Workgroup gather of a tile of rows.  Each thread brings up to K rows
+// [beg, end) with owner par (end == beg for none).  Long rows go to the grid
+// tier; the others are compacted into an LDS table of kBlock rows (row start,
+// edge offset, owner) and their edges spread evenly over the workgroup: each
+// round covers kBlock * 4 consecutive edges, edge j * kBlock + t of a round
+// going to thread t, so a load instruction of a wave reads consecutive
+// entries of a row.  A thread finds its edges' rows by searching the offsets,
+// and hands the four column positions (-1: none) and owners to `edges`, which
+// issues every memory trip of a round for all four before using the first
+// result.  Called by every thread; `edges` is called workgroup-converged, and
+// `begin` once before, with the tile's edge count.  Edge j of a call is edge
+// x0 + j * kBlock of the tile.
+//
+// A level is bound by its chain of dependent memory trips, not by bytes: one
+// row per thread gathered 64 edges a wave at a time (gather_rows) made the
+// 4318-vertex level of a 100 k-vertex random graph a chain of 16 such rounds
+// on nine workgroups, 76 us; spread over the grid it is one round.
+// ---------------------------------------------------------------------------
+// A tile of more than kHeavyTile edges sends its rows from kHeavyRow edges
+// on to the grid tier as well.  The first workgroups to claim anything in a
+// level claim its high-degree vertices (an edge leads to a vertex in
+// proportion to its degree), and with 2048 items a tile they kept the
+// 24.9 M-edge contract-expand step of an R-MAT scale 20 search busy for
+// 1200 us while the rest waited.
+constexpr int kHeavyTile = 1 << 15, kHeavyRow = 512;
+
+template <int K, typename Begin, typename Edges>
+__device__ __forceinline__ void gather_tile(const int (&beg)[K], int (&end)[K], const int (&par)[K],
+                                            const HubList &hub, RowTable &rt, Begin &&begin, Edges &&edges)
+{
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    int *tbeg = &rt.beg[0][0], *toff = &rt.excl[0][0], *tpar = &rt.par[0][0];
+    int rpos, epos, rtotal, etotal;
+    HubList h = hub;
+    while (true) {
+        int rows = 0, degs = 0;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            if (publish_hub_row(beg[k], end[k], par[k], h)) end[k] = beg[k];
+            rows += end[k] > beg[k] ? 1 : 0;
+            degs += end[k] - beg[k];
+        }
+        // exclusive sums of rows and edges over the workgroup, in one pass
+        const int rincl = wave_inclusive_sum(rows), dincl = wave_inclusive_sum(degs);
+        if (lane == kWave - 1) {
+            rt.scan[wave] = rincl;
+            rt.scan2[wave] = dincl;
+        }
+        __syncthreads();
+        rpos = rincl - rows;
+        epos = dincl - degs;
+        rtotal = etotal = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) {
+            const int a = rt.scan[w], b = rt.scan2[w];
+            if (w < wave) {
+                rpos += a;
+                epos += b;
+            }
+            rtotal += a;
+            etotal += b;
+        }
+        if (etotal <= kHeavyTile || h.grid_t <= kHeavyRow || h.grid_t == 0x7fffffff) break;
+        h.grid_t = kHeavyRow;
+        __syncthreads();  // the sums are written again
+    }
+    begin(etotal);
+    for (int r0 = 0; r0 < rtotal; r0 += kBlock) {
+        int p = rpos - r0, e = epos;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            if (end[k] > beg[k]) {
+                if (p >= 0 && p < kBlock) {
+                    tbeg[p] = beg[k] - e;  // column position of edge x of the tile: tbeg + x
+                    toff[p] = e;
+                    tpar[p] = par[k];
+                } else if (p == kBlock) {
+                    rt.end = e;
+                }
+                p++;
+                e += end[k] - beg[k];
+            }
+        }
+        const int nr = min(rtotal - r0, kBlock);
+        if (rtotal - r0 <= kBlock && tid == 0) rt.end = etotal;
+        __syncthreads();
+        const int e_begin = toff[0], e_end = rt.end;
+        int top = 1;  // first step of the search: the largest power of two below nr (uniform)
+        while (2 * top < nr) top *= 2;
+        // (unsigned: the last round of a tile may reach past 2^31)
+        for (unsigned b0 = (unsigned) e_begin; b0 < (unsigned) e_end; b0 += 4 * kBlock) {
+            int at[4], pv[4], r[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) r[j] = 0;
+            for (int st = top; st > 0; st >>= 1) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int q = r[j] + st;
+                    if (q < nr && (unsigned) toff[q] <= b0 + (unsigned) (j * kBlock + tid)) r[j] = q;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const unsigned x = b0 + (unsigned) (j * kBlock + tid);
+                at[j] = x < (unsigned) e_end ? tbeg[r[j]] + (int) x : -1;
+                pv[j] = tpar[r[j]];
+            }
+            edges(at, pv, b0 + (unsigned) tid);
+        }
+        __syncthreads();  // the table and the sums are written again next
+    }
+    if (rtotal == 0) __syncthreads();
+}
+
+// ---------------------------------------------------------------------------
 // Grid barrier for cooperatively launched (co-resident) grids.
 // Two-level arrival: workgroup b arrives on leaf counter b % kBarrierFanIn;
 // the last arrival at a leaf arrives at the root; the last root arrival
@@ -520,57 +667,54 @@ __device__ __forceinline__ void gather_rows(int beg, int end, int par, const int
 // release word, so waiting workgroups poll kBarrierFanIn different lines
 // instead of one.
 //
-// Memory ordering costs one agent-scope release fence (L2 write-back) and one
-// acquire fence (L1/L2 invalidate) per workgroup, issued by thread 0 around
-// the workgroup barriers.  Polling uses relaxed loads: an acquire load inside
+// Memory ordering of a full barrier costs one agent-scope release fence (L2
+// write-back) and one acquire fence (L1/L2 invalidate) per workgroup, issued
+// by thread 0 around the workgroup barriers.  Polling uses relaxed loads: an acquire load inside
 // the spin would invalidate the caches on every poll and slow every other
 // workgroup still working.  The last arrivers chain acquire/release fences so
 // every workgroup's pre-barrier writes happen-before every post-barrier read.
 // Replaces util::GlobalBarrier (b40c/util/global_barrier.cuh:80-126).
 // ---------------------------------------------------------------------------
-// Which leaf a workgroup arrives on, how many workgroups share it, and how
-// many leaves there are.  By block (b % kBarrierFanIn), every workgroup
-// writes back its XCD's L2 before arriving.  With XCD leaves (shared), the
-// leaf is the workgroup's XCD and only the leaf's last arriver writes back
-// that XCD's L2 -- once for all of them: the L1 is write-through, so a
-// workgroup's stores are in its XCD's L2 once they have completed, which
-// every workgroup waits for before it arrives.
-struct BarrierShape {
-    unsigned leaf, leaf_size, leaves, shared;
-};
-static_assert(kBarrierFanIn >= 8, "an XCD leaf indexes the leaf words");
+// Every wave drains its own outstanding memory operations first:
+// __syncthreads() alone does not wait for other waves' stores, and the
+// single write-back of thread 0's release fence must find all of this
+// workgroup's stores already in L2, or a store still in flight stays dirty
+// in this XCD's L2 and readers elsewhere see old memory.
+__device__ __forceinline__ void drain() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
 
-__device__ __forceinline__ BarrierShape barrier_shape_by_block()
+// Release and acquire of the whole caches, by thread 0 for its workgroup
+// (every thread of the workgroup calls them).
+__device__ __forceinline__ void release_caches()
+{
+    drain();
+    __syncthreads();
+    if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+}
+__device__ __forceinline__ void refresh_caches()
+{
+    if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    __syncthreads();
+}
+
+// MAINTAIN: plain stores before the barrier are visible to plain loads after
+// it, at the price of a write-back and an invalidate of the XCD's L2 per
+// workgroup.  Without it (light barriers) the barrier orders only what goes
+// past the XCDs' L2s by itself -- agent- and system-scope loads, stores and
+// atomics: a workgroup's have completed before it arrives.  At 256 workgroups
+// the maintenance is two thirds of the barrier (6.4 us with, 2.3 without).
+// The counter protocol is the same; each of its stores is waited for before
+// the store or atomic that may release someone who depends on it.
+template <bool MAINTAIN>
+__device__ __forceinline__ void grid_barrier_t(Control *ctl)
 {
     const unsigned nblocks = gridDim.x;
-    BarrierShape b;
-    b.leaf = blockIdx.x % kBarrierFanIn;
-    b.leaves = nblocks < (unsigned) kBarrierFanIn ? nblocks : (unsigned) kBarrierFanIn;
+    const unsigned leaf = blockIdx.x % kBarrierFanIn;
+    const unsigned leaves = nblocks < (unsigned) kBarrierFanIn ? nblocks : (unsigned) kBarrierFanIn;
     // workgroups on this leaf: ceil((nblocks - leaf) / fan_in)
-    b.leaf_size = (nblocks - b.leaf + kBarrierFanIn - 1) / kBarrierFanIn;
-    b.shared = 0u;
-    return b;
-}
-
-// The XCD (accelerator complex die) the calling wave runs on.
-__device__ __forceinline__ unsigned xcc_id()
-{
-    unsigned x;
-    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(x));
-    return x & 7u;
-}
-
-__device__ __forceinline__ void grid_barrier(Control *ctl, const BarrierShape &shape)
-{
-    // Every wave drains its own outstanding memory operations first:
-    // __syncthreads() alone does not wait for other waves' stores, and the
-    // single write-back below (thread 0's release fence) must find all of
-    // this workgroup's stores already in L2, or a store still in flight
-    // stays dirty in this XCD's L2 and readers elsewhere see old memory.
-    __builtin_amdgcn_s_waitcnt(0);
+    const unsigned leaf_size = (nblocks - leaf + kBarrierFanIn - 1) / kBarrierFanIn;
+    drain();
     __syncthreads();
     if (threadIdx.x == 0) {
-        const unsigned leaf = shape.leaf, leaves = shape.leaves, leaf_size = shape.leaf_size;
         unsigned *release = &ctl->bar_release[leaf * 32];
         // The generation comes from the one global word, which only the last
         // arriver of a barrier advances (after every workgroup has read it
@@ -578,31 +722,32 @@ __device__ __forceinline__ void grid_barrier(Control *ctl, const BarrierShape &s
         // Leaf words of leaves a smaller earlier grid never used may lag:
         // they are compared with gen + 1, never with each other.
         const unsigned gen = __hip_atomic_load(&ctl->bar_gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // (with XCD leaves the leaf's last arriver writes the L2 back; the
-        // generation must still be read before this arrival)
-        if (shape.shared) __builtin_amdgcn_s_waitcnt(0);
-        else __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        // (the generation must be read before this arrival)
+        if (MAINTAIN) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        drain();
         unsigned *lc = &ctl->bar_leaf[leaf * 32];
         unsigned arrived = __hip_atomic_fetch_add(lc, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         bool last = false;
         if (arrived == leaf_size - 1) {
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
+            if (MAINTAIN) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
             __hip_atomic_store(lc, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             // Relaxed stores to different lines may land in any order, and a
             // relaxed RMW does not wait for them: the reset must be visible
             // before the root arrival that can release this leaf's
             // workgroups, or their next arrival could be overwritten by it.
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            if (MAINTAIN) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            drain();
             unsigned r = __hip_atomic_fetch_add(&ctl->bar_root, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (r == leaves - 1) {
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
+                if (MAINTAIN) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
                 __hip_atomic_store(&ctl->bar_root, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(&ctl->bar_gen, gen + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 // the new generation and the root reset before any release
                 // word: a released workgroup reads bar_gen at its next
                 // barrier, and an old value there would let it straight
                 // through
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+                if (MAINTAIN) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+                drain();
                 for (unsigned l = 0; l < leaves; l++)
                     __hip_atomic_store(&ctl->bar_release[l * 32], gen + 1, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
@@ -611,73 +756,30 @@ __device__ __forceinline__ void grid_barrier(Control *ctl, const BarrierShape &s
         }
         if (!last) {
             while (__hip_atomic_load(release, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gen + 1)
-                __builtin_amdgcn_s_sleep(2);
+                __builtin_amdgcn_s_sleep(MAINTAIN ? 2 : 1);
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if (MAINTAIN) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
 }
 
-__device__ __forceinline__ void grid_barrier(Control *ctl) { grid_barrier(ctl, barrier_shape_by_block()); }
+__device__ __forceinline__ void grid_barrier(Control *ctl) { grid_barrier_t<true>(ctl); }
+__device__ __forceinline__ void grid_barrier_light(Control *ctl) { grid_barrier_t<false>(ctl); }
 
-// Thread 0 of block 0 only (shape: block 0's): waits until every other
-// workgroup has arrived at the grid barrier in progress (block 0 itself has
-// not), i.e. until every other workgroup is done with whatever it did
-// before that barrier.  Block 0's leaf then holds all its workgroups but
-// block 0 and the root all leaves but that one; neither count can move on
-// before block 0 arrives, so the wait ends exactly once they are reached.
-__device__ __forceinline__ void wait_other_arrivals(Control *ctl, const BarrierShape &shape)
+// Thread 0 of block 0 only: waits until every other workgroup has arrived at
+// the grid barrier in progress (block 0 itself has not), i.e. until every
+// other workgroup is done with whatever it did before that barrier.  Block
+// 0's leaf then holds all its workgroups but block 0 and the root all leaves
+// but that one; neither count can move on before block 0 arrives, so the wait
+// ends exactly once they are reached.
+__device__ __forceinline__ void wait_other_arrivals(Control *ctl)
 {
-    while (__hip_atomic_load(&ctl->bar_root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != shape.leaves - 1 ||
-           __hip_atomic_load(&ctl->bar_leaf[shape.leaf * 32], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) !=
-               shape.leaf_size - 1)
+    const unsigned nblocks = gridDim.x;
+    const unsigned leaves = nblocks < (unsigned) kBarrierFanIn ? nblocks : (unsigned) kBarrierFanIn;
+    const unsigned leaf_size = (nblocks + kBarrierFanIn - 1) / kBarrierFanIn;  // of leaf 0
+    while (__hip_atomic_load(&ctl->bar_root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != leaves - 1 ||
+           __hip_atomic_load(&ctl->bar_leaf[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != leaf_size - 1)
         __builtin_amdgcn_s_sleep(2);
-}
-
-// Thread 0 of every workgroup of a persistent launch (gridDim.x <=
-// kMaxXcdGrid), before its first barrier: records the workgroup's XCD.
-__device__ __forceinline__ void xcd_register(Control *ctl) { ctl->xcd_of[blockIdx.x] = xcc_id(); }
-
-// Thread 0, after the launch's first barrier (every workgroup recorded its
-// XCD before arriving at it): XCD leaves when all eight XCDs hold
-// workgroups of this launch, else leaves by block.  The counts are kept
-// in 16-bit fields, four XCDs to a word.
-__device__ __forceinline__ BarrierShape xcd_shape(Control *ctl)
-{
-    const unsigned x = xcc_id();
-    unsigned long long lo = 0, hi = 0;
-    const uint4 *rec = reinterpret_cast<const uint4 *>(ctl->xcd_of);
-    const unsigned words = gridDim.x / 4, tail = gridDim.x % 4;
-    for (unsigned i = 0; i < words; i++) {
-        const uint4 q = rec[i];
-        const unsigned v[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const unsigned y = v[k] & 7u;
-            if (y < 4) lo += 1ull << (16 * y);
-            else hi += 1ull << (16 * (y - 4));
-        }
-    }
-    for (unsigned i = 4 * words; i < 4 * words + tail; i++) {
-        const unsigned y = ctl->xcd_of[i] & 7u;
-        if (y < 4) lo += 1ull << (16 * y);
-        else hi += 1ull << (16 * (y - 4));
-    }
-    bool all = true;
-    unsigned mine = 0;
-#pragma unroll
-    for (unsigned k = 0; k < 8; k++) {
-        const unsigned c = (unsigned) (((k < 4 ? lo : hi) >> (16 * (k & 3))) & 0xFFFFull);
-        all = all && c > 0;
-        if (k == x) mine = c;
-    }
-    if (!all) return barrier_shape_by_block();
-    BarrierShape b;
-    b.leaf = x;
-    b.leaf_size = mine;
-    b.leaves = 8u;
-    b.shared = 1u;
-    return b;
 }
 
 }  // inline namespace (workgroup size)

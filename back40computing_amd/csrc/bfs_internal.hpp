@@ -53,6 +53,7 @@ struct SearchArgs {
     int instrument;
     int grab_max;          // most tiles taken per tile-counter atomic
     int coherent_filter;   // claim pre-test reads the device-coherent visited word
+    int max_degree;        // largest row (in-neighbour rows not counted)
     int spread;            // few-member top-down levels split their edges evenly over the grid
     int fast_visited;      // the fast path claims in an LDS copy of the visited bitmap (when it fits)
     // Chained compaction of contract and filter steps: one status word per

@@ -49,17 +49,30 @@ __device__ __forceinline__ unsigned next_item(unsigned *counter, Lds<PRED> &lds,
     return lds.tile;
 }
 
-// Guided grabs of kBlock-item tiles: one counter atomic hands a workgroup
-// `grab` consecutive tiles, about eight grabs per workgroup when a phase has
-// many tiles, so the single counter address (whose device-scope atomics
+// Guided grabs of tiles: one counter atomic hands a workgroup `grab`
+// consecutive tiles, about eight grabs per workgroup when a phase has many
+// tiles, so the single counter address (whose device-scope atomics
 // serialise) stays off the critical path of large levels.
-// A phase of at most one tile per workgroup that every workgroup runs needs
-// no counter: workgroup b takes tile b (grab 0), and the two round trips of
-// the counter atomics (the grab, and the one that finds nothing left) leave
-// the level's critical path.  A workgroup running a step alone (lds.solo)
-// grabs every tile itself.
+// A phase whose items fit one tile per workgroup and that every workgroup
+// runs needs no counter: workgroup b takes tile b (grab 0), and the two round
+// trips of the counter atomics (the grab, and the one that finds nothing
+// left) leave the level's critical path.  Its tiles are as narrow as spreads
+// the items over `want` workgroups.  A workgroup running a step alone
+// (lds.solo) grabs every tile itself.
 struct TileGrab {
     unsigned next, end, grab, tiles;
+    unsigned width;  // items per tile
+
+    // Item i of tile t when tiles are dealt the queue in runs of 16 entries
+    // (64 bytes): run k of the tile is the queue's run k * tiles + t.  The
+    // members a step claims first, where its output begins, are the
+    // high-degree ones; tiles of consecutive members left the first few
+    // with most of the edges (R-MAT scale 20, 437602 members, 24.9 M edges:
+    // waves lived a quarter of the expansion's 461 us on average).
+    __device__ __forceinline__ unsigned dealt(unsigned t, unsigned i) const
+    {
+        return (((i >> 4) * tiles + t) << 4) + (i & 15u);
+    }
 };
 
 // tiles per counter atomic of a dynamic assignment
@@ -68,13 +81,19 @@ __device__ __forceinline__ unsigned tile_grab_size(const SearchArgs &s, unsigned
     return max(1u, min((unsigned) s.grab_max, tiles / (gridDim.x * 8u)));
 }
 
+// Tiles of at most max_width items over n > 0 items.
 template <bool PRED>
-__device__ __forceinline__ TileGrab tile_grab(const SearchArgs &s, unsigned items, const Lds<PRED> &lds)
+__device__ __forceinline__ TileGrab tile_grab(const SearchArgs &s, unsigned n, const Lds<PRED> &lds,
+                                              unsigned max_width, unsigned want)
 {
-    unsigned tiles = (items + kBlock - 1) / kBlock;
-    if (tiles <= gridDim.x && !lds.solo)
-        return TileGrab{blockIdx.x, blockIdx.x < tiles ? blockIdx.x + 1 : blockIdx.x, 0u, tiles};
-    return TileGrab{0u, 0u, tile_grab_size(s, tiles), tiles};
+    if (!lds.solo && n <= gridDim.x * max_width) {
+        const unsigned wgs = max(min(want, gridDim.x), (n + max_width - 1) / max_width);
+        const unsigned width = min(((n + wgs - 1) / wgs + 15u) & ~15u, max_width);
+        const unsigned tiles = (n + width - 1) / width;
+        return TileGrab{blockIdx.x, blockIdx.x < tiles ? blockIdx.x + 1 : blockIdx.x, 0u, tiles, width};
+    }
+    const unsigned tiles = (n + max_width - 1) / max_width;
+    return TileGrab{0u, 0u, tile_grab_size(s, tiles), tiles, max_width};
 }
 
 // Next tile index of the workgroup (workgroup-uniform); with a static
@@ -110,8 +129,21 @@ __device__ __forceinline__ bool history_pass(Lds<PRED> &lds, int u)
     return true;
 }
 
+// How a grid-wide step meets the caches around it (grid-uniform):
+// light: a light barrier follows, so what other workgroups read next goes
+//   past the XCD's L2 (queue entries); the step is small, and reads the rows
+//   of its candidates before their claims have answered;
+// stale: a light barrier came before, so this XCD's L2 may hold visited words
+//   from before other workgroups' claims: pre-reads go past it.  (A word that
+//   is too old only costs a claim that fails, but on a lattice every second
+//   edge leads back to a vertex visited a level or two before.)
+struct StepIo {
+    bool light, stale;
+};
+
 template <bool PRED>
-__device__ __forceinline__ WaveQueue<PRED> make_queue(const SearchArgs &s, int step, Lds<PRED> &lds)
+__device__ __forceinline__ WaveQueue<PRED> make_queue(const SearchArgs &s, int step, Lds<PRED> &lds,
+                                                      bool through = false)
 {
     const int wave = threadIdx.x / kWave;
     WaveQueue<PRED> wq;
@@ -119,6 +151,7 @@ __device__ __forceinline__ WaveQueue<PRED> make_queue(const SearchArgs &s, int s
     if constexpr (PRED) wq.pbuf = lds.wqp.buf[wave];
     else wq.pbuf = nullptr;
     wq.count = 0;
+    wq.through = through;
     wq.out = s.q[(step + 1) & 1];
     wq.pout = PRED ? s.pq[(step + 1) & 1] : nullptr;
     wq.out_len = &s.ctl->qlen[(step + 1) % 3];
@@ -128,49 +161,42 @@ __device__ __forceinline__ WaveQueue<PRED> make_queue(const SearchArgs &s, int s
     return wq;
 }
 
-// Steps with fewer tiles than the grid has workgroups (a level of a handful
-// of hub vertices): most workgroups would idle while a few stride long rows
-// alone, so every row the workgroup tier would take goes to the grid tier
-// instead, in kBlock-edge chunks.  Grid-uniform (n is read after a barrier).
-__device__ __forceinline__ bool narrow_step(unsigned n) { return (n + kBlock - 1) / kBlock < gridDim.x; }
-
-// Grid-tier chunk of a step over n items.  Marked steps (see
-// body_expand_mark) keep kHubChunk chunks even when narrow: their chunks
-// are gathered four workgroup-widths at a time.
-__device__ __forceinline__ int hub_chunk(unsigned n, bool marked = false)
-{
-    return narrow_step(n) && !marked ? kBlock : kHubChunk;
-}
+// Steps of at most one kBlock-item tile per workgroup: rows of a grid-tier
+// chunk and more go to the grid tier, so that no workgroup of such a short
+// step strides a long row alone.  Grid-uniform (n is read after a barrier).
+__device__ __forceinline__ bool narrow_step(unsigned n) { return (n + kBlock - 1) / kBlock <= gridDim.x; }
 
 // Grid-tier list of a gathering step over n input items.
-__device__ __forceinline__ HubList hub_list(const SearchArgs &s, int step, bool enabled, unsigned n,
-                                            bool marked = false)
+__device__ __forceinline__ HubList hub_list(const SearchArgs &s, int step, bool enabled, unsigned n)
 {
     HubList h;
     h.entries = s.hubs[step & 1];
     h.cap = s.hub_cap;
     h.alloc = &s.ctl->hub_alloc[step & 1];
     h.grid_t = enabled ? s.grid_t : 0x7fffffff;
-    // a step of fewer tiles than workgroups leaves most workgroups idle:
-    // every row long enough for the wave tier goes to the grid instead
-    if (enabled && narrow_step(n)) h.grid_t = min(h.grid_t, max(s.wave_t, kWave));
+    if (enabled && narrow_step(n)) h.grid_t = min(h.grid_t, kHubChunk);
     h.tag = 0;
-    h.chunk = hub_chunk(n, marked);
+    h.chunk = kHubChunk;
+    h.out_len = nullptr;
     return h;
 }
 
 // End of a step for the whole workgroup (every thread calls it): the waves'
 // staged queue entries are reserved with one atomic, and their degree sums
-// and depth note are folded into one update each.  Per-wave updates would
-// put four times as many device-scope atomics on the same few addresses,
-// where they serialise across the grid.
+// are folded into one update.  256 workgroups' atomics on one address cost a
+// level about 2 us (8 ns each) on top of its barrier and plain stores to one
+// address 6 us, so a step keeps to these two: the deepest label is noted by
+// one workgroup at the top of the next step (prepare_step), and the visited
+// edges are summed by whoever decides on them.
 //
 // `uncounted` (per lane) adds frontier members that are not staged in the
 // queue: a bottom-up level records its output only in the frontier bitmap,
 // and the queue length alone carries its size.
+// `labeled` (per lane; contract-expand): labelled vertices with depth
+// `depth`, to be noted here if the workgroup stages no output at all.
 template <bool PRED>
-__device__ void finish_step(WaveQueue<PRED> &wq, Lds<PRED> &lds, Control *ctl, int step, bool labeled, int depth,
-                            unsigned fe, bool track, int uncounted = 0)
+__device__ void finish_step(WaveQueue<PRED> &wq, Lds<PRED> &lds, Control *ctl, int step, unsigned fe, bool track,
+                            int uncounted = 0, bool labeled = false, int depth = -1)
 {
     const int lane = lane_id(), wave = threadIdx.x / kWave;
     int lo = wave_inclusive_sum((int) (fe & 0xFFFFu));
@@ -195,11 +221,9 @@ __device__ void finish_step(WaveQueue<PRED> &wq, Lds<PRED> &lds, Control *ctl, i
             lab |= lds.ep_lab[w];
         }
         lds.ep_base = (tot | ext) ? add_agent(wq.out_len, tot + ext) : 0u;
-        if (track && fsum) {
+        if (track && fsum)
             __hip_atomic_fetch_add(&ctl->fedges[(step + 1) % 3], fsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_add(&ctl->visited_edges, fsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (lab) atomicMax(&ctl->max_depth, depth);
+        if (lab && tot == 0) atomicMax(&ctl->max_depth, depth);
     }
     __syncthreads();
     unsigned off = lds.ep_base;
@@ -210,10 +234,7 @@ __device__ void finish_step(WaveQueue<PRED> &wq, Lds<PRED> &lds, Control *ctl, i
         st_agent(wq.overflow, 1u);
         st_agent(wq.overflow_step, 1u);
     }
-    for (unsigned i = (unsigned) lane; i < lim; i += kWave) {
-        wq.out[off + i] = wq.buf[i];
-        if (PRED) wq.pout[off + i] = wq.pbuf[i];
-    }
+    for (unsigned i = (unsigned) lane; i < lim; i += kWave) wq.store(off + i, wq.buf[i], PRED ? wq.pbuf[i] : -1);
     wq.count = 0;
 }
 
@@ -226,30 +247,12 @@ __device__ __forceinline__ unsigned long long ld64_agent(const unsigned long lon
 // Generic phases
 // ---------------------------------------------------------------------------
 
-// Tile phase of a gathering step.  row_of(i, beg, end, par) turns input
-// element i (< n) into the adjacency row to gather (end == beg for none);
-// edge(ok, u, par) consumes each neighbour, wave-converged.
-template <bool PRED, typename RowOf, typename Edge>
-__device__ __forceinline__ void tile_phase(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n,
-                                           const HubList &hub, Lds<PRED> &lds, RowOf &&row_of, Edge &&edge)
-{
-    TileGrab tg = tile_grab(s, n, lds);
-    while (true) {
-        unsigned base = next_tile(&s.ctl->steal[c.step & 1], lds, tg) * kBlock;
-        if (base >= n) break;
-        unsigned i = base + threadIdx.x;
-        int beg = 0, end = 0, par = -1;
-        if (i < n) row_of(i, beg, end, par);
-        gather_rows<PRED>(beg, end, par, g.col, s.wave_t, s.cta_t, hub, lds, edge);
-    }
-}
-
-// Hub phase: every workgroup takes hub_chunk(n)-edge chunks of the rows that
+// Hub phase: every workgroup takes kHubChunk-edge chunks of the rows that
 // the tile phase published, until all chunks are done.  Must follow a grid
-// barrier (or kernel boundary) after the tile phase.
+// barrier (or kernel boundary) after the tile phase.  run_chunk(b, e, par)
+// consumes columns [b, e) of a row of par.
 template <bool PRED, typename Chunk>
-__device__ __forceinline__ void hub_phase_chunks(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n,
-                                                 Lds<PRED> &lds, bool marked, Chunk &&run_chunk)
+__device__ __forceinline__ void hub_phase_chunks(const SearchArgs &s, Cursor c, Lds<PRED> &lds, Chunk &&run_chunk)
 {
     unsigned long long a = __hip_atomic_load(&s.ctl->hub_alloc[c.step & 1], __ATOMIC_RELAXED,
                                              __HIP_MEMORY_SCOPE_AGENT);
@@ -258,11 +261,11 @@ __device__ __forceinline__ void hub_phase_chunks(const GraphArgs &g, const Searc
     if (entries == 0) return;
     const HubEntry *list = s.hubs[c.step & 1];
     HubEntry lastent = list[entries - 1];
-    const int chunk = hub_chunk(n, marked);
+    constexpr int chunk = kHubChunk;
     unsigned total = lastent.first_chunk + (unsigned) ((lastent.end - lastent.beg + chunk - 1) / chunk);
     // guided grabs of consecutive chunks, as for tiles: a level of many hub
     // chunks must not queue on the one chunk counter
-    TileGrab tg{0u, 0u, max(1u, min((unsigned) s.grab_max, total / (gridDim.x * 8u))), 0u};
+    TileGrab tg{0u, 0u, max(1u, min((unsigned) s.grab_max, total / (gridDim.x * 8u))), 0u, 1u};
     unsigned hint = 0;  // thread 0: entry of this workgroup's previous chunk
     while (true) {
         unsigned ch = next_tile(&s.ctl->hub_steal[c.step & 1], lds, tg);
@@ -275,6 +278,7 @@ __device__ __forceinline__ void hub_phase_chunks(const GraphArgs &g, const Searc
             lds.cta_beg = b;
             lds.cta_end = min(e.end, b + chunk);
             lds.cta_par = e.par;
+            lds.cta_out = (unsigned) e.tag + (unsigned) (b - e.beg);
         }
         __syncthreads();
         run_chunk(lds.cta_beg, lds.cta_end, lds.cta_par);
@@ -282,18 +286,163 @@ __device__ __forceinline__ void hub_phase_chunks(const GraphArgs &g, const Searc
 }
 
 
-template <bool PRED, typename Edge>
-__device__ __forceinline__ void hub_phase(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds,
-                                          Edge &&edge)
+// The same with gather_tile's edge consumer (four column positions per
+// thread and round).
+template <bool PRED, typename Edges>
+__device__ __forceinline__ void hub_phase(const SearchArgs &s, Cursor c, Lds<PRED> &lds, Edges &&edges)
 {
-    hub_phase_chunks<PRED>(g, s, c, n, lds, false, [&](int b, int e, int pv) {
-        for (int k = b; k < e; k += kBlock) {
-            int idx = k + threadIdx.x;
-            bool ok = idx < e;
-            int u = ok ? __builtin_nontemporal_load(g.col + idx) : -1;
-            edge(ok, u, pv);
+    hub_phase_chunks<PRED>(s, c, lds, [&](int b, int e, int par) {
+        for (int k = b; k < e; k += 4 * kBlock) {
+            int at[4], pv[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int x = k + j * kBlock + (int) threadIdx.x;
+                at[j] = x < e ? x : -1;
+                pv[j] = par;
+            }
+            edges(at, pv, 0u);
         }
     });
+}
+
+// Claims of one thread's edge slots: at[k] = column position of slot k (or
+// -1), pv[k] = its row's owner.  Claims the unvisited neighbours, labels
+// them, and returns the mask of the slots k that claimed u[k] (row
+// [ub[k], ud[k])).  Each memory trip (column entry, visited word, claim,
+// row bounds) is issued for every slot before the first result is used.
+//
+// LOCAL: the calling workgroup is the only one touching the labels and the
+// visited words (block 0's fast path, between two grid barriers).  Its
+// claims are then workgroup-scope atomics, done in this XCD's L2, where
+// agent-scope ones must be coherent across the eight XCDs; the barrier
+// before the path invalidated stale lines, and the one after it writes the
+// path's lines back.  Column entries are read through the caches: the next
+// level's rows sit next to this level's on a lattice.  With vbits (LOCAL
+// only) the claims are LDS atomics on the path's copy of the visited
+// bitmap: no pre-read and no memory trip between a column entry and the
+// claimed vertex's row bounds.
+// Without ROWS the row bounds are not read (the caller does not gather).
+// With best-effort culling the claims are atomic here too: with four edges
+// per thread in flight, racing plain stores (claim_best_effort) passed so
+// many duplicates that queues of four times the vertices overflowed.
+// fast_claim_vertices: the same for vertices u[k] (-1: none) already at hand.
+template <bool PRED, bool EXACT, bool LOCAL, int S, bool ROWS = true>
+__device__ __forceinline__ unsigned fast_claim_vertices(const GraphArgs &g, const SearchArgs &s, int next_depth,
+                                                        const int (&pv)[S], const int (&u)[S], int (&ub)[S],
+                                                        int (&ud)[S], bool ldsv, unsigned *vbits,
+                                                        StepIo io = StepIo{false, false})
+{
+    unsigned old[S];
+    const bool coherent = s.coherent_filter || (!LOCAL && io.stale);
+    // light steps: the candidates' rows, read beside their claims
+    int rb[S], rd[S];
+    if (LOCAL && ldsv) {
+#pragma unroll
+        for (int k = 0; k < S; k++) {
+            old[k] = ~0u;
+            if (u[k] >= 0)
+                old[k] = __hip_atomic_fetch_or(vbits + (u[k] >> 5), 1u << (u[k] & 31), __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+    } else {
+        // visited words (a set bit is final), then claims of the clear ones
+        unsigned cur[S];
+#pragma unroll
+        for (int k = 0; k < S; k++) {
+            cur[k] = ~0u;
+            if (u[k] >= 0) {
+                unsigned *w = s.visited + (u[k] >> 5);
+                cur[k] = coherent ? __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *w;
+            }
+        }
+        // The claims' results are read only after all are issued (a use
+        // next to its atomic would wait out each round trip in turn).
+#pragma unroll
+        for (int k = 0; k < S; k++) {
+            old[k] = ~0u;
+            const unsigned bit = 1u << (u[k] & 31);
+            if (u[k] >= 0 && !(cur[k] & bit)) {
+                // agent scope unless LOCAL: other workgroups claim
+                // concurrently, and another XCD's L2 may hold this word from
+                // before an earlier step's claims
+                if (LOCAL)
+                    old[k] = __hip_atomic_fetch_or(s.visited + (u[k] >> 5), bit, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+                else
+                    old[k] = __hip_atomic_fetch_or(s.visited + (u[k] >> 5), bit, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        if constexpr (!LOCAL && ROWS) {
+            if (io.light) {
+#pragma unroll
+                for (int k = 0; k < S; k++) {
+                    rb[k] = 0;
+                    rd[k] = 0;
+                    if (u[k] >= 0 && !((cur[k] >> (u[k] & 31)) & 1u)) {
+                        rb[k] = g.row[u[k]];
+                        rd[k] = g.row[u[k] + 1];
+                    }
+                }
+            }
+        }
+    }
+    // (the empty asm keeps the compiler from folding a use into the
+    // atomic's own block)
+#pragma unroll
+    for (int k = 0; k < S; k++) asm volatile("" : "+v"(old[k]));
+    unsigned fresh = 0;
+#pragma unroll
+    for (int k = 0; k < S; k++)
+        if (!((old[k] >> (u[k] & 31)) & 1u)) fresh |= 1u << k;
+    if (!EXACT) {
+        // best-effort culling elsewhere may have lost bits of labelled vertices
+        int dep[S];
+#pragma unroll
+        for (int k = 0; k < S; k++) dep[k] = ((fresh >> k) & 1) ? s.depth[u[k]] : -1;
+#pragma unroll
+        for (int k = 0; k < S; k++)
+            if (dep[k] != -1) fresh &= ~(1u << k);
+    }
+#pragma unroll
+    for (int k = 0; k < S; k++) {
+        ub[k] = 0;
+        ud[k] = 0;
+        if ((fresh >> k) & 1) {
+            s.depth[u[k]] = next_depth;
+            if (PRED) s.pred[u[k]] = pv[k];
+            if (!LOCAL && io.light) {
+                if (ROWS) {
+                    ub[k] = rb[k];
+                    ud[k] = rd[k];
+                }
+            } else if (ROWS) {
+                ub[k] = g.row[u[k]];
+                ud[k] = g.row[u[k] + 1];
+            }
+        }
+    }
+    return fresh;
+}
+
+template <bool PRED, bool EXACT, bool LOCAL, int S>
+__device__ __forceinline__ unsigned fast_claim_slots(const GraphArgs &g, const SearchArgs &s, int next_depth,
+                                                     const int (&at)[S], const int (&pv)[S], int (&u)[S],
+                                                     int (&ub)[S], int (&ud)[S], bool ldsv = false,
+                                                     unsigned *vbits = nullptr, StepIo io = StepIo{false, false})
+{
+#pragma unroll
+    for (int k = 0; k < S; k++)
+        u[k] = at[k] < 0 ? -1 : LOCAL ? g.col[at[k]] : __builtin_nontemporal_load(g.col + at[k]);
+    return fast_claim_vertices<PRED, EXACT, LOCAL, S>(g, s, next_depth, pv, u, ub, ud, ldsv, vbits, io);
+}
+
+// Workgroups worth running a top-down step of `fe` frontier edges: about
+// 1024 edges each (two per thread), fewer workgroups than that leave a
+// longer chain, more only add reservation atomics.
+__device__ __forceinline__ unsigned edge_workgroups(unsigned long long fe)
+{
+    return (unsigned) min(fe / 1024ull + 1ull, (unsigned long long) gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -303,34 +452,40 @@ __device__ __forceinline__ void hub_phase(const GraphArgs &g, const SearchArgs &
 // kernel's argument structs by address, and the compiler then copies them to
 // scratch and reads every field from there for the whole kernel.
 // ---------------------------------------------------------------------------
+// (fe_in: the step's frontier edges)
 template <bool PRED, bool EXACT>
 __device__ __forceinline__ void body_expand_contract(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds,
-                                     int sub, bool hubs, unsigned *next_bits = nullptr, bool from_bitmap = false)
+                                     int sub, bool hubs, unsigned long long fe_in, StepIo io,
+                                     unsigned *next_bits = nullptr, bool from_bitmap = false)
 {
-    WaveQueue<PRED> wq = make_queue<PRED>(s, c.step, lds);
+    WaveQueue<PRED> wq = make_queue<PRED>(s, c.step, lds, io.light);
     const int *in = s.q[c.step & 1];
     const int next_depth = c.iteration + 1;
-    bool labeled = false;
     unsigned fe = 0;
-    auto edge = [&](bool ok, int u, int par) {
-        bool fresh = ok && claim<EXACT>(s.visited, s.depth, u, s.coherent_filter);
-        if (fresh) {
-            s.depth[u] = next_depth;
-            if (PRED) s.pred[u] = par;
-            labeled = true;
-            if (s.track_edges) fe += (unsigned) (g.row[u + 1] - g.row[u]);
-            // a clear frontier bitmap becomes the next frontier's, exactly
-            if (next_bits)
-                __hip_atomic_fetch_or(next_bits + (u >> 5), 1u << (u & 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    auto begin = [](int) {};
+    auto edges = [&](const int (&at)[4], const int (&pv)[4], unsigned) {
+        int u[4], ub[4], ud[4];
+        const unsigned fresh =
+            fast_claim_slots<PRED, EXACT, false, 4>(g, s, next_depth, at, pv, u, ub, ud, false, nullptr, io);
+#pragma unroll
+        for (int j = 0; j < 4; j++) fe += (unsigned) (ud[j] - ub[j]);
+        // a clear frontier bitmap becomes the next frontier's, exactly
+        if (next_bits) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if ((fresh >> j) & 1)
+                    __hip_atomic_fetch_or(next_bits + (u[j] >> 5), 1u << (u[j] & 31), __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
         }
-        wq.push(fresh, u, par);
+#pragma unroll
+        for (int j = 0; j < 4; j++) wq.push((fresh >> j) & 1, u[j], pv[j]);
     };
     if (sub == 0 && from_bitmap) {
         // The frontier is frontier bitmap fbm[c.iteration & 1], as a
         // bottom-up level left it: each workgroup takes kBlock-word tiles
         // of it, clears them and the other bitmap's words (so both are
         // clear after the step, as a top-down level needs them), and
-        // gathers one member per thread per round.
+        // gathers up to two members per thread per round.
         const HubList hub = hub_list(s, c.step, hubs, n);
         unsigned *bm = s.fbm[c.iteration & 1];
         unsigned *other = s.fbm[(c.iteration + 1) & 1];
@@ -344,28 +499,43 @@ __device__ __forceinline__ void body_expand_contract(const GraphArgs &g, const S
                 other[w] = 0u;
             }
             while (__syncthreads_or(bits != 0u)) {
-                int beg = 0, end = 0, par = -1;
-                if (bits) {
-                    const int v = (int) ((w << 5) + (unsigned) __builtin_ctz(bits));
-                    bits &= bits - 1u;
-                    beg = g.row[v];
-                    end = g.row[v + 1];
-                    par = v;
+                int beg[2] = {0, 0}, end[2] = {0, 0}, par[2] = {-1, -1};
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    if (bits) {
+                        par[k] = (int) ((w << 5) + (unsigned) __builtin_ctz(bits));
+                        bits &= bits - 1u;
+                    }
                 }
-                gather_rows<PRED>(beg, end, par, g.col, s.wave_t, s.cta_t, hub, lds, edge);
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    if (par[k] >= 0) {
+                        beg[k] = g.row[par[k]];
+                        end[k] = g.row[par[k] + 1];
+                    }
+                }
+                gather_tile<2>(beg, end, par, hub, lds.rt, begin, edges);
             }
         }
     } else if (sub == 0) {
-        tile_phase<PRED>(g, s, c, n, hub_list(s, c.step, hubs, n), lds, [&](unsigned i, int &beg, int &end, int &par) {
-            int v = ld_queue(in + i);
-            beg = g.row[v];
-            end = g.row[v + 1];
-            par = v;
-        }, edge);
+        const HubList hub = hub_list(s, c.step, hubs, n);
+        TileGrab tg = tile_grab(s, n, lds, kBlock, edge_workgroups(fe_in));
+        while (true) {
+            const unsigned t = next_tile(&s.ctl->steal[c.step & 1], lds, tg);
+            if (t >= tg.tiles) break;
+            const unsigned i = tg.dealt(t, threadIdx.x);
+            int beg[1] = {0}, end[1] = {0}, par[1] = {-1};
+            if (threadIdx.x < tg.width && i < n) {
+                par[0] = ld_queue(in + i);
+                beg[0] = g.row[par[0]];
+                end[0] = g.row[par[0] + 1];
+            }
+            gather_tile<1>(beg, end, par, hub, lds.rt, begin, edges);
+        }
     } else {
-        hub_phase<PRED>(g, s, c, n, lds, edge);
+        hub_phase<PRED>(s, c, lds, edges);
     }
-    finish_step<PRED>(wq, lds, s.ctl, c.step, labeled, next_depth, fe, s.track_edges != 0);
+    finish_step<PRED>(wq, lds, s.ctl, c.step, fe, s.track_edges != 0);
 }
 
 // Bottom-up step of a direction-optimizing search (Beamer, Asanovic,
@@ -412,7 +582,6 @@ __device__ __forceinline__ void body_bottom_up(const GraphArgs &g, const SearchA
     const int wave = threadIdx.x / kWave;
     const int next_depth = c.iteration + 1;
     const unsigned words = ((unsigned) g.nodes + 31) >> 5;
-    bool labeled = false;
     unsigned fe = 0;
     int found = 0;
     int *qv = lds.wq[wave];
@@ -493,7 +662,6 @@ __device__ __forceinline__ void body_bottom_up(const GraphArgs &g, const SearchA
                 s.depth[v[h]] = next_depth;
                 if (PRED) s.pred[v[h]] = parent[h];
                 fe += (unsigned) (end[h] - beg[h]);
-                labeled = true;
                 found++;
                 __hip_atomic_fetch_or(&fbits[((unsigned) v[h] >> 5) - word0], 1u << (v[h] & 31), __ATOMIC_RELAXED,
                                       __HIP_MEMORY_SCOPE_WAVEFRONT);
@@ -602,7 +770,7 @@ __device__ __forceinline__ void body_bottom_up(const GraphArgs &g, const SearchA
     // The level's output is the bitmap nxt; only its size goes to the queue
     // length (queue_from_bitmap materialises the queue if the search turns
     // top-down again).
-    finish_step<PRED>(wq, lds, s.ctl, c.step, labeled, next_depth, fe, true, found);
+    finish_step<PRED>(wq, lds, s.ctl, c.step, fe, true, found);
 }
 
 // Writes the members of frontier bitmap fbm[c.iteration & 1] into the input
@@ -640,52 +808,180 @@ __device__ __forceinline__ void queue_from_bitmap(const GraphArgs &g, const Sear
     }
 }
 
-template <bool PRED, bool EXACT>
-__device__ __forceinline__ void body_contract_expand(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds,
-                                     int sub, bool hubs)
+// Contraction of one tile of an edge frontier: threads take up to kItems
+// items each (kBlock apart), cull them through the history hash, and claim
+// the rest with every memory trip in flight for all of them.  Returns the
+// mask of the items k that claimed u[k] (parent pv[k], row [ub[k], ud[k])).
+constexpr int kItems = 4;
+
+template <bool PRED, bool EXACT, bool ROWS>
+__device__ __forceinline__ unsigned contract_tile(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n,
+                                                  unsigned base, unsigned width, Lds<PRED> &lds, StepIo io,
+                                                  int (&u)[kItems], int (&pv)[kItems], int (&ub)[kItems],
+                                                  int (&ud)[kItems])
 {
-    WaveQueue<PRED> wq = make_queue<PRED>(s, c.step, lds);
     const int *in = s.q[c.step & 1];
     const int *pin = s.pq[c.step & 1];
-    bool labeled = false;
-    auto edge = [&](bool ok, int w, int par) { wq.push(ok, w, par); };
-    if (sub == 0) {
-        tile_phase<PRED>(g, s, c, n, hub_list(s, c.step, hubs, n), lds, [&](unsigned i, int &beg, int &end, int &par) {
-            int u = ld_queue(in + i);
-            int p = PRED ? ld_queue(pin + i) : -1;
-            if (history_pass<PRED>(lds, u) && claim<EXACT>(s.visited, s.depth, u, s.coherent_filter)) {
-                s.depth[u] = c.iteration;
-                if (PRED) s.pred[u] = p;
-                beg = g.row[u];
-                end = g.row[u + 1];
-                par = u;
-                labeled = true;
-            }
-        }, edge);
-    } else {
-        hub_phase<PRED>(g, s, c, n, lds, edge);
+#pragma unroll
+    for (int k = 0; k < kItems; k++) {
+        const unsigned o = (unsigned) (k * kBlock) + threadIdx.x;
+        const bool ok = o < width && base + o < n;
+        u[k] = ok ? ld_queue(in + base + o) : -1;
+        pv[k] = PRED && ok ? ld_queue(pin + base + o) : -1;
     }
-    finish_step<PRED>(wq, lds, s.ctl, c.step, labeled, c.iteration, 0u, false);
+#pragma unroll
+    for (int k = 0; k < kItems; k++)
+        if (u[k] >= 0 && !history_pass<PRED>(lds, u[k])) u[k] = -1;
+    return fast_claim_vertices<PRED, EXACT, false, kItems, ROWS>(g, s, c.iteration, pv, u, ub, ud, false, nullptr,
+                                                                 io);
+}
+
+// Expansion: every neighbour goes to the output queue.  A tile's edge count
+// is its output, so a tile of kDirectEdges and more reserves its place with
+// one atomic and writes there in order (the staging areas cost one atomic,
+// all on the queue's length, per 2048 edges: 12 k of them, 40 ns each,
+// were most of the 25 M-edge expansion of an R-MAT scale 20 search, 545 us
+// through staging); smaller tiles go through the waves' staging, which
+// gathers many of them per atomic.  Rows of the grid tier reserve theirs when
+// they are published.
+constexpr int kDirectEdges = 4096;
+
+template <bool PRED>
+struct Expansion {
+    const GraphArgs &g;
+    const SearchArgs &s;
+    const Cursor c;
+    Lds<PRED> &lds;
+    WaveQueue<PRED> wq;
+    bool direct;  // the current tile's form (workgroup-uniform)
+    bool wrote;   // some output did not go through the staging
+    bool lost;
+
+    __device__ __forceinline__ Expansion(const GraphArgs &g_, const SearchArgs &s_, Cursor c_, Lds<PRED> &lds_,
+                                         StepIo io)
+        : g(g_), s(s_), c(c_), lds(lds_), wq(make_queue<PRED>(s_, c_.step, lds_, io.light)), direct(false),
+          wrote(false), lost(false)
+    {
+    }
+    __device__ __forceinline__ void put(unsigned at, int u, int par)
+    {
+        if (at < s.cap) wq.store(at, u, par);
+        else lost = true;
+    }
+    __device__ __forceinline__ void begin(int edges)
+    {
+        direct = edges >= kDirectEdges;
+        wrote = wrote || direct;
+        // (the row table's barrier orders the word before its readers)
+        if (direct && threadIdx.x == 0) lds.ep_base = add_agent(wq.out_len, (unsigned) edges);
+    }
+    __device__ __forceinline__ void edges(const int (&at)[4], const int (&pv)[4], unsigned x0)
+    {
+        int u[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) u[j] = at[j] >= 0 ? __builtin_nontemporal_load(g.col + at[j]) : -1;
+        if (direct) {
+            const unsigned base = lds.ep_base + x0;
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (at[j] >= 0) put(base + (unsigned) (j * kBlock), u[j], pv[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) wq.push(at[j] >= 0, u[j], pv[j]);
+        }
+    }
+    template <int K>
+    __device__ __forceinline__ void tile(const int (&beg)[K], int (&end)[K], const int (&par)[K], const HubList &hub)
+    {
+        gather_tile<K>(
+            beg, end, par, hub, lds.rt, [&](int e) { begin(e); },
+            [&](const int (&at)[4], const int (&pv)[4], unsigned x0) { edges(at, pv, x0); });
+    }
+    __device__ __forceinline__ HubList hubs(unsigned n, bool enabled) const
+    {
+        HubList h = hub_list(s, c.step, enabled, n);
+        h.out_len = wq.out_len;
+        return h;
+    }
+    __device__ __forceinline__ void hub_chunks()
+    {
+        hub_phase_chunks<PRED>(s, c, lds, [&](int b, int e, int par) {
+            const unsigned out = lds.cta_out;
+            int u[kHubChunk / kBlock];
+#pragma unroll
+            for (int j = 0; j < kHubChunk / kBlock; j++) {
+                const int x = b + j * kBlock + (int) threadIdx.x;
+                u[j] = x < e ? __builtin_nontemporal_load(g.col + x) : -1;
+            }
+#pragma unroll
+            for (int j = 0; j < kHubChunk / kBlock; j++) {
+                const int o = j * kBlock + (int) threadIdx.x;
+                if (b + o < e) put(out + (unsigned) o, u[j], par);
+            }
+        });
+    }
+    __device__ __forceinline__ void report_lost()
+    {
+        if (lost) {
+            st_agent(wq.overflow, 1u);
+            st_agent(wq.overflow_step, 1u);
+        }
+    }
+};
+
+template <bool PRED, bool EXACT>
+__device__ __forceinline__ void body_contract_expand(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds,
+                                     int sub, bool hubs, StepIo io)
+{
+    Expansion<PRED> x(g, s, c, lds, io);
+    bool labeled = false;
+    if (sub == 0) {
+        const HubList hub = x.hubs(n, hubs);
+        TileGrab tg = tile_grab(s, n, lds, kItems * kBlock, (n + kBlock - 1) / kBlock);
+        while (true) {
+            const unsigned base = next_tile(&s.ctl->steal[c.step & 1], lds, tg) * tg.width;
+            if (base >= n) break;
+            int u[kItems], pv[kItems], beg[kItems], end[kItems];
+            const unsigned fresh = contract_tile<PRED, EXACT, true>(g, s, c, n, base, tg.width, lds, io, u, pv, beg, end);
+            labeled = labeled || fresh != 0;  // (rows of the other items are empty)
+            x.template tile<kItems>(beg, end, u, hub);
+        }
+    } else {
+        x.hub_chunks();
+    }
+    x.report_lost();
+    // Vertices labelled here show in the next step's input (prepare_step),
+    // unless none of them has neighbours.
+    const bool all_staged = !__syncthreads_or(x.wrote);
+    finish_step<PRED>(x.wq, lds, s.ctl, c.step, 0u, false, 0, labeled && all_staged, c.iteration);
 }
 
 template <bool PRED, bool EXACT>
 __device__ __forceinline__ void body_expand(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds, int sub,
-                            bool hubs)
+                            bool hubs, StepIo io)
 {
-    WaveQueue<PRED> wq = make_queue<PRED>(s, c.step, lds);
+    Expansion<PRED> x(g, s, c, lds, io);
     const int *in = s.q[c.step & 1];
-    auto edge = [&](bool ok, int w, int par) { wq.push(ok, w, par); };
     if (sub == 0) {
-        tile_phase<PRED>(g, s, c, n, hub_list(s, c.step, hubs, n), lds, [&](unsigned i, int &beg, int &end, int &par) {
-            int v = ld_queue(in + i);
-            beg = g.row[v];
-            end = g.row[v + 1];
-            par = v;
-        }, edge);
+        const HubList hub = x.hubs(n, hubs);
+        TileGrab tg = tile_grab(s, n, lds, kBlock, gridDim.x);
+        while (true) {
+            const unsigned t = next_tile(&s.ctl->steal[c.step & 1], lds, tg);
+            if (t >= tg.tiles) break;
+            const unsigned i = tg.dealt(t, threadIdx.x);
+            int beg[1] = {0}, end[1] = {0}, par[1] = {-1};
+            if (threadIdx.x < tg.width && i < n) {
+                par[0] = ld_queue(in + i);
+                beg[0] = g.row[par[0]];
+                end[0] = g.row[par[0] + 1];
+            }
+            x.template tile<1>(beg, end, par, hub);
+        }
     } else {
-        hub_phase<PRED>(g, s, c, n, lds, edge);
+        x.hub_chunks();
     }
-    finish_step<PRED>(wq, lds, s.ctl, c.step, false, 0, 0u, false);
+    x.report_lost();
+    finish_step<PRED>(x.wq, lds, s.ctl, c.step, 0u, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -709,8 +1005,7 @@ constexpr unsigned kChainGrabMax = kWave;  // tiles per grab: one lane each in t
 static_assert(kChainGrabMax * kWaves * 2 <= kWaves * kWaveQueueCap, "grab masks fit the staging area");
 
 template <bool PRED, bool EXACT, bool FILTER>
-__device__ __forceinline__ void chained_step(const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds,
-                                             bool &labeled)
+__device__ __forceinline__ void chained_step(const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds)
 {
     const int *in = s.q[c.step & 1];
     const int *pin = s.pq[c.step & 1];
@@ -718,7 +1013,7 @@ __device__ __forceinline__ void chained_step(const SearchArgs &s, Cursor c, unsi
     int *pout = PRED ? s.pq[(c.step + 1) & 1] : nullptr;
     // the wave-queue staging is idle: ballot masks [tile][wave]
     unsigned long long *masks = reinterpret_cast<unsigned long long *>(&lds.wq[0][0]);
-    int *tile_off = &lds.sc_excl[0][0];
+    int *tile_off = &lds.rt.excl[0][0];
     const int lane = lane_id(), wave = threadIdx.x / kWave;
     const unsigned tiles = (n + kBlock - 1) / kBlock;
     // (grabs in increasing order, as the look-back needs: always dynamic)
@@ -742,7 +1037,6 @@ __device__ __forceinline__ void chained_step(const SearchArgs &s, Cursor c, unsi
                     if (keep) {
                         s.depth[u] = c.iteration;
                         if (PRED) s.pred[u] = p;
-                        labeled = true;
                     }
                 }
             }
@@ -797,71 +1091,62 @@ __device__ __forceinline__ void chained_step(const SearchArgs &s, Cursor c, unsi
 }
 
 template <bool PRED, bool EXACT>
-__device__ __forceinline__ void body_contract(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds)
+__device__ __forceinline__ void body_contract(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds,
+                                              StepIo io)
 {
-    (void) g;
-    WaveQueue<PRED> wq = make_queue<PRED>(s, c.step, lds);
-    const int *in = s.q[c.step & 1];
-    const int *pin = s.pq[c.step & 1];
-    bool labeled = false;
+    WaveQueue<PRED> wq = make_queue<PRED>(s, c.step, lds, io.light);
     if (s.tile_status) {
-        chained_step<PRED, EXACT, false>(s, c, n, lds, labeled);
+        chained_step<PRED, EXACT, false>(s, c, n, lds);
     } else {
-        TileGrab tg = tile_grab(s, n, lds);
+        TileGrab tg = tile_grab(s, n, lds, kItems * kBlock, (n + kBlock - 1) / kBlock);
         while (true) {
-            unsigned base = next_tile(&s.ctl->steal[c.step & 1], lds, tg) * kBlock;
+            const unsigned base = next_tile(&s.ctl->steal[c.step & 1], lds, tg) * tg.width;
             if (base >= n) break;
-            unsigned i = base + threadIdx.x;
-            int u = -1, p = -1;
-            if (i < n) {
-                u = ld_queue(in + i);
-                if (PRED) p = ld_queue(pin + i);
-            }
-            bool keep = u >= 0 && history_pass<PRED>(lds, u) && claim<EXACT>(s.visited, s.depth, u, s.coherent_filter);
-            if (keep) {
-                s.depth[u] = c.iteration;
-                if (PRED) s.pred[u] = p;
-                labeled = true;
-            }
-            wq.push(keep, u, -1);
+            int u[kItems], pv[kItems], ub[kItems], ud[kItems];
+            const unsigned fresh =
+                contract_tile<PRED, EXACT, false>(g, s, c, n, base, tg.width, lds, io, u, pv, ub, ud);
+#pragma unroll
+            for (int k = 0; k < kItems; k++) wq.push((fresh >> k) & 1, u[k], -1);
         }
     }
-    finish_step<PRED>(wq, lds, s.ctl, c.step, labeled, c.iteration, 0u, false);
+    finish_step<PRED>(wq, lds, s.ctl, c.step, 0u, false);
 }
 
 template <bool PRED, bool EXACT>
-__device__ __forceinline__ void body_filter(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds)
+__device__ __forceinline__ void body_filter(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds,
+                                            StepIo io)
 {
     (void) g;
-    WaveQueue<PRED> wq = make_queue<PRED>(s, c.step, lds);
+    WaveQueue<PRED> wq = make_queue<PRED>(s, c.step, lds, io.light);
     const int *in = s.q[c.step & 1];
     const int *pin = s.pq[c.step & 1];
     if (s.tile_status) {
-        bool unused = false;
-        chained_step<PRED, EXACT, true>(s, c, n, lds, unused);
+        chained_step<PRED, EXACT, true>(s, c, n, lds);
     } else {
-        TileGrab tg = tile_grab(s, n, lds);
+        TileGrab tg = tile_grab(s, n, lds, kItems * kBlock, (n + kBlock - 1) / kBlock);
         while (true) {
-            unsigned base = next_tile(&s.ctl->steal[c.step & 1], lds, tg) * kBlock;
+            const unsigned base = next_tile(&s.ctl->steal[c.step & 1], lds, tg) * tg.width;
             if (base >= n) break;
-            unsigned i = base + threadIdx.x;
-            int u = -1, p = -1;
-            if (i < n) {
-                u = ld_queue(in + i);
-                if (PRED) p = ld_queue(pin + i);
+            int u[kItems], p[kItems];
+            unsigned w[kItems];
+#pragma unroll
+            for (int k = 0; k < kItems; k++) {
+                const unsigned o = (unsigned) (k * kBlock) + threadIdx.x;
+                const bool ok = o < tg.width && base + o < n;
+                u[k] = ok ? ld_queue(in + base + o) : -1;
+                p[k] = PRED && ok ? ld_queue(pin + base + o) : -1;
             }
             // Bitmask only: the history hash is reserved for claims, because a
             // hit there must mean the vertex has already been claimed or found
             // visited by this workgroup.
-            bool keep = false;
-            if (u >= 0) {
-                unsigned w = s.visited[u >> 5];
-                keep = ((w >> (u & 31)) & 1u) == 0;
-            }
-            wq.push(keep, u, p);
+#pragma unroll
+            for (int k = 0; k < kItems; k++)
+                w[k] = u[k] < 0 ? ~0u : io.stale ? ld_agent(s.visited + (u[k] >> 5)) : s.visited[u[k] >> 5];
+#pragma unroll
+            for (int k = 0; k < kItems; k++) wq.push(u[k] >= 0 && !((w[k] >> (u[k] & 31)) & 1u), u[k], p[k]);
         }
     }
-    finish_step<PRED>(wq, lds, s.ctl, c.step, false, 0, 0u, false);
+    finish_step<PRED>(wq, lds, s.ctl, c.step, 0u, false);
 }
 
 __device__ __forceinline__ bool gathers(int phase)
@@ -871,15 +1156,16 @@ __device__ __forceinline__ bool gathers(int phase)
 
 template <bool PRED, bool EXACT>
 __device__ __forceinline__ void run_body(int phase, const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n,
-                                         Lds<PRED> &lds, int sub, bool hubs)
+                                         Lds<PRED> &lds, int sub, bool hubs, unsigned long long fe)
 {
+    const StepIo io{false, false};
     switch (phase) {
-    case kPhaseExpandContract: body_expand_contract<PRED, EXACT>(g, s, c, n, lds, sub, hubs); break;
-    case kPhaseContractExpand: body_contract_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs); break;
-    case kPhaseContract: body_contract<PRED, EXACT>(g, s, c, n, lds); break;
-    case kPhaseExpand: body_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs); break;
+    case kPhaseExpandContract: body_expand_contract<PRED, EXACT>(g, s, c, n, lds, sub, hubs, fe, io); break;
+    case kPhaseContractExpand: body_contract_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs, io); break;
+    case kPhaseContract: body_contract<PRED, EXACT>(g, s, c, n, lds, io); break;
+    case kPhaseExpand: body_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs, io); break;
     case kPhaseBottomUp: body_bottom_up<PRED, EXACT>(g, s, c, lds); break;
-    default: body_filter<PRED, EXACT>(g, s, c, n, lds); break;
+    default: body_filter<PRED, EXACT>(g, s, c, n, lds, io); break;
     }
 }
 
@@ -887,22 +1173,22 @@ __device__ __forceinline__ void run_body(int phase, const GraphArgs &g, const Se
 // its kernel, which keeps their registers out of its budget).
 template <bool PRED, bool EXACT, int LOOP>
 __device__ __forceinline__ void loop_body(int phase, const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n,
-                                          Lds<PRED> &lds, int sub, bool hubs, unsigned *next_bits = nullptr,
-                                          bool from_bitmap = false)
+                                          Lds<PRED> &lds, int sub, bool hubs, unsigned long long fe, StepIo io,
+                                          unsigned *next_bits = nullptr, bool from_bitmap = false)
 {
     if constexpr (LOOP == kLoopEC) {
-        body_expand_contract<PRED, EXACT>(g, s, c, n, lds, sub, hubs);
+        body_expand_contract<PRED, EXACT>(g, s, c, n, lds, sub, hubs, fe, io);
     } else if constexpr (LOOP == kLoopCE) {
         // (expand: the step that ends a contract-expand fast path)
-        if (phase == kPhaseExpand) body_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs);
-        else body_contract_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs);
+        if (phase == kPhaseExpand) body_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs, io);
+        else body_contract_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs, io);
     } else if constexpr (LOOP == kLoopDO) {
         if (phase == kPhaseBottomUp) body_bottom_up<PRED, EXACT>(g, s, c, lds);
-        else body_expand_contract<PRED, EXACT>(g, s, c, n, lds, sub, hubs, next_bits, from_bitmap);
+        else body_expand_contract<PRED, EXACT>(g, s, c, n, lds, sub, hubs, fe, io, next_bits, from_bitmap);
     } else {
-        if (phase == kPhaseContract) body_contract<PRED, EXACT>(g, s, c, n, lds);
-        else if (phase == kPhaseExpand) body_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs);
-        else body_filter<PRED, EXACT>(g, s, c, n, lds);
+        if (phase == kPhaseContract) body_contract<PRED, EXACT>(g, s, c, n, lds, io);
+        else if (phase == kPhaseExpand) body_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs, io);
+        else body_filter<PRED, EXACT>(g, s, c, n, lds, io);
     }
 }
 
@@ -968,18 +1254,18 @@ __device__ __forceinline__ void body_expand_mark(const GraphArgs &g, const Searc
         // four consecutive edges per thread per round with every load of a
         // round in flight -- instead of the gather tiers' one chain per
         // round of 64 edges.
-        const HubList hub = hub_list(s, c.step, hubs, n, true);
+        const HubList hub = hub_list(s, c.step, hubs, n);
         int *tbeg = lds.wq[0];  // the wave-queue staging is idle in a marked step
         int *tpar = lds.wq[1];
         int *toff = lds.wq[2];
         static_assert(kWaveQueueCap >= kBlock && kWaves >= 3, "tile tables fit the staging area");
-        TileGrab tg = tile_grab(s, n, lds);
+        TileGrab tg = tile_grab(s, n, lds, kBlock, gridDim.x);
         while (true) {
-            const unsigned base = next_tile(&s.ctl->steal[c.step & 1], lds, tg) * kBlock;
-            if (base >= n) break;
-            const unsigned i = base + threadIdx.x;
+            const unsigned t = next_tile(&s.ctl->steal[c.step & 1], lds, tg);
+            if (t >= tg.tiles) break;
+            const unsigned i = tg.dealt(t, threadIdx.x);
             int v = -1, beg = 0, end = 0;
-            if (i < n) {
+            if (threadIdx.x < tg.width && i < n) {
                 v = ld_queue(in + i);
                 beg = g.row[v];
                 end = g.row[v + 1];
@@ -1047,7 +1333,7 @@ __device__ __forceinline__ void body_expand_mark(const GraphArgs &g, const Searc
     // load of a round in flight together (the per-edge chain -- column,
     // visited word, mark -- is the cost of these levels, not bytes).
     constexpr int U = 4;
-    hub_phase_chunks<PRED>(g, s, c, n, lds, true, [&](int b, int e, int pv) {
+    hub_phase_chunks<PRED>(s, c, lds, [&](int b, int e, int pv) {
         for (int k = b; k < e; k += U * kBlock) {
             int u[U];
             unsigned w[U];
@@ -1101,7 +1387,6 @@ __device__ __forceinline__ void mark_compact(const GraphArgs &g, const SearchArg
     int *stage = &lds.wq[0][0];
     constexpr int kStage = kWaves * kWaveQueueCap;
     unsigned fe = 0;
-    bool labeled = false;
     bool over = false;
     for (unsigned w0 = blockIdx.x * kBlock; w0 < words; w0 += gridDim.x * kBlock) {
         const unsigned w = w0 + threadIdx.x;
@@ -1131,7 +1416,6 @@ __device__ __forceinline__ void mark_compact(const GraphArgs &g, const SearchArg
         const int excl = block_exclusive_sum(__popc(bits), lds.ep_scan, &total);
         if (total == 0) continue;  // block-uniform
         if (threadIdx.x == 0) lds.ep_base = add_agent(&s.ctl->qlen[(c.step + 1) % 3], (unsigned) total);
-        labeled = labeled || bits != 0;
         if (total <= kStage) {
             // labels, queue entries and degrees spread over the workgroup,
             // four vertices per thread per round with their row loads in
@@ -1177,9 +1461,9 @@ __device__ __forceinline__ void mark_compact(const GraphArgs &g, const SearchArg
         st_agent(&s.ctl->overflow, 1u);
         st_agent(&s.ctl->ovf[(c.step + 1) % 3], 1u);
     }
-    // frontier-edge, visited-edge and depth counters: one update per workgroup
+    // frontier-edge counter: one update per workgroup
     WaveQueue<PRED> wq = make_queue<PRED>(s, c.step, lds);
-    finish_step<PRED>(wq, lds, s.ctl, c.step, labeled, next_depth, fe, s.track_edges != 0);
+    finish_step<PRED>(wq, lds, s.ctl, c.step, fe, s.track_edges != 0);
 }
 
 // Direction choice of a direction-optimizing search at the top of a level
@@ -1252,6 +1536,10 @@ __device__ __forceinline__ void prepare_step(Control *ctl, Cursor c, unsigned n)
     __hip_atomic_store(&ctl->hub_alloc[(c.step + 1) & 1], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(&ctl->fedges[(c.step + 2) % 3], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     ctl->total_queued += n;
+    // deepest label so far: the members of a vertex frontier carry the step's
+    // iteration, those whose neighbours form an edge frontier the one before
+    const bool members = c.phase == kPhaseExpandContract || c.phase == kPhaseBottomUp || c.phase == kPhaseExpand;
+    if (n > 0) atomicMax(&ctl->max_depth, members ? c.iteration : c.iteration - 1);
     if (c.step < kLevelLog) {
         ctl->level_len[c.step] = n;
         ctl->level_clock[c.step] = wall_clock64();
@@ -1370,110 +1658,6 @@ __device__ int fast_scan(FastFront &F, int b, unsigned n)
     return total;
 }
 
-// Claims of one thread's edge slots: at[k] = column position of slot k (or
-// -1), pv[k] = its row's owner.  Claims the unvisited neighbours, labels
-// them, and returns the mask of the slots k that claimed u[k] (row
-// [ub[k], ud[k])).  Each memory trip (column entry, visited word, claim,
-// row bounds) is issued for every slot before the first result is used.
-//
-// LOCAL: the calling workgroup is the only one touching the labels and the
-// visited words (block 0's fast path, between two grid barriers).  Its
-// claims are then workgroup-scope atomics, done in this XCD's L2, where
-// agent-scope ones must be coherent across the eight XCDs; the barrier
-// before the path invalidated stale lines, and the one after it writes the
-// path's lines back.  Column entries are read through the caches: the next
-// level's rows sit next to this level's on a lattice.  With vbits (LOCAL
-// only) the claims are LDS atomics on the path's copy of the visited
-// bitmap: no pre-read and no memory trip between a column entry and the
-// claimed vertex's row bounds.
-// fast_claim_vertices: the same for vertices u[k] (-1: none) already at hand.
-template <bool PRED, bool EXACT, bool LOCAL, int S>
-__device__ __forceinline__ unsigned fast_claim_vertices(const GraphArgs &g, const SearchArgs &s, int next_depth,
-                                                        const int (&pv)[S], const int (&u)[S], int (&ub)[S],
-                                                        int (&ud)[S], bool ldsv, unsigned *vbits)
-{
-    unsigned old[S];
-    if (LOCAL && ldsv) {
-#pragma unroll
-        for (int k = 0; k < S; k++) {
-            old[k] = ~0u;
-            if (u[k] >= 0)
-                old[k] = __hip_atomic_fetch_or(vbits + (u[k] >> 5), 1u << (u[k] & 31), __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
-    } else {
-        // visited words (a set bit is final), then claims of the clear ones
-        unsigned cur[S];
-#pragma unroll
-        for (int k = 0; k < S; k++) {
-            cur[k] = ~0u;
-            if (u[k] >= 0) {
-                unsigned *w = s.visited + (u[k] >> 5);
-                cur[k] = s.coherent_filter ? __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *w;
-            }
-        }
-        // The claims' results are read only after all are issued (a use
-        // next to its atomic would wait out each round trip in turn).
-#pragma unroll
-        for (int k = 0; k < S; k++) {
-            old[k] = ~0u;
-            const unsigned bit = 1u << (u[k] & 31);
-            if (u[k] >= 0 && !(cur[k] & bit)) {
-                // agent scope unless LOCAL: other workgroups claim
-                // concurrently, and another XCD's L2 may hold this word from
-                // before an earlier step's claims
-                if (LOCAL)
-                    old[k] = __hip_atomic_fetch_or(s.visited + (u[k] >> 5), bit, __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-                else
-                    old[k] = __hip_atomic_fetch_or(s.visited + (u[k] >> 5), bit, __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-    }
-    // (the empty asm keeps the compiler from folding a use into the
-    // atomic's own block)
-#pragma unroll
-    for (int k = 0; k < S; k++) asm volatile("" : "+v"(old[k]));
-    unsigned fresh = 0;
-#pragma unroll
-    for (int k = 0; k < S; k++)
-        if (!((old[k] >> (u[k] & 31)) & 1u)) fresh |= 1u << k;
-    if (!EXACT) {
-        // best-effort culling elsewhere may have lost bits of labelled vertices
-        int dep[S];
-#pragma unroll
-        for (int k = 0; k < S; k++) dep[k] = ((fresh >> k) & 1) ? s.depth[u[k]] : -1;
-#pragma unroll
-        for (int k = 0; k < S; k++)
-            if (dep[k] != -1) fresh &= ~(1u << k);
-    }
-#pragma unroll
-    for (int k = 0; k < S; k++) {
-        ub[k] = 0;
-        ud[k] = 0;
-        if ((fresh >> k) & 1) {
-            s.depth[u[k]] = next_depth;
-            if (PRED) s.pred[u[k]] = pv[k];
-            ub[k] = g.row[u[k]];
-            ud[k] = g.row[u[k] + 1];
-        }
-    }
-    return fresh;
-}
-
-template <bool PRED, bool EXACT, bool LOCAL, int S>
-__device__ __forceinline__ unsigned fast_claim_slots(const GraphArgs &g, const SearchArgs &s, int next_depth,
-                                                     const int (&at)[S], const int (&pv)[S], int (&u)[S],
-                                                     int (&ub)[S], int (&ud)[S], bool ldsv = false,
-                                                     unsigned *vbits = nullptr)
-{
-#pragma unroll
-    for (int k = 0; k < S; k++)
-        u[k] = at[k] < 0 ? -1 : LOCAL ? g.col[at[k]] : __builtin_nontemporal_load(g.col + at[k]);
-    return fast_claim_vertices<PRED, EXACT, LOCAL, S>(g, s, next_depth, pv, u, ub, ud, ldsv, vbits);
-}
-
 // kFastK consecutive edges from e0 (one thread's share of a batch) of an
 // LDS-resident frontier: offs = the exclusive scan of its n members' degrees
 // (total edges in all), begs = their row starts, vs = the members.  Returns
@@ -1483,7 +1667,7 @@ __device__ __forceinline__ unsigned fast_edges(const GraphArgs &g, const SearchA
                                                const int *offs, const int *begs, const int *vs, unsigned n,
                                                int total, int e0, int (&u)[kFastK], int (&pv)[kFastK],
                                                int (&ub)[kFastK], int (&ud)[kFastK], bool ldsv = false,
-                                               unsigned *vbits = nullptr)
+                                               unsigned *vbits = nullptr, StepIo io = StepIo{false, false})
 {
     // member holding edge e0: the last i with offs[i] <= e0 (it has edges)
     int i = 0;
@@ -1510,7 +1694,7 @@ __device__ __forceinline__ unsigned fast_edges(const GraphArgs &g, const SearchA
             pv[k] = vs[i];
         }
     }
-    return fast_claim_slots<PRED, EXACT, LOCAL, kFastK>(g, s, next_depth, at, pv, u, ub, ud, ldsv, vbits);
+    return fast_claim_slots<PRED, EXACT, LOCAL, kFastK>(g, s, next_depth, at, pv, u, ub, ud, ldsv, vbits, io);
 }
 
 // Appends one thread's claimed slots to LDS buffer dst (one LDS reservation
@@ -1667,7 +1851,7 @@ __device__ __forceinline__ void fast_lds_level(const GraphArgs &g, const SearchA
 // Every thread of every workgroup calls it; F must not be live.
 template <bool PRED, bool EXACT>
 __device__ __forceinline__ void spread_step(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, FastFront &F,
-                            unsigned *next_bits)
+                            StepIo io, unsigned *next_bits)
 {
     const int lane = lane_id(), wave = threadIdx.x / kWave;
     const int *in = s.q[c.step & 1];
@@ -1685,12 +1869,12 @@ __device__ __forceinline__ void spread_step(const GraphArgs &g, const SearchArgs
     int *out = s.q[(c.step + 1) & 1];
     int *pout = PRED ? s.pq[(c.step + 1) & 1] : nullptr;
     unsigned long long fe = 0;
-    bool labeled = false;
     const int stride = (int) gridDim.x * kBlock * kFastK;
     for (int b0 = (int) blockIdx.x * kBlock * kFastK; b0 < total; b0 += stride) {
         int u[kFastK], pv[kFastK], ub[kFastK], ud[kFastK];
         const unsigned fresh = fast_edges<PRED, EXACT, false>(g, s, next_depth, F.deg[0], F.beg[0], F.v[0], n, total,
-                                                       b0 + (int) threadIdx.x * kFastK, u, pv, ub, ud);
+                                                       b0 + (int) threadIdx.x * kFastK, u, pv, ub, ud, false, nullptr,
+                                                       io);
         int got;
         const int off = block_exclusive_sum(__popc(fresh), F.scan, &got);
         // (every thread read the previous batch's base before the scan's
@@ -1704,7 +1888,10 @@ __device__ __forceinline__ void spread_step(const GraphArgs &g, const SearchArgs
             const unsigned p = p0 + (unsigned) __popc(fresh & ((1u << k) - 1u));
             if ((fresh >> k) & 1) {
                 fe += (unsigned) (ud[k] - ub[k]);
-                if (p < s.cap) {
+                if (p < s.cap && io.light) {
+                    st_agent(out + p, u[k]);
+                    if (PRED) st_agent(pout + p, pv[k]);
+                } else if (p < s.cap) {
                     out[p] = u[k];
                     if (PRED) pout[p] = pv[k];
                 } else {
@@ -1712,7 +1899,6 @@ __device__ __forceinline__ void spread_step(const GraphArgs &g, const SearchArgs
                 }
             }
         }
-        labeled |= fresh != 0;
         if (lost) {
             st_agent(&ctl->overflow, 1u);
             st_agent(&ctl->ovf[(c.step + 1) % 3], 1u);
@@ -1725,27 +1911,18 @@ __device__ __forceinline__ void spread_step(const GraphArgs &g, const SearchArgs
                                           __HIP_MEMORY_SCOPE_AGENT);
         }
     }
-    // one update per workgroup of the next frontier's edges and the depth
+    // one update per workgroup of the next frontier's edges
     const int lo = wave_inclusive_sum((int) (fe & 0xFFFFu));
     const int hi = wave_inclusive_sum((int) (fe >> 16));
-    const bool any = ballot(labeled) != 0;
     if (lane == kWave - 1) {
         F.wfe[wave] = ((unsigned long long) (unsigned) hi << 16) + (unsigned long long) (unsigned) lo;
-        F.wlab[wave] = any ? 1 : 0;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         unsigned long long f = 0;
-        int l = 0;
-        for (int w = 0; w < kWaves; w++) {
-            f += F.wfe[w];
-            l |= F.wlab[w];
-        }
-        if (s.track_edges && f) {
+        for (int w = 0; w < kWaves; w++) f += F.wfe[w];
+        if (s.track_edges && f)
             __hip_atomic_fetch_add(&ctl->fedges[(c.step + 1) % 3], f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_add(&ctl->visited_edges, f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (l) atomicMax(&ctl->max_depth, next_depth);
     }
 }
 
@@ -1757,8 +1934,7 @@ __device__ __forceinline__ void spread_step(const GraphArgs &g, const SearchArgs
 // (see direction_rule).  Block 0 only; every thread calls it.
 template <bool PRED, bool EXACT, bool FASTV>
 __device__ __forceinline__ void fast_lds_path(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, int loop,
-                              unsigned long long fv, unsigned long long fe_in, FastLds<FASTV> &L, bool wait_others,
-                              const BarrierShape &bshape)
+                              unsigned long long fv, unsigned long long fe_in, FastLds<FASTV> &L, bool wait_others)
 {
     FastFront &F = L.f;
     const int *in = s.q[c.step & 1];
@@ -1789,8 +1965,9 @@ __device__ __forceinline__ void fast_lds_path(const GraphArgs &g, const SearchAr
         for (int i = 4 * chunks + (int) threadIdx.x; i < vwords; i += kBlock) L.vbits[i] = s.visited[i];
     }
     int src = 0;
-    unsigned long long ve_add = 0, queued = 0;
-    int maxd = -1;
+    unsigned long long queued = 0;
+    // deepest label so far (as prepare_step notes it for the entry step)
+    int maxd = c.phase == kPhaseExpandContract ? c.iteration : c.iteration - 1;
     unsigned n2 = 0;
     unsigned long long fe2 = 0;
     // frontier edges of the members and of the level before them
@@ -1880,7 +2057,6 @@ __device__ __forceinline__ void fast_lds_path(const GraphArgs &g, const SearchAr
         n2 = F.count;
         fe2 = F.fe;
         if (F.labeled) maxd = c.iteration + 1;
-        ve_add += fe2;
         src ^= 1;
         c = advance(loop, c);
         if (tp) {
@@ -1926,7 +2102,7 @@ __device__ __forceinline__ void fast_lds_path(const GraphArgs &g, const SearchAr
     // be reading at the top of the step the path started from, unless they
     // have all arrived at the barrier that ends the path.
     if (wait_others) {
-        if (threadIdx.x == 0) wait_other_arrivals(s.ctl, bshape);
+        if (threadIdx.x == 0) wait_other_arrivals(s.ctl);
         __syncthreads();
     }
     // The next step (c) reads its input from the global queue: copy the
@@ -1949,7 +2125,6 @@ __device__ __forceinline__ void fast_lds_path(const GraphArgs &g, const SearchAr
         st_agent(&ctl->ovf[c.step % 3], n2 > s.cap ? 1u : 0u);
         if (n2 > s.cap) st_agent(&ctl->overflow, 1u);
         __hip_atomic_store(&ctl->fedges[c.step % 3], fe2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_fetch_add(&ctl->visited_edges, ve_add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (maxd >= 0) atomicMax(&ctl->max_depth, maxd);
         ctl->total_queued += queued;
         st_agent(&ctl->fast_step, c.step);
@@ -2011,7 +2186,6 @@ __device__ __forceinline__ void search_prologue(const GraphArgs &g, const Search
             ctl->max_depth = 0;
             const unsigned long long deg = (unsigned long long) (g.row[src + 1] - g.row[src]);
             ctl->fedges[0] = deg;
-            ctl->visited_edges = deg;
         }
     }
 }
@@ -2039,11 +2213,11 @@ __device__ __forceinline__ void publish_status(const SearchArgs &s)
 // ---------------------------------------------------------------------------
 // One instantiation per strategy (LOOP), so profiles attribute time to the
 // strategy and the level loop carries no dead strategy branches.
-// Most work of a step whose grid barrier leaves the L2 write-back to each
-// XCD's last arriver, and the barrier of a launch from which XCD leaves
-// are used.
+// Most work (frontier edges, or items when edges are not tracked) of a step
+// that ends in a light barrier: up to here a step is bound by its chain of
+// memory trips, past it the stores past the L2 and the row reads beside the
+// claims would cost more than the cache maintenance they replace.
 constexpr unsigned long long kLightWork = 1ull << 19;
-constexpr unsigned kXcdBarrierFrom = 32;
 
 template <bool PRED, bool EXACT, int LOOP, bool FASTV>
 __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchArgs s, Cursor c)
@@ -2066,27 +2240,24 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
     // 0 is still writing, and the step's first grid barrier orders the
     // label rewrite before any claim.
     bool start = s.init_src >= 0;
-    // Grid barriers: leaves by block, and from the kXcdBarrierFrom-th
-    // barrier of a long launch on (a high-diameter search) the XCDs, counted
-    // from the records every workgroup left before its first barrier
-    // (thread 0's shape is the one used; the count costs a few
-    // microseconds, which a short launch does not win back).  After a light
-    // phase (little written) only each XCD's last arriver then writes its L2
-    // back; after a heavy one every workgroup still writes back its XCD's L2
-    // before arriving, which spreads the write-back over the arrivals
-    // instead of leaving it all to the last one.
-    BarrierShape bshape = barrier_shape_by_block();
-    bool shape_pending = gridDim.x >= 8u && gridDim.x <= (unsigned) kMaxXcdGrid;
-    unsigned barriers = 0;
-    if (shape_pending && threadIdx.x == 0) xcd_register(s.ctl);
+    // Barriers: full ones order plain stores before plain loads; light ones
+    // (after light steps, see StepIo) only what goes past the XCDs' L2s, and
+    // leave the caches stale: the next step that is not light itself
+    // refreshes them first.  Best-effort culling reads labels, which are
+    // plain stores, so its barriers are all full.
+    bool stale = false;
     auto bar = [&](bool light) {
-        BarrierShape b = bshape;
-        b.shared = bshape.shared && light ? 1u : 0u;
-        grid_barrier(s.ctl, b);
-        if (shape_pending && ++barriers == kXcdBarrierFrom) {
-            shape_pending = false;
-            if (threadIdx.x == 0) bshape = xcd_shape(s.ctl);
+        if (EXACT && light) {
+            grid_barrier_light(s.ctl);
+            stale = true;
+        } else {
+            grid_barrier(s.ctl);
+            stale = false;
         }
+    };
+    auto refresh = [&]() {
+        if (stale) refresh_caches();
+        stale = false;
     };
     if (start) search_prologue(g, s, LOOP == kLoopDO);
     // Frontier bitmaps of a direction-optimizing loop (grid-uniform state):
@@ -2125,6 +2296,7 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
                 bar(false);
                 start = false;
             }
+            if (dir == kPhaseBottomUp) refresh();
             if (dir == kPhaseBottomUp && c.phase != kPhaseBottomUp) {
                 if (fbm_exact_step != c.step) {
                     if (fbm_dirty & (1u << (c.iteration & 1))) {
@@ -2189,8 +2361,9 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
                 // frontier kept in LDS between levels
                 if (blockIdx.x == 0) {
                     unsigned long long t0 = s.instrument ? wall_clock64() : 0;
-                    fast_lds_path<PRED, EXACT, FASTV>(g, s, c, n, loop, vsum, fe, shared.fast, lds_path && !first,
-                                                      bshape);
+                    refresh();
+                    fast_lds_path<PRED, EXACT, FASTV>(g, s, c, n, loop, vsum, fe, shared.fast, lds_path && !first);
+                    release_caches();
                     __syncthreads();
                     init_lds(lds);
                     if (s.instrument) busy += wall_clock64() - t0;
@@ -2198,12 +2371,13 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
             } else if (blockIdx.x == 0) {
                 unsigned long long t0 = s.instrument ? wall_clock64() : 0;
                 unsigned long long fv = vsum;  // sum through the step being run
+                refresh();
                 // (the step bodies grab every tile: see tile_grab)
                 if (threadIdx.x == 0) lds.solo = 1;
                 __syncthreads();
                 while (true) {
                     if (threadIdx.x == 0) prepare_step(s.ctl, c, n);
-                    loop_body<PRED, EXACT, LOOP>(c.phase, g, s, c, n, lds, 0, false);
+                    loop_body<PRED, EXACT, LOOP>(c.phase, g, s, c, n, lds, 0, false, 0ull, StepIo{false, false});
                     // the next level reads queue entries other waves just
                     // stored: each wave's stores must have completed, which
                     // __syncthreads() alone does not wait for
@@ -2227,9 +2401,10 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
                     __hip_atomic_store(&s.ctl->fast_vsum, fv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     lds.solo = 0;  // (the grid barrier below orders it)
                 }
+                release_caches();
                 if (s.instrument) busy += wall_clock64() - t0;
             }
-            bar(true);
+            bar(true);  // (block 0 alone wrote anything, and has written its L2 back)
             c.step = ld_agent(&s.ctl->fast_step);
             c.iteration = ld_agent(&s.ctl->fast_iteration);
             c.phase = ld_agent(&s.ctl->fast_phase);
@@ -2250,29 +2425,33 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
             fbm_exact_step = c.step + 1;
         }
         if (blockIdx.x == 0 && threadIdx.x == 0) prepare_step(s.ctl, c, n);
+        // (chained compaction keeps plain status words; it takes full barriers)
+        const bool light_step = EXACT && c.phase != kPhaseBottomUp && !mark && !from_bitmap && !s.tile_status &&
+                                (s.track_edges ? fe : (unsigned long long) n) <= kLightWork;
+        if (!light_step) refresh();
+        const StepIo io{light_step, stale};
         if (spread) {
             if constexpr (LOOP == kLoopEC || LOOP == kLoopDO) {
-                spread_step<PRED, EXACT>(g, s, c, n, shared.fast.f, next_bits);
+                spread_step<PRED, EXACT>(g, s, c, n, shared.fast.f, io, next_bits);
                 __syncthreads();
                 init_lds(lds);
             }
         } else if (mark) {
             body_expand_mark<PRED, EXACT>(g, s, c, n, lds, 0, true);
         } else {
-            loop_body<PRED, EXACT, LOOP>(c.phase, g, s, c, n, lds, 0, true, next_bits, from_bitmap);
+            loop_body<PRED, EXACT, LOOP>(c.phase, g, s, c, n, lds, 0, true, fe, io, next_bits, from_bitmap);
         }
         if (s.instrument) busy += wall_clock64() - t0;
-        // (light: a top-down or contract/expand step of at most
-        // kLightWork frontier edges, or items when edges are not tracked)
-        const bool light_step = c.phase != kPhaseBottomUp && !mark &&
-                                (s.track_edges ? fe : (unsigned long long) n) <= kLightWork;
         bar(light_step);
-        if (!spread && gathers(c.phase) && hubs_pending(s, c.step)) {
+        // (graphs whose longest row no step publishes have no list to look at)
+        if (!spread && gathers(c.phase) && s.max_degree >= min(s.grid_t, kHeavyRow) && hubs_pending(s, c.step)) {
             t0 = s.instrument ? wall_clock64() : 0;
+            refresh();  // (the list is read through the caches)
+            const StepIo io{light_step, false};
             if (mark) body_expand_mark<PRED, EXACT>(g, s, c, n, lds, 1, true);
-            else loop_body<PRED, EXACT, LOOP>(c.phase, g, s, c, n, lds, 1, true, next_bits, from_bitmap);
+            else loop_body<PRED, EXACT, LOOP>(c.phase, g, s, c, n, lds, 1, true, fe, io, next_bits, from_bitmap);
             if (s.instrument) busy += wall_clock64() - t0;
-            bar(false);
+            bar(light_step);
         }
         if (mark) {
             t0 = s.instrument ? wall_clock64() : 0;
@@ -2296,6 +2475,8 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
         s.ctl->exit_step = c.step;
         s.ctl->exit_iteration = c.iteration;
         s.ctl->exit_phase = c.phase;
+        // (agent-scope loads of the words this block stored plainly)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         if (s.host_head) publish_status(s);
     }
     if (s.instrument && threadIdx.x == 0) {
@@ -2309,12 +2490,14 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
 // Launches per step: the tile phase, then (for gathering phases) the hub
 // phase as its own launch.
 // ---------------------------------------------------------------------------
-template <bool PRED, bool EXACT, int PHASE>
-__global__ __launch_bounds__(kBlock) void step_kernel(GraphArgs g, SearchArgs s, Cursor c)
+
+// The step's input length n, or false when the launch has nothing to do
+// (grid-uniform: every workgroup sees the same counters).
+template <int PHASE>
+__device__ __forceinline__ bool step_begins(const SearchArgs &s, Cursor c, unsigned &n)
 {
-    __shared__ Lds<PRED> lds;
-    if (s.hybrid_steps && ld_agent(&s.ctl->hybrid_stop)) return;
-    unsigned n = frontier_length(s, c.step);
+    if (s.hybrid_steps && ld_agent(&s.ctl->hybrid_stop)) return false;
+    n = frontier_length(s, c.step);
     if (ld_agent(&s.ctl->overflow)) n = 0;
     if (PHASE == kPhaseContract && s.hybrid_steps && n > 0 && n <= (unsigned) s.sat_t) {
         // The filtered edge frontier fits the persistent kernel again: it
@@ -2325,12 +2508,28 @@ __global__ __launch_bounds__(kBlock) void step_kernel(GraphArgs g, SearchArgs s,
             s.ctl->exit_iteration = c.iteration;
             st_agent(&s.ctl->hybrid_stop, 1u);
         }
-        return;
+        return false;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) prepare_step(s.ctl, c, n);
+    return true;
+}
+
+template <bool PRED, bool EXACT, int PHASE>
+__global__ __launch_bounds__(kBlock) void step_kernel(GraphArgs g, SearchArgs s, Cursor c)
+{
+    __shared__ Lds<PRED> lds;
+    unsigned n;
+    if (!step_begins<PHASE>(s, c, n)) return;
+    // (the step's frontier edges; a bottom-up step's are read for the sum alone)
+    const unsigned long long fe = PHASE == kPhaseExpandContract || PHASE == kPhaseBottomUp
+                                      ? ld64_agent(&s.ctl->fedges[c.step % 3])
+                                      : 0ull;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        prepare_step(s.ctl, c, n);
+        s.ctl->visited_edges += fe;  // (the host's direction rule reads it)
+    }
     if (n == 0) return;
     init_lds(lds);
-    run_body<PRED, EXACT>(PHASE, g, s, c, n, lds, 0, true);
+    run_body<PRED, EXACT>(PHASE, g, s, c, n, lds, 0, true, fe);
 }
 
 template <bool PRED, bool EXACT, int PHASE>
@@ -2340,8 +2539,7 @@ __global__ __launch_bounds__(kBlock) void hub_kernel(GraphArgs g, SearchArgs s, 
     if (s.hybrid_steps && ld_agent(&s.ctl->hybrid_stop)) return;
     if (!hubs_pending(s, c.step)) return;
     init_lds(lds);
-    // the tile step's input length: it sets the chunk size of the list
-    run_body<PRED, EXACT>(PHASE, g, s, c, frontier_length(s, c.step), lds, 1, true);
+    run_body<PRED, EXACT>(PHASE, g, s, c, frontier_length(s, c.step), lds, 1, true, 0ull);
 }
 
 __global__ __launch_bounds__(kBlock) void frontier_bitmap_kernel(GraphArgs g, SearchArgs s, Cursor c, int pass)
@@ -2409,7 +2607,6 @@ __global__ void init_search_kernel(SearchArgs s, const int *row, int src, int la
             ctl->max_depth = 0;
             unsigned long long deg = (unsigned long long) (row[src + 1] - row[src]);
             ctl->fedges[0] = deg;
-            ctl->visited_edges = deg;
         }
     }
 }
