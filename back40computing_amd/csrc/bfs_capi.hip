@@ -105,6 +105,7 @@ struct bfs_problem {
     Control *h_ctl_dev = nullptr;  // its device-side address
     HubEntry *d_hubs = nullptr;  // two grid-tier lists of kHubCapacity entries
     unsigned *d_fbm = nullptr;   // two frontier bitmaps (bottom-up levels)
+    unsigned *d_slabs = nullptr;  // bit marks: one bitmap per workgroup (graphs of few vertices)
     unsigned char *d_marks = nullptr;  // discovery marks of large top-down levels (32 per visited word)
     int wall_khz = 100000;
     bfs_config cfg = kDefaults;
@@ -149,6 +150,8 @@ SearchArgs search_args(const bfs_problem *p, int grid)
     s.fbm[0] = p->d_fbm;
     s.fbm[1] = p->d_fbm + words;
     s.marks = p->d_marks;
+    s.slabs = p->d_slabs;
+    s.slab_count = p->num_cus;
     s.tile_status = p->cfg.compaction == 2 ? p->d_tile_status : nullptr;
     s.scan_epoch = p->scan_epoch;
     s.nodes = p->nodes;
@@ -456,6 +459,10 @@ bfs_status bfs_problem_create(const int32_t *h_row_offsets, const int32_t *h_col
         (e = hipMalloc(&p->d_fbm, sizeof(unsigned) * 2 * words)) != hipSuccess ||
         (e = hipMalloc(&p->d_marks, 32 * words)) != hipSuccess)
         return cleanup(hip_fail(e, "allocate problem"));
+    // (steps of kMarkEdges edges and more use them: smaller graphs have none)
+    if (nodes <= BFS_FAST_VISITED_MAX && edges >= (1 << 20) &&
+        (e = hipMalloc(&p->d_slabs, 16 * slab_quads(nodes) * (size_t) p->num_cus)) != hipSuccess)
+        return cleanup(hip_fail(e, "allocate bit-mark slabs"));
     // marks are clear between steps (each compaction clears what it reads)
     if ((e = hipMemset(p->d_marks, 0, 32 * words)) != hipSuccess) return cleanup(hip_fail(e, "clear marks"));
     if (p->mark_pred && (e = hipMalloc(&p->d_pred, sizeof(int) * (size_t) nodes)) != hipSuccess)
@@ -720,6 +727,7 @@ void bfs_problem_destroy(bfs_problem *p)
     if (p->d_hubs) (void) hipFree(p->d_hubs);
     if (p->d_fbm) (void) hipFree(p->d_fbm);
     if (p->d_marks) (void) hipFree(p->d_marks);
+    if (p->d_slabs) (void) hipFree(p->d_slabs);
     if (p->h_ctl) (void) hipHostFree(p->h_ctl);
     if (p->ev_start) (void) hipEventDestroy(p->ev_start);
     if (p->ev_stop) (void) hipEventDestroy(p->ev_stop);
@@ -735,6 +743,7 @@ bfs_status bfs_problem_device_info(const bfs_problem *p, int32_t *num_cus, int32
     if (device_bytes) {
         int64_t b = 4 * ((int64_t) p->nodes + 1) + 4 * p->edges + 4 * (int64_t) p->nodes * (p->mark_pred ? 2 : 1) +
                     (4 + 8 + 32) * (((int64_t) p->nodes + 31) / 32) + (int64_t) sizeof(Control) +
+                    (p->d_slabs ? 16 * (int64_t) slab_quads(p->nodes) * p->num_cus : 0) +
                     (int64_t) p->q_cap * 4 * 2 * (p->mark_pred ? 2 : 1);
         *device_bytes = b;
     }

@@ -41,6 +41,10 @@ struct SearchArgs {
     unsigned hub_cap;      // entries per list
     unsigned *fbm[2];      // frontier bitmaps of the bottom-up levels, by iteration & 1
     unsigned char *marks;  // [32 * ceil(V / 32)] discovery marks of large top-down levels, clear between steps
+    // Bit marks (graphs whose visited bitmap fits LDS; null otherwise): one
+    // bitmap of slab_quads(V) 16-byte units per workgroup of a persistent launch.
+    unsigned *slabs;
+    int slab_count;
     int nodes;
     unsigned long long total_edges;
     int track_edges;       // accumulate frontier edge counts (direction switching)
@@ -72,6 +76,15 @@ struct SearchArgs {
     // persistent launch when its level loop ends (null: none).
     Control *host_head;
 };
+
+// 16-byte units of a bit-mark slab of V vertices, an odd number of 256-byte
+// lines: every workgroup reads the same range of all slabs, and a stride of a
+// power of two would put those on a few memory channels.
+__host__ __device__ inline size_t slab_quads(int nodes)
+{
+    const size_t quads = ((size_t) nodes + 127) / 128;
+    return (((quads + 15) / 16) | 1) * 16;
+}
 
 // Loop position: step index (selects queues and counters), BFS iteration
 // (depth written by the next claim), and phase (two-phase cycle).

@@ -1839,6 +1839,355 @@ __device__ __forceinline__ void fast_lds_level(const GraphArgs &g, const SearchA
     fast_fold(F, dst, fe, labeled, dmax);
 }
 
+// ---------------------------------------------------------------------------
+// Bit marks: the large top-down and contraction steps of graphs whose
+// visited bitmap fits the workgroup's LDS (FASTV).  A workgroup sets the bits
+// of the targets of its share of the step's edges (or queue items) in an LDS
+// bitmap of all vertices, writes the bitmap to its slab in device memory, and
+// after a grid barrier every workgroup ORs its range of words over all the
+// slabs: new vertices are the bits not visited yet, and get their labels,
+// queue entries (in vertex order) and degree sums there, as in mark_compact.
+//
+// An LDS atomic costs a few cycles where a claim costs the device 1/27 ns and
+// a byte mark 1/84 ns, so the marking streams the columns; the price is the
+// slabs, V / 8 bytes per workgroup written and read once (64 MB at 2^20
+// vertices), past the L2 so that a light barrier orders them.
+// R-MAT scale 20, edge factor 16 (31 M edges): expand-contract 430 -> 313 us,
+// its 24.9 M-edge level 190 -> 135 us; a contraction of 5.1 M queued edges
+// 133 -> 25 us (hybrid 800 -> 650 us, contract-expand 1140 -> 600 us).
+// ---------------------------------------------------------------------------
+struct BitLds {
+    RowTable rt;
+    int list[64 * kWave];            // new vertices of 128 words
+    unsigned acc[2 * kWave];         // the words being collected
+    unsigned base;
+    int scan[kWaves];
+    unsigned long long wfe[kWaves];
+};
+static_assert(sizeof(BitLds) <= sizeof(FastFront), "the bitmap stays free of the step's other variables");
+
+// Whether a step of `work` edges or items takes bit marks (grid-uniform): the
+// rule of the byte marks, whose passes over V cost about as much.
+__device__ __forceinline__ bool bit_step(const SearchArgs &s, unsigned long long work)
+{
+    return s.slabs != nullptr && gridDim.x <= (unsigned) s.slab_count && s.nodes <= kFastVisitedWords * 32 &&
+           work >= kMarkEdges && work >= (unsigned long long) s.nodes / 2;
+}
+
+template <bool PRED, bool EXACT>
+__device__ __forceinline__ void bit_mark(const SearchArgs &s, unsigned *vbits, int u, int par)
+{
+    const unsigned bit = 1u << (u & 31);
+    if (PRED) {
+        // the workgroup's first edge to an unvisited vertex leaves its source
+        // (any of the level's sources is a valid parent)
+        const unsigned old =
+            __hip_atomic_fetch_or(vbits + (u >> 5), bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (!(old & bit) && !((s.visited[u >> 5] >> (u & 31)) & 1u) && (EXACT || s.depth[u] == -1)) s.pred[u] = par;
+    } else {
+        __hip_atomic_fetch_or(vbits + (u >> 5), bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+}
+
+__device__ __forceinline__ void bits_clear(const SearchArgs &s, unsigned *vbits)
+{
+    const int chunks = (s.nodes + 127) >> 7;
+    uint4 *p = reinterpret_cast<uint4 *>(vbits);
+    for (int i = threadIdx.x; i < chunks; i += kBlock) p[i] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+}
+static_assert(kFastVisitedWords % 4 == 0, "the bitmap is cleared 16 bytes at a time");
+
+// Marks the targets of the rows of the vertex frontier of step c.  Waves work
+// alone: wave w takes runs w, w + waves, ... of up to 64 queue entries (the
+// high-degree members, claimed first, are spread over all of them), and
+// nothing but the published rows waits for the workgroup.  Rows of
+// kBitWaveRow edges and more are read a row per load instruction, eight rows
+// in flight; shorter ones share load instructions through the wave's edge
+// offsets, four of them in flight.  Rows of kBitHubRow edges and more are
+// published: bits_from_hubs follows behind a grid barrier.
+// (A workgroup's row table, as gather_tile has it, left the waves in step:
+// 166 us for 437602 rows of 24.9 M edges, about 80 like this.)
+constexpr int kBitWaveRow = 32, kBitHubRow = 512;
+
+template <bool PRED, bool EXACT>
+__device__ __forceinline__ void bits_from_rows(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n,
+                                               BitLds &B, unsigned *vbits)
+{
+    const int *in = s.q[c.step & 1];
+    HubList hub = hub_list(s, c.step, true, n);
+    hub.grid_t = min(s.grid_t, kBitHubRow);
+    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    int *excl = B.rt.excl[wave], *rb = B.rt.beg[wave], *rp = B.rt.par[wave];
+    // runs of equal length, as many for every wave
+    const unsigned stride = gridDim.x * kWaves;
+    const unsigned rounds = (n + stride * kWave - 1) / (stride * kWave);
+    const unsigned width = (n + stride * rounds - 1) / (stride * rounds), runs = (n + width - 1) / width;
+    unsigned t = (unsigned) wave * gridDim.x + blockIdx.x;
+    auto member = [&](unsigned run) {
+        const unsigned long long i = (unsigned long long) run * width + (unsigned) lane;
+        return (unsigned) lane < width && i < n ? ld_queue(in + i) : -1;
+    };
+    int v_next = member(t), b_next = 0, e_next = 0;
+    if (v_next >= 0) {
+        b_next = g.row[v_next];
+        e_next = g.row[v_next + 1];
+    }
+    constexpr int U = 8;  // rows in flight
+    for (; t < runs; t += stride) {
+        const int v = v_next, beg = b_next;
+        int end = e_next;
+        v_next = member(t + stride);
+        if (publish_hub_row(beg, end, v, hub)) end = beg;
+        uint64_t wm = ballot(end - beg >= kBitWaveRow);
+        while (wm) {
+            int b[U], e[U], p[U], longest = 0;
+#pragma unroll
+            for (int q = 0; q < U; q++) {
+                const int l = wm ? uniform(__builtin_ctzll(wm)) : 0;
+                b[q] = readlane(beg, l);
+                e[q] = wm ? readlane(end, l) : b[q];
+                p[q] = readlane(v, l);
+                wm &= wm - 1;  // (0 stays 0)
+                longest = max(longest, e[q] - b[q]);
+            }
+            for (int k = lane; k - lane < longest; k += kWave) {
+                int u[U];
+#pragma unroll
+                for (int q = 0; q < U; q++) u[q] = k < e[q] - b[q] ? __builtin_nontemporal_load(g.col + b[q] + k) : -1;
+#pragma unroll
+                for (int q = 0; q < U; q++)
+                    if (u[q] >= 0) bit_mark<PRED, EXACT>(s, vbits, u[q], p[q]);
+            }
+        }
+        // the next run's row bounds, behind its members
+        b_next = e_next = 0;
+        if (v_next >= 0) {
+            b_next = g.row[v_next];
+            e_next = g.row[v_next + 1];
+        }
+        const int len = end - beg < kBitWaveRow ? end - beg : 0;
+        const int incl = wave_inclusive_sum(len);
+        const int total = readlane(incl, kWave - 1);
+        if (total == 0) continue;
+        excl[lane] = incl - len;
+        rb[lane] = beg - (incl - len);
+        rp[lane] = v;
+        wave_lds_sync();
+        for (int r = 0; r < total; r += 4 * kWave) {
+            int u[4], p[4], at[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) at[q] = 0;
+#pragma unroll
+            for (int st = 32; st > 0; st >>= 1) {
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (excl[at[q] + st] <= r + q * kWave + lane) at[q] += st;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int x = r + q * kWave + lane;
+                u[q] = x < total ? __builtin_nontemporal_load(g.col + rb[at[q]] + x) : -1;
+                p[q] = rp[at[q]];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (u[q] >= 0) bit_mark<PRED, EXACT>(s, vbits, u[q], p[q]);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// Index of the last grid-tier entry whose first chunk is <= ch, by the whole
+// wave: 64 probes at a time, so even a full list takes three dependent loads.
+__device__ __forceinline__ unsigned hub_entry_of_wave(const HubEntry *list, unsigned entries, unsigned ch)
+{
+    unsigned lo = 0, count = entries;
+    while (count > 1) {
+        const unsigned step = (count + kWave - 1) / kWave;
+        const unsigned at = (unsigned) lane_id() * step;
+        const uint64_t below = ballot(at < count && list[lo + at].first_chunk <= ch);
+        const unsigned k = (unsigned) __popcll(below) - 1u;  // (probe 0 is always below)
+        lo += k * step;
+        count = min(step, count - k * step);
+    }
+    return lo;
+}
+
+// The published rows, a wave per chunk.
+template <bool PRED, bool EXACT>
+__device__ __forceinline__ void bits_from_hubs(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned *vbits)
+{
+    const unsigned long long a = ld64_agent(&s.ctl->hub_alloc[c.step & 1]);
+    const unsigned entries = min((unsigned) (a >> 32), s.hub_cap);
+    if (entries == 0) return;
+    const HubEntry *list = s.hubs[c.step & 1];
+    const HubEntry last = list[entries - 1];
+    const unsigned total = last.first_chunk + (unsigned) ((last.end - last.beg + kHubChunk - 1) / kHubChunk);
+    for (unsigned ch = (threadIdx.x / kWave) * gridDim.x + blockIdx.x; ch < total; ch += gridDim.x * kWaves) {
+        const HubEntry e = list[hub_entry_of_wave(list, entries, (unsigned) uniform((int) ch))];
+        const int b = e.beg + (int) (ch - e.first_chunk) * kHubChunk;
+        const int end = min(e.end, b + kHubChunk);
+        constexpr int U = 8;
+        for (int k = b; k < end; k += U * kWave) {
+            int u[U];
+#pragma unroll
+            for (int j = 0; j < U; j++) {
+                const int x = k + j * kWave + lane_id();
+                u[j] = x < end ? __builtin_nontemporal_load(g.col + x) : -1;
+            }
+#pragma unroll
+            for (int j = 0; j < U; j++)
+                if (u[j] >= 0) bit_mark<PRED, EXACT>(s, vbits, u[j], e.par);
+        }
+    }
+}
+
+// Marks the items of the edge frontier of step c (with their parents).
+template <bool PRED, bool EXACT>
+__device__ __forceinline__ void bits_from_items(const SearchArgs &s, Cursor c, unsigned n, unsigned *vbits)
+{
+    const int *in = s.q[c.step & 1];
+    const int *pin = s.pq[c.step & 1];
+    constexpr unsigned U = 8;
+    for (unsigned long long base = blockIdx.x * (unsigned long long) (U * kBlock); base < n;
+         base += gridDim.x * (unsigned long long) (U * kBlock)) {
+        int u[U], p[U];
+#pragma unroll
+        for (unsigned j = 0; j < U; j++) {
+            const unsigned long long i = base + j * kBlock + threadIdx.x;
+            u[j] = i < n ? ld_queue(in + i) : -1;
+            p[j] = PRED && i < n ? ld_queue(pin + i) : -1;
+        }
+#pragma unroll
+        for (unsigned j = 0; j < U; j++)
+            if (u[j] >= 0) bit_mark<PRED, EXACT>(s, vbits, u[j], p[j]);
+    }
+}
+
+// Writes the bitmap to the workgroup's slab (a light barrier may follow).
+__device__ __forceinline__ void bits_dump(const SearchArgs &s, const unsigned *vbits)
+{
+    __syncthreads();
+    const int pairs = ((s.nodes + 127) >> 7) * 2;
+    const unsigned long long *from = reinterpret_cast<const unsigned long long *>(vbits);
+    unsigned long long *to =
+        reinterpret_cast<unsigned long long *>(s.slabs) + 2 * (size_t) blockIdx.x * slab_quads(s.nodes);
+    for (int i = threadIdx.x; i < pairs; i += kBlock)
+        __hip_atomic_store(to + i, from[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Collects the slabs behind a grid barrier and a refresh of the caches: new vertices get label `depth`,
+// a place in `out` (whose length is *out_len, overflow flags at step + 1)
+// and, with fbm_out, their bit in every word of that frontier bitmap; with
+// track their degrees are added to *fedges.  A full grid barrier must follow.
+template <bool EXACT>
+__device__ __forceinline__ void bits_collect(const GraphArgs &g, const SearchArgs &s, Cursor c, int depth, BitLds &B,
+                                             int *out, unsigned *out_len, unsigned *fbm_out, bool track)
+{
+    const int words = (s.nodes + 31) >> 5;
+    const int quads = (words + 3) >> 2;
+    const size_t stride = slab_quads(s.nodes);
+    const int per = (quads + (int) gridDim.x - 1) / (int) gridDim.x;
+    const int p0 = (int) blockIdx.x * per, p1 = min(quads, p0 + per);
+    const int tid = threadIdx.x;
+    unsigned fe = 0;
+    bool over = false;
+    __syncthreads();
+    for (int pb = p0; pb < p1; pb += kWave / 2) {
+        const int np = min(kWave / 2, p1 - pb);
+        if (tid < 2 * kWave) B.acc[tid] = 0u;
+        __syncthreads();
+        // P lanes (a power of two) cover the quads, the rest of the workgroup
+        // further slabs, sixteen loads a thread in flight
+        int lg = 0;
+        while ((1 << lg) < np) lg++;
+        const int lp = tid & ((1 << lg) - 1);
+        const int groups = kBlock >> lg;
+        if (lp < np) {
+            u32x4 a = {0u, 0u, 0u, 0u};
+            const u32x4 *from = reinterpret_cast<const u32x4 *>(s.slabs) + pb + lp;
+            const int count = (int) gridDim.x;
+            for (int sl = tid >> lg; sl < count; sl += 16 * groups) {
+                u32x4 v[16];
+#pragma unroll
+                for (int j = 0; j < 16; j++) {
+                    v[j] = u32x4{0u, 0u, 0u, 0u};
+                    if (sl + j * groups < count)
+                        v[j] = __builtin_nontemporal_load(from + (size_t) (sl + j * groups) * stride);
+                }
+#pragma unroll
+                for (int j = 0; j < 16; j++) a |= v[j];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (a[j]) atomicOr(&B.acc[4 * lp + j], a[j]);
+        }
+        __syncthreads();
+        const int w = 4 * pb + tid;
+        unsigned bits = 0;
+        if (tid < 4 * np && w < words) {
+            bits = B.acc[tid];
+            const unsigned vis = s.visited[w];
+            bits &= ~vis;
+            if (!EXACT) {
+                // best-effort levels may have lost bits of labelled vertices
+                for (unsigned b = bits; b; b &= b - 1) {
+                    const int v = (w << 5) + __builtin_ctz(b);
+                    if (s.depth[v] != -1) bits &= ~(1u << (v & 31));
+                }
+            }
+            if (bits) s.visited[w] = vis | bits;
+            if (fbm_out) fbm_out[w] = bits;
+        }
+        int total = 0;
+        int k = block_exclusive_sum(__popc(bits), B.scan, &total);
+        if (total == 0) continue;  // workgroup-uniform
+        if (tid == 0) B.base = add_agent(out_len, (unsigned) total);
+        for (unsigned b = bits; b; b &= b - 1) B.list[k++] = (w << 5) + __builtin_ctz(b);
+        __syncthreads();
+        const unsigned base = B.base;
+        for (int i0 = 0; i0 < total; i0 += 4 * kBlock) {
+            int v[4], r0[4], r1[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int i = i0 + j * kBlock + tid;
+                v[j] = i < total ? B.list[i] : -1;
+                r0[j] = v[j] >= 0 && track ? g.row[v[j]] : 0;
+                r1[j] = v[j] >= 0 && track ? g.row[v[j] + 1] : 0;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (v[j] < 0) continue;
+                s.depth[v[j]] = depth;
+                const unsigned pos = base + (unsigned) (i0 + j * kBlock + tid);
+                if (pos < s.cap) out[pos] = v[j];
+                else over = true;
+                fe += (unsigned) (r1[j] - r0[j]);
+            }
+        }
+        __syncthreads();  // the list and the words are used again
+    }
+    if (over) {
+        st_agent(&s.ctl->overflow, 1u);
+        st_agent(&s.ctl->ovf[(c.step + 1) % 3], 1u);
+    }
+    if (track) {
+        const int lo = wave_inclusive_sum((int) (fe & 0xFFFFu));
+        const int hi = wave_inclusive_sum((int) (fe >> 16));
+        if (lane_id() == kWave - 1)
+            B.wfe[tid / kWave] = ((unsigned long long) (unsigned) hi << 16) + (unsigned long long) (unsigned) lo;
+        __syncthreads();
+        if (tid == 0) {
+            unsigned long long f = 0;
+            for (int w = 0; w < kWaves; w++) f += B.wfe[w];
+            if (f)
+                __hip_atomic_fetch_add(&s.ctl->fedges[(c.step + 1) % 3], f, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+
 // Spread step: a top-down level of few members (n <= kFastCap) with more
 // edges than the fast path takes -- typically the first level after the
 // source, a handful of hubs.  The tile phase would hand each row to one
@@ -2326,6 +2675,12 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
         // edges over the grid
         const bool mark =
             (LOOP == kLoopEC || LOOP == kLoopDO) && c.phase == kPhaseExpandContract && marked_step(s, fe);
+        // large steps of graphs with an LDS bitmap take bit marks instead
+        // (contractions chained through tile status words keep their order)
+        const bool bits = FASTV && !fast &&
+                          ((LOOP == kLoopEC || LOOP == kLoopDO) ? mark && bit_step(s, fe)
+                           : LOOP == kLoopTP                     ? c.phase == kPhaseContract && !s.tile_status && bit_step(s, n)
+                                                                 : c.phase == kPhaseContractExpand && bit_step(s, n));
         const bool spread = (LOOP == kLoopEC || LOOP == kLoopDO) && c.phase == kPhaseExpandContract && !mark &&
                             n <= (unsigned) kFastCap && s.spread;
         // The first top-down step after bottom-up levels reads its frontier
@@ -2426,10 +2781,71 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
         }
         if (blockIdx.x == 0 && threadIdx.x == 0) prepare_step(s.ctl, c, n);
         // (chained compaction keeps plain status words; it takes full barriers)
-        const bool light_step = EXACT && c.phase != kPhaseBottomUp && !mark && !from_bitmap && !s.tile_status &&
+        const bool light_step = EXACT && c.phase != kPhaseBottomUp && !mark && !bits && !from_bitmap && !s.tile_status &&
                                 (s.track_edges ? fe : (unsigned long long) n) <= kLightWork;
         if (!light_step) refresh();
         const StepIo io{light_step, stale};
+        if (bits) {
+            if constexpr (FASTV) {
+                BitLds &B = *reinterpret_cast<BitLds *>(&shared.fast.f);
+                unsigned *vbits = shared.fast.vbits;
+                __syncthreads();
+                bits_clear(s, vbits);
+                if constexpr (LOOP == kLoopEC || LOOP == kLoopDO) {
+                    bits_from_rows<PRED, EXACT>(g, s, c, n, B, vbits);
+                    if (s.max_degree >= min(s.grid_t, kBitHubRow)) {
+                        bar(true);
+                        refresh();  // (the list is read through the caches)
+                        bits_from_hubs<PRED, EXACT>(g, s, c, vbits);
+                    }
+                } else {
+                    bits_from_items<PRED, EXACT>(s, c, n, vbits);
+                }
+                bits_dump(s, vbits);
+                if (s.instrument) busy += wall_clock64() - t0;
+                bar(true);
+                t0 = s.instrument ? wall_clock64() : 0;
+                unsigned *fbm_out = nullptr;
+                if (LOOP == kLoopDO) {
+                    fbm_out = s.fbm[(c.iteration + 1) & 1];
+                    fbm_dirty |= 1u << ((c.iteration + 1) & 1);
+                    fbm_exact_step = c.step + 1;
+                }
+                refresh();  // (visited words are read and written plainly)
+                if (LOOP == kLoopEC || LOOP == kLoopDO)
+                    bits_collect<EXACT>(g, s, c, c.iteration + 1, B, s.q[(c.step + 1) & 1],
+                                        &s.ctl->qlen[(c.step + 1) % 3], fbm_out, s.track_edges != 0);
+                else if (LOOP == kLoopTP)
+                    bits_collect<EXACT>(g, s, c, c.iteration, B, s.q[(c.step + 1) & 1],
+                                        &s.ctl->qlen[(c.step + 1) % 3], nullptr, false);
+                else  // (the input is spent: its queue takes the members)
+                    bits_collect<EXACT>(g, s, c, c.iteration, B, s.q[c.step & 1], &s.ctl->compact, nullptr, false);
+                __syncthreads();
+                init_lds(lds);
+                if (s.instrument) busy += wall_clock64() - t0;
+                bar(false);
+                if constexpr (LOOP == kLoopCE) {
+                    // the members expand into the next edge frontier
+                    const unsigned m = ld_agent(&s.ctl->compact);
+                    const StepIo xio{false, false};
+                    if (m > 0) {
+                        if (blockIdx.x == 0 && threadIdx.x == 0) atomicMax(&s.ctl->max_depth, c.iteration);
+                        t0 = s.instrument ? wall_clock64() : 0;
+                        body_expand<PRED, EXACT>(g, s, c, m, lds, 0, true, xio);
+                        if (s.instrument) busy += wall_clock64() - t0;
+                        bar(false);
+                        if (s.max_degree >= min(s.grid_t, kHeavyRow) && hubs_pending(s, c.step)) {
+                            t0 = s.instrument ? wall_clock64() : 0;
+                            body_expand<PRED, EXACT>(g, s, c, m, lds, 1, true, xio);
+                            if (s.instrument) busy += wall_clock64() - t0;
+                            bar(false);
+                        }
+                    }
+                }
+            }
+            c = advance(loop, c);
+            continue;
+        }
         if (spread) {
             if constexpr (LOOP == kLoopEC || LOOP == kLoopDO) {
                 spread_step<PRED, EXACT>(g, s, c, n, shared.fast.f, io, next_bits);
@@ -2540,6 +2956,36 @@ __global__ __launch_bounds__(kBlock) void hub_kernel(GraphArgs g, SearchArgs s, 
     if (!hubs_pending(s, c.step)) return;
     init_lds(lds);
     run_body<PRED, EXACT>(PHASE, g, s, c, frontier_length(s, c.step), lds, 1, true, 0ull);
+}
+
+// Contract steps of graphs with bit-mark slabs: large ones set bits here and
+// are collected by the launch that follows, on the same grid.
+template <bool PRED, bool EXACT>
+__global__ __launch_bounds__(kBlock) void contract_bits_kernel(GraphArgs g, SearchArgs s, Cursor c)
+{
+    __shared__ LoopLds<PRED, true> shared;
+    unsigned n;
+    if (!step_begins<kPhaseContract>(s, c, n)) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) prepare_step(s.ctl, c, n);
+    if (n == 0) return;
+    if (bit_step(s, n)) {
+        bits_clear(s, shared.fast.vbits);
+        bits_from_items<PRED, EXACT>(s, c, n, shared.fast.vbits);
+        bits_dump(s, shared.fast.vbits);
+    } else {
+        init_lds(shared.step);
+        body_contract<PRED, EXACT>(g, s, c, n, shared.step, StepIo{false, false});
+    }
+}
+
+template <bool EXACT>
+__global__ __launch_bounds__(kBlock) void contract_collect_kernel(GraphArgs g, SearchArgs s, Cursor c)
+{
+    __shared__ BitLds B;
+    if (s.hybrid_steps && ld_agent(&s.ctl->hybrid_stop)) return;
+    const unsigned n = ld_agent(&s.ctl->overflow) ? 0u : frontier_length(s, c.step);
+    if (n == 0 || !bit_step(s, n)) return;
+    bits_collect<EXACT>(g, s, c, c.iteration, B, s.q[(c.step + 1) & 1], &s.ctl->qlen[(c.step + 1) % 3], nullptr, false);
 }
 
 __global__ __launch_bounds__(kBlock) void frontier_bitmap_kernel(GraphArgs g, SearchArgs s, Cursor c, int pass)
@@ -2680,6 +3126,13 @@ bool uses_fast_visited(const SearchArgs &s) { return s.fast_visited && s.nodes <
 template <bool PRED, bool EXACT, int PHASE>
 hipError_t launch_phase(const GraphArgs &g, const SearchArgs &s, Cursor c, int grid, hipStream_t st, int *launches)
 {
+    if (PHASE == kPhaseContract && s.slabs && !s.tile_status) {
+        const int marking = std::min(grid, s.slab_count);
+        hipLaunchKernelGGL((contract_bits_kernel<PRED, EXACT>), dim3(marking), dim3(kBlock), 0, st, g, s, c);
+        hipLaunchKernelGGL((contract_collect_kernel<EXACT>), dim3(marking), dim3(kBlock), 0, st, g, s, c);
+        *launches += 2;
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL((step_kernel<PRED, EXACT, PHASE>), dim3(grid), dim3(kBlock), 0, st, g, s, c);
     (*launches)++;
     if (PHASE == kPhaseExpandContract || PHASE == kPhaseContractExpand || PHASE == kPhaseExpand) {
