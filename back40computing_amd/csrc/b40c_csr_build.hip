@@ -5,7 +5,7 @@
 // the COO tuples by row (b40c/graph/csr_graph.cuh:108-152), after builders
 // and file readers produced them (b40c/graph/builder/*.cuh).  Here the
 // tuples become 64-bit keys (row << b | column, b = bits of V - 1) that an
-// LSD radix sort orders on the device (8-bit digits, 2b bits in all: a
+// LSD radix sort orders on the device (digits of up to 9 bits, 2b bits in all: a
 // per-tile digit histogram, one chained scan of the digit-major count matrix,
 // then a stable scatter ranked by wave ballots); duplicates are dropped by a
 // chained stream compaction; row offsets are written at the row boundaries
@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <mutex>
 #include <vector>
 
 using namespace b40c_hip;
@@ -34,44 +35,51 @@ constexpr int kWaves = kThreads / prim::kWave;
 constexpr int kRounds = 16;                          // keys per lane
 constexpr int kTile = kThreads * kRounds;            // 4096 keys per tile
 constexpr int kWaveKeys = prim::kWave * kRounds;     // 1024 contiguous keys per wave
-constexpr int kDigits = 256;
+constexpr int kDigitBits = 9;                        // most bits per sorting pass
+constexpr int kDigits = 1 << kDigitBits;
 
-__device__ __forceinline__ unsigned digit_of(unsigned long long key, int shift)
+__device__ __forceinline__ unsigned digit_of(unsigned long long key, int shift, int bits)
 {
-    return (unsigned) (key >> shift) & (kDigits - 1);
+    return (unsigned) (key >> shift) & ((1u << bits) - 1u);
 }
 
 // Per-tile digit counts, digit-major: counts[d * tiles + tile].
 __global__ __launch_bounds__(kThreads) void sort_upsweep_kernel(const unsigned long long *keys, long long n, int shift,
-                                                                unsigned *counts, long long tiles)
+                                                                int bits, unsigned *counts, long long tiles)
 {
     __shared__ unsigned hist[kDigits];
-    hist[threadIdx.x] = 0u;
+    const int digits = 1 << bits;
+    for (int d = threadIdx.x; d < digits; d += kThreads) hist[d] = 0u;
     __syncthreads();
     const long long tile = blockIdx.x;
     const int wave = threadIdx.x / prim::kWave, lane = prim::lane();
     const long long base = tile * kTile + (long long) wave * kWaveKeys + lane;
-#pragma unroll 4
+    unsigned long long key[kRounds];
+#pragma unroll
     for (int r = 0; r < kRounds; r++) {
         const long long i = base + (long long) r * prim::kWave;
-        if (i < n) atomicAdd(&hist[digit_of(keys[i], shift)], 1u);
+        key[r] = i < n ? keys[i] : 0ull;
     }
+#pragma unroll
+    for (int r = 0; r < kRounds; r++)
+        if (base + (long long) r * prim::kWave < n) atomicAdd(&hist[digit_of(key[r], shift, bits)], 1u);
     __syncthreads();
-    counts[(long long) threadIdx.x * tiles + tile] = hist[threadIdx.x];
+    for (int d = threadIdx.x; d < digits; d += kThreads) counts[(long long) d * tiles + tile] = hist[d];
 }
 
 // Stable scatter by digit.  Wave w of a tile owns keys [w * 1024, (w + 1) *
 // 1024) of the tile and walks them in 16 rounds of 64; a key's slot is its
 // digit's scanned offset for this tile, plus the keys of that digit in the
 // tile's lower waves, plus those earlier in its own wave (ballot match of
-// the eight digit bits).
+// the digit bits).
 __global__ __launch_bounds__(kThreads) void sort_downsweep_kernel(const unsigned long long *keys_in,
                                                                   unsigned long long *keys_out, long long n, int shift,
-                                                                  const unsigned *offsets, long long tiles)
+                                                                  int bits, const unsigned *offsets, long long tiles)
 {
     __shared__ unsigned base_of[kWaves][kDigits];
-    unsigned *flat = &base_of[0][0];
-    for (int i = threadIdx.x; i < kWaves * kDigits; i += kThreads) flat[i] = 0u;
+    const int digits = 1 << bits;
+    for (int d = threadIdx.x; d < digits; d += kThreads)
+        for (int w = 0; w < kWaves; w++) base_of[w][d] = 0u;
     __syncthreads();
     const long long tile = blockIdx.x;
     const int wave = threadIdx.x / prim::kWave, lane = prim::lane();
@@ -81,15 +89,17 @@ __global__ __launch_bounds__(kThreads) void sort_downsweep_kernel(const unsigned
     for (int r = 0; r < kRounds; r++) {
         const long long i = base + (long long) r * prim::kWave;
         key[r] = i < n ? keys_in[i] : 0ull;
-        if (i < n) atomicAdd(&base_of[wave][digit_of(key[r], shift)], 1u);
     }
+#pragma unroll
+    for (int r = 0; r < kRounds; r++)
+        if (base + (long long) r * prim::kWave < n) atomicAdd(&base_of[wave][digit_of(key[r], shift, bits)], 1u);
     __syncthreads();
-    {
-        // thread = digit: this tile's offset, then the lower waves' counts
-        unsigned run = offsets[(long long) threadIdx.x * tiles + tile];
+    for (int d = threadIdx.x; d < digits; d += kThreads) {
+        // this tile's offset, then the lower waves' counts
+        unsigned run = offsets[(long long) d * tiles + tile];
         for (int w = 0; w < kWaves; w++) {
-            const unsigned c = base_of[w][threadIdx.x];
-            base_of[w][threadIdx.x] = run;
+            const unsigned c = base_of[w][d];
+            base_of[w][d] = run;
             run += c;
         }
     }
@@ -99,10 +109,10 @@ __global__ __launch_bounds__(kThreads) void sort_downsweep_kernel(const unsigned
     for (int r = 0; r < kRounds; r++) {
         const long long i = base + (long long) r * prim::kWave;
         const bool valid = i < n;
-        const unsigned d = digit_of(key[r], shift);
+        const unsigned d = digit_of(key[r], shift, bits);
         uint64_t peers = __ballot(valid);
 #pragma unroll
-        for (int b = 0; b < 8; b++) {
+        for (int b = 0; b < kDigitBits; b++) {  // (bits past the digit's are clear in all)
             const bool bit = (d >> b) & 1u;
             const uint64_t m = __ballot(valid && bit);
             peers &= bit ? m : ~m;
@@ -118,24 +128,35 @@ __global__ __launch_bounds__(kThreads) void sort_downsweep_kernel(const unsigned
     }
 }
 
+// What a keys kernel counts; read back before the sort.
+struct KeyCounts {
+    unsigned long long loops;  // keys dropped
+    unsigned outside;          // pairs with an end outside the graph
+    unsigned pad;
+};
+
 // Keys of (src, dst) pairs; with symmetrize also (dst, src); self-loops to
-// drop become the loop key (2^b - 1, 2^b - 1) and are counted in *loops.
-__global__ __launch_bounds__(kThreads) void pair_keys_kernel(const int *src, const int *dst, long long pairs, int bits,
-                                                             int symmetrize, int drop_loops,
-                                                             unsigned long long *keys, unsigned long long *loops)
+// drop become the loop key (2^b - 1, 2^b - 1) and are counted.  Pairs with
+// an end outside [0, nodes) are counted too (the caller rejects the list).
+__global__ __launch_bounds__(kThreads) void pair_keys_kernel(const int *src, const int *dst, long long pairs, int nodes,
+                                                             int bits, int symmetrize, int drop_loops,
+                                                             unsigned long long *keys, KeyCounts *counts)
 {
+    unsigned outside = 0;
     const unsigned long long loop_key = ((1ull << bits) - 1ull) << bits | ((1ull << bits) - 1ull);
     unsigned long long dropped = 0;
     for (long long i = blockIdx.x * (long long) kThreads + threadIdx.x; i < pairs;
          i += (long long) gridDim.x * kThreads) {
         const unsigned long long u = (unsigned) src[i], v = (unsigned) dst[i];
+        if (u >= (unsigned) nodes || v >= (unsigned) nodes) outside++;
         const bool drop = drop_loops && u == v;
         const long long at = symmetrize ? 2 * i : i;
         keys[at] = drop ? loop_key : (u << bits) | v;
         if (symmetrize) keys[at + 1] = drop ? loop_key : (v << bits) | u;
         if (drop) dropped += symmetrize ? 2 : 1;
     }
-    if (dropped) atomicAdd(loops, dropped);
+    if (dropped) atomicAdd(&counts->loops, dropped);
+    if (outside) atomicAdd(&counts->outside, outside);
 }
 
 // SplitMix64 (Steele, Lea, Flood, OOPSLA 2014) and the counter-based stream of
@@ -190,31 +211,51 @@ __global__ __launch_bounds__(kThreads) void rmat_keys_kernel(long long samples, 
 }
 
 // Chained stable compaction of sorted keys: keeps key i when it differs from
-// key i - 1 (consecutive duplicates collapse to the first).
+// key i - 1 (consecutive duplicates collapse to the first).  Wave w of a tile
+// owns 1024 consecutive keys and walks them in rounds of 64, so every load
+// and store instruction covers consecutive keys (sixteen consecutive keys a
+// thread made 8 M keys 100 us; 49 us now).
 __global__ __launch_bounds__(kThreads) void unique_kernel(const unsigned long long *in, unsigned long long *out,
                                                           long long n, ChainArgs c, unsigned *d_count)
 {
     __shared__ long long s_tile;
     __shared__ unsigned s_wave[kWaves], s_prefix;
     const long long tile = prim::take_tile(c, &s_tile);
-    const long long base = tile * kTile + (long long) threadIdx.x * kRounds;
+    const int wave = threadIdx.x / prim::kWave, lane = prim::lane();
+    const long long base = tile * kTile + (long long) wave * kWaveKeys;
     unsigned long long v[kRounds];
-    unsigned long long prev = base > 0 && base - 1 < n ? in[base - 1] : 0ull;
-    unsigned keep = 0;
 #pragma unroll
-    for (int k = 0; k < kRounds; k++) {
-        const long long i = base + k;
-        v[k] = i < n ? in[i] : 0ull;
-        if (i < n && (i == 0 || v[k] != prev)) keep |= 1u << k;
-        prev = v[k];
+    for (int r = 0; r < kRounds; r++) {
+        const long long i = base + r * prim::kWave + lane;
+        v[r] = i < n ? in[i] : 0ull;
     }
-    unsigned agg;
-    const unsigned before = prim::block_exclusive_sum_u32<kThreads>((unsigned) __popc(keep), s_wave, &agg);
-    const unsigned prefix = prim::chain_prefix(c, tile, agg, &s_prefix);
-    unsigned at = prefix + before;
+    unsigned long long before = base > 0 && base <= n ? in[base - 1] : 0ull;  // the key before the round's first
+    uint64_t keep[kRounds];
+    unsigned run = 0;
 #pragma unroll
-    for (int k = 0; k < kRounds; k++)
-        if ((keep >> k) & 1u) out[at++] = v[k];
+    for (int r = 0; r < kRounds; r++) {
+        const long long i = base + r * prim::kWave + lane;
+        unsigned long long prev = __shfl_up(v[r], 1);
+        if (lane == 0) prev = before;
+        keep[r] = __ballot(i < n && (i == 0 || v[r] != prev));
+        run += (unsigned) __popcll(keep[r]);
+        before = __shfl(v[r], prim::kWave - 1);
+    }
+    if (lane == 0) s_wave[wave] = run;
+    __syncthreads();
+    unsigned off = 0, agg = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) {
+        if (w < wave) off += s_wave[w];
+        agg += s_wave[w];
+    }
+    const unsigned prefix = prim::chain_prefix(c, tile, agg, &s_prefix);
+    unsigned at = prefix + off;
+#pragma unroll
+    for (int r = 0; r < kRounds; r++) {
+        if ((keep[r] >> lane) & 1u) out[at + (unsigned) prim::lanes_below(keep[r])] = v[r];
+        at += (unsigned) __popcll(keep[r]);
+    }
     if (tile == c.tiles - 1 && threadIdx.x == 0) *d_count = prefix + agg;
 }
 
@@ -243,22 +284,67 @@ __global__ __launch_bounds__(kThreads) void fill_int_kernel(int *p, long long n,
         p[i] = value;
 }
 
-// (column, row) keys of every edge of a CSR: the transpose's tuples.  Each
-// edge finds its row by a binary search of the row offsets.
+// Last u in [0, nodes) with row[u] <= e.
+__device__ __forceinline__ int row_of_edge(const int *row, int nodes, long long e)
+{
+    int lo = 0, hi = nodes - 1;
+    while (lo < hi) {
+        const int mid = lo + (hi - lo + 1) / 2;
+        if ((long long) row[mid] <= e) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+// (column, row) keys of every edge of a CSR: the transpose's tuples.  A tile
+// of 4096 edges finds its first and last row by two searches; the rows
+// starting inside it leave their numbers at their first edges in LDS (the
+// last of several starting at one edge is the one with edges), and a running
+// maximum hands every edge its row.  (A search per edge, 20 dependent loads,
+// made 16 M edges 249 us; 55 now.)
 __global__ __launch_bounds__(kThreads) void transpose_keys_kernel(const int *row, const int *col, int nodes,
                                                                   long long edges, int bits,
                                                                   unsigned long long *keys)
 {
-    for (long long e = blockIdx.x * (long long) kThreads + threadIdx.x; e < edges;
-         e += (long long) gridDim.x * kThreads) {
-        int lo = 0, hi = nodes - 1;  // last u with row[u] <= e
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if ((long long) row[mid] <= e) lo = mid;
-            else hi = mid - 1;
-        }
-        keys[e] = ((unsigned long long) (unsigned) col[e] << bits) | (unsigned) lo;
+    __shared__ int s_row[kTile];
+    __shared__ int s_wave[kWaves], s_first, s_last;
+    const long long e0 = (long long) blockIdx.x * kTile;
+    const int count = (int) (edges - e0 < (long long) kTile ? edges - e0 : (long long) kTile);
+    for (int i = threadIdx.x; i < kTile; i += kThreads) s_row[i] = 0;
+    if (threadIdx.x == 0) s_first = row_of_edge(row, nodes, e0);
+    if (threadIdx.x == prim::kWave) s_last = row_of_edge(row, nodes, e0 + count - 1);
+    __syncthreads();
+    const int first = s_first, last = s_last;
+    for (int u = first + 1 + (int) threadIdx.x; u <= last; u += kThreads) {
+        const int at = (int) ((long long) row[u] - e0);
+        if (at >= 0 && at < count) atomicMax(&s_row[at], u);
     }
+    __syncthreads();
+    // running maximum: sixteen consecutive edges a thread, then the threads before it
+    int r[kRounds], top = 0;
+#pragma unroll
+    for (int k = 0; k < kRounds; k++) {
+        top = max(top, s_row[threadIdx.x * kRounds + k]);
+        r[k] = top;
+    }
+    int incl = top;
+#pragma unroll
+    for (int d = 1; d < prim::kWave; d <<= 1) {
+        const int below = __shfl_up(incl, d);
+        if (prim::lane() >= d) incl = max(incl, below);
+    }
+    const int wave = threadIdx.x / prim::kWave;
+    if (prim::lane() == prim::kWave - 1) s_wave[wave] = incl;
+    int before = __shfl_up(incl, 1);
+    if (prim::lane() == 0) before = 0;
+    __syncthreads();
+    before = max(before, first);
+    for (int w = 0; w < wave; w++) before = max(before, s_wave[w]);
+#pragma unroll
+    for (int k = 0; k < kRounds; k++) s_row[threadIdx.x * kRounds + k] = max(r[k], before);
+    __syncthreads();
+    for (int i = threadIdx.x; i < count; i += kThreads)
+        keys[e0 + i] = ((unsigned long long) (unsigned) col[e0 + i] << bits) | (unsigned) s_row[i];
 }
 
 unsigned grid_for(long long n)
@@ -273,12 +359,73 @@ int bits_for(int nodes)
     return b;
 }
 
-// Device storage and stream of one build.
-struct Builder {
-    int device = 0;
+// What a build needs besides its result -- a stream, events, chain state and
+// one block of device memory -- is kept per device between builds: allocating
+// and freeing 260 MB took longer than transposing 16 M edges (1.3 ms of 2.7,
+// on some boxes 8 of 9.5).  One build at a time has the kept set; others at
+// the same time make their own.  The block stays below kKeepBytes, and goes
+// back to the device when the last device CSR built here is freed.
+constexpr size_t kKeepBytes = (size_t) 512 << 20;
+constexpr int kKeepDevices = 64;
+
+struct BuildSet {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     ChainState chain;
+    char *block = nullptr;
+    size_t bytes = 0;
+    bool busy = false;
+
+    hipError_t make(int device)
+    {
+        if (stream) return hipSuccess;
+        hipError_t e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking);
+        if (e == hipSuccess) e = hipEventCreate(&ev0);
+        if (e == hipSuccess) e = hipEventCreate(&ev1);
+        if (e == hipSuccess) e = chain.init(device);
+        if (e != hipSuccess) drop();
+        return e;
+    }
+    hipError_t reserve(size_t need)
+    {
+        if (need <= bytes) return hipSuccess;
+        release_block();
+        hipError_t e = hipMalloc(reinterpret_cast<void **>(&block), need);
+        if (e != hipSuccess) {
+            block = nullptr;
+            return e;
+        }
+        bytes = need;
+        return hipSuccess;
+    }
+    void release_block()
+    {
+        if (block) (void) hipFree(block);
+        block = nullptr;
+        bytes = 0;
+    }
+    void drop()
+    {
+        if (stream) (void) hipStreamSynchronize(stream);
+        release_block();
+        chain.release();
+        if (ev0) (void) hipEventDestroy(ev0);
+        if (ev1) (void) hipEventDestroy(ev1);
+        if (stream) (void) hipStreamDestroy(stream);
+        ev0 = ev1 = nullptr;
+        stream = nullptr;
+    }
+};
+
+std::mutex g_keep_mu;
+BuildSet g_keep[kKeepDevices];
+int64_t g_live[kKeepDevices];  // device CSRs built and not yet freed
+
+// One build: the kept set of its device, or a set of its own.
+struct Builder {
+    int device = 0;
+    BuildSet own, *set = nullptr;
+    hipStream_t stream = nullptr;
     unsigned long long *keys[2] = {nullptr, nullptr};
     unsigned *counts = nullptr;
     int *perm = nullptr;
@@ -287,17 +434,15 @@ struct Builder {
 
     ~Builder()
     {
+        if (!set) return;
         if (stream) (void) hipStreamSynchronize(stream);
-        for (auto *k : keys)
-            if (k) (void) hipFree(k);
-        if (counts) (void) hipFree(counts);
-        if (perm) (void) hipFree(perm);
-        if (src) (void) hipFree(src);
-        if (dst) (void) hipFree(dst);
-        chain.release();
-        if (ev0) (void) hipEventDestroy(ev0);
-        if (ev1) (void) hipEventDestroy(ev1);
-        if (stream) (void) hipStreamDestroy(stream);
+        if (set == &own) {
+            own.drop();
+            return;
+        }
+        std::lock_guard<std::mutex> lock(g_keep_mu);
+        if (set->bytes > kKeepBytes || g_live[device] == 0) set->release_block();
+        set->busy = false;
     }
 
     bool ok(hipError_t e)
@@ -310,40 +455,74 @@ struct Builder {
     bool start(int dev)
     {
         device = dev;
-        return ok(hipSetDevice(dev)) && ok(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking)) &&
-               ok(hipEventCreate(&ev0)) && ok(hipEventCreate(&ev1)) && ok(chain.init(dev)) &&
-               ok(hipEventRecord(ev0, stream));
+        if (!ok(hipSetDevice(dev))) return false;
+        set = &own;
+        if (dev < kKeepDevices) {
+            std::lock_guard<std::mutex> lock(g_keep_mu);
+            if (!g_keep[dev].busy) {
+                set = &g_keep[dev];
+                set->busy = true;
+            }
+        }
+        if (!ok(set->make(dev))) return false;
+        stream = set->stream;
+        return ok(hipEventRecord(set->ev0, stream));
     }
 
-    bool alloc_keys(long long n)
+    // Device memory of a build over n keys: the keys twice, the digit counts,
+    // the vertex permutation (perm_n) and the pairs (pairs_n), 256-byte aligned.
+    bool alloc(long long n, long long perm_n, long long pairs_n)
     {
-        const size_t b = sizeof(unsigned long long) * (size_t) std::max(1LL, n);
-        return ok(hipMalloc(&keys[0], b)) && ok(hipMalloc(&keys[1], b));
+        auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+        const size_t kb = up(sizeof(unsigned long long) * (size_t) std::max(1LL, n));
+        const size_t tiles = ((size_t) std::max(1LL, n) + kTile - 1) / kTile;
+        const size_t cb = up(sizeof(unsigned) * tiles * kDigits);
+        const size_t pb = up(sizeof(int) * (size_t) perm_n), qb = up(sizeof(int) * (size_t) pairs_n);
+        if (!ok(set->reserve(2 * kb + cb + pb + 2 * qb))) return false;
+        char *at = set->block;
+        keys[0] = reinterpret_cast<unsigned long long *>(at);
+        keys[1] = reinterpret_cast<unsigned long long *>(at + kb);
+        counts = reinterpret_cast<unsigned *>(at + 2 * kb);
+        perm = reinterpret_cast<int *>(at + 2 * kb + cb);
+        src = reinterpret_cast<int *>(at + 2 * kb + cb + pb);
+        dst = reinterpret_cast<int *>(at + 2 * kb + cb + pb + qb);
+        return true;
     }
 
-    // LSD radix sort of keys[0][0, n) over bits [0, key_bits); the result
-    // is in keys[0].
-    bool sort(long long n, int key_bits)
+    KeyCounts *key_counts() const { return reinterpret_cast<KeyCounts *>(set->chain.d_word); }
+
+    bool read_key_counts(KeyCounts *c)
+    {
+        return ok(hipMemcpyAsync(c, key_counts(), sizeof(*c), hipMemcpyDeviceToHost, stream)) &&
+               ok(hipStreamSynchronize(stream));
+    }
+
+    // LSD radix sort of keys[0][0, n) over bits [low_bit, key_bits); the result
+    // is in keys[0].  Every pass takes the same number of bits, at most 8.
+    bool sort(long long n, int key_bits, int low_bit = 0)
     {
         if (n <= 1) return true;
         const long long tiles = (n + kTile - 1) / kTile;
-        if (!ok(hipMalloc(&counts, sizeof(unsigned) * (size_t) (tiles * kDigits)))) return false;
+        // as few passes as kDigitBits allow, then digits as narrow as those
+        // passes allow: fewer digits leave longer runs per tile to write
+        const int passes = std::max(1, (key_bits - low_bit + kDigitBits - 1) / kDigitBits);
         int cur = 0;
-        for (int shift = 0; shift < key_bits; shift += 8) {
+        for (int p = 0, shift = low_bit; p < passes; p++) {
+            const int bits = (key_bits - shift + (passes - p) - 1) / (passes - p);
+            const long long counts_n = tiles << bits;
             hipLaunchKernelGGL(sort_upsweep_kernel, dim3((unsigned) tiles), dim3(kThreads), 0, stream, keys[cur], n,
-                               shift, counts, tiles);
+                               shift, bits, counts, tiles);
             if (!ok(hipGetLastError())) return false;
             ChainArgs c;
-            if (!ok(chain.prepare(tiles * kDigits, scan_tile_items(tiles * kDigits), &c, stream))) return false;
-            if (!ok(launch_scan_u32(counts, counts, tiles * kDigits, true, c, nullptr, stream))) return false;
+            if (!ok(set->chain.prepare(counts_n, scan_tile_items(counts_n), &c, stream))) return false;
+            if (!ok(launch_scan_u32(counts, counts, counts_n, true, c, nullptr, stream))) return false;
             hipLaunchKernelGGL(sort_downsweep_kernel, dim3((unsigned) tiles), dim3(kThreads), 0, stream, keys[cur],
-                               keys[cur ^ 1], n, shift, counts, tiles);
+                               keys[cur ^ 1], n, shift, bits, counts, tiles);
             if (!ok(hipGetLastError())) return false;
             cur ^= 1;
+            shift += bits;
         }
         if (cur == 1) std::swap(keys[0], keys[1]);
-        (void) hipFree(counts);
-        counts = nullptr;
         return true;
     }
 
@@ -354,12 +533,12 @@ struct Builder {
         long long m = n - loops;
         if (dedup && m > 0) {
             ChainArgs c;
-            if (!ok(chain.prepare(m, kTile, &c, stream))) return false;
+            if (!ok(set->chain.prepare(m, kTile, &c, stream))) return false;
             hipLaunchKernelGGL(unique_kernel, dim3((unsigned) c.tiles), dim3(kThreads), 0, stream, keys[0], keys[1],
-                               m, c, chain.d_word);
+                               m, c, set->chain.d_word);
             if (!ok(hipGetLastError())) return false;
             unsigned k = 0;
-            if (!ok(hipMemcpyAsync(&k, chain.d_word, sizeof(unsigned), hipMemcpyDeviceToHost, stream)) ||
+            if (!ok(hipMemcpyAsync(&k, set->chain.d_word, sizeof(unsigned), hipMemcpyDeviceToHost, stream)) ||
                 !ok(hipStreamSynchronize(stream)))
                 return false;
             m = k;
@@ -386,8 +565,8 @@ struct Builder {
         else hipLaunchKernelGGL(csr_from_keys_kernel, dim3(grid_for(edges)), dim3(kThreads), 0, stream, keys[0],
                                 edges, bits, nodes, row, col);
         float ms = 0.f;
-        if (!ok(hipGetLastError()) || !ok(hipEventRecord(ev1, stream)) || !ok(hipEventSynchronize(ev1)) ||
-            !ok(hipEventElapsedTime(&ms, ev0, ev1))) {
+        if (!ok(hipGetLastError()) || !ok(hipEventRecord(set->ev1, stream)) || !ok(hipEventSynchronize(set->ev1)) ||
+            !ok(hipEventElapsedTime(&ms, set->ev0, set->ev1))) {
             (void) hipFree(row);
             (void) hipFree(col);
             return false;
@@ -399,6 +578,10 @@ struct Builder {
         out->column_indices = col;
         out->symmetric = symmetric ? 1 : 0;
         out->build_ms = ms;
+        if (device < kKeepDevices) {
+            std::lock_guard<std::mutex> lock(g_keep_mu);
+            g_live[device]++;
+        }
         return true;
     }
 };
@@ -410,7 +593,22 @@ int device_ok(int32_t device)
     return device >= 0 && device < count ? 0 : 1;
 }
 
+bool pairs_inside(const int32_t *src, const int32_t *dst, int64_t pairs, int32_t nodes)
+{
+    for (int64_t i = 0; i < pairs; i++)
+        if (src[i] < 0 || src[i] >= nodes || dst[i] < 0 || dst[i] >= nodes) return false;
+    return true;
+}
+
 }  // namespace
+
+void device_csr_gone(int device)
+{
+    if (device < 0 || device >= kKeepDevices) return;
+    std::lock_guard<std::mutex> lock(g_keep_mu);
+    if (g_live[device] > 0 && --g_live[device] == 0 && !g_keep[device].busy) g_keep[device].release_block();
+}
+
 }  // namespace b40c_hip
 
 extern "C" {
@@ -421,32 +619,28 @@ int b40c_device_csr_from_coo(int32_t device, int32_t nodes, int64_t num_pairs, c
 {
     if (!out || nodes <= 0 || num_pairs < 0 || (num_pairs > 0 && (!h_src || !h_dst))) return 1;
     *out = b40c_device_csr{};
-    for (int64_t i = 0; i < num_pairs; i++)
-        if (h_src[i] < 0 || h_src[i] >= nodes || h_dst[i] < 0 || h_dst[i] >= nodes) return 1;
     const long long n = (symmetrize ? 2 : 1) * (long long) num_pairs;
-    if (n > (long long) UINT32_MAX) return 3;  // sort offsets are 32-bit
-    if (int rc = device_ok(device)) return rc;
+    // the device checks the pairs; where it does not get to see them, they
+    // are checked here (an invalid pair is the first error reported)
+    const int rc = n > (long long) UINT32_MAX ? 3 : device_ok(device);  // (sort offsets are 32-bit)
+    if (rc) return pairs_inside(h_src, h_dst, num_pairs, nodes) ? rc : 1;
     Builder b;
     if (!b.start(device)) return b.status;
     const int bits = bits_for(nodes);
     long long edges = 0;
     if (n > 0) {
-        unsigned long long *d_loops = reinterpret_cast<unsigned long long *>(b.chain.d_word);  // 8-byte aligned
-        unsigned long long loops = 0;
         const size_t pb = sizeof(int) * (size_t) num_pairs;
-        if (!b.alloc_keys(n) || !b.ok(hipMalloc(&b.src, pb)) || !b.ok(hipMalloc(&b.dst, pb)) ||
-            !b.ok(hipMemcpyAsync(b.src, h_src, pb, hipMemcpyHostToDevice, b.stream)) ||
+        KeyCounts kc;
+        if (!b.alloc(n, 0, num_pairs) || !b.ok(hipMemcpyAsync(b.src, h_src, pb, hipMemcpyHostToDevice, b.stream)) ||
             !b.ok(hipMemcpyAsync(b.dst, h_dst, pb, hipMemcpyHostToDevice, b.stream)) ||
-            !b.ok(hipMemsetAsync(d_loops, 0, sizeof(unsigned long long), b.stream)))
+            !b.ok(hipMemsetAsync(b.key_counts(), 0, sizeof(KeyCounts), b.stream)))
             return b.status;
         hipLaunchKernelGGL(pair_keys_kernel, dim3(grid_for(num_pairs)), dim3(kThreads), 0, b.stream, b.src, b.dst,
-                           (long long) num_pairs, bits, symmetrize ? 1 : 0, drop_self_loops ? 1 : 0, b.keys[0],
-                           d_loops);
-        if (!b.ok(hipGetLastError()) ||
-            !b.ok(hipMemcpyAsync(&loops, d_loops, sizeof(loops), hipMemcpyDeviceToHost, b.stream)) ||
-            !b.ok(hipStreamSynchronize(b.stream)))
-            return b.status;
-        if (!b.sort(n, 2 * bits) || !b.compact(n, (long long) loops, dedup != 0, &edges)) return b.status;
+                           (long long) num_pairs, nodes, bits, symmetrize ? 1 : 0, drop_self_loops ? 1 : 0, b.keys[0],
+                           b.key_counts());
+        if (!b.ok(hipGetLastError()) || !b.read_key_counts(&kc)) return b.status;
+        if (kc.outside) return 1;
+        if (!b.sort(n, 2 * bits) || !b.compact(n, (long long) kc.loops, dedup != 0, &edges)) return b.status;
     }
     if (!b.finish(nodes, edges, bits, symmetrize != 0, out)) return b.status ? b.status : 4;
     return 0;
@@ -471,23 +665,20 @@ int b40c_device_csr_rmat(int32_t device, int32_t scale, int32_t edge_factor, dou
     if (!bld.start(device)) return bld.status;
     const int bits = scale;
     const long long n = 2 * samples;
-    unsigned long long *d_loops = reinterpret_cast<unsigned long long *>(bld.chain.d_word);
-    unsigned long long loops = 0;
-    if (!bld.alloc_keys(n) || !bld.ok(hipMemsetAsync(d_loops, 0, sizeof(unsigned long long), bld.stream)))
+    KeyCounts kc;
+    if (!bld.alloc(n, scramble ? nodes : 0, 0) ||
+        !bld.ok(hipMemsetAsync(bld.key_counts(), 0, sizeof(KeyCounts), bld.stream)))
         return bld.status;
-    if (scramble && (!bld.ok(hipMalloc(&bld.perm, sizeof(int) * (size_t) nodes)) ||
-                     !bld.ok(hipMemcpyAsync(bld.perm, perm.data(), sizeof(int) * (size_t) nodes,
-                                            hipMemcpyHostToDevice, bld.stream))))
+    if (scramble && !bld.ok(hipMemcpyAsync(bld.perm, perm.data(), sizeof(int) * (size_t) nodes,
+                                           hipMemcpyHostToDevice, bld.stream)))
         return bld.status;
     hipLaunchKernelGGL(rmat_keys_kernel, dim3(grid_for(samples)), dim3(kThreads), 0, bld.stream, samples, scale,
                        (unsigned long long) seed, (unsigned long long) t_a, (unsigned long long) t_ab,
-                       (unsigned long long) t_abc, bld.perm, bits, bld.keys[0], d_loops);
-    if (!bld.ok(hipGetLastError()) ||
-        !bld.ok(hipMemcpyAsync(&loops, d_loops, sizeof(loops), hipMemcpyDeviceToHost, bld.stream)) ||
-        !bld.ok(hipStreamSynchronize(bld.stream)))
-        return bld.status;
+                       (unsigned long long) t_abc, scramble ? bld.perm : nullptr, bits, bld.keys[0],
+                       &bld.key_counts()->loops);
+    if (!bld.ok(hipGetLastError()) || !bld.read_key_counts(&kc)) return bld.status;
     long long edges = 0;
-    if (!bld.sort(n, 2 * bits) || !bld.compact(n, (long long) loops, true, &edges)) return bld.status;
+    if (!bld.sort(n, 2 * bits) || !bld.compact(n, (long long) kc.loops, true, &edges)) return bld.status;
     if (!bld.finish(nodes, edges, bits, true, out)) return bld.status ? bld.status : 4;
     return 0;
 }
@@ -502,10 +693,12 @@ int b40c_device_csr_transpose(const b40c_device_csr *g, b40c_device_csr *out)
     const int bits = bits_for(g->nodes);
     const long long n = g->edges;
     if (n > 0) {
-        if (!b.alloc_keys(n)) return b.status;
-        hipLaunchKernelGGL(transpose_keys_kernel, dim3(grid_for(n)), dim3(kThreads), 0, b.stream, g->row_offsets,
-                           g->column_indices, g->nodes, n, bits, b.keys[0]);
-        if (!b.ok(hipGetLastError()) || !b.sort(n, 2 * bits)) return b.status;
+        if (!b.alloc(n, 0, 0)) return b.status;
+        hipLaunchKernelGGL(transpose_keys_kernel, dim3((unsigned) ((n + kTile - 1) / kTile)), dim3(kThreads), 0,
+                           b.stream, g->row_offsets, g->column_indices, g->nodes, n, bits, b.keys[0]);
+        // the tuples come in row order, and the passes are stable: sorting by
+        // the column leaves every column's rows in order
+        if (!b.ok(hipGetLastError()) || !b.sort(n, 2 * bits, bits)) return b.status;
     }
     if (!b.finish(g->nodes, n, bits, g->symmetric != 0, out)) return b.status ? b.status : 4;
     return 0;
@@ -537,6 +730,7 @@ void b40c_device_csr_free(b40c_device_csr *g)
 {
     if (!g) return;
     if (g->row_offsets || g->column_indices) (void) hipSetDevice(g->device);
+    if (g->row_offsets) device_csr_gone(g->device);
     if (g->row_offsets) (void) hipFree(g->row_offsets);
     if (g->column_indices) (void) hipFree(g->column_indices);
     g->row_offsets = g->column_indices = nullptr;

@@ -16,6 +16,7 @@
 #include "bfs_batch.hpp"
 #include "bfs_batch_internal.hpp"
 #include "bfs_internal.hpp"
+#include "graph_builder_internal.hpp"
 
 #include <algorithm>
 #include <chrono>
@@ -372,6 +373,7 @@ bfs_status bfs_pool_add_device_graph(bfs_graph_pool *p, const b40c_device_csr *d
         if (b40c_device_csr_transpose(dg, &t) != 0) return host_fail(BFS_ERR_OOM, "device transpose failed");
         g.rrow = t.row_offsets;
         g.rcol = t.column_indices;
+        device_csr_gone(t.device);
         p->bytes += (int64_t) (rb + cb);
     }
     p->graphs.push_back(g);
