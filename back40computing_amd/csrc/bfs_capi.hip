@@ -66,6 +66,7 @@ const bfs_config kDefaults = {
     /*compaction*/ 1,
     /*fast_visited*/ 1};
 
+constexpr long long kWorkPerWorkgroup = 2048;
 constexpr unsigned kHubCapacity = 1u << 16;  // grid-tier entries per step list
 
 }  // namespace
@@ -106,6 +107,8 @@ struct bfs_problem {
     HubEntry *d_hubs = nullptr;  // two grid-tier lists of kHubCapacity entries
     unsigned *d_fbm = nullptr;   // two frontier bitmaps (bottom-up levels)
     unsigned *d_slabs = nullptr;  // bit marks: one bitmap per workgroup (graphs of few vertices)
+    unsigned *d_adj = nullptr;             // adjacency records (low-degree graphs), adj_width words each
+    int adj_width = 0;
     unsigned char *d_marks = nullptr;  // discovery marks of large top-down levels (32 per visited word)
     int wall_khz = 100000;
     bfs_config cfg = kDefaults;
@@ -152,6 +155,8 @@ SearchArgs search_args(const bfs_problem *p, int grid)
     s.marks = p->d_marks;
     s.slabs = p->d_slabs;
     s.slab_count = p->num_cus;
+    s.adj = p->d_adj;
+    s.adj_width = p->adj_width;
     s.tile_status = p->cfg.compaction == 2 ? p->d_tile_status : nullptr;
     s.scan_epoch = p->scan_epoch;
     s.nodes = p->nodes;
@@ -480,6 +485,15 @@ bfs_status bfs_problem_create(const int32_t *h_row_offsets, const int32_t *h_col
         (e = hipMemcpy(p->d_col, h_column_indices, sizeof(int) * (size_t) edges, hipMemcpyHostToDevice)) != hipSuccess)
         return cleanup(hip_fail(e, "copy column indices"));
 
+    p->adj_width = adjacency_width(nodes, p->max_degree);
+    if (p->adj_width) {
+        if ((e = hipMalloc(&p->d_adj, sizeof(unsigned) * (size_t) p->adj_width * (size_t) nodes)) != hipSuccess)
+            return cleanup(hip_fail(e, "allocate adjacency records"));
+        if ((e = launch_adjacency(p->d_row, p->d_col, nodes, p->adj_width, p->d_adj, p->stream)) != hipSuccess ||
+            (e = hipStreamSynchronize(p->stream)) != hipSuccess)
+            return cleanup(hip_fail(e, "write adjacency records"));
+    }
+
     // Bottom-up levels scan in-neighbours: reuse the CSR when the graph is
     // symmetric, otherwise upload its transpose.
     p->symmetric = csr_is_symmetric(h_row_offsets, h_column_indices, nodes);
@@ -596,6 +610,12 @@ bfs_status bfs_enact(bfs_problem *p, bfs_strategy strategy, int32_t fused, int32
     int pgrid = persistent_grid(p, loop, max_grid_size);
     if (pgrid > p->num_cus * std::max(1, persistent_max_blocks_per_cu(loop, p->mark_pred, exact)))
         return fail(BFS_ERR_LAUNCH, "grid exceeds co-resident capacity");
+    // A small graph meets at cheaper barriers on fewer workgroups: one per
+    // kWorkPerWorkgroup vertices and edges, about one round of a gathering
+    // step's workgroup, and never fewer than eight (R-MAT scale 10: 15
+    // workgroups 70 us a launch, 256 of them 86).
+    if (max_grid_size <= 0)
+        pgrid = (int) std::min<long long>(pgrid, std::max<long long>(8, (p->nodes + p->edges) / kWorkPerWorkgroup));
     int sgrid = step_grid(p, max_grid_size);
     GraphArgs g{p->d_row, p->d_col, p->nodes, p->d_rrow, p->d_rcol};
     // Chained compaction tags each step's tile words with scan_epoch + step.
@@ -728,6 +748,7 @@ void bfs_problem_destroy(bfs_problem *p)
     if (p->d_fbm) (void) hipFree(p->d_fbm);
     if (p->d_marks) (void) hipFree(p->d_marks);
     if (p->d_slabs) (void) hipFree(p->d_slabs);
+    if (p->d_adj) (void) hipFree(p->d_adj);
     if (p->h_ctl) (void) hipHostFree(p->h_ctl);
     if (p->ev_start) (void) hipEventDestroy(p->ev_start);
     if (p->ev_stop) (void) hipEventDestroy(p->ev_stop);
@@ -744,6 +765,7 @@ bfs_status bfs_problem_device_info(const bfs_problem *p, int32_t *num_cus, int32
         int64_t b = 4 * ((int64_t) p->nodes + 1) + 4 * p->edges + 4 * (int64_t) p->nodes * (p->mark_pred ? 2 : 1) +
                     (4 + 8 + 32) * (((int64_t) p->nodes + 31) / 32) + (int64_t) sizeof(Control) +
                     (p->d_slabs ? 16 * (int64_t) slab_quads(p->nodes) * p->num_cus : 0) +
+                    4 * (int64_t) p->adj_width * p->nodes +
                     (int64_t) p->q_cap * 4 * 2 * (p->mark_pred ? 2 : 1);
         *device_bytes = b;
     }

@@ -45,6 +45,10 @@ struct SearchArgs {
     // bitmap of slab_quads(V) 16-byte units per workgroup of a persistent launch.
     unsigned *slabs;
     int slab_count;
+    // Adjacency records of low-degree graphs (null: none), adj_width (4 or 8)
+    // words per vertex.
+    const unsigned *adj;
+    int adj_width;
     int nodes;
     unsigned long long total_edges;
     int track_edges;       // accumulate frontier edge counts (direction switching)
@@ -106,6 +110,9 @@ hipError_t launch_init_search(const SearchArgs &s, const int *row, int src, int 
 hipError_t launch_build_frontier_bitmap(const SearchArgs &s, Cursor c, int grid, hipStream_t st, int *launches);
 // Bitmap fbm[c.iteration & 1] -> input queue of step c (bottom-up -> top-down).
 hipError_t launch_queue_from_bitmap(const SearchArgs &s, Cursor c, int grid, hipStream_t st, int *launches);
+// Words per adjacency record of a graph (0: none), and their construction.
+int adjacency_width(int nodes, int max_degree);
+hipError_t launch_adjacency(const int *row, const int *col, int nodes, int width, unsigned *adj, hipStream_t st);
 hipError_t launch_reset_labels(int *depth, int *pred, unsigned *visited, int nodes, hipStream_t st);
 // One step as a kernel launch; gathering phases are followed by the
 // grid-tier launch for rows published to the hub list.

@@ -2275,6 +2275,112 @@ __device__ __forceinline__ void spread_step(const GraphArgs &g, const SearchArgs
     }
 }
 
+// ---------------------------------------------------------------------------
+// Adjacency records of low-degree graphs (lattices, road networks): every
+// vertex's neighbours in one aligned record of 4 or 8 words, each the
+// neighbour's number and, above it, that neighbour's degree (all ones: none),
+// written once when the problem is created.  A level of the LDS path then
+// costs one memory trip -- the members' records -- where it took two (column
+// entries, then the claimed vertices' row bounds): the claims are LDS
+// atomics, and a claimed vertex comes with its degree.  Bound: that trip, the
+// one CU's line requests on wide levels, and one workgroup barrier; grid2d
+// 1000^2 (1999 levels) 6.8 -> 4.0 ms, a level of tens of members 1.9 -> 1.6 us
+// and of a thousand 5 -> 2.4.
+// ---------------------------------------------------------------------------
+constexpr int kAdjDegreeShift = 24;                 // vertices below 2^24, degrees up to 8
+constexpr int kAdjMaxDegree = 8;
+constexpr unsigned kAdjNone = ~0u;
+static_assert(kFastVisitedWords * 32 <= (1 << kAdjDegreeShift), "a record holds the vertex number");
+constexpr int kAdjCap = 3 * kFastCap;               // members kept in LDS: the frontier buffers hold numbers only
+static_assert(2 * kAdjCap * sizeof(int) <= offsetof(FastFront, maxdeg), "two buffers fit the frontier arrays");
+
+__global__ void adjacency_kernel(const int *row, const int *col, int nodes, int width, unsigned *adj)
+{
+    const long long count = (long long) nodes * width;
+    for (long long i = blockIdx.x * (long long) blockDim.x + threadIdx.x; i < count;
+         i += (long long) gridDim.x * blockDim.x) {
+        const int v = (int) (i / width), e = row[v] + (int) (i % width);
+        unsigned x = kAdjNone;
+        if (e < row[v + 1]) {
+            const int u = col[e];
+            x = (unsigned) u | (unsigned) (row[u + 1] - row[u]) << kAdjDegreeShift;
+        }
+        adj[i] = x;
+    }
+}
+
+// One level: the n members of src claim their neighbours (LDS bitmap vbits),
+// label them, and append them to dst (past kAdjCap to the global queue
+// `spill`).  *count and *edges, zero before, get the new members and their
+// degree sum; a workgroup barrier must follow.  Every thread calls it.
+template <bool PRED, int W>
+__device__ __forceinline__ void adjacency_level(const SearchArgs &s, int next_depth, unsigned n, const int *src,
+                                                int *dst, int *spill, unsigned *vbits, unsigned *count,
+                                                unsigned *edges)
+{
+    constexpr int M = 8 / W;  // members per thread and round
+    const unsigned wave0 = threadIdx.x & ~(unsigned) (kWave - 1);
+    // (waves past the members skip the round together)
+    for (unsigned base = 0; base + wave0 < n; base += M * kBlock) {
+        int v[M];
+        u32x4 a[M][W / 4];
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            const unsigned i = base + (unsigned) (m * kBlock) + threadIdx.x;
+            v[m] = i < n ? src[i] : -1;
+        }
+#pragma unroll
+        for (int m = 0; m < M; m++)
+#pragma unroll
+            for (int q = 0; q < W / 4; q++) {
+                a[m][q] = u32x4{kAdjNone, kAdjNone, kAdjNone, kAdjNone};
+                if (v[m] >= 0)
+                    a[m][q] = *reinterpret_cast<const u32x4 *>(s.adj + (size_t) v[m] * W + 4 * q);
+            }
+        unsigned old[8], fresh = 0;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const unsigned x = a[k / W][(k % W) / 4][k % 4], u = x & ((1u << kAdjDegreeShift) - 1u);
+            old[k] = ~0u;
+            if (x != kAdjNone)
+                old[k] = __hip_atomic_fetch_or(vbits + (u >> 5), 1u << (u & 31u), __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        // (all claims are issued before the first result is used)
+#pragma unroll
+        for (int k = 0; k < 8; k++) asm volatile("" : "+v"(old[k]));
+        int fe = 0;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const unsigned x = a[k / W][(k % W) / 4][k % 4], u = x & ((1u << kAdjDegreeShift) - 1u);
+            if (!((old[k] >> (u & 31u)) & 1u)) {
+                fresh |= 1u << k;
+                fe += (int) (x >> kAdjDegreeShift);
+                s.depth[u] = next_depth;
+                if (PRED) s.pred[u] = v[k / W];
+            }
+        }
+        const int cnt = __popc(fresh);
+        const int incl = wave_inclusive_sum(cnt | fe << 16);  // (at most 512 and 4096 a wave)
+        const int tot = readlane(incl, kWave - 1);
+        if ((tot & 0xFFFF) == 0) continue;
+        unsigned at = 0;
+        if (lane_id() == 0) {
+            at = atomicAdd(count, (unsigned) (tot & 0xFFFF));
+            atomicAdd(edges, (unsigned) (tot >> 16));
+        }
+        unsigned p = (unsigned) readlane((int) at, 0) + (unsigned) ((incl & 0xFFFF) - cnt);
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            if (!((fresh >> k) & 1u)) continue;
+            const int u = (int) (a[k / W][(k % W) / 4][k % 4] & ((1u << kAdjDegreeShift) - 1u));
+            if (p < (unsigned) kAdjCap) dst[p] = u;
+            else if (p < s.cap) spill[p] = u;
+            p++;
+        }
+    }
+}
+
 // Runs LDS fast levels from step c (input: n <= kFastCap members in the
 // global queue) until a level's output is empty, too large for the path, or
 // (direction-optimizing) calls for bottom-up.  Leaves the global queue,
@@ -2382,7 +2488,64 @@ __device__ __forceinline__ void fast_lds_path(const GraphArgs &g, const SearchAr
         }
         __syncthreads();
     }
-    while (n > 0) {
+    // Adjacency levels (see above): members' numbers only, in two buffers over
+    // the frontier arrays; one workgroup barrier a level, with three sets of
+    // counters (a level's set was last read before the level before it).
+    const bool adjacent = EXACT && FASTV && !tp && ldsv && s.adj != nullptr;
+    int *abuf = &F.v[0][0];
+    unsigned *acount = reinterpret_cast<unsigned *>(F.scan), *aedges = reinterpret_cast<unsigned *>(F.wmax);
+    int acur = 0;
+    if (adjacent) {
+        __syncthreads();
+        if (threadIdx.x < 3) {
+            acount[threadIdx.x] = 0u;
+            aedges[threadIdx.x] = 0u;
+        }
+        __syncthreads();
+        const unsigned most = (unsigned) min((long long) kAdjCap, 3ll * s.fast_t);
+        int set = 0;
+        while (n > 0) {
+            const int logged = c.step + (ce ? 1 : 0);
+            const unsigned long long step_input = ce ? fe2 : n;
+            if (threadIdx.x == 0 && logged < kLevelLog) {
+                s.ctl->level_len[logged] = (unsigned) step_input;
+                s.ctl->level_clock[logged] = wall_clock64();
+            }
+            queued += step_input;
+            const int after = set == 2 ? 0 : set + 1;
+            if (threadIdx.x == 0) {
+                acount[after] = 0u;
+                aedges[after] = 0u;
+            }
+            const int *from = abuf + acur * kAdjCap;
+            int *to = abuf + (acur ^ 1) * kAdjCap;
+            if (s.adj_width == 4)
+                adjacency_level<PRED, 4>(s, c.iteration + 1, n, from, to, s.q[(c.step + 1) & 1], L.vbits,
+                                         acount + set, aedges + set);
+            else
+                adjacency_level<PRED, 8>(s, c.iteration + 1, n, from, to, s.q[(c.step + 1) & 1], L.vbits,
+                                         acount + set, aedges + set);
+            __syncthreads();
+            n2 = acount[set];
+            fe2 = aedges[set];
+            if (n2 > 0) maxd = c.iteration + 1;
+            acur ^= 1;
+            set = after;
+            c = advance(loop, c);
+            bool go = n2 > 0 && n2 <= most;
+            if (go && loop == kLoopDO) {
+                const unsigned long long fv2 = fv + fe2;
+                if (direction_rule(s, c.phase, fe2, n2, fv2, cur_fe) != c.phase) go = false;
+                else fv = fv2;
+            }
+            prev_fe = cur_fe;
+            cur_fe = fe2;
+            if (go && ce && s.sat_t >= 0 && fe2 > (unsigned long long) s.sat_t) go = false;
+            n = n2;
+            if (!go) break;
+        }
+    }
+    while (!adjacent && n > 0) {
         // Two-phase counts a contraction's input -- every edge the filter
         // passes, i.e. every edge to a vertex the level claims -- which
         // direct levels count; the grid takes the others.
@@ -2456,9 +2619,10 @@ __device__ __forceinline__ void fast_lds_path(const GraphArgs &g, const SearchAr
     }
     // The next step (c) reads its input from the global queue: copy the
     // LDS-resident members (those past kFastCap were written there already).
-    const unsigned held = min(n2, (unsigned) kFastCap);
+    const unsigned held = min(n2, (unsigned) (adjacent ? kAdjCap : kFastCap));
+    const int *members = adjacent ? abuf + acur * kAdjCap : F.v[src];
     int *q = s.q[c.step & 1];
-    for (unsigned i = threadIdx.x; i < held && i < s.cap; i += kBlock) q[i] = F.v[src][i];
+    for (unsigned i = threadIdx.x; i < held && i < s.cap; i += kBlock) q[i] = members[i];
     if (threadIdx.x == 0) {
         Control *ctl = s.ctl;
         // what the previous step's prepare_step would have left for step c
@@ -3158,6 +3322,20 @@ hipError_t launch_step_t(int phase, const GraphArgs &g, const SearchArgs &s, Cur
 }
 
 }  // namespace
+
+int adjacency_width(int nodes, int max_degree)
+{
+    if (nodes > kFastVisitedWords * 32 || max_degree < 1 || max_degree > kAdjMaxDegree) return 0;
+    return max_degree <= 4 ? 4 : 8;
+}
+
+hipError_t launch_adjacency(const int *row, const int *col, int nodes, int width, unsigned *adj, hipStream_t st)
+{
+    const long long count = (long long) nodes * width;
+    const int grid = (int) std::min<long long>(16384, (count + 255) / 256);
+    hipLaunchKernelGGL(adjacency_kernel, dim3(grid), dim3(256), 0, st, row, col, nodes, width, adj);
+    return hipGetLastError();
+}
 
 hipError_t launch_reset_labels(int *depth, int *pred, unsigned *visited, int nodes, hipStream_t st)
 {
