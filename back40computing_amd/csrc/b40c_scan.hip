@@ -289,6 +289,46 @@ hipError_t noalloc_scratch(int device, unsigned long long **out)
 }  // namespace
 
 // ---------------------------------------------------------------------------
+// Pinned host words for enactors' totals, handed out from one page that the
+// process keeps (pinning memory for every enactor took 55 us of its creation);
+// past the page's words an enactor pins its own.
+// ---------------------------------------------------------------------------
+namespace {
+
+constexpr int kPinnedWords = 1024;
+std::mutex g_word_mu;
+uint32_t *g_word_page = nullptr;
+bool g_word_used[kPinnedWords];
+
+hipError_t take_pinned_word(uint32_t **word)
+{
+    std::lock_guard<std::mutex> lock(g_word_mu);
+    if (!g_word_page) {
+        hipError_t e = hipHostMalloc(&g_word_page, kPinnedWords * sizeof(uint32_t), hipHostMallocPortable);
+        if (e != hipSuccess) {
+            g_word_page = nullptr;
+            return e;
+        }
+    }
+    for (int i = 0; i < kPinnedWords; i++) {
+        if (g_word_used[i]) continue;
+        g_word_used[i] = true;
+        *word = g_word_page + i;
+        return hipSuccess;
+    }
+    return hipHostMalloc(word, sizeof(uint32_t), hipHostMallocPortable);
+}
+
+void give_pinned_word(uint32_t *word)
+{
+    std::lock_guard<std::mutex> lock(g_word_mu);
+    if (g_word_page && word >= g_word_page && word < g_word_page + kPinnedWords) g_word_used[word - g_word_page] = false;
+    else (void) hipHostFree(word);
+}
+
+}  // namespace
+
+// ---------------------------------------------------------------------------
 // Chain state: the tile counter and the per-tile status words.
 // ---------------------------------------------------------------------------
 hipError_t ChainState::init(int dev)
@@ -386,7 +426,7 @@ bfs_status b40c_scan_enactor_create(int32_t device, b40c_scan_enactor **out)
     if ((e = hipStreamCreateWithFlags(&en->stream, hipStreamNonBlocking)) != hipSuccess ||
         (e = hipEventCreate(&en->ev0)) != hipSuccess || (e = hipEventCreate(&en->ev1)) != hipSuccess ||
         (e = en->chain.init(device)) != hipSuccess ||
-        (e = hipHostMalloc(&en->h_word, sizeof(uint32_t), hipHostMallocDefault)) != hipSuccess ||
+        (e = take_pinned_word(&en->h_word)) != hipSuccess ||
         (e = hipHostGetDevicePointer(reinterpret_cast<void **>(&en->h_word_dev), en->h_word, 0)) != hipSuccess) {
         b40c_scan_enactor_destroy(en);
         return host_hip_fail(e, "create scan enactor");
@@ -401,7 +441,7 @@ void b40c_scan_enactor_destroy(b40c_scan_enactor *e)
     (void) hipSetDevice(e->device);
     if (e->stream) (void) hipStreamSynchronize(e->stream);
     e->chain.release();
-    if (e->h_word) (void) hipHostFree(e->h_word);
+    if (e->h_word) give_pinned_word(e->h_word);
     if (e->ev0) (void) hipEventDestroy(e->ev0);
     if (e->ev1) (void) hipEventDestroy(e->ev1);
     if (e->stream) (void) hipStreamDestroy(e->stream);
