@@ -39,9 +39,6 @@ TABLE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned.jso
 SPACE_SINGLE = {
     "blocks_per_cu": [1, 2],
     "tile_grab_max": [1, 4, 16, 32, 64],
-    "wave_gather_threshold": [32, 64, 128],
-    # rows shorter than a 512-thread workgroup waste most of it in the CTA tier
-    "cta_gather_threshold": [256, 512, 1024],
     "grid_gather_threshold": [2048, 4096, 8192, 32768, -1],
     "do_alpha": [2, 4, 8, 14, 24],
     "do_beta": [8, 16, 24, 48],
@@ -55,8 +52,6 @@ SPACE_LATTICE = {
     "blocks_per_cu": [1, 2],
     "fast_path_threshold": [256, 512, 1024],
     "tile_grab_max": [1, 4, 16, 32],
-    "wave_gather_threshold": [8, 32, 64],
-    "cta_gather_threshold": [256, 512, 1024],
     "compaction": [1, 2],
     "fast_visited": [1, 2],
 }
@@ -67,9 +62,7 @@ SPACE_BATCH = {
     # an upper bound: each level shrinks it to give every workgroup tiles
     "bu_tile_blocks": [16, 64, 256],
     "grab_strided": [1, 2],
-    "wave_gather_threshold": [32, 64, 128],
-    "cta_gather_threshold": [256, 512, 1024],
-    "grid_gather_threshold": [256, 512, 1024, 4096],
+    "grid_gather_threshold": [1024, 2048, 4096],
     "do_alpha": [4, 8, 12],
     "do_beta": [8, 24, 48],
 }

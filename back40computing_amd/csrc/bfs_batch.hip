@@ -162,8 +162,6 @@ struct SlotTable {
         a.slots = d_slots;
         a.ctl = d_ctl;
         a.nslots = nslots;
-        a.wave_t = cfg.wave_gather_threshold;
-        a.cta_t = cfg.cta_gather_threshold;
         a.direction = direction;
         a.do_alpha = cfg.do_alpha;
         a.do_beta = cfg.do_beta;

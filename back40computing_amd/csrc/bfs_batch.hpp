@@ -8,6 +8,10 @@
 namespace b40c_hip {
 
 constexpr int kMaxSlots = 256;  // queries advanced by one launch
+// Groups of workgroups with a tile counter of their own: 512 workgroups on
+// one counter waited about 5 us for each tile (its atomics serialise, some
+// 10 ns each).
+constexpr int kTileGroups = 8;
 
 struct BatchGraph {
     const int *row, *col;    // CSR
@@ -30,7 +34,7 @@ struct alignas(128) BatchSlot {
     unsigned cap;             // queue capacity (elements)
     unsigned qlen[3];
     unsigned long long fedges[3];
-    unsigned long long visited_edges;
+    unsigned long long pad;
     unsigned long long t_begin, t_end;  // wall clock at seeding / completion
     unsigned ovf[3];          // per-step overflow of the output queue, by step % 3
     int bits;                 // fbm[iteration & 1] holds exactly the current frontier
@@ -38,15 +42,16 @@ struct alignas(128) BatchSlot {
 };
 
 struct alignas(256) BatchControl {
-    unsigned steal[2];        // tile counters by level parity
+    unsigned pad2[2];
     int level;                // levels completed by the batch
     int pad0;
     unsigned long long t_start;
     unsigned bar_pad[26];
     unsigned long long hub_alloc[2];  // grid tier: (entries << 32) | chunks, by level & 1
     unsigned hub_steal[2];            // grid tier: chunk counter, by level & 1
-    int hub_chunk[2];                 // grid tier: edges per chunk, by level & 1
-    unsigned pad1[26];
+    unsigned pad1[28];
+    // tile counters by level parity and group of workgroups, a 128-byte line each
+    unsigned group_steal[2 * kTileGroups * 32];
     // grid barrier state (same layout discipline as Control)
     Control bar;
     // per-level record: wall clock at the level start, top-down and
@@ -61,7 +66,6 @@ struct BatchArgs {
     BatchSlot *slots;
     BatchControl *ctl;
     int nslots;
-    int wave_t, cta_t;
     int direction;            // 0: top-down only, 1: direction-optimizing
     int do_alpha, do_beta;
     HubEntry *hubs[2];        // grid-tier rows of all queries, by level & 1

@@ -5,7 +5,7 @@
 // plans the level for all queries (frontier length, direction, tile count),
 // then workgroups take tiles from one batch-wide counter; a tile belongs to
 // one query and is either a top-down tile (256 frontier vertices, gathered
-// by the CTA / wave / scan tiers with exact claims) or a bottom-up tile (256
+// by the whole workgroup with exact claims) or a bottom-up tile (256
 // consecutive vertices looking for a parent at the current depth).  Levels
 // are separated by the grid barrier of a persistent launch, or by kernel
 // boundaries when each level is a launch (those launches are captured into a
@@ -32,8 +32,8 @@ struct BatchLds {
     unsigned long long vsum[kMaxSlots];
     unsigned long long vtop[kMaxSlots];
     unsigned char bits[kMaxSlots];  // the current frontier bitmap is exact (BatchSlot::bits)
-    int grid_t;              // grid-tier row threshold of this level
-    int chunk;               // grid-tier chunk of this level
+    int grid_t;              // grid-tier row threshold
+    int width[kMaxSlots];    // frontier vertices per top-down tile of each query this level
     int bu_tile;             // kBlock-vertex blocks per bottom-up tile of this level
 };
 
@@ -74,6 +74,8 @@ __device__ __forceinline__ int batch_direction(const BatchArgs &a, const BatchSl
 // frontier lengths, directions and the tile prefix.  Block 0 also zeroes the
 // counters the next level appends to and marks finished queries.  Returns
 // the total number of tiles (grid-uniform).
+constexpr int kTileEdges = 4 * kBlock;  // one round of a workgroup's gather
+
 __device__ int batch_plan(const BatchArgs &a, BatchLds &L, int level)
 {
     const int tid = threadIdx.x;
@@ -91,8 +93,15 @@ __device__ int batch_plan(const BatchArgs &a, BatchLds &L, int level)
             L.vtop[tid] = L.vsum[tid] + ld64(&sl.fedges[step % 3]);
             if (n > 0) {
                 dir = batch_direction(a, sl, g, L.phase[tid], step, (unsigned) n, L.vtop[tid]);
+                // top-down tiles: about kTileEdges edges each, so that a
+                // level of a few high-degree vertices is spread over the
+                // grid instead of gathered in a few long chains
+                const unsigned long long mf = L.vtop[tid] - L.vsum[tid];
+                const unsigned long long fit = (unsigned long long) n * kTileEdges / (mf ? mf : 1ull);
+                const int width = (int) max(1ull, min((unsigned long long) kBlock, fit));
+                L.width[tid] = width;
                 // bottom-up: kBlock-vertex blocks here, grouped into tiles below
-                tiles = dir == kPhaseBottomUp ? (g.nodes + kBlock - 1) / kBlock : (n + kBlock - 1) / kBlock;
+                tiles = dir == kPhaseBottomUp ? (g.nodes + kBlock - 1) / kBlock : (n + width - 1) / width;
                 if (blockIdx.x == 0) {
                     st_agent(&sl.qlen[(step + 2) % 3], 0u);
                     st_agent(&sl.ovf[(step + 2) % 3], 0u);
@@ -114,17 +123,18 @@ __device__ int batch_plan(const BatchArgs &a, BatchLds &L, int level)
         }
     }
     if (blockIdx.x == 0 && tid == 0) {
-        st_agent(&a.ctl->steal[(level + 1) & 1], 0u);
+        for (int k = 0; k < kTileGroups; k++)
+            st_agent(&a.ctl->group_steal[(((level + 1) & 1) * kTileGroups + k) * 32], 0u);
         st_agent(&a.ctl->hub_steal[(level + 1) & 1], 0u);
         __hip_atomic_store(&a.ctl->hub_alloc[(level + 1) & 1], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     // Bottom-up tile size of this level: up to bu_tile blocks, fewer when
-    // the level has too few blocks to give every workgroup about eight
+    // the level has too few blocks to give every workgroup about four
     // tiles (one tile of a small graph would otherwise hold a whole
     // level up while the grid waits at the barrier).
     int bu_blocks = 0;
     (void) block_exclusive_sum(tid < a.nslots && L.dir[tid] == kPhaseBottomUp ? tiles : 0, L.wave_tot, &bu_blocks);
-    const int bu_tile = max(1, min(a.bu_tile, bu_blocks / (8 * (int) gridDim.x)));
+    const int bu_tile = max(1, min(a.bu_tile, bu_blocks / (4 * (int) gridDim.x)));
     if (tid < a.nslots && L.dir[tid] == kPhaseBottomUp) tiles = (tiles + bu_tile - 1) / bu_tile;
     if (tid == 0) L.bu_tile = bu_tile;
     int total = 0;
@@ -133,13 +143,9 @@ __device__ int batch_plan(const BatchArgs &a, BatchLds &L, int level)
     int excl = block_exclusive_sum(tiles, L.wave_tot, &total);
     if (tid < a.nslots) L.prefix[tid] = excl;
     if (tid == 0) L.prefix[a.nslots] = total;
-    // A level of fewer tiles than workgroups leaves most of them idle while
-    // a few gather long rows alone: every row long enough for the wave tier
-    // then goes to the grid tier, in workgroup-sized chunks.
-    const bool narrow = total < (int) gridDim.x;
-    L.grid_t = narrow ? min(a.grid_t, max(a.wave_t, kWave)) : a.grid_t;
-    L.chunk = narrow ? kBlock : kHubChunk;
-    if (blockIdx.x == 0 && tid == 0) a.ctl->hub_chunk[level & 1] = L.chunk;
+    // Shorter rows than half a grid-tier chunk are no work to share: a tile
+    // spreads its rows over its workgroup anyway.
+    if (tid == 0) L.grid_t = a.grid_t == 0x7fffffff ? a.grid_t : max(a.grid_t, kHubChunk / 2);
     if (blockIdx.x == 0 && tid == 0 && level < kLevelLog) {
         a.ctl->level_clock[level] = wall_clock64();
         a.ctl->level_td_tiles[level] = (unsigned) (total - bu_total);
@@ -155,10 +161,8 @@ __device__ __forceinline__ void slot_edges(BatchSlot &sl, int step, unsigned fe)
     int hi = wave_inclusive_sum((int) (fe >> 16));
     unsigned long long tot = ((unsigned long long) (unsigned) readlane(hi, kWave - 1) << 16) +
                              (unsigned long long) (unsigned) readlane(lo, kWave - 1);
-    if (tot != 0 && lane_id() == 0) {
+    if (tot != 0 && lane_id() == 0)
         __hip_atomic_fetch_add(&sl.fedges[(step + 1) % 3], tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_fetch_add(&sl.visited_edges, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
 }
 
 // Per-wave output of the query whose tiles the workgroup is processing: the
@@ -201,24 +205,60 @@ __device__ __forceinline__ void out_open(SlotOut &o, const BatchArgs &a, BatchLd
     o.step = step;
 }
 
-// Top-down edge visit of query q: exact claim, label, frontier edge count,
-// append to the query's next frontier.
-struct TdEdge {
+// Top-down edge visits of query q, four per thread: exact claims, labels,
+// frontier edge counts, appends to the query's next frontier.  Every memory
+// trip (column, visited word, claim, row bounds) is issued for all four
+// before the first result is used: a level is bound by that chain.  With the
+// tile widths and counter groups below, 64 queries over 16 R-MAT graphs of scale
+// 14 to 17 went from 770 to 500 us of kernel time.
+struct TdEdges {
     BatchSlot &sl;
     const BatchGraph &g;
     int next_depth;
     SlotOut &o;
     bool coherent;
     unsigned *bits;  // next frontier's bitmap to mark claims in, or null
-    __device__ __forceinline__ void operator()(bool ok, int u, int par) const
+    __device__ __forceinline__ void operator()(const int (&at)[4], const int (&pv)[4], unsigned) const
     {
-        bool fresh = ok && claim_exact(sl.visited, u, coherent);
-        if (fresh) {
-            sl.depth[u] = next_depth;
-            o.fe += (unsigned) (g.row[u + 1] - g.row[u]);
-            if (bits) __hip_atomic_fetch_or(bits + (u >> 5), 1u << (u & 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        int u[4];
+        unsigned cur[4], old[4], fresh = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) u[j] = at[j] >= 0 ? __builtin_nontemporal_load(g.col + at[j]) : -1;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const unsigned *w = sl.visited + (u[j] >> 5);
+            cur[j] = u[j] < 0 ? ~0u : coherent ? ld_agent(w) : *w;
         }
-        o.wq.push(fresh, u, par);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const unsigned bit = 1u << (u[j] & 31);
+            old[j] = ~0u;
+            if (u[j] >= 0 && !(cur[j] & bit))
+                old[j] = __hip_atomic_fetch_or(sl.visited + (u[j] >> 5), bit, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+        // (a use next to its atomic would wait out each round trip in turn)
+#pragma unroll
+        for (int j = 0; j < 4; j++) asm volatile("" : "+v"(old[j]));
+        int r0[4], r1[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            r0[j] = r1[j] = 0;
+            if (!((old[j] >> (u[j] & 31)) & 1u)) {
+                fresh |= 1u << j;
+                sl.depth[u[j]] = next_depth;
+                r0[j] = g.row[u[j]];
+                r1[j] = g.row[u[j] + 1];
+                if (bits)
+                    __hip_atomic_fetch_or(bits + (u[j] >> 5), 1u << (u[j] & 31), __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            o.fe += (unsigned) (r1[j] - r0[j]);
+            o.wq.push((fresh >> j) & 1u, u[j], pv[j]);
+        }
     }
 };
 
@@ -244,25 +284,27 @@ __device__ void batch_td_tile(const BatchArgs &a, BatchLds &L, int q, unsigned l
     const BatchGraph g = a.graphs[sl.graph];
     const int step = L.step[q];
     const unsigned n = (unsigned) L.n[q];
-    HubList hub{a.hubs[level & 1], a.hub_cap, &a.ctl->hub_alloc[level & 1], L.grid_t, q, L.chunk, nullptr};
-    unsigned i = local * kBlock + threadIdx.x;
-    int v = -1, beg = 0, end = 0;
-    if (i < n) {
-        v = ld_queue(sl.q[step & 1] + i);
-        beg = g.row[v];
-        end = g.row[v + 1];
+    HubList hub{a.hubs[level & 1], a.hub_cap, &a.ctl->hub_alloc[level & 1], L.grid_t, q, kHubChunk, nullptr, kHeavyTile, kHeavyRow};
+    const unsigned width = (unsigned) L.width[q];
+    const unsigned i = local * width + threadIdx.x;
+    int v[1] = {-1}, beg[1] = {0}, end[1] = {0};
+    if (threadIdx.x < width && i < n) {
+        v[0] = ld_queue(sl.q[step & 1] + i);
+        beg[0] = g.row[v[0]];
+        end[0] = g.row[v[0] + 1];
     }
     {
         // this tile's share of clearing fbm[d & 1] (see td_bits)
         const unsigned words = ((unsigned) g.nodes + 31) >> 5;
-        const unsigned ntiles = (n + kBlock - 1) / kBlock;
+        const unsigned ntiles = (n + width - 1) / width;
         const unsigned share = (words + ntiles - 1) / ntiles;
         unsigned *old = sl.fbm[L.it[q] & 1];
         const unsigned w_end = min(words, (local + 1) * share);
         for (unsigned w = local * share + threadIdx.x; w < w_end; w += kBlock) old[w] = 0u;
     }
-    gather_rows<false>(beg, end, v, g.col, a.wave_t, a.cta_t, hub, L.base,
-                       TdEdge{sl, g, L.it[q] + 1, o, a.coherent_filter != 0, td_bits(L, sl, q)});
+    __syncthreads();  // (the row table served the previous tile)
+    gather_tile<1>(beg, end, v, hub, L.base.rt, [](int) {},
+                   TdEdges{sl, g, L.it[q] + 1, o, a.coherent_filter != 0, td_bits(L, sl, q)});
 }
 
 // Grid-tier phase of a level: every workgroup takes chunks of
@@ -276,8 +318,7 @@ __device__ void batch_hub_phase(const BatchArgs &a, BatchLds &L, int level)
     if (entries == 0) return;
     const HubEntry *list = a.hubs[level & 1];
     HubEntry last = list[entries - 1];
-    // the chunk the level's tiles published with (set when it was planned)
-    const int chunk = ld_agent(&a.ctl->hub_chunk[level & 1]);
+    constexpr int chunk = kHubChunk;
     unsigned total = last.first_chunk + (unsigned) ((last.end - last.beg + chunk - 1) / chunk);
     SlotOut o;
     o.q = -1;
@@ -318,12 +359,16 @@ __device__ void batch_hub_phase(const BatchArgs &a, BatchLds &L, int level)
         out_open(o, a, L, q);
         BatchSlot &sl = a.slots[q];
         const BatchGraph g = a.graphs[sl.graph];
-        TdEdge edge{sl, g, L.it[q] + 1, o, a.coherent_filter != 0, td_bits(L, sl, q)};
-        for (int k = b; k < e; k += kBlock) {
-            int idx = k + threadIdx.x;
-            bool ok = idx < e;
-            int u = ok ? __builtin_nontemporal_load(g.col + idx) : -1;
-            edge(ok, u, pv);
+        const TdEdges edges{sl, g, L.it[q] + 1, o, a.coherent_filter != 0, td_bits(L, sl, q)};
+        for (int k = b; k < e; k += 4 * kBlock) {
+            int at[4], par[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int x = k + j * kBlock + (int) threadIdx.x;
+                at[j] = x < e ? x : -1;
+                par[j] = pv;
+            }
+            edges(at, par, 0u);
         }
     }
     out_close(o, a);
@@ -353,7 +398,7 @@ __device__ __forceinline__ void wave_lds_sync_b()
 // lane busy; parents found become bits per window of kBatchBuWindow blocks
 // (two words per wave and block) written once per word.  The wave's queue
 // lives in LDS the batch kernels leave idle during a tile: the history-hash
-// area and the scan-tier staging of gather_rows (used only inside a call).
+// area and the row table of gather_tile (used only inside a call).
 constexpr int kBatchBuWindow = 32;
 
 __device__ void batch_bu_tile(const BatchArgs &a, BatchLds &L, int q, unsigned local, SlotOut &o)
@@ -378,10 +423,6 @@ __device__ void batch_bu_tile(const BatchArgs &a, BatchLds &L, int q, unsigned l
     int *qe1 = L.base.rt.beg[wave];      // row ends, entries 64..127
     unsigned *fb = reinterpret_cast<unsigned *>(L.base.rt.par[wave]);  // found bits of the window
 
-    auto in_frontier = [&](int u) {
-        if (use_bitmap) return ((cur[u >> 5] >> (u & 31)) & 1u) != 0;
-        return ((sl.visited[u >> 5] >> (u & 31)) & 1u) != 0 && sl.depth[u] == d;
-    };
     // Scans the first cnt (1..64) queued vertices of the window starting at block wb0.
     auto scan = [&](int cnt, unsigned wb0) {
         int v = -1, beg = 0, end = 0;
@@ -409,23 +450,20 @@ __device__ void batch_bu_tile(const BatchArgs &a, BatchLds &L, int q, unsigned l
                 if (u[j] >= 0 && ((fw[j] >> (u[j] & 31)) & 1u) && lab[j] == d) parent = u[j];
             pos += 4;
         }
-        uint64_t lm = ballot(parent < 0 && lim < end);
-        while (lm) {
-            const int l = uniform(__builtin_ctzll(lm));
-            lm &= lm - 1;
-            const int b = readlane(lim, l), e = readlane(end, l);
-            int hit = -1;
-            for (int r = b; r < e; r += kWave) {
-                const int idx = r + lane;
-                const int uu = idx < e ? g.rcol[idx] : -1;
-                const uint64_t hm = ballot(uu >= 0 && in_frontier(uu));
-                if (hm) {
-                    hit = readlane(uu, uniform(__builtin_ctzll(hm)));
-                    break;
+        const uint64_t lm = ballot(parent < 0 && lim < end);
+        if (lm)
+            parent = scan_long_rows(lm, lim, end, parent, g.rcol, [&](const int (&u)[kLongRows], bool (&in)[kLongRows]) {
+                unsigned fw[kLongRows];
+                int lab[kLongRows];
+#pragma unroll
+                for (int r = 0; r < kLongRows; r++) {
+                    fw[r] = u[r] >= 0 ? (use_bitmap ? cur[u[r] >> 5] : sl.visited[u[r] >> 5]) : 0u;
+                    lab[r] = u[r] >= 0 && !use_bitmap ? sl.depth[u[r]] : d;
                 }
-            }
-            if (lane == l) parent = hit;
-        }
+#pragma unroll
+                for (int r = 0; r < kLongRows; r++)
+                    in[r] = u[r] >= 0 && ((fw[r] >> (u[r] & 31)) & 1u) && lab[r] == d;
+            });
         const bool got = parent >= 0;
         if (got) {
             sl.depth[v] = d + 1;
@@ -519,26 +557,30 @@ __device__ void batch_tiles(const BatchArgs &a, BatchLds &L, int level, int tota
 {
     SlotOut o;
     o.q = -1;
-    // Grabs: one counter atomic hands a workgroup `grab` tiles, so the
-    // single counter address (whose device-scope atomics serialise) is not
-    // the bottleneck of levels with many tiles.  Strided: counter value i
-    // takes tiles i0, i0 + W, ... (W = gridDim.x), so W consecutive grabs
-    // cover W * grab consecutive tiles and the tiles in flight across the
-    // grid stay a window about W wide.  Consecutive: counter value t0 takes
-    // [t0, t0 + grab).
-    const unsigned W = gridDim.x;
-    const unsigned grab = (unsigned) max(1, min(a.grab_max, total / ((int) W * 8)));
+    // Tiles t with t % groups == b % groups go to workgroup b's group; one
+    // counter atomic hands a workgroup `grab` of them.  Strided: counter
+    // value i takes the group's tiles i0, i0 + W, ... (W workgroups in the
+    // group), so W consecutive grabs cover W * grab consecutive ones and the
+    // tiles in flight stay a window of the level.  Consecutive: counter value
+    // t0 takes [t0, t0 + grab).
+    const unsigned groups = min((unsigned) kTileGroups, gridDim.x);
+    const unsigned group = blockIdx.x % groups;
+    const unsigned W = (gridDim.x - group + groups - 1) / groups;
+    const unsigned mine = ((unsigned) total + groups - 1 - group) / groups;  // the group's tiles
+    const unsigned grab = (unsigned) max(1, min(a.grab_max, (int) (mine / (W * 8))));
     const unsigned step = a.strided ? W : 1u;
+    unsigned *counter = &a.ctl->group_steal[((level & 1) * kTileGroups + group) * 32];
     while (true) {
         unsigned t0;
         if (a.strided) {
-            const unsigned i = next_item_batch(&a.ctl->steal[level & 1], L.base);
+            const unsigned i = next_item_batch(counter, L.base);
             t0 = (i / W) * W * grab + i % W;
         } else {
-            t0 = next_item_batch(&a.ctl->steal[level & 1], L.base, grab);
+            t0 = next_item_batch(counter, L.base, grab);
         }
-        if (t0 >= (unsigned) total) break;
-        for (unsigned t = t0, k = 0; k < grab && t < (unsigned) total; k++, t += step) {
+        if (t0 >= mine) break;
+        for (unsigned ti = t0, k = 0; k < grab && ti < mine; k++, ti += step) {
+            const unsigned t = ti * groups + group;
             // last query whose first tile is <= t (queries without tiles
             // repeat the prefix value and are skipped by taking the last match)
             int lo = 0, hi = a.nslots - 1;
@@ -559,7 +601,6 @@ __device__ void batch_tiles(const BatchArgs &a, BatchLds &L, int level, int tota
 __device__ void batch_load_cursors(const BatchArgs &a, BatchLds &L)
 {
     for (int i = threadIdx.x; i < kHistory; i += kBlock) L.base.hist[i] = -1;
-    if (threadIdx.x == 0) L.base.cta_owner = -1;
     int tid = threadIdx.x;
     if (tid < a.nslots) {
         const BatchSlot &sl = a.slots[tid];
@@ -697,7 +738,6 @@ __global__ void batch_seed_kernel(BatchArgs a, const int *list, int count)
     sl.fedges[0] = deg;
     sl.fedges[1] = 0;
     sl.fedges[2] = 0;
-    sl.visited_edges = deg;
     sl.step = 0;
     sl.iteration = 0;
     sl.phase = kPhaseExpandContract;

@@ -931,8 +931,6 @@ bfs_status host_fail(bfs_status s, const char *msg) { return fail(s, msg); }
 
 void apply_search_config(SearchArgs &s, const bfs_config &cfg, int grid)
 {
-    s.wave_t = cfg.wave_gather_threshold;
-    s.cta_t = cfg.cta_gather_threshold;
     s.grid_t = cfg.grid_gather_threshold > 0 ? cfg.grid_gather_threshold : 0x7fffffff;
     s.grab_max = cfg.tile_grab_max > 0 ? cfg.tile_grab_max : 1;
     s.coherent_filter = cfg.claim_filter == 2;

@@ -1,7 +1,7 @@
 // bfs_device.hpp -- gfx950 device building blocks of the BFS kernels.
 //
 // Wave64 primitives (DPP prefix sum, ballot/mbcnt compaction), the per-wave
-// LDS-staged frontier queue, the visited-bitmask claims, the three-tier
+// LDS-staged frontier queue, the visited-bitmask claims, the workgroup
 // neighbour gather and the hierarchical grid barrier.  These replace the
 // reference's CTA raking scans, warp scans, tile I/O, culls and software
 // global barrier (b40c/util/scan/*.cuh, b40c/util/io/*.cuh,
@@ -266,9 +266,9 @@ struct PredStore<false> {
     int buf[1][1];
 };
 
-// Row table of gather_tile (and the scan tier's staging of gather_rows).
+// Row table of gather_tile, in parts a wave can use by itself.
 struct RowTable {
-    int excl[kWaves][kWave];             // edge offset (scan tier: exclusive rank per lane)
+    int excl[kWaves][kWave];             // edge offset
     int beg[kWaves][kWave];              // row begin (gather_tile: less the edge offset)
     int par[kWaves][kWave];              // row owner
     int scan[kWaves], scan2[kWaves];
@@ -281,7 +281,7 @@ struct Lds {
     PredStore<PRED> wqp;                 // per-wave predecessor staging
     RowTable rt;
     int hist[kHistory];                  // history hash (contract / filter)
-    int cta_owner, cta_beg, cta_end, cta_par;
+    int cta_beg, cta_end, cta_par;
     unsigned cta_out;                    // expansions: the chunk's place in the output queue
     unsigned tile;
     unsigned nb;                         // broadcast frontier length
@@ -365,19 +365,7 @@ struct WaveQueue {
     }
 };
 
-// ---------------------------------------------------------------------------
-// Three-tier neighbour gather.  Each thread owns one adjacency row
-// [beg, end) with owner `par` (end == beg for none).  fn(valid, u, par) is
-// called wave-converged for every neighbour u exactly once:
-//   CTA tier  (len >= cta_t):  the whole workgroup strides through the row;
-//   wave tier (len >= wave_t): one wave strides through the row;
-//   scan tier (len <  wave_t): a wave-wide DPP prefix sum ranks the short
-//       rows, and each lane locates its edge by a 6-step search over the 64
-//       LDS-staged exclusive ranks, so the wave's lanes stay fully occupied
-//       whatever the mix of short lengths.
-// Replaces ExpandByCta / ExpandByWarp / ExpandByScan
-// (b40c/graph/bfs/two_phase/expand_atomic/cta.cuh:215-423).
-// ---------------------------------------------------------------------------
+// Grid tier of a gathering step: where its long rows are published.
 struct HubList {
     HubEntry *entries;
     unsigned cap;
@@ -386,6 +374,7 @@ struct HubList {
     int tag;           // stored with every published row
     int chunk;         // edges per chunk
     unsigned *out_len; // expansions: length of the output queue (null: none reserved)
+    int heavy, heavy_row;  // edges from which a tile publishes its rows of heavy_row and more (gather_tile)
 };
 
 // Index of the last grid-tier entry whose first chunk is <= ch (entries are
@@ -460,90 +449,6 @@ __device__ __forceinline__ bool publish_hub_row(int beg, int end, int par, const
     return done;
 }
 
-template <bool PRED, typename Fn>
-__device__ __forceinline__ void gather_rows(int beg, int end, int par, const int *__restrict__ col,
-                                            int wave_t, int cta_t, const HubList &hub, Lds<PRED> &lds, Fn &&fn)
-{
-    const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
-    const int wave = tid / kWave;
-    int len = end - beg;
-
-    // Grid tier: publish the row as chunks for every workgroup of the grid
-    // (processed after this tile phase).  A full list falls back to the CTA
-    // tier below.
-    if (publish_hub_row(beg, end, par, hub)) len = 0;
-
-    // CTA tier
-    while (true) {
-        __syncthreads();
-        if (len >= cta_t) lds.cta_owner = tid;
-        __syncthreads();
-        int owner = lds.cta_owner;
-        if (owner < 0) break;
-        if (tid == owner) {
-            lds.cta_beg = beg;
-            lds.cta_end = end;
-            lds.cta_par = par;
-            len = 0;
-        }
-        __syncthreads();
-        int b = lds.cta_beg, e = lds.cta_end, pv = lds.cta_par;
-        __syncthreads();
-        if (tid == 0) lds.cta_owner = -1;
-        for (int k = b; k < e; k += kBlock) {
-            int idx = k + tid;
-            bool ok = idx < e;
-            int u = ok ? __builtin_nontemporal_load(col + idx) : -1;
-            fn(ok, u, pv);
-        }
-    }
-
-    // Wave tier
-    uint64_t wm = ballot(len >= wave_t);
-    while (wm) {
-        int l = uniform(__builtin_ctzll(wm));
-        wm &= wm - 1;
-        int b = readlane(beg, l), e = readlane(end, l), pv = readlane(par, l);
-        for (int k = b; k < e; k += kWave) {
-            int idx = k + lane;
-            bool ok = idx < e;
-            int u = ok ? __builtin_nontemporal_load(col + idx) : -1;
-            fn(ok, u, pv);
-        }
-    }
-    if (len >= wave_t) len = 0;
-
-    // Scan tier
-    int incl = wave_inclusive_sum(len);
-    int total = readlane(incl, kWave - 1);
-    if (total == 0) return;
-    int *excl = lds.rt.excl[wave];
-    int *rb = lds.rt.beg[wave];
-    int *rp = lds.rt.par[wave];
-    excl[lane] = incl - len;
-    rb[lane] = beg;
-    rp[lane] = par;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    for (int r = 0; r < total; r += kWave) {
-        int idx = r + lane;
-        bool ok = idx < total;
-        int u = -1, pv = -1;
-        if (ok) {
-            int l = 0;
-#pragma unroll
-            for (int s = 32; s > 0; s >>= 1)
-                if (excl[l + s] <= idx) l += s;
-            u = __builtin_nontemporal_load(col + rb[l] + (idx - excl[l]));
-            pv = rp[l];
-        }
-        fn(ok, u, pv);
-    }
-    __builtin_amdgcn_wave_barrier();
-}
-
 // ---------------------------------------------------------------------------
 // Workgroup gather of a tile of rows.  Each thread brings up to K rows
 // [beg, end) with owner par (end == beg for none).  Long rows go to the grid
@@ -554,22 +459,26 @@ __device__ __forceinline__ void gather_rows(int beg, int end, int par, const int
 // entries of a row.  A thread finds its edges' rows by searching the offsets,
 // and hands the four column positions (-1: none) and owners to `edges`, which
 // issues every memory trip of a round for all four before using the first
-// result.  Called by every thread; `edges` is called workgroup-converged, and
+// result.  Replaces ExpandByCta / ExpandByWarp / ExpandByScan
+// (b40c/graph/bfs/two_phase/expand_atomic/cta.cuh:215-423).
+// Called by every thread; `edges` is called workgroup-converged, and
 // `begin` once before, with the tile's edge count.  Edge j of a call is edge
 // x0 + j * kBlock of the tile.
 //
 // A level is bound by its chain of dependent memory trips, not by bytes: one
-// row per thread gathered 64 edges a wave at a time (gather_rows) made the
+// row per thread gathered 64 edges a wave at a time made the
 // 4318-vertex level of a 100 k-vertex random graph a chain of 16 such rounds
 // on nine workgroups, 76 us; spread over the grid it is one round.
 // ---------------------------------------------------------------------------
-// A tile of more than kHeavyTile edges sends its rows from kHeavyRow edges
+// A tile of more than hub.heavy edges sends its rows from hub.heavy_row edges
 // on to the grid tier as well.  The first workgroups to claim anything in a
 // level claim its high-degree vertices (an edge leads to a vertex in
 // proportion to its degree), and with 2048 items a tile they kept the
 // 24.9 M-edge contract-expand step of an R-MAT scale 20 search busy for
-// 1200 us while the rest waited.
-constexpr int kHeavyTile = 1 << 15, kHeavyRow = 512;
+// 1200 us while the rest waited.  In a step of one tile per workgroup the
+// others have nothing else to do, so there two rounds' edges are heavy.
+constexpr int kHeavyTile = 1 << 15, kHeavyTileNarrow = 2 * 4 * kBlock;
+constexpr int kHeavyRow = 512, kHeavyRowNarrow = 256;
 
 template <int K, typename Begin, typename Edges>
 __device__ __forceinline__ void gather_tile(const int (&beg)[K], int (&end)[K], const int (&par)[K],
@@ -607,8 +516,8 @@ __device__ __forceinline__ void gather_tile(const int (&beg)[K], int (&end)[K], 
             rtotal += a;
             etotal += b;
         }
-        if (etotal <= kHeavyTile || h.grid_t <= kHeavyRow || h.grid_t == 0x7fffffff) break;
-        h.grid_t = kHeavyRow;
+        if (etotal <= h.heavy || h.grid_t <= h.heavy_row || h.grid_t == 0x7fffffff) break;
+        h.grid_t = h.heavy_row;
         __syncthreads();  // the sums are written again
     }
     begin(etotal);
@@ -657,6 +566,60 @@ __device__ __forceinline__ void gather_tile(const int (&beg)[K], int (&end)[K], 
         __syncthreads();  // the table and the sums are written again next
     }
     if (rtotal == 0) __syncthreads();
+}
+
+// ---------------------------------------------------------------------------
+// Long rows of a bottom-up step: the lanes of mask lm look for the first
+// neighbour in the frontier among columns [beg, end) of their rows; returns
+// it to them (other lanes, and rows without one: `none`).  The whole wave
+// reads 64 neighbours of each of kLongRows rows at a time, so as many chains
+// (column, frontier word) run together; a row that is done makes room for the
+// next.  in_frontier(u, in) tests kLongRows neighbours per lane (-1: none).
+// (One row at a time made these rows most of a first bottom-up level: 8 to 30
+// of them per wave, two memory trips each.)
+// ---------------------------------------------------------------------------
+constexpr int kLongRows = 4;
+
+template <typename Test>
+__device__ __forceinline__ int scan_long_rows(uint64_t lm, int beg, int end, int none, const int *col, Test &&in_frontier)
+{
+    const int lane = lane_id();
+    int found = none;
+    int row[kLongRows], at[kLongRows], stop[kLongRows];  // wave-uniform; row: the lane, -1 none
+#pragma unroll
+    for (int q = 0; q < kLongRows; q++) row[q] = -1;
+    while (true) {
+        bool any = false;
+#pragma unroll
+        for (int q = 0; q < kLongRows; q++) {
+            if (row[q] < 0 && lm) {
+                row[q] = uniform(__builtin_ctzll(lm));
+                lm &= lm - 1;
+                at[q] = readlane(beg, row[q]);
+                stop[q] = readlane(end, row[q]);
+            }
+            any = any || row[q] >= 0;
+        }
+        if (!any) return found;
+        int u[kLongRows];
+        bool in[kLongRows];
+#pragma unroll
+        for (int q = 0; q < kLongRows; q++) u[q] = row[q] >= 0 && at[q] + lane < stop[q] ? col[at[q] + lane] : -1;
+        in_frontier(u, in);
+#pragma unroll
+        for (int q = 0; q < kLongRows; q++) {
+            if (row[q] < 0) continue;
+            const uint64_t hm = ballot(in[q]);
+            if (hm) {  // (the first in row order)
+                const int hit = readlane(u[q], uniform(__builtin_ctzll(hm)));
+                if (lane == row[q]) found = hit;
+                row[q] = -1;
+            } else {
+                at[q] += kWave;
+                if (at[q] >= stop[q]) row[q] = -1;
+            }
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------

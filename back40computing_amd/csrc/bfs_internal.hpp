@@ -53,7 +53,7 @@ struct SearchArgs {
     unsigned long long total_edges;
     int track_edges;       // accumulate frontier edge counts (direction switching)
     int do_alpha, do_beta; // top-down -> bottom-up when m_f * alpha > m_u; back when n_f * beta < V
-    int wave_t, cta_t, grid_t, fast_t, sat_t;
+    int grid_t, fast_t, sat_t;
     // Hybrid two-phase launches: a contract step whose input is at most
     // sat_t hands the search back to the persistent contract-expand kernel
     // (sets Control::hybrid_stop), and every step launched after it returns.

@@ -13,7 +13,7 @@
 //   filter           edge frontier -> visited-bitmask cull -> edge frontier
 //                    (b40c/graph/bfs/two_phase/filter_atomic/cta.cuh:308-388)
 // Gathering steps have two sub-phases: the tile phase (frontier tiles taken
-// dynamically by workgroups, rows gathered by the CTA / wave / scan tiers)
+// by workgroups, their rows' edges spread over the workgroup)
 // and, when some rows were long enough for the grid tier, the hub phase in
 // which every workgroup takes fixed-size chunks of those rows.
 // Each step runs either inside a persistent, cooperatively launched loop with
@@ -32,10 +32,7 @@ template <bool PRED>
 __device__ __forceinline__ void init_lds(Lds<PRED> &lds)
 {
     for (int i = threadIdx.x; i < kHistory; i += kBlock) lds.hist[i] = -1;
-    if (threadIdx.x == 0) {
-        lds.cta_owner = -1;
-        lds.solo = 0;
-    }
+    if (threadIdx.x == 0) lds.solo = 0;
     __syncthreads();
 }
 
@@ -178,6 +175,8 @@ __device__ __forceinline__ HubList hub_list(const SearchArgs &s, int step, bool 
     h.tag = 0;
     h.chunk = kHubChunk;
     h.out_len = nullptr;
+    h.heavy = narrow_step(n) ? kHeavyTileNarrow : kHeavyTile;
+    h.heavy_row = narrow_step(n) ? kHeavyRowNarrow : kHeavyRow;
     return h;
 }
 
@@ -554,8 +553,8 @@ __device__ __forceinline__ void body_expand_contract(const GraphArgs &g, const S
 //   2. every 128 queued vertices are scanned with all lanes busy, two per
 //      lane: four neighbours of each per round, all eight loads of a round
 //      in flight; rows of kBuLong+ neighbours get one such round and then a
-//      wave-wide scan of the rest (a high-degree vertex usually finds a
-//      frontier neighbour among its first four).
+//      wave-wide scan of the rest, several rows at a time (a high-degree
+//      vertex usually finds a frontier neighbour among its first four).
 // Parents found are collected as bits in LDS per window of kBuWindow groups
 // and written once per word: visited |= found, next frontier = found (the
 // next-frontier word is overwritten in full, which also clears it).
@@ -635,26 +634,21 @@ __device__ __forceinline__ void body_bottom_up(const GraphArgs &g, const SearchA
             pos[1] += 4;
         }
         // rows of kBuLong+ neighbours with no parent among their first four:
-        // a wave-wide scan of the rest, one row at a time
+        // a wave-wide scan of the rest
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            uint64_t lm = ballot(parent[h] < 0 && lim[h] < end[h]);
-            while (lm) {
-                const int l = uniform(__builtin_ctzll(lm));
-                lm &= lm - 1;
-                const int b = readlane(lim[h], l), e = readlane(end[h], l);
-                int hit = -1;
-                for (int q = b; q < e; q += kWave) {
-                    const int idx = q + lane;
-                    const int uu = idx < e ? g.rcol[idx] : -1;
-                    const uint64_t hm = ballot(uu >= 0 && ((cur[uu >> 5] >> (uu & 31)) & 1u));
-                    if (hm) {
-                        hit = readlane(uu, uniform(__builtin_ctzll(hm)));
-                        break;
-                    }
-                }
-                if (lane == l) parent[h] = hit;
-            }
+            const uint64_t lm = ballot(parent[h] < 0 && lim[h] < end[h]);
+            if (lm)
+                parent[h] = scan_long_rows(lm, lim[h], end[h], parent[h], g.rcol,
+                                           [&](const int (&u)[kLongRows], bool (&in)[kLongRows]) {
+                                               unsigned fw[kLongRows];
+#pragma unroll
+                                               for (int q = 0; q < kLongRows; q++)
+                                                   fw[q] = u[q] >= 0 ? cur[u[q] >> 5] : 0u;
+#pragma unroll
+                                               for (int q = 0; q < kLongRows; q++)
+                                                   in[q] = u[q] >= 0 && ((fw[q] >> (u[q] & 31)) & 1u);
+                                           });
         }
 #pragma unroll
         for (int h = 0; h < 2; h++) {
@@ -2998,7 +2992,7 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
                         body_expand<PRED, EXACT>(g, s, c, m, lds, 0, true, xio);
                         if (s.instrument) busy += wall_clock64() - t0;
                         bar(false);
-                        if (s.max_degree >= min(s.grid_t, kHeavyRow) && hubs_pending(s, c.step)) {
+                        if (s.max_degree >= min(s.grid_t, kHeavyRowNarrow) && hubs_pending(s, c.step)) {
                             t0 = s.instrument ? wall_clock64() : 0;
                             body_expand<PRED, EXACT>(g, s, c, m, lds, 1, true, xio);
                             if (s.instrument) busy += wall_clock64() - t0;
@@ -3024,7 +3018,7 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
         if (s.instrument) busy += wall_clock64() - t0;
         bar(light_step);
         // (graphs whose longest row no step publishes have no list to look at)
-        if (!spread && gathers(c.phase) && s.max_degree >= min(s.grid_t, kHeavyRow) && hubs_pending(s, c.step)) {
+        if (!spread && gathers(c.phase) && s.max_degree >= min(s.grid_t, kHeavyRowNarrow) && hubs_pending(s, c.step)) {
             t0 = s.instrument ? wall_clock64() : 0;
             refresh();  // (the list is read through the caches)
             const StepIo io{light_step, false};

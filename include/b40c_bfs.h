@@ -91,18 +91,25 @@ typedef enum bfs_cull_mode {
  * Zero in any field selects the library default.
  */
 typedef struct bfs_config {
-    int32_t wave_gather_threshold;  /* row length >= this: one wave gathers the row   */
-    int32_t cta_gather_threshold;   /* row length >= this: the whole workgroup gathers */
+    int32_t wave_gather_threshold;  /* accepted and checked (>= 1), selects nothing:  */
+    int32_t cta_gather_threshold;   /* a tile's edges are spread over the workgroup
+                                       whatever the lengths of its rows               */
     int32_t fast_path_threshold;    /* frontier <= this: one workgroup runs the level
-                                       with no grid barrier (-1 disables)             */
+                                       with no grid barrier (-1 disables); up to three
+                                       times this where no row is longer than 8 and
+                                       the graph has at most BFS_FAST_VISITED_MAX
+                                       vertices                                       */
     int32_t saturation_threshold;   /* hybrid: edge frontier > this leaves the
                                        persistent contract-expand kernel (-1: never;
                                        default: 4 items per thread of the grid)       */
     int32_t blocks_per_cu;          /* persistent grid = CUs * this (capped by occupancy) */
     int32_t cull_mode;              /* bfs_cull_mode */
     int32_t instrument;             /* 1: collect per-workgroup duty statistics */
-    int32_t grid_gather_threshold;  /* row length >= this: the row is split into
-                                       2048-edge chunks shared by the whole grid */
+    int32_t grid_gather_threshold;  /* row length >= this: the row is split into chunks
+                                       shared by the whole grid (-1: never).  Steps of
+                                       few vertices, and tiles with many edges, share
+                                       shorter rows too; batched searches share none
+                                       below half a chunk */
     int32_t do_alpha;               /* direction-optimizing: go bottom-up when
                                        frontier edges * alpha > unexplored edges */
     int32_t do_beta;                /* direction-optimizing: back to top-down when
