@@ -464,8 +464,8 @@ bfs_status bfs_problem_create(const int32_t *h_row_offsets, const int32_t *h_col
         (e = hipMalloc(&p->d_fbm, sizeof(unsigned) * 2 * words)) != hipSuccess ||
         (e = hipMalloc(&p->d_marks, 32 * words)) != hipSuccess)
         return cleanup(hip_fail(e, "allocate problem"));
-    // (steps of kMarkEdges edges and more use them: smaller graphs have none)
-    if (nodes <= BFS_FAST_VISITED_MAX && edges >= (1 << 20) &&
+    // (no step of a graph with fewer edges uses them)
+    if (nodes <= BFS_FAST_VISITED_MAX && (unsigned long long) edges >= bit_mark_work(nodes) &&
         (e = hipMalloc(&p->d_slabs, 16 * slab_quads(nodes) * (size_t) p->num_cus)) != hipSuccess)
         return cleanup(hip_fail(e, "allocate bit-mark slabs"));
     // marks are clear between steps (each compaction clears what it reads)
@@ -617,6 +617,9 @@ bfs_status bfs_enact(bfs_problem *p, bfs_strategy strategy, int32_t fused, int32
     if (max_grid_size <= 0)
         pgrid = (int) std::min<long long>(pgrid, std::max<long long>(8, (p->nodes + p->edges) / kWorkPerWorkgroup));
     int sgrid = step_grid(p, max_grid_size);
+    // (launches per step have no barriers, but a reservation atomic per workgroup)
+    if (max_grid_size <= 0)
+        sgrid = (int) std::min<long long>(sgrid, std::max<long long>(16, (p->nodes + p->edges) / (kWorkPerWorkgroup / 2)));
     GraphArgs g{p->d_row, p->d_col, p->nodes, p->d_rrow, p->d_rcol};
     // Chained compaction tags each step's tile words with scan_epoch + step.
     // A search has fewer than 3 (V + 2) steps (every level but the last

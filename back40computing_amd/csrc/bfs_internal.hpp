@@ -90,6 +90,12 @@ __host__ __device__ inline size_t slab_quads(int nodes)
     return (((quads + 15) / 16) | 1) * 16;
 }
 
+// Fewest edges or items of a step that takes bit marks on a graph of V vertices.
+__host__ __device__ inline unsigned long long bit_mark_work(int nodes)
+{
+    return (1ull << 16) + (unsigned long long) nodes / 2;
+}
+
 // Loop position: step index (selects queues and counters), BFS iteration
 // (depth written by the next claim), and phase (two-phase cycle).
 struct Cursor {

@@ -931,7 +931,9 @@ __device__ __forceinline__ void body_contract_expand(const GraphArgs &g, const S
     bool labeled = false;
     if (sub == 0) {
         const HubList hub = x.hubs(n, hubs);
-        TileGrab tg = tile_grab(s, n, lds, kItems * kBlock, (n + kBlock - 1) / kBlock);
+        // (an item may claim a row of any length: few items go to as many
+        // workgroups as runs of the queue allow)
+        TileGrab tg = tile_grab(s, n, lds, kItems * kBlock, (n + 15) / 16);
         while (true) {
             const unsigned base = next_tile(&s.ctl->steal[c.step & 1], lds, tg) * tg.width;
             if (base >= n) break;
@@ -1860,12 +1862,15 @@ struct BitLds {
 };
 static_assert(sizeof(BitLds) <= sizeof(FastFront), "the bitmap stays free of the step's other variables");
 
-// Whether a step of `work` edges or items takes bit marks (grid-uniform): the
-// rule of the byte marks, whose passes over V cost about as much.
+// Whether a step of `work` edges or items takes bit marks (grid-uniform).  The
+// passes over the slabs cost 10 us and more with V (30 us at 2^20 vertices);
+// claims cost the more the fewer lines the bitmap has, as atomics on a line
+// serialise (69 k claims of a 100 k-vertex graph take 18 us, as many as 27
+// G/s would do in 2.5).
 __device__ __forceinline__ bool bit_step(const SearchArgs &s, unsigned long long work)
 {
     return s.slabs != nullptr && gridDim.x <= (unsigned) s.slab_count && s.nodes <= kFastVisitedWords * 32 &&
-           work >= kMarkEdges && work >= (unsigned long long) s.nodes / 2;
+           work >= bit_mark_work(s.nodes);
 }
 
 template <bool PRED, bool EXACT>
@@ -2074,10 +2079,12 @@ __device__ __forceinline__ void bits_dump(const SearchArgs &s, const unsigned *v
 // Collects the slabs behind a grid barrier and a refresh of the caches: new vertices get label `depth`,
 // a place in `out` (whose length is *out_len, overflow flags at step + 1)
 // and, with fbm_out, their bit in every word of that frontier bitmap; with
-// track their degrees are added to *fedges.  A full grid barrier must follow.
+// track their degrees are added to fedges.  A full grid barrier must follow,
+// or with `through` a light one.
 template <bool EXACT>
 __device__ __forceinline__ void bits_collect(const GraphArgs &g, const SearchArgs &s, Cursor c, int depth, BitLds &B,
-                                             int *out, unsigned *out_len, unsigned *fbm_out, bool track)
+                                             int *out, unsigned *out_len, unsigned *fbm_out, bool track,
+                                             bool through = false)
 {
     const int words = (s.nodes + 31) >> 5;
     const int quads = (words + 3) >> 2;
@@ -2131,8 +2138,13 @@ __device__ __forceinline__ void bits_collect(const GraphArgs &g, const SearchArg
                     if (s.depth[v] != -1) bits &= ~(1u << (v & 31));
                 }
             }
-            if (bits) s.visited[w] = vis | bits;
-            if (fbm_out) fbm_out[w] = bits;
+            if (through) {
+                if (bits) st_agent(s.visited + w, vis | bits);
+                if (fbm_out) st_agent(fbm_out + w, bits);
+            } else {
+                if (bits) s.visited[w] = vis | bits;
+                if (fbm_out) fbm_out[w] = bits;
+            }
         }
         int total = 0;
         int k = block_exclusive_sum(__popc(bits), B.scan, &total);
@@ -2155,8 +2167,9 @@ __device__ __forceinline__ void bits_collect(const GraphArgs &g, const SearchArg
                 if (v[j] < 0) continue;
                 s.depth[v[j]] = depth;
                 const unsigned pos = base + (unsigned) (i0 + j * kBlock + tid);
-                if (pos < s.cap) out[pos] = v[j];
-                else over = true;
+                if (pos >= s.cap) over = true;
+                else if (through) st_agent(out + pos, v[j]);
+                else out[pos] = v[j];
                 fe += (unsigned) (r1[j] - r0[j]);
             }
         }
@@ -2835,16 +2848,19 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
             (LOOP == kLoopEC || LOOP == kLoopDO) && c.phase == kPhaseExpandContract && marked_step(s, fe);
         // large steps of graphs with an LDS bitmap take bit marks instead
         // (contractions chained through tile status words keep their order)
-        const bool bits = FASTV && !fast &&
-                          ((LOOP == kLoopEC || LOOP == kLoopDO) ? mark && bit_step(s, fe)
-                           : LOOP == kLoopTP                     ? c.phase == kPhaseContract && !s.tile_status && bit_step(s, n)
-                                                                 : c.phase == kPhaseContractExpand && bit_step(s, n));
+        // (few members keep the spread form up to the byte marks' rule)
+        const bool bits =
+            FASTV && !fast &&
+            ((LOOP == kLoopEC || LOOP == kLoopDO)
+                 ? c.phase == kPhaseExpandContract && (mark || n > (unsigned) kFastCap) && bit_step(s, fe)
+             : LOOP == kLoopTP ? c.phase == kPhaseContract && !s.tile_status && bit_step(s, n)
+                               : c.phase == kPhaseContractExpand && bit_step(s, n));
         const bool spread = (LOOP == kLoopEC || LOOP == kLoopDO) && c.phase == kPhaseExpandContract && !mark &&
                             n <= (unsigned) kFastCap && s.spread;
         // The first top-down step after bottom-up levels reads its frontier
         // from the bitmap they left, unless its form needs the queue (the
         // fast path, spread and marked steps index it).
-        const bool from_bitmap = bu_exit && !fast && !mark && !spread;
+        const bool from_bitmap = bu_exit && !fast && !mark && !bits && !spread;
         if (bu_exit && !from_bitmap) {
             queue_from_bitmap<PRED>(g, s, c, lds);  // clears both bitmaps
             bar(false);
@@ -2969,19 +2985,23 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
                     fbm_dirty |= 1u << ((c.iteration + 1) & 1);
                     fbm_exact_step = c.step + 1;
                 }
-                refresh();  // (visited words are read and written plainly)
+                refresh();  // (slabs and visited words are read plainly)
+                // (what others read next goes past the L2 and a light barrier
+                // follows: R-MAT scale 19 expand-contract 244 -> 235 us)
+                const bool through = EXACT;
                 if (LOOP == kLoopEC || LOOP == kLoopDO)
                     bits_collect<EXACT>(g, s, c, c.iteration + 1, B, s.q[(c.step + 1) & 1],
-                                        &s.ctl->qlen[(c.step + 1) % 3], fbm_out, s.track_edges != 0);
+                                        &s.ctl->qlen[(c.step + 1) % 3], fbm_out, s.track_edges != 0, through);
                 else if (LOOP == kLoopTP)
                     bits_collect<EXACT>(g, s, c, c.iteration, B, s.q[(c.step + 1) & 1],
-                                        &s.ctl->qlen[(c.step + 1) % 3], nullptr, false);
+                                        &s.ctl->qlen[(c.step + 1) % 3], nullptr, false, through);
                 else  // (the input is spent: its queue takes the members)
-                    bits_collect<EXACT>(g, s, c, c.iteration, B, s.q[c.step & 1], &s.ctl->compact, nullptr, false);
+                    bits_collect<EXACT>(g, s, c, c.iteration, B, s.q[c.step & 1], &s.ctl->compact, nullptr, false,
+                                        through);
                 __syncthreads();
                 init_lds(lds);
                 if (s.instrument) busy += wall_clock64() - t0;
-                bar(false);
+                bar(through);
                 if constexpr (LOOP == kLoopCE) {
                     // the members expand into the next edge frontier
                     const unsigned m = ld_agent(&s.ctl->compact);
@@ -2989,6 +3009,7 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
                     if (m > 0) {
                         if (blockIdx.x == 0 && threadIdx.x == 0) atomicMax(&s.ctl->max_depth, c.iteration);
                         t0 = s.instrument ? wall_clock64() : 0;
+                        refresh();
                         body_expand<PRED, EXACT>(g, s, c, m, lds, 0, true, xio);
                         if (s.instrument) busy += wall_clock64() - t0;
                         bar(false);

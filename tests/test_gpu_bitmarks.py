@@ -49,3 +49,11 @@ def test_rmat_repeated(gpu):
     # marks, slabs and counters left by one search do not show in the next
     g = CsrGraph.rmat(17, 24, seed=9)
     check(g, sources=tuple(int(s) for s in g.sample_sources(3, seed=2)))
+
+
+@pytest.mark.parametrize("targets", [20000, (1 << 18) - 1501, (1 << 18) - 1500])
+@pytest.mark.parametrize("below", [0, 1])
+def test_smallest_marked_step(gpu, targets, below):
+    # the second step has exactly the edges of the rule, or one less
+    work = (1 << 16) + (1501 + targets) // 2 - below
+    check(layered(1500, targets, work, 40))
