@@ -203,12 +203,36 @@ Cursor next_same(Cursor c)
     return c;
 }
 
+// (the expand step filters as well, except before a chained filter step)
 Cursor next_two_phase(Cursor c)
 {
     c.step++;
     if (c.phase == kPhaseContract) c.phase = kPhaseExpand;
-    else if (c.phase == kPhaseExpand) c.phase = kPhaseFilter;
     else { c.phase = kPhaseContract; c.iteration++; }
+    return c;
+}
+
+Cursor next_two_phase_chained(Cursor c)
+{
+    if (c.phase != kPhaseExpand) return next_two_phase(c);
+    c.step++;
+    c.phase = kPhaseFilter;
+    return c;
+}
+
+// Hybrid levels begin with the filter of their edge frontier, which with
+// `chained` off only the first has left to do.
+Cursor next_hybrid(Cursor c, bool chained)
+{
+    c.step++;
+    if (c.phase == kPhaseFilter) {
+        c.phase = kPhaseContract;
+    } else if (c.phase == kPhaseContract) {
+        c.phase = kPhaseExpand;
+    } else {
+        c.phase = chained ? kPhaseFilter : kPhaseContract;
+        c.iteration++;
+    }
     return c;
 }
 
@@ -237,20 +261,18 @@ bfs_status enact_hybrid(bfs_problem *p, const GraphArgs &g, const SearchArgs &s,
         // Two-phase levels: filter -> contract -> expand, until the filtered
         // edge frontier fits the persistent kernel again
         // (enactor_hybrid.cuh:386-532); the contract step that finds it so
-        // records where and stops the rest of the chunk.
+        // records where and stops the rest of the chunk.  The first filter
+        // step runs by itself, the others with the expand before them
+        // (chained compaction keeps them all).
         c = Cursor{h.exit_step, h.exit_iteration, kPhaseFilter};
         HIP_TRY(hipMemsetAsync(&p->d_ctl->hybrid_stop, 0, sizeof(unsigned), p->stream), "clear hand-back flag");
         while (true) {
             for (int k = 0; k < chunk; k++) {
-                HIP_TRY(launch_step(kPhaseFilter, p->mark_pred, exact, g, ts, c, sgrid, p->stream, launches),
-                        "launch filter");
-                Cursor cc{c.step + 1, c.iteration, kPhaseContract};
-                HIP_TRY(launch_step(kPhaseContract, p->mark_pred, exact, g, ts, cc, sgrid, p->stream, launches),
-                        "launch contract");
-                Cursor ce{c.step + 2, c.iteration, kPhaseExpand};
-                HIP_TRY(launch_step(kPhaseExpand, p->mark_pred, exact, g, ts, ce, sgrid, p->stream, launches),
-                        "launch expand");
-                c = Cursor{c.step + 3, c.iteration + 1, kPhaseFilter};
+                for (int level = c.iteration; c.iteration == level;) {
+                    HIP_TRY(launch_step(c.phase, p->mark_pred, exact, g, ts, c, sgrid, p->stream, launches),
+                            "launch two-phase step");
+                    c = next_hybrid(c, s.tile_status != nullptr);
+                }
             }
             st = read_control(p);
             if (st != BFS_OK) return st;
@@ -678,7 +700,8 @@ bfs_status bfs_enact(bfs_problem *p, bfs_strategy strategy, int32_t fused, int32
             HIP_TRY(launch_persistent(kLoopTP, p->mark_pred, exact, g, s, c, pgrid, p->stream), "launch persistent");
             launches++;
         } else {
-            st = run_iterative(p, g, s, c, sgrid, &launches, next_two_phase, nullptr);
+            st = run_iterative(p, g, s, c, sgrid, &launches,
+                               s.tile_status ? next_two_phase_chained : next_two_phase, nullptr);
         }
         break;
     case BFS_HYBRID:
