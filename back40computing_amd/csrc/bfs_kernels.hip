@@ -2897,7 +2897,11 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
         const bool contract_lds = ((LOOP == kLoopCE && c.phase == kPhaseContractExpand) ||
                                    (LOOP == kLoopTP && c.phase == kPhaseContract)) &&
                                   n <= (unsigned) kFastCap;
+        // Two-phase expand steps always take the grid: one workgroup alone
+        // also costs an entry barrier, and their rows may be long (a 1 M-vertex
+        // random tree 943 -> 900 us, R-MAT scale 15 186 -> 155 us).
         const bool fast = fast_level(s, c, n, fe) && gridDim.x > 1 && !(LOOP == kLoopCE && c.phase == kPhaseExpand) &&
+                          (LOOP != kLoopTP || c.phase == kPhaseContract) &&
                           ((LOOP != kLoopEC && LOOP != kLoopDO) || (n <= (unsigned) kFastCap && fe <= kFastEdges));
         // large top-down levels mark instead of claiming (grid-uniform: fe
         // is this step's frontier-edge count); few-member ones spread their
