@@ -830,6 +830,104 @@ __device__ __forceinline__ unsigned contract_tile(const GraphArgs &g, const Sear
                                                                  io);
 }
 
+// The rows of a large vertex frontier, waves alone: wave w takes runs w, w + waves, ... of up to 64 queue entries (the
+// high-degree members, claimed first, are spread over all of them), and
+// nothing but the published rows waits for the workgroup.  Rows of
+// kWaveRow edges and more are read a row per load instruction, eight rows
+// in flight; shorter ones share load instructions through the wave's edge
+// offsets, four of them in flight.  Rows of kWaveHubRow edges and more are
+// published: the grid tier follows behind a grid barrier.  `edges` gets the
+// neighbours (-1: none) and owners of four or eight edges per lane, called
+// wave-converged.  Returns this lane's share of the edges not published.
+// (A workgroup's row table, as gather_tile has it, left the waves of a
+// bit-marked step in step: 166 us for 437602 rows of 24.9 M edges, about 80
+// like this.)
+constexpr int kWaveRow = 32, kWaveHubRow = 512;
+
+template <typename Edges>
+__device__ __forceinline__ unsigned long long wave_rows(const GraphArgs &g, const int *in, unsigned n,
+                                                        const HubList &hub, RowTable &rt, Edges &&edges)
+{
+    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    int *excl = rt.excl[wave], *rb = rt.beg[wave], *rp = rt.par[wave];
+    unsigned long long met = 0;
+    // runs of equal length, as many for every wave
+    const unsigned stride = gridDim.x * kWaves;
+    const unsigned rounds = (n + stride * kWave - 1) / (stride * kWave);
+    const unsigned width = (n + stride * rounds - 1) / (stride * rounds), runs = (n + width - 1) / width;
+    unsigned t = (unsigned) wave * gridDim.x + blockIdx.x;
+    auto member = [&](unsigned run) {
+        const unsigned long long i = (unsigned long long) run * width + (unsigned) lane;
+        return (unsigned) lane < width && i < n ? ld_queue(in + i) : -1;
+    };
+    int v_next = member(t), b_next = 0, e_next = 0;
+    if (v_next >= 0) {
+        b_next = g.row[v_next];
+        e_next = g.row[v_next + 1];
+    }
+    constexpr int U = 8;  // rows in flight
+    for (; t < runs; t += stride) {
+        const int v = v_next, beg = b_next;
+        int end = e_next;
+        v_next = member(t + stride);
+        if (publish_hub_row(beg, end, v, hub)) end = beg;
+        met += (unsigned long long) (end - beg);
+        uint64_t wm = ballot(end - beg >= kWaveRow);
+        while (wm) {
+            int b[U], e[U], p[U], longest = 0;
+#pragma unroll
+            for (int q = 0; q < U; q++) {
+                const int l = wm ? uniform(__builtin_ctzll(wm)) : 0;
+                b[q] = readlane(beg, l);
+                e[q] = wm ? readlane(end, l) : b[q];
+                p[q] = readlane(v, l);
+                wm &= wm - 1;  // (0 stays 0)
+                longest = max(longest, e[q] - b[q]);
+            }
+            for (int k = lane; k - lane < longest; k += kWave) {
+                int u[U];
+#pragma unroll
+                for (int q = 0; q < U; q++) u[q] = k < e[q] - b[q] ? __builtin_nontemporal_load(g.col + b[q] + k) : -1;
+                edges(u, p);
+            }
+        }
+        // the next run's row bounds, behind its members
+        b_next = e_next = 0;
+        if (v_next >= 0) {
+            b_next = g.row[v_next];
+            e_next = g.row[v_next + 1];
+        }
+        const int len = end - beg < kWaveRow ? end - beg : 0;
+        const int incl = wave_inclusive_sum(len);
+        const int total = readlane(incl, kWave - 1);
+        if (total == 0) continue;
+        excl[lane] = incl - len;
+        rb[lane] = beg - (incl - len);
+        rp[lane] = v;
+        wave_lds_sync();
+        for (int r = 0; r < total; r += 4 * kWave) {
+            int u[4], p[4], at[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) at[q] = 0;
+#pragma unroll
+            for (int st = 32; st > 0; st >>= 1) {
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (excl[at[q] + st] <= r + q * kWave + lane) at[q] += st;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int x = r + q * kWave + lane;
+                u[q] = x < total ? __builtin_nontemporal_load(g.col + rb[at[q]] + x) : -1;
+                p[q] = rp[at[q]];
+            }
+            edges(u, p);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    return met;
+}
+
 // Expansion: every neighbour goes to the output queue.  A tile's edge count
 // is its output, so a tile of kDirectEdges and more reserves its place with
 // one atomic and writes there in order (the staging areas cost one atomic,
@@ -847,6 +945,13 @@ __device__ __forceinline__ unsigned contract_tile(const GraphArgs &g, const Sear
 // factor 24, went from 605 to 489 us, of a 1 M-vertex random tree with
 // predecessors from 1150 to 943 us.
 constexpr int kDirectEdges = 4096;
+// Rows per wave past which the waves of a filtering expansion work alone in a
+// persistent loop (two-phase search of R-MAT scale 19, edge factor 24: 449 us
+// with workgroup tiles, 389 / 383 / 385 / 385 from 0 / 1 / 4 / 16 rows; scale
+// 18, edge factor 8: 282, and 238 / 237 / 240 / 250).  A launch per step has
+// two workgroups a CU to cover the tiles' barriers (the 24.4 M-edge step of
+// an R-MAT scale 20 hybrid search: 20 us slower with waves alone).
+constexpr unsigned kRowsPerWave = 1;
 
 template <bool PRED, bool MAYFILTER = false>
 struct Expansion {
@@ -867,14 +972,15 @@ struct Expansion {
           wrote(false), lost(false), filter(MAYFILTER && filter_), coherent(io.stale), seen(0)
     {
     }
-    __device__ __forceinline__ void push_unvisited(const int (&u)[4], const int (&pv)[4])
+    template <int N>
+    __device__ __forceinline__ void push_unvisited(const int (&u)[N], const int (&pv)[N])
     {
-        unsigned w[4];
+        unsigned w[N];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < N; j++)
             w[j] = u[j] < 0 ? ~0u : coherent ? ld_agent(s.visited + (u[j] >> 5)) : s.visited[u[j] >> 5];
 #pragma unroll
-        for (int j = 0; j < 4; j++) wq.push(!((w[j] >> (u[j] & 31)) & 1u), u[j], pv[j]);
+        for (int j = 0; j < N; j++) wq.push(!((w[j] >> (u[j] & 31)) & 1u), u[j], pv[j]);
     }
     // Accounts the filter step's input: its length, and the overflow of an
     // edge queue that could not have held it.
@@ -995,13 +1101,24 @@ __device__ __forceinline__ void body_contract_expand(const GraphArgs &g, const S
 }
 
 // filter: the filter step runs with it (see Expansion).
-template <bool PRED, bool EXACT, bool MAYFILTER = false>
+template <bool PRED, bool EXACT, bool MAYFILTER = false, bool WAVES = false>
 __device__ __forceinline__ void body_expand(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds, int sub,
                             bool hubs, StepIo io, bool filter = false)
 {
     Expansion<PRED, MAYFILTER> x(g, s, c, lds, io, filter);
     const int *in = s.q[c.step & 1];
-    if (sub == 0) {
+    if (sub == 0 && WAVES && filter && hubs && n > gridDim.x * kWaves * kRowsPerWave) {
+        HubList hub = x.hubs(n, hubs);
+        if (hub.grid_t != 0x7fffffff) hub.grid_t = min(hub.grid_t, kWaveHubRow);
+        const unsigned long long met = wave_rows(
+            g, in, n, hub, lds.rt, [&](const auto &u, const auto &p) { x.push_unvisited(u, p); });
+        // (fewer than 2^31 edges in all)
+        const int sum = wave_inclusive_sum((int) met);
+        if (lane_id() == kWave - 1) lds.ep_fe[threadIdx.x / kWave] = (unsigned long long) (unsigned) sum;
+        __syncthreads();
+        for (int w = 0; w < kWaves; w++) x.seen += lds.ep_fe[w];
+        __syncthreads();  // (finish_step writes them again)
+    } else if (sub == 0) {
         const HubList hub = x.hubs(n, hubs);
         TileGrab tg = tile_grab(s, n, lds, kBlock, gridDim.x);
         while (true) {
@@ -1231,7 +1348,8 @@ __device__ __forceinline__ void loop_body(int phase, const GraphArgs &g, const S
         else body_expand_contract<PRED, EXACT>(g, s, c, n, lds, sub, hubs, fe, io, next_bits, from_bitmap);
     } else {
         if (phase == kPhaseContract) body_contract<PRED, EXACT>(g, s, c, n, lds, io);
-        else if (phase == kPhaseExpand) body_expand<PRED, EXACT, true>(g, s, c, n, lds, sub, hubs, io, filters(s));
+        else if (phase == kPhaseExpand)
+            body_expand<PRED, EXACT, true, true>(g, s, c, n, lds, sub, hubs, io, filters(s));
         else body_filter<PRED, EXACT>(g, s, c, n, lds, io);
     }
 }
@@ -1946,104 +2064,19 @@ __device__ __forceinline__ void bits_clear(const SearchArgs &s, unsigned *vbits)
 }
 static_assert(kFastVisitedWords % 4 == 0, "the bitmap is cleared 16 bytes at a time");
 
-// Marks the targets of the rows of the vertex frontier of step c.  Waves work
-// alone: wave w takes runs w, w + waves, ... of up to 64 queue entries (the
-// high-degree members, claimed first, are spread over all of them), and
-// nothing but the published rows waits for the workgroup.  Rows of
-// kBitWaveRow edges and more are read a row per load instruction, eight rows
-// in flight; shorter ones share load instructions through the wave's edge
-// offsets, four of them in flight.  Rows of kBitHubRow edges and more are
-// published: bits_from_hubs follows behind a grid barrier.
-// (A workgroup's row table, as gather_tile has it, left the waves in step:
-// 166 us for 437602 rows of 24.9 M edges, about 80 like this.)
-constexpr int kBitWaveRow = 32, kBitHubRow = 512;
-
+// Marks the targets of the rows of the vertex frontier of step c (the rows
+// published for the grid tier follow in bits_from_hubs, behind a barrier).
 template <bool PRED, bool EXACT>
 __device__ __forceinline__ void bits_from_rows(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n,
                                                BitLds &B, unsigned *vbits)
 {
-    const int *in = s.q[c.step & 1];
     HubList hub = hub_list(s, c.step, true, n);
-    hub.grid_t = min(s.grid_t, kBitHubRow);
-    const int lane = lane_id(), wave = threadIdx.x / kWave;
-    int *excl = B.rt.excl[wave], *rb = B.rt.beg[wave], *rp = B.rt.par[wave];
-    // runs of equal length, as many for every wave
-    const unsigned stride = gridDim.x * kWaves;
-    const unsigned rounds = (n + stride * kWave - 1) / (stride * kWave);
-    const unsigned width = (n + stride * rounds - 1) / (stride * rounds), runs = (n + width - 1) / width;
-    unsigned t = (unsigned) wave * gridDim.x + blockIdx.x;
-    auto member = [&](unsigned run) {
-        const unsigned long long i = (unsigned long long) run * width + (unsigned) lane;
-        return (unsigned) lane < width && i < n ? ld_queue(in + i) : -1;
-    };
-    int v_next = member(t), b_next = 0, e_next = 0;
-    if (v_next >= 0) {
-        b_next = g.row[v_next];
-        e_next = g.row[v_next + 1];
-    }
-    constexpr int U = 8;  // rows in flight
-    for (; t < runs; t += stride) {
-        const int v = v_next, beg = b_next;
-        int end = e_next;
-        v_next = member(t + stride);
-        if (publish_hub_row(beg, end, v, hub)) end = beg;
-        uint64_t wm = ballot(end - beg >= kBitWaveRow);
-        while (wm) {
-            int b[U], e[U], p[U], longest = 0;
+    hub.grid_t = min(s.grid_t, kWaveHubRow);
+    wave_rows(g, s.q[c.step & 1], n, hub, B.rt, [&](const auto &u, const auto &p) {
 #pragma unroll
-            for (int q = 0; q < U; q++) {
-                const int l = wm ? uniform(__builtin_ctzll(wm)) : 0;
-                b[q] = readlane(beg, l);
-                e[q] = wm ? readlane(end, l) : b[q];
-                p[q] = readlane(v, l);
-                wm &= wm - 1;  // (0 stays 0)
-                longest = max(longest, e[q] - b[q]);
-            }
-            for (int k = lane; k - lane < longest; k += kWave) {
-                int u[U];
-#pragma unroll
-                for (int q = 0; q < U; q++) u[q] = k < e[q] - b[q] ? __builtin_nontemporal_load(g.col + b[q] + k) : -1;
-#pragma unroll
-                for (int q = 0; q < U; q++)
-                    if (u[q] >= 0) bit_mark<PRED, EXACT>(s, vbits, u[q], p[q]);
-            }
-        }
-        // the next run's row bounds, behind its members
-        b_next = e_next = 0;
-        if (v_next >= 0) {
-            b_next = g.row[v_next];
-            e_next = g.row[v_next + 1];
-        }
-        const int len = end - beg < kBitWaveRow ? end - beg : 0;
-        const int incl = wave_inclusive_sum(len);
-        const int total = readlane(incl, kWave - 1);
-        if (total == 0) continue;
-        excl[lane] = incl - len;
-        rb[lane] = beg - (incl - len);
-        rp[lane] = v;
-        wave_lds_sync();
-        for (int r = 0; r < total; r += 4 * kWave) {
-            int u[4], p[4], at[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) at[q] = 0;
-#pragma unroll
-            for (int st = 32; st > 0; st >>= 1) {
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-                    if (excl[at[q] + st] <= r + q * kWave + lane) at[q] += st;
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int x = r + q * kWave + lane;
-                u[q] = x < total ? __builtin_nontemporal_load(g.col + rb[at[q]] + x) : -1;
-                p[q] = rp[at[q]];
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                if (u[q] >= 0) bit_mark<PRED, EXACT>(s, vbits, u[q], p[q]);
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
+        for (int q = 0; q < (int) (sizeof(u) / sizeof(u[0])); q++)
+            if (u[q] >= 0) bit_mark<PRED, EXACT>(s, vbits, u[q], p[q]);
+    });
 }
 
 // Index of the last grid-tier entry whose first chunk is <= ch, by the whole
@@ -3029,7 +3062,7 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
                 bits_clear(s, vbits);
                 if constexpr (LOOP == kLoopEC || LOOP == kLoopDO) {
                     bits_from_rows<PRED, EXACT>(g, s, c, n, B, vbits);
-                    if (s.max_degree >= min(s.grid_t, kBitHubRow)) {
+                    if (s.max_degree >= min(s.grid_t, kWaveHubRow)) {
                         bar(true);
                         refresh();  // (the list is read through the caches)
                         bits_from_hubs<PRED, EXACT>(g, s, c, vbits);

@@ -60,3 +60,23 @@ def test_edges_past_the_queue(gpu, compaction, strategy, fused):
     p.enact(strategy, 0, fused=fused)
     assert oracle.compare(p.extract_depths(), oracle.bfs(g.row_offsets, g.column_indices, 0)[0]) == -1
     p.destroy()
+
+
+@pytest.mark.parametrize("members", [2047, 2048, 2049, 131072, 131073])
+@pytest.mark.parametrize("cull", [b40c.CULL_EXACT, b40c.CULL_BEST_EFFORT], ids=["exact", "best_effort"])
+def test_rows_of_a_step_by_waves(gpu, members, cull):
+    # 0 -> members, whose rows have 0, 1, 31, 32, 33 and 511 to 513 edges: as
+    # many members as the waves of a full grid, and a full run for each wave
+    rng = np.random.default_rng(members)
+    deg = rng.integers(0, 3, members)
+    deg[rng.choice(members, 40, replace=False)] = np.tile([31, 32, 33, 511, 512, 513, 64, 2049], 5)
+    targets = 600000
+    src = np.concatenate([np.zeros(members, np.int64), np.repeat(1 + np.arange(members), deg)])
+    dst = np.concatenate([1 + np.arange(members), 1 + members + rng.integers(0, targets, int(deg.sum()))])
+    g = CsrGraph.from_coo(1 + members + targets, src, dst)
+    p = CsrProblem(mark_predecessors=members % 2 == 0).from_host_problem(g)
+    p.set_config(cull_mode=cull)
+    p.reset(b40c.EDGE_FRONTIERS, 2.0)
+    p.enact(b40c.TWO_PHASE, 0)
+    assert oracle.compare(p.extract_depths(), oracle.bfs(g.row_offsets, g.column_indices, 0)[0]) == -1
+    p.destroy()
