@@ -34,7 +34,8 @@ struct ChainState {
     long long capacity = 0;                   // status words allocated
     unsigned epoch = 0;
 
-    hipError_t init(int dev);
+    // The launches that follow are all on st.
+    hipError_t init(int dev, hipStream_t st);
     // Status words and a fresh epoch for a launch over `items` in tiles of
     // tile_items.  (The tile counter needs no clearing: the workgroup that
     // takes a launch's last tile sets it back to zero, prim::take_tile.)

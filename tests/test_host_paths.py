@@ -1,0 +1,54 @@
+"""The library's host paths over a stand-in HIP runtime (hip_stub.c, built
+here with the host compiler): what they order before a launch, and what they
+do where device memory ends.  Kernels do not run, so results are not looked
+at; every test is a process of its own."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    d = tmp_path_factory.mktemp("hip_stub")
+    so = d / "libamdhip64.so.7"
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-Wl,-soname,libamdhip64.so.7", "-o", str(so),
+                    os.path.join(HERE, "hip_stub", "hip_stub.c")], check=True)
+    return str(d)
+
+
+def run(stub, body):
+    script = textwrap.dedent("""
+        import ctypes, sys
+        import numpy as np
+        sys.path.insert(0, %r)
+        from back40computing_amd import BfsError, CsrGraph, CsrProblem, _native
+        from back40computing_amd.primitives import DeviceCsr, ScanEnactor
+        hip = ctypes.CDLL("libamdhip64.so.7")
+        hip.stub_used.restype = ctypes.c_size_t
+        hip.stub_budget.argtypes = [ctypes.c_size_t]
+        hip.stub_refuse.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
+        _native.load()
+    """ % ROOT) + textwrap.dedent(body)
+    env = dict(os.environ, LD_LIBRARY_PATH=stub)
+    p = subprocess.run([sys.executable, "-c", script], env=env, capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0, p.stdout + p.stderr
+
+
+def test_tile_counters_are_clear_before_the_first_launch(stub):
+    # an enactor's and a builder's streams do not wait for the null stream
+    run(stub, """
+        for n in (1, 100000):
+            e = ScanEnactor()
+            a = np.zeros(n, np.uint32)
+            e.scan(a.ctypes.data, a.ctypes.data, n)
+            e.copy_if(a.ctypes.data, a.ctypes.data, n)
+        DeviceCsr.from_coo(100, np.zeros(5000, np.int32), np.ones(5000, np.int32), dedup=True)
+        assert hip.stub_launches() > 0
+        assert hip.stub_unordered() == 0, hip.stub_unordered()
+    """)
