@@ -302,6 +302,13 @@ __device__ __forceinline__ int row_of_edge(const int *row, int nodes, long long 
 // last of several starting at one edge is the one with edges), and a running
 // maximum hands every edge its row.  (A search per edge, 20 dependent loads,
 // made 16 M edges 249 us; 55 now.)
+// A tile of more than kWalkRows rows an edge searches all the same, a thread's
+// sixteen edges together: its empty rows have no bound, and one workgroup
+// walked all of them (whole transposes of 1000 edges over 2^21 vertices
+// 3051 us walked, 680 searched; of 5000 over 20 M 19360 and 1250; 300 k over
+// 2^21, seven rows an edge, 83 to 109 us either way, as from 1 to 16).
+constexpr int kWalkRows = 4;
+
 __global__ __launch_bounds__(kThreads) void transpose_keys_kernel(const int *row, const int *col, int nodes,
                                                                   long long edges, int bits,
                                                                   unsigned long long *keys)
@@ -315,6 +322,28 @@ __global__ __launch_bounds__(kThreads) void transpose_keys_kernel(const int *row
     if (threadIdx.x == prim::kWave) s_last = row_of_edge(row, nodes, e0 + count - 1);
     __syncthreads();
     const int first = s_first, last = s_last;
+    if (last - first > kWalkRows * kTile) {  // workgroup-uniform
+        int r[kRounds], top = 1;
+#pragma unroll
+        for (int k = 0; k < kRounds; k++) r[k] = first;
+        while (2 * (long long) top <= last - first) top *= 2;
+        for (int st = top; st > 0; st >>= 1) {
+            int at[kRounds];
+#pragma unroll
+            for (int k = 0; k < kRounds; k++) at[k] = row[min((long long) r[k] + st, (long long) last)];
+#pragma unroll
+            for (int k = 0; k < kRounds; k++) {
+                const int i = min(k * kThreads + (int) threadIdx.x, count - 1);
+                if ((long long) r[k] + st <= last && at[k] <= e0 + i) r[k] += st;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kRounds; k++) {
+            const int i = k * kThreads + (int) threadIdx.x;
+            if (i < count) keys[e0 + i] = ((unsigned long long) (unsigned) col[e0 + i] << bits) | (unsigned) r[k];
+        }
+        return;
+    }
     for (int u = first + 1 + (int) threadIdx.x; u <= last; u += kThreads) {
         const int at = (int) ((long long) row[u] - e0);
         if (at >= 0 && at < count) atomicMax(&s_row[at], u);
