@@ -391,6 +391,40 @@ void free_queues(bfs_problem *p)
     p->q_cap = 0;
 }
 
+// Both queues (of cap elements) and the tile status words; none on failure.
+hipError_t allocate_queues(bfs_problem *p, size_t cap, size_t words)
+{
+    hipError_t e = hipMalloc(&p->d_tile_status, sizeof(unsigned long long) * words);
+    for (int i = 0; i < 2 && e == hipSuccess; i++) {
+        e = hipMalloc(&p->d_q[i], sizeof(int) * cap);
+        if (e == hipSuccess && p->mark_pred) e = hipMalloc(&p->d_pq[i], sizeof(int) * cap);
+    }
+    if (e != hipSuccess) free_queues(p);
+    return e;
+}
+
+// Device memory that only makes searches faster: what does not fit is done
+// without (every search has a form that needs none of it), and given up where
+// the queues need the room.
+bool optional_malloc(unsigned **buffer, size_t bytes)
+{
+    if (hipMalloc(buffer, bytes) == hipSuccess) return true;
+    (void) hipGetLastError();  // (no error of the launches that follow)
+    *buffer = nullptr;
+    return false;
+}
+
+bool drop_optional(bfs_problem *p)
+{
+    if (!p->d_slabs && !p->d_adj) return false;
+    (void) hipGetLastError();
+    if (p->d_slabs) (void) hipFree(p->d_slabs);
+    if (p->d_adj) (void) hipFree(p->d_adj);
+    p->d_slabs = p->d_adj = nullptr;
+    p->adj_width = 0;
+    return true;
+}
+
 }  // namespace
 
 extern "C" {
@@ -486,10 +520,6 @@ bfs_status bfs_problem_create(const int32_t *h_row_offsets, const int32_t *h_col
         (e = hipMalloc(&p->d_fbm, sizeof(unsigned) * 2 * words)) != hipSuccess ||
         (e = hipMalloc(&p->d_marks, 32 * words)) != hipSuccess)
         return cleanup(hip_fail(e, "allocate problem"));
-    // (no step of a graph with fewer edges uses them)
-    if (nodes <= BFS_FAST_VISITED_MAX && (unsigned long long) edges >= bit_mark_work(nodes) &&
-        (e = hipMalloc(&p->d_slabs, 16 * slab_quads(nodes) * (size_t) p->num_cus)) != hipSuccess)
-        return cleanup(hip_fail(e, "allocate bit-mark slabs"));
     // marks are clear between steps (each compaction clears what it reads)
     if ((e = hipMemset(p->d_marks, 0, 32 * words)) != hipSuccess) return cleanup(hip_fail(e, "clear marks"));
     if (p->mark_pred && (e = hipMalloc(&p->d_pred, sizeof(int) * (size_t) nodes)) != hipSuccess)
@@ -506,15 +536,6 @@ bfs_status bfs_problem_create(const int32_t *h_row_offsets, const int32_t *h_col
     if (edges > 0 &&
         (e = hipMemcpy(p->d_col, h_column_indices, sizeof(int) * (size_t) edges, hipMemcpyHostToDevice)) != hipSuccess)
         return cleanup(hip_fail(e, "copy column indices"));
-
-    p->adj_width = adjacency_width(nodes, p->max_degree);
-    if (p->adj_width) {
-        if ((e = hipMalloc(&p->d_adj, sizeof(unsigned) * (size_t) p->adj_width * (size_t) nodes)) != hipSuccess)
-            return cleanup(hip_fail(e, "allocate adjacency records"));
-        if ((e = launch_adjacency(p->d_row, p->d_col, nodes, p->adj_width, p->d_adj, p->stream)) != hipSuccess ||
-            (e = hipStreamSynchronize(p->stream)) != hipSuccess)
-            return cleanup(hip_fail(e, "write adjacency records"));
-    }
 
     // Bottom-up levels scan in-neighbours: reuse the CSR when the graph is
     // symmetric, otherwise upload its transpose.
@@ -538,6 +559,16 @@ bfs_status bfs_problem_create(const int32_t *h_row_offsets, const int32_t *h_col
         b40c_graph_free(&t);
         if (!ok) return cleanup(fail(BFS_ERR_OOM, "allocate or copy the transpose"));
     }
+    const int width = adjacency_width(nodes, p->max_degree);
+    if (width && optional_malloc(&p->d_adj, sizeof(unsigned) * (size_t) width * (size_t) nodes)) {
+        p->adj_width = width;
+        if ((e = launch_adjacency(p->d_row, p->d_col, nodes, p->adj_width, p->d_adj, p->stream)) != hipSuccess ||
+            (e = hipStreamSynchronize(p->stream)) != hipSuccess)
+            return cleanup(hip_fail(e, "write adjacency records"));
+    }
+    // (no step of a graph with fewer edges uses them)
+    if (nodes <= BFS_FAST_VISITED_MAX && (unsigned long long) edges >= bit_mark_work(nodes))
+        (void) optional_malloc(&p->d_slabs, 16 * slab_quads(nodes) * (size_t) p->num_cus);
     *out = p;
     return BFS_OK;
 }
@@ -555,12 +586,10 @@ bfs_status bfs_problem_reset(bfs_problem *p, bfs_frontier_type ft, double queue_
     size_t cap = (size_t) want;
     if (cap > p->q_cap) {
         free_queues(p);
-        for (int i = 0; i < 2; i++) {
-            HIP_TRY(hipMalloc(&p->d_q[i], sizeof(int) * cap), "allocate frontier queue");
-            if (p->mark_pred) HIP_TRY(hipMalloc(&p->d_pq[i], sizeof(int) * cap), "allocate predecessor queue");
-        }
         const size_t words = cap / kBlock + 2;
-        HIP_TRY(hipMalloc(&p->d_tile_status, sizeof(unsigned long long) * words), "allocate tile status words");
+        hipError_t e = allocate_queues(p, cap, words);
+        if (e == hipErrorOutOfMemory && drop_optional(p)) e = allocate_queues(p, cap, words);
+        HIP_TRY(e, "allocate frontier queues");
         HIP_TRY(hipMemsetAsync(p->d_tile_status, 0, sizeof(unsigned long long) * words, p->stream),
                 "clear tile status words");
         p->scan_epoch = 1;

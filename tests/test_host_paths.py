@@ -52,3 +52,46 @@ def test_tile_counters_are_clear_before_the_first_launch(stub):
         assert hip.stub_launches() > 0
         assert hip.stub_unordered() == 0, hip.stub_unordered()
     """)
+
+
+@pytest.mark.parametrize("graph,extra", [
+    ("CsrGraph.random(50000, 200000, seed=1)", "16 * 400 * 256"),   # a bit-mark slab for each of 256 CUs
+    ("CsrGraph.grid2d(100)", "4 * 4 * 10000"),                      # adjacency records of four words
+])
+def test_problems_do_without_memory_that_only_speeds_them_up(stub, graph, extra):
+    run(stub, """
+        import back40computing_amd as b40c
+        g, extra = %s, %s
+        p = CsrProblem(mark_predecessors=True).from_host_problem(g)
+        with_it = hip.stub_used()
+        assert p.device_info()["device_bytes"] > extra
+        p.destroy()
+        hip.stub_refuse(extra, extra)
+        p = CsrProblem(mark_predecessors=True).from_host_problem(g)
+        assert with_it - hip.stub_used() == extra
+        p.reset(b40c.bfs._native.load().bfs_strategy_frontier_type(b40c.HYBRID), 1.3)
+        for s in (b40c.CONTRACT_EXPAND, b40c.TWO_PHASE, b40c.HYBRID):
+            for fused in (True, False):
+                p.enact(s, 0, fused=fused)
+    """ % (graph, extra))
+
+
+@pytest.mark.parametrize("graph", ["CsrGraph.random(50000, 200000, seed=1)", "CsrGraph.grid2d(100)"])
+def test_queues_come_before_such_memory(stub, graph):
+    run(stub, """
+        import back40computing_amd as b40c
+        p = CsrProblem().from_host_problem(%s)
+        edges = b40c.bfs._native.load().bfs_strategy_frontier_type(b40c.HYBRID)
+        full = hip.stub_used()
+        need = 2 * 4 * int(np.ceil(1.3 * p.edges)) + 8 * (int(np.ceil(1.3 * p.edges)) // 512 + 2)
+        hip.stub_budget(full + need - 1)
+        p.reset(edges, 1.3)
+        assert hip.stub_used() < full + need
+        p.enact(b40c.HYBRID, 0)
+        hip.stub_budget(hip.stub_used())
+        try:
+            p.reset(edges, 2.6)
+            raise SystemExit("a queue larger than the device")
+        except BfsError:
+            pass
+    """ % graph)
