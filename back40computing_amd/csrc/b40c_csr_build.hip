@@ -651,10 +651,11 @@ int b40c_device_csr_from_coo(int32_t device, int32_t nodes, int64_t num_pairs, c
     const long long n = (symmetrize ? 2 : 1) * (long long) num_pairs;
     // the device checks the pairs; where it does not get to see them, they
     // are checked here (an invalid pair is the first error reported)
-    const int rc = n > (long long) UINT32_MAX ? 3 : device_ok(device);  // (sort offsets are 32-bit)
-    if (rc) return pairs_inside(h_src, h_dst, num_pairs, nodes) ? rc : 1;
+    auto unseen = [&](int rc) { return pairs_inside(h_src, h_dst, num_pairs, nodes) ? rc : 1; };
+    if (n > (long long) UINT32_MAX) return unseen(3);  // (sort offsets are 32-bit)
+    if (int rc = device_ok(device)) return unseen(rc);
     Builder b;
-    if (!b.start(device)) return b.status;
+    if (!b.start(device)) return unseen(b.status);
     const int bits = bits_for(nodes);
     long long edges = 0;
     if (n > 0) {
@@ -663,11 +664,11 @@ int b40c_device_csr_from_coo(int32_t device, int32_t nodes, int64_t num_pairs, c
         if (!b.alloc(n, 0, num_pairs) || !b.ok(hipMemcpyAsync(b.src, h_src, pb, hipMemcpyHostToDevice, b.stream)) ||
             !b.ok(hipMemcpyAsync(b.dst, h_dst, pb, hipMemcpyHostToDevice, b.stream)) ||
             !b.ok(hipMemsetAsync(b.key_counts(), 0, sizeof(KeyCounts), b.stream)))
-            return b.status;
+            return unseen(b.status);
         hipLaunchKernelGGL(pair_keys_kernel, dim3(grid_for(num_pairs)), dim3(kThreads), 0, b.stream, b.src, b.dst,
                            (long long) num_pairs, nodes, bits, symmetrize ? 1 : 0, drop_self_loops ? 1 : 0, b.keys[0],
                            b.key_counts());
-        if (!b.ok(hipGetLastError()) || !b.read_key_counts(&kc)) return b.status;
+        if (!b.ok(hipGetLastError()) || !b.read_key_counts(&kc)) return unseen(b.status);
         if (kc.outside) return 1;
         if (!b.sort(n, 2 * bits) || !b.compact(n, (long long) kc.loops, dedup != 0, &edges)) return b.status;
     }

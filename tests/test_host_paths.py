@@ -95,3 +95,20 @@ def test_queues_come_before_such_memory(stub, graph):
         except BfsError:
             pass
     """ % graph)
+
+
+def test_invalid_pairs_are_reported_before_a_lack_of_memory(stub):
+    # the pairs are the first thing wrong with the call, whatever else would have failed
+    run(stub, """
+        lib = _native.load()
+        out = _native.DeviceCsrStruct()
+        src, dst = np.zeros(5000, np.int32), np.ones(5000, np.int32)
+        bad = dst.copy()
+        bad[4999] = 100
+        call = lambda d: lib.b40c_device_csr_from_coo(0, 100, 5000, _native.i32ptr(src), _native.i32ptr(d), 1, 0, 0,
+                                                      ctypes.byref(out))
+        for room in (0, 100, 1000, 50000):
+            hip.stub_budget(room)
+            assert call(dst) == 2, room
+            assert call(bad) == 1, room
+    """)
