@@ -393,7 +393,8 @@ int bits_for(int nodes)
 // and freeing 260 MB took longer than transposing 16 M edges (1.3 ms of 2.7,
 // on some boxes 8 of 9.5).  One build at a time has the kept set; others at
 // the same time make their own.  The block stays below kKeepBytes, and goes
-// back to the device when the last device CSR built here is freed.
+// back to the device when the last device CSR built here is freed, or when
+// an allocation of the library finds no room (device_malloc, run_build).
 constexpr size_t kKeepBytes = (size_t) 512 << 20;
 constexpr int kKeepDevices = 64;
 
@@ -419,7 +420,7 @@ struct BuildSet {
     {
         if (need <= bytes) return hipSuccess;
         release_block();
-        hipError_t e = hipMalloc(reinterpret_cast<void **>(&block), need);
+        hipError_t e = device_malloc(&block, need);
         if (e != hipSuccess) {
             block = nullptr;
             return e;
@@ -460,6 +461,7 @@ struct Builder {
     int *perm = nullptr;
     int *src = nullptr, *dst = nullptr;
     int status = 0;  // first failure: 1 invalid, 2 out of memory, 4 device error
+    size_t need = 0; // bytes of the block that the build uses
 
     ~Builder()
     {
@@ -472,6 +474,17 @@ struct Builder {
         std::lock_guard<std::mutex> lock(g_keep_mu);
         if (set->bytes > kKeepBytes || g_live[device] == 0) set->release_block();
         set->busy = false;
+    }
+
+    // After a build that ran out of memory: whether the kept block held more
+    // than it needed; the block is released.
+    bool gives_room()
+    {
+        if (!set || set == &own || set->bytes <= need) return false;
+        (void) hipStreamSynchronize(stream);
+        set->release_block();
+        (void) hipGetLastError();
+        return true;
     }
 
     bool ok(hipError_t e)
@@ -507,7 +520,8 @@ struct Builder {
         const size_t tiles = ((size_t) std::max(1LL, n) + kTile - 1) / kTile;
         const size_t cb = up(sizeof(unsigned) * tiles * kDigits);
         const size_t pb = up(sizeof(int) * (size_t) perm_n), qb = up(sizeof(int) * (size_t) pairs_n);
-        if (!ok(set->reserve(2 * kb + cb + pb + 2 * qb))) return false;
+        need = 2 * kb + cb + pb + 2 * qb;
+        if (!ok(set->reserve(need))) return false;
         char *at = set->block;
         keys[0] = reinterpret_cast<unsigned long long *>(at);
         keys[1] = reinterpret_cast<unsigned long long *>(at + kb);
@@ -584,8 +598,8 @@ struct Builder {
             return false;
         }
         int *row = nullptr, *col = nullptr;
-        if (!ok(hipMalloc(&row, sizeof(int) * ((size_t) nodes + 1))) ||
-            !ok(hipMalloc(&col, sizeof(int) * (size_t) std::max(1LL, edges)))) {
+        if (!ok(device_malloc(&row, sizeof(int) * ((size_t) nodes + 1))) ||
+            !ok(device_malloc(&col, sizeof(int) * (size_t) std::max(1LL, edges)))) {
             if (row) (void) hipFree(row);
             return false;
         }
@@ -615,6 +629,18 @@ struct Builder {
     }
 };
 
+// Runs one build, and once more if it ran out of memory beside a kept block
+// larger than its own.
+template <typename Build>
+int run_build(int device, Build &&build)
+{
+    for (bool again = false;; again = true) {
+        Builder b;
+        const int rc = b.start(device) ? build(b) : b.status;
+        if (rc != 2 || again || !b.gives_room()) return rc;
+    }
+}
+
 int device_ok(int32_t device)
 {
     int count = 0;
@@ -630,6 +656,24 @@ bool pairs_inside(const int32_t *src, const int32_t *dst, int64_t pairs, int32_t
 }
 
 }  // namespace
+
+hipError_t device_malloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    {
+        std::lock_guard<std::mutex> lock(g_keep_mu);
+        bool room = false;
+        for (BuildSet &k : g_keep) {
+            if (k.busy || !k.block) continue;
+            k.release_block();
+            room = true;
+        }
+        if (!room) return e;
+    }
+    (void) hipGetLastError();
+    return hipMalloc(p, bytes);
+}
 
 void device_csr_gone(int device)
 {
@@ -654,26 +698,30 @@ int b40c_device_csr_from_coo(int32_t device, int32_t nodes, int64_t num_pairs, c
     auto unseen = [&](int rc) { return pairs_inside(h_src, h_dst, num_pairs, nodes) ? rc : 1; };
     if (n > (long long) UINT32_MAX) return unseen(3);  // (sort offsets are 32-bit)
     if (int rc = device_ok(device)) return unseen(rc);
-    Builder b;
-    if (!b.start(device)) return unseen(b.status);
-    const int bits = bits_for(nodes);
-    long long edges = 0;
-    if (n > 0) {
-        const size_t pb = sizeof(int) * (size_t) num_pairs;
-        KeyCounts kc;
-        if (!b.alloc(n, 0, num_pairs) || !b.ok(hipMemcpyAsync(b.src, h_src, pb, hipMemcpyHostToDevice, b.stream)) ||
-            !b.ok(hipMemcpyAsync(b.dst, h_dst, pb, hipMemcpyHostToDevice, b.stream)) ||
-            !b.ok(hipMemsetAsync(b.key_counts(), 0, sizeof(KeyCounts), b.stream)))
-            return unseen(b.status);
-        hipLaunchKernelGGL(pair_keys_kernel, dim3(grid_for(num_pairs)), dim3(kThreads), 0, b.stream, b.src, b.dst,
-                           (long long) num_pairs, nodes, bits, symmetrize ? 1 : 0, drop_self_loops ? 1 : 0, b.keys[0],
-                           b.key_counts());
-        if (!b.ok(hipGetLastError()) || !b.read_key_counts(&kc)) return unseen(b.status);
-        if (kc.outside) return 1;
-        if (!b.sort(n, 2 * bits) || !b.compact(n, (long long) kc.loops, dedup != 0, &edges)) return b.status;
-    }
-    if (!b.finish(nodes, edges, bits, symmetrize != 0, out)) return b.status ? b.status : 4;
-    return 0;
+    bool seen = n == 0;
+    const int rc = run_build(device, [&](Builder &b) {
+        const int bits = bits_for(nodes);
+        long long edges = 0;
+        if (n > 0) {
+            const size_t pb = sizeof(int) * (size_t) num_pairs;
+            KeyCounts kc;
+            if (!b.alloc(n, 0, num_pairs) ||
+                !b.ok(hipMemcpyAsync(b.src, h_src, pb, hipMemcpyHostToDevice, b.stream)) ||
+                !b.ok(hipMemcpyAsync(b.dst, h_dst, pb, hipMemcpyHostToDevice, b.stream)) ||
+                !b.ok(hipMemsetAsync(b.key_counts(), 0, sizeof(KeyCounts), b.stream)))
+                return b.status;
+            hipLaunchKernelGGL(pair_keys_kernel, dim3(grid_for(num_pairs)), dim3(kThreads), 0, b.stream, b.src, b.dst,
+                               (long long) num_pairs, nodes, bits, symmetrize ? 1 : 0, drop_self_loops ? 1 : 0,
+                               b.keys[0], b.key_counts());
+            if (!b.ok(hipGetLastError()) || !b.read_key_counts(&kc)) return b.status;
+            seen = true;
+            if (kc.outside) return 1;
+            if (!b.sort(n, 2 * bits) || !b.compact(n, (long long) kc.loops, dedup != 0, &edges)) return b.status;
+        }
+        if (!b.finish(nodes, edges, bits, symmetrize != 0, out)) return b.status ? b.status : 4;
+        return 0;
+    });
+    return rc && !seen ? unseen(rc) : rc;
 }
 
 int b40c_device_csr_rmat(int32_t device, int32_t scale, int32_t edge_factor, double a, double b, double c,
@@ -691,26 +739,26 @@ int b40c_device_csr_rmat(int32_t device, int32_t scale, int32_t edge_factor, dou
                    t_abc = (uint64_t) ((a + b + c) * two32);
     std::vector<int32_t> perm;
     if (scramble) b40c_rmat_permutation(scale, seed, &perm);
-    Builder bld;
-    if (!bld.start(device)) return bld.status;
-    const int bits = scale;
-    const long long n = 2 * samples;
-    KeyCounts kc;
-    if (!bld.alloc(n, scramble ? nodes : 0, 0) ||
-        !bld.ok(hipMemsetAsync(bld.key_counts(), 0, sizeof(KeyCounts), bld.stream)))
-        return bld.status;
-    if (scramble && !bld.ok(hipMemcpyAsync(bld.perm, perm.data(), sizeof(int) * (size_t) nodes,
-                                           hipMemcpyHostToDevice, bld.stream)))
-        return bld.status;
-    hipLaunchKernelGGL(rmat_keys_kernel, dim3(grid_for(samples)), dim3(kThreads), 0, bld.stream, samples, scale,
-                       (unsigned long long) seed, (unsigned long long) t_a, (unsigned long long) t_ab,
-                       (unsigned long long) t_abc, scramble ? bld.perm : nullptr, bits, bld.keys[0],
-                       &bld.key_counts()->loops);
-    if (!bld.ok(hipGetLastError()) || !bld.read_key_counts(&kc)) return bld.status;
-    long long edges = 0;
-    if (!bld.sort(n, 2 * bits) || !bld.compact(n, (long long) kc.loops, true, &edges)) return bld.status;
-    if (!bld.finish(nodes, edges, bits, true, out)) return bld.status ? bld.status : 4;
-    return 0;
+    return run_build(device, [&](Builder &bld) {
+        const int bits = scale;
+        const long long n = 2 * samples;
+        KeyCounts kc;
+        if (!bld.alloc(n, scramble ? nodes : 0, 0) ||
+            !bld.ok(hipMemsetAsync(bld.key_counts(), 0, sizeof(KeyCounts), bld.stream)))
+            return bld.status;
+        if (scramble && !bld.ok(hipMemcpyAsync(bld.perm, perm.data(), sizeof(int) * (size_t) nodes,
+                                               hipMemcpyHostToDevice, bld.stream)))
+            return bld.status;
+        hipLaunchKernelGGL(rmat_keys_kernel, dim3(grid_for(samples)), dim3(kThreads), 0, bld.stream, samples, scale,
+                           (unsigned long long) seed, (unsigned long long) t_a, (unsigned long long) t_ab,
+                           (unsigned long long) t_abc, scramble ? bld.perm : nullptr, bits, bld.keys[0],
+                           &bld.key_counts()->loops);
+        if (!bld.ok(hipGetLastError()) || !bld.read_key_counts(&kc)) return bld.status;
+        long long edges = 0;
+        if (!bld.sort(n, 2 * bits) || !bld.compact(n, (long long) kc.loops, true, &edges)) return bld.status;
+        if (!bld.finish(nodes, edges, bits, true, out)) return bld.status ? bld.status : 4;
+        return 0;
+    });
 }
 
 int b40c_device_csr_transpose(const b40c_device_csr *g, b40c_device_csr *out)
@@ -718,20 +766,20 @@ int b40c_device_csr_transpose(const b40c_device_csr *g, b40c_device_csr *out)
     if (!g || !out || g->nodes <= 0 || g->edges < 0 || !g->row_offsets) return 1;
     *out = b40c_device_csr{};
     if (int rc = device_ok(g->device)) return rc;
-    Builder b;
-    if (!b.start(g->device)) return b.status;
-    const int bits = bits_for(g->nodes);
-    const long long n = g->edges;
-    if (n > 0) {
-        if (!b.alloc(n, 0, 0)) return b.status;
-        hipLaunchKernelGGL(transpose_keys_kernel, dim3((unsigned) ((n + kTile - 1) / kTile)), dim3(kThreads), 0,
-                           b.stream, g->row_offsets, g->column_indices, g->nodes, n, bits, b.keys[0]);
-        // the tuples come in row order, and the passes are stable: sorting by
-        // the column leaves every column's rows in order
-        if (!b.ok(hipGetLastError()) || !b.sort(n, 2 * bits, bits)) return b.status;
-    }
-    if (!b.finish(g->nodes, n, bits, g->symmetric != 0, out)) return b.status ? b.status : 4;
-    return 0;
+    return run_build(g->device, [&](Builder &b) {
+        const int bits = bits_for(g->nodes);
+        const long long n = g->edges;
+        if (n > 0) {
+            if (!b.alloc(n, 0, 0)) return b.status;
+            hipLaunchKernelGGL(transpose_keys_kernel, dim3((unsigned) ((n + kTile - 1) / kTile)), dim3(kThreads), 0,
+                               b.stream, g->row_offsets, g->column_indices, g->nodes, n, bits, b.keys[0]);
+            // the tuples come in row order, and the passes are stable: sorting by
+            // the column leaves every column's rows in order
+            if (!b.ok(hipGetLastError()) || !b.sort(n, 2 * bits, bits)) return b.status;
+        }
+        if (!b.finish(g->nodes, n, bits, g->symmetric != 0, out)) return b.status ? b.status : 4;
+        return 0;
+    });
 }
 
 int b40c_device_csr_to_host(const b40c_device_csr *g, b40c_csr *out)

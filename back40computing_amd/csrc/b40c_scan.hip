@@ -334,7 +334,7 @@ void give_pinned_word(uint32_t *word)
 hipError_t ChainState::init(int dev, hipStream_t st)
 {
     device = dev;
-    hipError_t e = hipMalloc(&d_counter, sizeof(unsigned long long) + 4 * sizeof(uint32_t));
+    hipError_t e = device_malloc(&d_counter, sizeof(unsigned long long) + 4 * sizeof(uint32_t));
     if (e != hipSuccess) return e;
     d_word = reinterpret_cast<uint32_t *>(d_counter + 1);
     // on the launches' own stream: non-blocking streams do not wait for the
@@ -354,7 +354,7 @@ hipError_t ChainState::prepare(long long items, int tile_items, ChainArgs *c, hi
         }
         d_status = nullptr;
         capacity = 0;
-        hipError_t e = hipMalloc(&d_status, sizeof(unsigned long long) * (size_t) tiles);
+        hipError_t e = device_malloc(&d_status, sizeof(unsigned long long) * (size_t) tiles);
         if (e != hipSuccess) return e;
         // state 0 (unpublished) under every epoch; ordered on the launch's
         // (non-blocking) stream

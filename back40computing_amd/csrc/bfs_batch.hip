@@ -121,13 +121,13 @@ struct SlotTable {
         max_slots = slots;
         HIP_OK(hipSetDevice(dev), "hipSetDevice");
         HIP_OK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "create stream");
-        HIP_OK(hipMalloc(&d_slots, sizeof(BatchSlot) * slots), "allocate slots");
+        HIP_OK(device_malloc(&d_slots, sizeof(BatchSlot) * slots), "allocate slots");
         HIP_OK(hipHostMalloc(&h_slots, sizeof(BatchSlot) * slots, hipHostMallocDefault), "allocate pinned slots");
-        HIP_OK(hipMalloc(&d_ctl, sizeof(BatchControl)), "allocate batch control");
-        HIP_OK(hipMalloc(&d_list, sizeof(int) * slots), "allocate seed list");
-        HIP_OK(hipMalloc(&d_alive, sizeof(int)), "allocate alive counter");
+        HIP_OK(device_malloc(&d_ctl, sizeof(BatchControl)), "allocate batch control");
+        HIP_OK(device_malloc(&d_list, sizeof(int) * slots), "allocate seed list");
+        HIP_OK(device_malloc(&d_alive, sizeof(int)), "allocate alive counter");
         HIP_OK(hipHostMalloc(&h_alive, sizeof(int), hipHostMallocDefault), "allocate pinned counter");
-        HIP_OK(hipMalloc(&d_hubs, sizeof(HubEntry) * 2 * kBatchHubCapacity), "allocate grid-tier lists");
+        HIP_OK(device_malloc(&d_hubs, sizeof(HubEntry) * 2 * kBatchHubCapacity), "allocate grid-tier lists");
         memset(h_slots, 0, sizeof(BatchSlot) * slots);
         HIP_OK(hipMemcpy(d_slots, h_slots, sizeof(BatchSlot) * slots, hipMemcpyHostToDevice), "clear slots");
         HIP_OK(hipMemset(d_ctl, 0, sizeof(BatchControl)), "clear batch control");
@@ -230,7 +230,7 @@ bfs_status refresh_table(bfs_graph_pool *p)
     if (host.size() > p->table_cap) {
         size_t cap = std::max<size_t>(64, 2 * host.size());
         BatchGraph *nt = nullptr;
-        HIP_OK(hipMalloc(&nt, sizeof(BatchGraph) * cap), "allocate graph table");
+        HIP_OK(device_malloc(&nt, sizeof(BatchGraph) * cap), "allocate graph table");
         if (p->d_table) (void) hipFree(p->d_table);
         p->d_table = nt;
         p->table_cap = cap;
@@ -313,8 +313,8 @@ bfs_status bfs_pool_add_graph(bfs_graph_pool *p, const int32_t *h_row, const int
     g.nodes = nodes;
     g.edges = edges;
     size_t rb = sizeof(int) * ((size_t) nodes + 1), cb = sizeof(int) * (size_t) std::max<int64_t>(edges, 1);
-    HIP_OK(hipMalloc(&g.row, rb), "allocate row offsets");
-    HIP_OK(hipMalloc(&g.col, cb), "allocate column indices");
+    HIP_OK(device_malloc(&g.row, rb), "allocate row offsets");
+    HIP_OK(device_malloc(&g.col, cb), "allocate column indices");
     HIP_OK(hipMemcpy(g.row, h_row, rb, hipMemcpyHostToDevice), "copy row offsets");
     if (edges > 0) HIP_OK(hipMemcpy(g.col, h_col, sizeof(int) * (size_t) edges, hipMemcpyHostToDevice), "copy columns");
     p->bytes += (int64_t) (rb + cb);
@@ -328,7 +328,7 @@ bfs_status bfs_pool_add_graph(bfs_graph_pool *p, const int32_t *h_row, const int
         b40c_csr tr{};
         if (b40c_graph_from_coo(nodes, edges, h_col, src.data(), 0, 0, 0, &tr) != 0)
             return host_fail(BFS_ERR_OOM, "transpose construction failed");
-        bool ok = hipMalloc(&g.rrow, rb) == hipSuccess && hipMalloc(&g.rcol, cb) == hipSuccess &&
+        bool ok = device_malloc(&g.rrow, rb) == hipSuccess && device_malloc(&g.rcol, cb) == hipSuccess &&
                   hipMemcpy(g.rrow, tr.row_offsets, rb, hipMemcpyHostToDevice) == hipSuccess &&
                   (edges == 0 || hipMemcpy(g.rcol, tr.column_indices, sizeof(int) * (size_t) edges,
                                            hipMemcpyHostToDevice) == hipSuccess);
@@ -355,8 +355,8 @@ bfs_status bfs_pool_add_device_graph(bfs_graph_pool *p, const b40c_device_csr *d
     g.nodes = dg->nodes;
     g.edges = dg->edges;
     size_t rb = sizeof(int) * ((size_t) g.nodes + 1), cb = sizeof(int) * (size_t) std::max<int64_t>(g.edges, 1);
-    HIP_OK(hipMalloc(&g.row, rb), "allocate row offsets");
-    HIP_OK(hipMalloc(&g.col, cb), "allocate column indices");
+    HIP_OK(device_malloc(&g.row, rb), "allocate row offsets");
+    HIP_OK(device_malloc(&g.col, cb), "allocate column indices");
     HIP_OK(hipMemcpy(g.row, dg->row_offsets, rb, hipMemcpyDeviceToDevice), "copy row offsets");
     if (g.edges > 0)
         HIP_OK(hipMemcpy(g.col, dg->column_indices, sizeof(int) * (size_t) g.edges, hipMemcpyDeviceToDevice),
@@ -475,7 +475,7 @@ bfs_status bfs_batch_enact(bfs_batch *b, const int32_t *graph_ids, const int32_t
         if (b->arena) (void) hipFree(b->arena);
         b->arena = nullptr;
         b->arena_bytes = 0;
-        HIP_OK(hipMalloc(&b->arena, total), "allocate query state");
+        HIP_OK(device_malloc(&b->arena, total), "allocate query state");
         b->arena_bytes = total;
     }
     size_t off = 0;
@@ -914,14 +914,14 @@ bfs_status bfs_server_create(bfs_graph_pool *pool, const bfs_server_config *cfg,
         std::lock_guard<std::mutex> lk(pool->mu);
         s->graphs = pool->graphs;
         if (!s->graphs.empty()) {
-            if (hipMalloc(&s->d_table, sizeof(BatchGraph) * s->graphs.size()) != hipSuccess ||
+            if (device_malloc(&s->d_table, sizeof(BatchGraph) * s->graphs.size()) != hipSuccess ||
                 hipMemcpy(s->d_table, pool->d_table, sizeof(BatchGraph) * s->graphs.size(),
                           hipMemcpyDeviceToDevice) != hipSuccess)
                 return fail_out(host_fail(BFS_ERR_OOM, "copy graph table"));
         }
     }
     if (s->graphs.empty()) return fail_out(host_fail(BFS_ERR_INVALID_ARG, "pool has no graphs"));
-    if (hipMalloc(&s->d_arena, (size_t) c.hbm_budget_bytes) != hipSuccess)
+    if (device_malloc(&s->d_arena, (size_t) c.hbm_budget_bytes) != hipSuccess)
         return fail_out(host_fail(BFS_ERR_OOM, "allocate the query-state budget"));
     s->arena.reset((size_t) c.hbm_budget_bytes);
     if (hipStreamCreateWithFlags(&s->copy_stream, hipStreamNonBlocking) != hipSuccess)

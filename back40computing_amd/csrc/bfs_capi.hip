@@ -394,10 +394,10 @@ void free_queues(bfs_problem *p)
 // Both queues (of cap elements) and the tile status words; none on failure.
 hipError_t allocate_queues(bfs_problem *p, size_t cap, size_t words)
 {
-    hipError_t e = hipMalloc(&p->d_tile_status, sizeof(unsigned long long) * words);
+    hipError_t e = device_malloc(&p->d_tile_status, sizeof(unsigned long long) * words);
     for (int i = 0; i < 2 && e == hipSuccess; i++) {
-        e = hipMalloc(&p->d_q[i], sizeof(int) * cap);
-        if (e == hipSuccess && p->mark_pred) e = hipMalloc(&p->d_pq[i], sizeof(int) * cap);
+        e = device_malloc(&p->d_q[i], sizeof(int) * cap);
+        if (e == hipSuccess && p->mark_pred) e = device_malloc(&p->d_pq[i], sizeof(int) * cap);
     }
     if (e != hipSuccess) free_queues(p);
     return e;
@@ -408,7 +408,7 @@ hipError_t allocate_queues(bfs_problem *p, size_t cap, size_t words)
 // the queues need the room.
 bool optional_malloc(unsigned **buffer, size_t bytes)
 {
-    if (hipMalloc(buffer, bytes) == hipSuccess) return true;
+    if (device_malloc(buffer, bytes) == hipSuccess) return true;
     (void) hipGetLastError();  // (no error of the launches that follow)
     *buffer = nullptr;
     return false;
@@ -511,18 +511,18 @@ bfs_status bfs_problem_create(const int32_t *h_row_offsets, const int32_t *h_col
     if ((e = hipEventCreate(&p->ev_start)) != hipSuccess || (e = hipEventCreate(&p->ev_stop)) != hipSuccess)
         return cleanup(hip_fail(e, "create events"));
     size_t words = ((size_t) nodes + 31) / 32;
-    if ((e = hipMalloc(&p->d_row, sizeof(int) * ((size_t) nodes + 1))) != hipSuccess ||
-        (e = hipMalloc(&p->d_col, sizeof(int) * (size_t) std::max<int64_t>(edges, 1))) != hipSuccess ||
-        (e = hipMalloc(&p->d_depth, sizeof(int) * (size_t) nodes)) != hipSuccess ||
-        (e = hipMalloc(&p->d_visited, sizeof(unsigned) * words)) != hipSuccess ||
-        (e = hipMalloc(&p->d_ctl, sizeof(Control))) != hipSuccess ||
-        (e = hipMalloc(&p->d_hubs, sizeof(HubEntry) * 2 * kHubCapacity)) != hipSuccess ||
-        (e = hipMalloc(&p->d_fbm, sizeof(unsigned) * 2 * words)) != hipSuccess ||
-        (e = hipMalloc(&p->d_marks, 32 * words)) != hipSuccess)
+    if ((e = device_malloc(&p->d_row, sizeof(int) * ((size_t) nodes + 1))) != hipSuccess ||
+        (e = device_malloc(&p->d_col, sizeof(int) * (size_t) std::max<int64_t>(edges, 1))) != hipSuccess ||
+        (e = device_malloc(&p->d_depth, sizeof(int) * (size_t) nodes)) != hipSuccess ||
+        (e = device_malloc(&p->d_visited, sizeof(unsigned) * words)) != hipSuccess ||
+        (e = device_malloc(&p->d_ctl, sizeof(Control))) != hipSuccess ||
+        (e = device_malloc(&p->d_hubs, sizeof(HubEntry) * 2 * kHubCapacity)) != hipSuccess ||
+        (e = device_malloc(&p->d_fbm, sizeof(unsigned) * 2 * words)) != hipSuccess ||
+        (e = device_malloc(&p->d_marks, 32 * words)) != hipSuccess)
         return cleanup(hip_fail(e, "allocate problem"));
     // marks are clear between steps (each compaction clears what it reads)
     if ((e = hipMemset(p->d_marks, 0, 32 * words)) != hipSuccess) return cleanup(hip_fail(e, "clear marks"));
-    if (p->mark_pred && (e = hipMalloc(&p->d_pred, sizeof(int) * (size_t) nodes)) != hipSuccess)
+    if (p->mark_pred && (e = device_malloc(&p->d_pred, sizeof(int) * (size_t) nodes)) != hipSuccess)
         return cleanup(hip_fail(e, "allocate predecessors"));
     if ((e = hipHostMalloc(&p->h_ctl, sizeof(Control), hipHostMallocDefault)) != hipSuccess)
         return cleanup(hip_fail(e, "allocate pinned control block"));
@@ -550,8 +550,8 @@ bfs_status bfs_problem_create(const int32_t *h_row_offsets, const int32_t *h_col
         b40c_csr t{};
         if (b40c_graph_from_coo(nodes, edges, h_column_indices, src.data(), 0, 0, 0, &t) != 0)
             return cleanup(fail(BFS_ERR_OOM, "transpose construction failed"));
-        bool ok = hipMalloc(&p->d_rrow, sizeof(int) * ((size_t) nodes + 1)) == hipSuccess &&
-                  hipMalloc(&p->d_rcol, sizeof(int) * (size_t) std::max<int64_t>(edges, 1)) == hipSuccess &&
+        bool ok = device_malloc(&p->d_rrow, sizeof(int) * ((size_t) nodes + 1)) == hipSuccess &&
+                  device_malloc(&p->d_rcol, sizeof(int) * (size_t) std::max<int64_t>(edges, 1)) == hipSuccess &&
                   hipMemcpy(p->d_rrow, t.row_offsets, sizeof(int) * ((size_t) nodes + 1), hipMemcpyHostToDevice) ==
                       hipSuccess &&
                   (edges == 0 || hipMemcpy(p->d_rcol, t.column_indices, sizeof(int) * (size_t) edges,
@@ -879,7 +879,7 @@ bfs_status bfs_barrier_benchmark(int32_t device, int32_t blocks_per_cu, int32_t 
     bfs_status rc = BFS_OK;
     do {
         hipError_t e;
-        if ((e = hipMalloc(&d_ctl, sizeof(Control))) != hipSuccess) { rc = hip_fail(e, "allocate"); break; }
+        if ((e = device_malloc(&d_ctl, sizeof(Control))) != hipSuccess) { rc = hip_fail(e, "allocate"); break; }
         if ((e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking)) != hipSuccess) { rc = hip_fail(e, "stream"); break; }
         if ((e = hipEventCreate(&e0)) != hipSuccess || (e = hipEventCreate(&e1)) != hipSuccess) {
             rc = hip_fail(e, "events");
@@ -914,7 +914,7 @@ bfs_status bfs_copy_calibration(int32_t device, int64_t bytes, double *ms)
     bfs_status rc = BFS_OK;
     do {
         hipError_t e;
-        if ((e = hipMalloc(&a, bytes)) != hipSuccess || (e = hipMalloc(&b, bytes)) != hipSuccess) {
+        if ((e = device_malloc(&a, bytes)) != hipSuccess || (e = device_malloc(&b, bytes)) != hipSuccess) {
             rc = hip_fail(e, "allocate");
             break;
         }
@@ -952,9 +952,9 @@ bfs_status bfs_selftest_wave_primitives(int32_t device, int32_t *mismatches)
         in[i] = (int) ((x >> 16) % 97);
     }
     int *d_in = nullptr, *d_scan = nullptr, *d_rank = nullptr;
-    HIP_TRY(hipMalloc(&d_in, sizeof(int) * n), "allocate");
-    HIP_TRY(hipMalloc(&d_scan, sizeof(int) * n), "allocate");
-    HIP_TRY(hipMalloc(&d_rank, sizeof(int) * n), "allocate");
+    HIP_TRY(device_malloc(&d_in, sizeof(int) * n), "allocate");
+    HIP_TRY(device_malloc(&d_scan, sizeof(int) * n), "allocate");
+    HIP_TRY(device_malloc(&d_rank, sizeof(int) * n), "allocate");
     HIP_TRY(hipMemcpy(d_in, in.data(), sizeof(int) * n, hipMemcpyHostToDevice), "copy");
     HIP_TRY(launch_wave_selftest(d_in, d_scan, d_rank, n, nullptr), "launch");
     HIP_TRY(hipDeviceSynchronize(), "synchronize");

@@ -156,6 +156,15 @@ int persistent_grid_for(int num_cus, int loop, bool pred, bool exact, int blocks
 // first such refusal the process launches plainly.
 hipError_t launch_coresident(const void *kernel, dim3 grid, dim3 block, void **args, hipStream_t st);
 
+// hipMalloc for the library's device memory: where there is no room, the idle
+// memory that the device CSR builder keeps is given back first.
+hipError_t device_malloc(void **p, size_t bytes);
+template <typename T>
+hipError_t device_malloc(T **p, size_t bytes)
+{
+    return device_malloc(reinterpret_cast<void **>(p), bytes);
+}
+
 // Error helpers (they record the message bfs_last_error_message returns).
 bfs_status host_fail(bfs_status s, const char *msg);
 bfs_status host_hip_fail(hipError_t e, const char *what);

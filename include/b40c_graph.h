@@ -89,6 +89,12 @@ void b40c_coo_free(b40c_coo *c);
  *   b40c_device_csr_rmat     <- b40c_graph_rmat (same samples, drawn on the device)
  *   b40c_device_csr_transpose: the in-neighbour CSR of a device CSR
  * Return codes as above, plus 4 = device error (no device, HIP failure).
+ *
+ * What a build works in (about 16 bytes a key and 8 a pair, at most 512 MB)
+ * is kept for the next one while any device CSR built on that device is
+ * alive.  It goes back to the device when the last one is freed (or taken
+ * over by a pool), and before that when an allocation of this library finds
+ * no room.  Allocations made elsewhere do not reach it.
  */
 typedef struct b40c_device_csr {
     int32_t device;

@@ -112,3 +112,31 @@ def test_invalid_pairs_are_reported_before_a_lack_of_memory(stub):
             assert call(dst) == 2, room
             assert call(bad) == 1, room
     """)
+
+
+@pytest.mark.parametrize("use,room", [
+    ("CsrProblem().from_host_problem(g)", 0),
+    ("p.reset(1, 1.3)", 0),
+    ("pool.add(g)", 0),
+    ("pool.add_device(d)", 4 << 20),
+    ("Batch(full, max_queries=4).enact(np.zeros(4, np.int32), np.zeros(4, np.int32))", 0),
+    ("DeviceCsr.from_coo(400000, src[:10], dst[:10])", 0),
+    ("DeviceCsr.rmat(17, 1)", 0),
+    ("d.transpose()", 0),
+    ("ScanEnactor().scan(a.ctypes.data, a.ctypes.data, 1 << 20)", 0),
+])
+def test_idle_build_memory_is_given_back_to_other_allocations(stub, use, room):
+    run(stub, """
+        from back40computing_amd.batch import Batch, GraphPool
+        g = CsrGraph.random(60000, 100000, seed=1)
+        p = CsrProblem().from_host_problem(g)
+        pool, full = GraphPool(), GraphPool()
+        full.add(g)
+        a = np.zeros(1 << 20, np.uint32)
+        src, dst = np.zeros(1000000, np.int32), np.ones(1000000, np.int32)
+        d = DeviceCsr.from_coo(60000, src, dst)   # while it lives, the builder keeps what it built it with
+        used = hip.stub_used()
+        hip.stub_budget(used + %d)
+        keep = [%s]
+        assert hip.stub_used() <= used + %d
+    """ % (room, use, room))
