@@ -661,6 +661,7 @@ bfs_status bfs_enact(bfs_problem *p, bfs_strategy strategy, int32_t fused, int32
     int pgrid = persistent_grid(p, loop, max_grid_size);
     if (pgrid > p->num_cus * std::max(1, persistent_max_blocks_per_cu(loop, p->mark_pred, exact)))
         return fail(BFS_ERR_LAUNCH, "grid exceeds co-resident capacity");
+    const int full_grid = pgrid;
     // A small graph meets at cheaper barriers on fewer workgroups: one per
     // kWorkPerWorkgroup vertices and edges, about one round of a gathering
     // step's workgroup, and never fewer than eight (R-MAT scale 10: 15
@@ -682,7 +683,9 @@ bfs_status bfs_enact(bfs_problem *p, bfs_strategy strategy, int32_t fused, int32
                 "clear tile status words");
         p->scan_epoch = 1;
     }
-    SearchArgs s = search_args(p, pgrid);
+    // (the hybrid's threshold stays that of the full grid: a level of a small
+    // dense graph may hold nearly all its edges)
+    SearchArgs s = search_args(p, full_grid);
     if (p->cfg.compaction == 2) p->scan_epoch += (unsigned) stride;
     if (strategy != BFS_HYBRID) s.sat_t = -1;
 

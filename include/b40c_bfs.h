@@ -101,7 +101,8 @@ typedef struct bfs_config {
                                        vertices                                       */
     int32_t saturation_threshold;   /* hybrid: edge frontier > this leaves the
                                        persistent contract-expand kernel (-1: never;
-                                       default: 4 items per thread of the grid)       */
+                                       default: 4 items per thread of the grid that
+                                       blocks_per_cu and max_grid_size give)          */
     int32_t blocks_per_cu;          /* persistent grid = CUs * this (capped by occupancy) */
     int32_t cull_mode;              /* bfs_cull_mode */
     int32_t instrument;             /* 1: collect per-workgroup duty statistics */
