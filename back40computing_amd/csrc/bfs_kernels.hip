@@ -1162,7 +1162,7 @@ constexpr unsigned kChainGrabMax = kWave;  // tiles per grab: one lane each in t
 static_assert(kChainGrabMax * kWaves * 2 <= kWaves * kWaveQueueCap, "grab masks fit the staging area");
 
 template <bool PRED, bool EXACT, bool FILTER>
-__device__ __forceinline__ void chained_step(const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds)
+__device__ __forceinline__ void chained_step(const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds, StepIo io)
 {
     const int *in = s.q[c.step & 1];
     const int *pin = s.pq[c.step & 1];
@@ -1187,10 +1187,14 @@ __device__ __forceinline__ void chained_step(const SearchArgs &s, Cursor c, unsi
             if (i < n) {
                 const int u = ld_queue(in + i);
                 if (FILTER) {
-                    if (u >= 0) keep = ((s.visited[u >> 5] >> (u & 31)) & 1u) == 0;
+                    if (u >= 0) {
+                        const unsigned w = io.stale ? ld_agent(s.visited + (u >> 5)) : s.visited[u >> 5];
+                        keep = ((w >> (u & 31)) & 1u) == 0;
+                    }
                 } else {
                     const int p = PRED ? ld_queue(pin + i) : -1;
-                    keep = u >= 0 && history_pass<PRED>(lds, u) && claim<EXACT>(s.visited, s.depth, u, s.coherent_filter);
+                    keep = u >= 0 && history_pass<PRED>(lds, u) &&
+                           claim<EXACT>(s.visited, s.depth, u, s.coherent_filter || io.stale);
                     if (keep) {
                         s.depth[u] = c.iteration;
                         if (PRED) s.pred[u] = p;
@@ -1233,8 +1237,14 @@ __device__ __forceinline__ void chained_step(const SearchArgs &s, Cursor c, unsi
             const unsigned i = (first + k) * kBlock + threadIdx.x;
             const unsigned at = prefix + rank;
             if (at < s.cap) {
-                out[at] = ld_queue(in + i);
-                if (PRED) pout[at] = FILTER ? ld_queue(pin + i) : -1;
+                const int u = ld_queue(in + i), p = PRED && FILTER ? ld_queue(pin + i) : -1;
+                if (io.light) {
+                    st_agent(out + at, u);
+                    if (PRED) st_agent(pout + at, p);
+                } else {
+                    out[at] = u;
+                    if (PRED) pout[at] = p;
+                }
             } else {
                 lost = true;
             }
@@ -1253,7 +1263,7 @@ __device__ __forceinline__ void body_contract(const GraphArgs &g, const SearchAr
 {
     WaveQueue<PRED> wq = make_queue<PRED>(s, c.step, lds, io.light);
     if (s.tile_status) {
-        chained_step<PRED, EXACT, false>(s, c, n, lds);
+        chained_step<PRED, EXACT, false>(s, c, n, lds, io);
     } else {
         TileGrab tg = tile_grab(s, n, lds, kItems * kBlock, (n + kBlock - 1) / kBlock);
         while (true) {
@@ -1278,7 +1288,7 @@ __device__ __forceinline__ void body_filter(const GraphArgs &g, const SearchArgs
     const int *in = s.q[c.step & 1];
     const int *pin = s.pq[c.step & 1];
     if (s.tile_status) {
-        chained_step<PRED, EXACT, true>(s, c, n, lds);
+        chained_step<PRED, EXACT, true>(s, c, n, lds, io);
     } else {
         TileGrab tg = tile_grab(s, n, lds, kItems * kBlock, (n + kBlock - 1) / kBlock);
         while (true) {
@@ -3049,8 +3059,7 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
             fbm_exact_step = c.step + 1;
         }
         if (blockIdx.x == 0 && threadIdx.x == 0) prepare_step(s.ctl, c, n);
-        // (chained compaction keeps plain status words; it takes full barriers)
-        const bool light_step = EXACT && c.phase != kPhaseBottomUp && !mark && !bits && !from_bitmap && !s.tile_status &&
+        const bool light_step = EXACT && c.phase != kPhaseBottomUp && !mark && !bits && !from_bitmap &&
                                 (LOOP == kLoopTP ? item_work(s, c.phase, n) : s.track_edges ? fe : (unsigned long long) n) <= kLightWork;
         if (!light_step) refresh();
         const StepIo io{light_step, stale};
