@@ -134,8 +134,9 @@ __device__ __forceinline__ bool history_pass(Lds<PRED> &lds, int u)
 //   from before other workgroups' claims: pre-reads go past it.  (A word that
 //   is too old only costs a claim that fails, but on a lattice every second
 //   edge leads back to a vertex visited a level or two before.)
+// launched: the step is a launch of its own, whose hub launch follows anyway.
 struct StepIo {
-    bool light, stale;
+    bool light, stale, launched = false;
 };
 
 template <bool PRED>
@@ -517,7 +518,12 @@ __device__ __forceinline__ void body_expand_contract(const GraphArgs &g, const S
             }
         }
     } else if (sub == 0) {
-        const HubList hub = hub_list(s, c.step, hubs, n);
+        HubList hub = hub_list(s, c.step, hubs, n);
+        // The few members of a launched step lie on a workgroup or two, and
+        // its hub launch follows anyway: rows of a wave and more go there
+        // (R-MAT scale 20, a level of 10 members and 73 k new vertices: 60
+        // us with rows of 2048 alone, 48 from 64 on, 50 from 256 and 512).
+        if (io.launched && n < (unsigned) kBlock) hub.grid_t = min(hub.grid_t, kWave);
         TileGrab tg = tile_grab(s, n, lds, kBlock, edge_workgroups(fe_in));
         while (true) {
             const unsigned t = next_tile(&s.ctl->steal[c.step & 1], lds, tg);
@@ -1329,7 +1335,7 @@ template <bool PRED, bool EXACT>
 __device__ __forceinline__ void run_body(int phase, const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n,
                                          Lds<PRED> &lds, int sub, bool hubs, unsigned long long fe)
 {
-    const StepIo io{false, false};
+    const StepIo io{false, false, true};
     switch (phase) {
     case kPhaseExpandContract: body_expand_contract<PRED, EXACT>(g, s, c, n, lds, sub, hubs, fe, io); break;
     case kPhaseContractExpand: body_contract_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs, io); break;
