@@ -125,6 +125,15 @@ int persistent_grid(const bfs_problem *p, int loop, int max_grid_size)
                                p->cfg.blocks_per_cu, max_grid_size);
 }
 
+// Only chained contractions claim without atomics (best effort).  Every other
+// claim sets its visited bit for good, and then neither the labels nor the
+// barriers that would keep them fresh for a check are needed.
+bool exact_claims(const bfs_problem *p, bfs_strategy strategy)
+{
+    const bool chains = p->cfg.compaction == 2 && (strategy == BFS_TWO_PHASE || strategy == BFS_HYBRID);
+    return p->cfg.cull_mode == BFS_CULL_EXACT || !chains;
+}
+
 int step_grid(const bfs_problem *p, int max_grid_size)
 {
     int occ = step_max_blocks_per_cu(p->mark_pred);
@@ -176,10 +185,9 @@ bfs_status read_control(bfs_problem *p)
 // frontier is empty.  Steps are issued in chunks; an empty frontier makes
 // the remaining launches of a chunk return immediately.
 template <typename Next>
-bfs_status run_iterative(bfs_problem *p, const GraphArgs &g, const SearchArgs &s, Cursor &c, int grid,
+bfs_status run_iterative(bfs_problem *p, bool exact, const GraphArgs &g, const SearchArgs &s, Cursor &c, int grid,
                          int *launches, Next next, bool (*stop)(const Control &, Cursor, unsigned))
 {
-    const bool exact = p->cfg.cull_mode == BFS_CULL_EXACT;
     const int chunk = 6;
     while (true) {
         for (int k = 0; k < chunk; k++) {
@@ -239,7 +247,7 @@ Cursor next_hybrid(Cursor c, bool chained)
 bfs_status enact_hybrid(bfs_problem *p, const GraphArgs &g, const SearchArgs &s, int pgrid, int sgrid,
                         int *launches)
 {
-    const bool exact = p->cfg.cull_mode == BFS_CULL_EXACT;
+    const bool exact = exact_claims(p, BFS_HYBRID);
     // Two-phase levels per host check: the launches of a chunk past the
     // hand-back (or past an empty frontier) return at once, so the host
     // waits once per chunk rather than once per level
@@ -292,7 +300,6 @@ bfs_status enact_hybrid(bfs_problem *p, const GraphArgs &g, const SearchArgs &s,
 bfs_status enact_direction_iterative(bfs_problem *p, const GraphArgs &g, const SearchArgs &s, int grid,
                                      int *launches)
 {
-    const bool exact = p->cfg.cull_mode == BFS_CULL_EXACT;
     Cursor c{0, 0, kPhaseExpandContract};
     unsigned long long prev_mf = 0;  // the previous frontier's edges
     while (true) {
@@ -317,7 +324,7 @@ bfs_status enact_direction_iterative(bfs_problem *p, const GraphArgs &g, const S
         else if (dir != kPhaseBottomUp && c.phase == kPhaseBottomUp)
             HIP_TRY(launch_queue_from_bitmap(s, c, grid, p->stream, launches), "queue from bitmap");
         c.phase = dir;
-        HIP_TRY(launch_step(c.phase, p->mark_pred, exact, g, s, c, grid, p->stream, launches), "launch step");
+        HIP_TRY(launch_step(c.phase, p->mark_pred, true, g, s, c, grid, p->stream, launches), "launch step");
         c.step++;
         c.iteration++;
     }
@@ -652,7 +659,7 @@ bfs_status bfs_enact(bfs_problem *p, bfs_strategy strategy, int32_t fused, int32
     const bool reset = p->dirty;
     p->dirty = true;
 
-    const bool exact = p->cfg.cull_mode == BFS_CULL_EXACT;
+    const bool exact = exact_claims(p, strategy);
     int loop = strategy == BFS_EXPAND_CONTRACT ? kLoopEC
                : strategy == BFS_TWO_PHASE       ? kLoopTP
                : strategy == BFS_DIRECTION_OPTIMIZING ? kLoopDO
@@ -714,7 +721,7 @@ bfs_status bfs_enact(bfs_problem *p, bfs_strategy strategy, int32_t fused, int32
             HIP_TRY(launch_persistent(kLoopEC, p->mark_pred, exact, g, s, c, pgrid, p->stream), "launch persistent");
             launches++;
         } else {
-            st = run_iterative(p, g, s, c, sgrid, &launches, next_same, nullptr);
+            st = run_iterative(p, exact, g, s, c, sgrid, &launches, next_same, nullptr);
         }
         break;
     case BFS_CONTRACT_EXPAND:
@@ -723,7 +730,7 @@ bfs_status bfs_enact(bfs_problem *p, bfs_strategy strategy, int32_t fused, int32
             HIP_TRY(launch_persistent(kLoopCE, p->mark_pred, exact, g, s, c, pgrid, p->stream), "launch persistent");
             launches++;
         } else {
-            st = run_iterative(p, g, s, c, sgrid, &launches, next_same, nullptr);
+            st = run_iterative(p, exact, g, s, c, sgrid, &launches, next_same, nullptr);
         }
         break;
     case BFS_TWO_PHASE:
@@ -732,7 +739,7 @@ bfs_status bfs_enact(bfs_problem *p, bfs_strategy strategy, int32_t fused, int32
             HIP_TRY(launch_persistent(kLoopTP, p->mark_pred, exact, g, s, c, pgrid, p->stream), "launch persistent");
             launches++;
         } else {
-            st = run_iterative(p, g, s, c, sgrid, &launches,
+            st = run_iterative(p, exact, g, s, c, sgrid, &launches,
                                s.tile_status ? next_two_phase_chained : next_two_phase, nullptr);
         }
         break;

@@ -322,9 +322,11 @@ __device__ __forceinline__ void hub_phase(const SearchArgs &s, Cursor c, Lds<PRE
 // bitmap: no pre-read and no memory trip between a column entry and the
 // claimed vertex's row bounds.
 // Without ROWS the row bounds are not read (the caller does not gather).
-// With best-effort culling the claims are atomic here too: with four edges
-// per thread in flight, racing plain stores (claim_best_effort) passed so
-// many duplicates that queues of four times the vertices overflowed.
+// The claims are atomic whatever the cull mode: with four edges per thread in
+// flight, racing plain stores (claim_best_effort) passed so many duplicates
+// that queues of four times the vertices overflowed.  EXACT says that no step
+// of the search claims otherwise (only best-effort chained contractions do,
+// chained_step), so that every labelled vertex has its visited bit.
 // fast_claim_vertices: the same for vertices u[k] (-1: none) already at hand.
 template <bool PRED, bool EXACT, bool LOCAL, int S, bool ROWS = true>
 __device__ __forceinline__ unsigned fast_claim_vertices(const GraphArgs &g, const SearchArgs &s, int next_depth,
@@ -396,7 +398,7 @@ __device__ __forceinline__ unsigned fast_claim_vertices(const GraphArgs &g, cons
     for (int k = 0; k < S; k++)
         if (!((old[k] >> (u[k] & 31)) & 1u)) fresh |= 1u << k;
     if (!EXACT) {
-        // best-effort culling elsewhere may have lost bits of labelled vertices
+        // chained contractions may have lost bits of labelled vertices
         int dep[S];
 #pragma unroll
         for (int k = 0; k < S; k++) dep[k] = ((fresh >> k) & 1) ? s.depth[u[k]] : -1;
@@ -453,7 +455,7 @@ __device__ __forceinline__ unsigned edge_workgroups(unsigned long long fe)
 // scratch and reads every field from there for the whole kernel.
 // ---------------------------------------------------------------------------
 // (fe_in: the step's frontier edges)
-template <bool PRED, bool EXACT>
+template <bool PRED>
 __device__ __forceinline__ void body_expand_contract(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds,
                                      int sub, bool hubs, unsigned long long fe_in, StepIo io,
                                      unsigned *next_bits = nullptr, bool from_bitmap = false)
@@ -466,7 +468,7 @@ __device__ __forceinline__ void body_expand_contract(const GraphArgs &g, const S
     auto edges = [&](const int (&at)[4], const int (&pv)[4], unsigned) {
         int u[4], ub[4], ud[4];
         const unsigned fresh =
-            fast_claim_slots<PRED, EXACT, false, 4>(g, s, next_depth, at, pv, u, ub, ud, false, nullptr, io);
+            fast_claim_slots<PRED, true, false, 4>(g, s, next_depth, at, pv, u, ub, ud, false, nullptr, io);
 #pragma unroll
         for (int j = 0; j < 4; j++) fe += (unsigned) (ud[j] - ub[j]);
         // a clear frontier bitmap becomes the next frontier's, exactly
@@ -577,7 +579,7 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <bool PRED, bool EXACT>
+template <bool PRED>
 __device__ __forceinline__ void body_bottom_up(const GraphArgs &g, const SearchArgs &s, Cursor c, Lds<PRED> &lds)
 {
     WaveQueue<PRED> wq = make_queue<PRED>(s, c.step, lds);
@@ -721,16 +723,6 @@ __device__ __forceinline__ void body_bottom_up(const GraphArgs &g, const SearchA
                 const int v = (int) ((gi + (unsigned) k) * kWave + (unsigned) lane);
                 todo[k] = gi + (unsigned) k < w_end && v < g.nodes && ((vis[k] >> (v & 31)) & 1u) == 0 &&
                           end[k] > beg[k];
-            }
-            if (!EXACT) {
-                // Best-effort top-down levels may have lost visited bits to
-                // racing read-modify-writes; the label stays the authority.
-                int dep[kBuGroups];
-#pragma unroll
-                for (int k = 0; k < kBuGroups; k++)
-                    dep[k] = todo[k] ? s.depth[(gi + (unsigned) k) * kWave + (unsigned) lane] : -1;
-#pragma unroll
-                for (int k = 0; k < kBuGroups; k++) todo[k] = todo[k] && dep[k] == -1;
             }
 #pragma unroll
             for (int k = 0; k < kBuGroups; k++) {
@@ -1337,11 +1329,11 @@ __device__ __forceinline__ void run_body(int phase, const GraphArgs &g, const Se
 {
     const StepIo io{false, false, true};
     switch (phase) {
-    case kPhaseExpandContract: body_expand_contract<PRED, EXACT>(g, s, c, n, lds, sub, hubs, fe, io); break;
+    case kPhaseExpandContract: body_expand_contract<PRED>(g, s, c, n, lds, sub, hubs, fe, io); break;
     case kPhaseContractExpand: body_contract_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs, io); break;
     case kPhaseContract: body_contract<PRED, EXACT>(g, s, c, n, lds, io); break;
     case kPhaseExpand: body_expand<PRED, EXACT, true>(g, s, c, n, lds, sub, hubs, io, filters(s)); break;
-    case kPhaseBottomUp: body_bottom_up<PRED, EXACT>(g, s, c, lds); break;
+    case kPhaseBottomUp: body_bottom_up<PRED>(g, s, c, lds); break;
     default: body_filter<PRED, EXACT>(g, s, c, n, lds, io); break;
     }
 }
@@ -1354,14 +1346,14 @@ __device__ __forceinline__ void loop_body(int phase, const GraphArgs &g, const S
                                           unsigned *next_bits = nullptr, bool from_bitmap = false)
 {
     if constexpr (LOOP == kLoopEC) {
-        body_expand_contract<PRED, EXACT>(g, s, c, n, lds, sub, hubs, fe, io);
+        body_expand_contract<PRED>(g, s, c, n, lds, sub, hubs, fe, io);
     } else if constexpr (LOOP == kLoopCE) {
         // (expand: the step that ends a contract-expand fast path)
         if (phase == kPhaseExpand) body_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs, io);
         else body_contract_expand<PRED, EXACT>(g, s, c, n, lds, sub, hubs, io);
     } else if constexpr (LOOP == kLoopDO) {
-        if (phase == kPhaseBottomUp) body_bottom_up<PRED, EXACT>(g, s, c, lds);
-        else body_expand_contract<PRED, EXACT>(g, s, c, n, lds, sub, hubs, fe, io, next_bits, from_bitmap);
+        if (phase == kPhaseBottomUp) body_bottom_up<PRED>(g, s, c, lds);
+        else body_expand_contract<PRED>(g, s, c, n, lds, sub, hubs, fe, io, next_bits, from_bitmap);
     } else {
         if (phase == kPhaseContract) body_contract<PRED, EXACT>(g, s, c, n, lds, io);
         else if (phase == kPhaseExpand)
@@ -1409,21 +1401,16 @@ __device__ __forceinline__ void frontier_bitmap_pass(const GraphArgs &g, const S
 // ---------------------------------------------------------------------------
 constexpr unsigned long long kMarkEdges = 1ull << 20;  // fewest frontier edges for the marked form
 
-// fe counts the frontier's edges with multiplicity (best-effort levels may
-// queue a vertex more than once).
 __device__ __forceinline__ bool marked_step(const SearchArgs &s, unsigned long long fe)
 {
     return s.marks != nullptr && fe >= kMarkEdges && fe >= (unsigned long long) s.nodes / 2;
 }
 
-template <bool PRED, bool EXACT>
+template <bool PRED>
 __device__ __forceinline__ void body_expand_mark(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, Lds<PRED> &lds,
                                  int sub, bool hubs)
 {
-    // An edge marks its target when the target's visited bit is clear and,
-    // in best-effort mode, its label is still -1: that mode may have lost
-    // visited bits of labelled vertices, whose predecessors a mark would
-    // overwrite.
+    // An edge marks its target when the target's visited bit is clear.
     const int *in = s.q[c.step & 1];
     if (sub == 0) {
         // Tiles of kBlock frontier vertices: rows of the grid tier are
@@ -1489,13 +1476,6 @@ __device__ __forceinline__ void body_expand_mark(const GraphArgs &g, const Searc
                 bool todo[4];
 #pragma unroll
                 for (int j = 0; j < 4; j++) todo[j] = u[j] >= 0 && !((w[j] >> (u[j] & 31)) & 1u);
-                if (!EXACT) {
-                    int dep[4];
-#pragma unroll
-                    for (int j = 0; j < 4; j++) dep[j] = todo[j] ? s.depth[u[j]] : -1;
-#pragma unroll
-                    for (int j = 0; j < 4; j++) todo[j] = todo[j] && dep[j] == -1;
-                }
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     if (todo[j]) {
@@ -1525,13 +1505,6 @@ __device__ __forceinline__ void body_expand_mark(const GraphArgs &g, const Searc
             bool todo[U];
 #pragma unroll
             for (int j = 0; j < U; j++) todo[j] = u[j] >= 0 && !((w[j] >> (u[j] & 31)) & 1u);
-            if (!EXACT) {
-                int dep[U];
-#pragma unroll
-                for (int j = 0; j < U; j++) dep[j] = todo[j] ? s.depth[u[j]] : -1;
-#pragma unroll
-                for (int j = 0; j < U; j++) todo[j] = todo[j] && dep[j] == -1;
-            }
 #pragma unroll
             for (int j = 0; j < U; j++) {
                 if (todo[j]) {
@@ -1555,7 +1528,7 @@ __device__ __forceinline__ unsigned byte_bits(unsigned x)
 // order.  With fbm_out set, also writes every word of that frontier bitmap
 // (the next step's frontier, exactly: a direction-optimizing search that
 // turns bottom-up next needs no bitmap pass).
-template <bool PRED, bool EXACT>
+template <bool PRED>
 __device__ __forceinline__ void mark_compact(const GraphArgs &g, const SearchArgs &s, Cursor c, Lds<PRED> &lds, unsigned *fbm_out)
 {
     const unsigned words = ((unsigned) g.nodes + 31) >> 5;
@@ -1579,13 +1552,6 @@ __device__ __forceinline__ void mark_compact(const GraphArgs &g, const SearchArg
                 m[1] = make_uint4(0u, 0u, 0u, 0u);
                 const unsigned vis = s.visited[w];
                 bits &= ~vis;
-                if (!EXACT) {
-                    // best-effort levels may have lost bits of labelled vertices
-                    for (unsigned b = bits; b; b &= b - 1) {
-                        const int v = (int) ((w << 5) + (unsigned) __builtin_ctz(b));
-                        if (s.depth[v] != -1) bits &= ~(1u << (v & 31));
-                    }
-                }
                 if (bits) s.visited[w] = vis | bits;
             }
             if (fbm_out) fbm_out[w] = bits;
@@ -2082,7 +2048,7 @@ static_assert(kFastVisitedWords % 4 == 0, "the bitmap is cleared 16 bytes at a t
 
 // Marks the targets of the rows of the vertex frontier of step c (the rows
 // published for the grid tier follow in bits_from_hubs, behind a barrier).
-template <bool PRED, bool EXACT>
+template <bool PRED>
 __device__ __forceinline__ void bits_from_rows(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n,
                                                BitLds &B, unsigned *vbits)
 {
@@ -2091,7 +2057,7 @@ __device__ __forceinline__ void bits_from_rows(const GraphArgs &g, const SearchA
     wave_rows(g, s.q[c.step & 1], n, hub, B.rt, [&](const auto &u, const auto &p) {
 #pragma unroll
         for (int q = 0; q < (int) (sizeof(u) / sizeof(u[0])); q++)
-            if (u[q] >= 0) bit_mark<PRED, EXACT>(s, vbits, u[q], p[q]);
+            if (u[q] >= 0) bit_mark<PRED, true>(s, vbits, u[q], p[q]);
     });
 }
 
@@ -2112,7 +2078,7 @@ __device__ __forceinline__ unsigned hub_entry_of_wave(const HubEntry *list, unsi
 }
 
 // The published rows, a wave per chunk.
-template <bool PRED, bool EXACT>
+template <bool PRED>
 __device__ __forceinline__ void bits_from_hubs(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned *vbits)
 {
     const unsigned long long a = ld64_agent(&s.ctl->hub_alloc[c.step & 1]);
@@ -2135,7 +2101,7 @@ __device__ __forceinline__ void bits_from_hubs(const GraphArgs &g, const SearchA
             }
 #pragma unroll
             for (int j = 0; j < U; j++)
-                if (u[j] >= 0) bit_mark<PRED, EXACT>(s, vbits, u[j], e.par);
+                if (u[j] >= 0) bit_mark<PRED, true>(s, vbits, u[j], e.par);
         }
     }
 }
@@ -2230,7 +2196,7 @@ __device__ __forceinline__ void bits_collect(const GraphArgs &g, const SearchArg
             const unsigned vis = s.visited[w];
             bits &= ~vis;
             if (!EXACT) {
-                // best-effort levels may have lost bits of labelled vertices
+                // chained contractions may have lost bits of labelled vertices
                 for (unsigned b = bits; b; b &= b - 1) {
                     const int v = (w << 5) + __builtin_ctz(b);
                     if (s.depth[v] != -1) bits &= ~(1u << (v & 31));
@@ -2303,7 +2269,7 @@ __device__ __forceinline__ void bits_collect(const GraphArgs &g, const SearchArg
 // barrier whatever its row lengths.  Each batch reserves its queue slots
 // with one atomic per workgroup.  next_bits as for body_expand_contract.
 // Every thread of every workgroup calls it; F must not be live.
-template <bool PRED, bool EXACT>
+template <bool PRED>
 __device__ __forceinline__ void spread_step(const GraphArgs &g, const SearchArgs &s, Cursor c, unsigned n, FastFront &F,
                             StepIo io, unsigned *next_bits)
 {
@@ -2326,7 +2292,7 @@ __device__ __forceinline__ void spread_step(const GraphArgs &g, const SearchArgs
     const int stride = (int) gridDim.x * kBlock * kFastK;
     for (int b0 = (int) blockIdx.x * kBlock * kFastK; b0 < total; b0 += stride) {
         int u[kFastK], pv[kFastK], ub[kFastK], ud[kFastK];
-        const unsigned fresh = fast_edges<PRED, EXACT, false>(g, s, next_depth, F.deg[0], F.beg[0], F.v[0], n, total,
+        const unsigned fresh = fast_edges<PRED, true, false>(g, s, next_depth, F.deg[0], F.beg[0], F.v[0], n, total,
                                                        b0 + (int) threadIdx.x * kFastK, u, pv, ub, ud, false, nullptr,
                                                        io);
         int got;
@@ -2870,8 +2836,8 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
     // Barriers: full ones order plain stores before plain loads; light ones
     // (after light steps, see StepIo) only what goes past the XCDs' L2s, and
     // leave the caches stale: the next step that is not light itself
-    // refreshes them first.  Best-effort culling reads labels, which are
-    // plain stores, so its barriers are all full.
+    // refreshes them first.  Searches with best-effort contractions read
+    // labels, which are plain stores, so their barriers are all full.
     bool stale = false;
     auto bar = [&](bool light) {
         if (EXACT && light) {
@@ -3076,11 +3042,11 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
                 __syncthreads();
                 bits_clear(s, vbits);
                 if constexpr (LOOP == kLoopEC || LOOP == kLoopDO) {
-                    bits_from_rows<PRED, EXACT>(g, s, c, n, B, vbits);
+                    bits_from_rows<PRED>(g, s, c, n, B, vbits);
                     if (s.max_degree >= min(s.grid_t, kWaveHubRow)) {
                         bar(true);
                         refresh();  // (the list is read through the caches)
-                        bits_from_hubs<PRED, EXACT>(g, s, c, vbits);
+                        bits_from_hubs<PRED>(g, s, c, vbits);
                     }
                 } else {
                     bits_from_items<PRED, EXACT>(s, c, n, vbits);
@@ -3137,12 +3103,12 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
         }
         if (spread) {
             if constexpr (LOOP == kLoopEC || LOOP == kLoopDO) {
-                spread_step<PRED, EXACT>(g, s, c, n, shared.fast.f, io, next_bits);
+                spread_step<PRED>(g, s, c, n, shared.fast.f, io, next_bits);
                 __syncthreads();
                 init_lds(lds);
             }
         } else if (mark) {
-            body_expand_mark<PRED, EXACT>(g, s, c, n, lds, 0, true);
+            body_expand_mark<PRED>(g, s, c, n, lds, 0, true);
         } else {
             loop_body<PRED, EXACT, LOOP>(c.phase, g, s, c, n, lds, 0, true, fe, io, next_bits, from_bitmap);
         }
@@ -3153,7 +3119,7 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
             t0 = s.instrument ? wall_clock64() : 0;
             refresh();  // (the list is read through the caches)
             const StepIo io{light_step, false};
-            if (mark) body_expand_mark<PRED, EXACT>(g, s, c, n, lds, 1, true);
+            if (mark) body_expand_mark<PRED>(g, s, c, n, lds, 1, true);
             else loop_body<PRED, EXACT, LOOP>(c.phase, g, s, c, n, lds, 1, true, fe, io, next_bits, from_bitmap);
             if (s.instrument) busy += wall_clock64() - t0;
             bar(light_step);
@@ -3166,7 +3132,7 @@ __global__ __launch_bounds__(kBlock) void persistent_kernel(GraphArgs g, SearchA
                 fbm_dirty |= 1u << ((c.iteration + 1) & 1);
                 fbm_exact_step = c.step + 1;
             }
-            mark_compact<PRED, EXACT>(g, s, c, lds, fbm_out);
+            mark_compact<PRED>(g, s, c, lds, fbm_out);
             if (s.instrument) busy += wall_clock64() - t0;
             bar(false);
         }
@@ -3389,8 +3355,8 @@ const void *persistent_ptr(int loop, bool fastv)
 {
     switch (loop) {
     case kLoopEC:
-        return fastv ? reinterpret_cast<const void *>(&persistent_kernel<PRED, EXACT, kLoopEC, true>)
-                     : reinterpret_cast<const void *>(&persistent_kernel<PRED, EXACT, kLoopEC, false>);
+        return fastv ? reinterpret_cast<const void *>(&persistent_kernel<PRED, true, kLoopEC, true>)
+                     : reinterpret_cast<const void *>(&persistent_kernel<PRED, true, kLoopEC, false>);
     case kLoopCE:
         return fastv ? reinterpret_cast<const void *>(&persistent_kernel<PRED, EXACT, kLoopCE, true>)
                      : reinterpret_cast<const void *>(&persistent_kernel<PRED, EXACT, kLoopCE, false>);
@@ -3398,8 +3364,8 @@ const void *persistent_ptr(int loop, bool fastv)
         return fastv ? reinterpret_cast<const void *>(&persistent_kernel<PRED, EXACT, kLoopTP, true>)
                      : reinterpret_cast<const void *>(&persistent_kernel<PRED, EXACT, kLoopTP, false>);
     default:
-        return fastv ? reinterpret_cast<const void *>(&persistent_kernel<PRED, EXACT, kLoopDO, true>)
-                     : reinterpret_cast<const void *>(&persistent_kernel<PRED, EXACT, kLoopDO, false>);
+        return fastv ? reinterpret_cast<const void *>(&persistent_kernel<PRED, true, kLoopDO, true>)
+                     : reinterpret_cast<const void *>(&persistent_kernel<PRED, true, kLoopDO, false>);
     }
 }
 
@@ -3436,12 +3402,12 @@ hipError_t launch_step_t(int phase, const GraphArgs &g, const SearchArgs &s, Cur
                          int *launches)
 {
     switch (phase) {
-    case kPhaseExpandContract: return launch_phase<PRED, EXACT, kPhaseExpandContract>(g, s, c, grid, st, launches);
+    case kPhaseExpandContract: return launch_phase<PRED, true, kPhaseExpandContract>(g, s, c, grid, st, launches);
     case kPhaseContractExpand: return launch_phase<PRED, EXACT, kPhaseContractExpand>(g, s, c, grid, st, launches);
     case kPhaseContract: return launch_phase<PRED, EXACT, kPhaseContract>(g, s, c, grid, st, launches);
     case kPhaseExpand: return launch_phase<PRED, EXACT, kPhaseExpand>(g, s, c, grid, st, launches);
     case kPhaseFilter: return launch_phase<PRED, EXACT, kPhaseFilter>(g, s, c, grid, st, launches);
-    case kPhaseBottomUp: return launch_phase<PRED, EXACT, kPhaseBottomUp>(g, s, c, grid, st, launches);
+    case kPhaseBottomUp: return launch_phase<PRED, true, kPhaseBottomUp>(g, s, c, grid, st, launches);
     default: return hipErrorInvalidValue;
     }
 }

@@ -82,8 +82,11 @@ typedef enum bfs_frontier_type {
 /* Visited-culling discipline. */
 typedef enum bfs_cull_mode {
     BFS_CULL_EXACT = 0,        /* atomic visited bitmask: every vertex enqueued once */
-    BFS_CULL_BEST_EFFORT = 1   /* reference discipline: racy bitmask + label check;
-                                  duplicates possible, labels still exact */
+    BFS_CULL_BEST_EFFORT = 1   /* reference discipline (racy bitmask + label check;
+                                  duplicates possible, labels still exact) in the
+                                  contract steps of chained compaction; all other
+                                  claims are exact, faster with several edges a
+                                  thread in flight */
 } bfs_cull_mode;
 
 /*
