@@ -144,7 +144,8 @@ __device__ int batch_plan(const BatchArgs &a, BatchLds &L, int level)
     if (tid < a.nslots) L.prefix[tid] = excl;
     if (tid == 0) L.prefix[a.nslots] = total;
     // Shorter rows than half a grid-tier chunk are no work to share: a tile
-    // spreads its rows over its workgroup anyway.
+    // spreads its rows over its workgroup anyway.  (Tiles of more than
+    // kHeavyTile edges share rows from kHeavyRow on, gather_tile.)
     if (tid == 0) L.grid_t = a.grid_t == 0x7fffffff ? a.grid_t : max(a.grid_t, kHubChunk / 2);
     if (blockIdx.x == 0 && tid == 0 && level < kLevelLog) {
         a.ctl->level_clock[level] = wall_clock64();

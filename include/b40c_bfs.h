@@ -110,10 +110,13 @@ typedef struct bfs_config {
     int32_t cull_mode;              /* bfs_cull_mode */
     int32_t instrument;             /* 1: collect per-workgroup duty statistics */
     int32_t grid_gather_threshold;  /* row length >= this: the row is split into chunks
-                                       shared by the whole grid (-1: never).  Steps of
-                                       few vertices, and tiles with many edges, share
-                                       shorter rows too; batched searches share none
-                                       below half a chunk */
+                                       shared by the whole grid.  Steps of few vertices,
+                                       bit-marked steps (2^16 + V/2 edges and more, at
+                                       most BFS_FAST_VISITED_MAX vertices) and tiles with
+                                       many edges share shorter rows too.  -1: only steps
+                                       of few vertices and bit-marked ones share rows.
+                                       Batched searches share none below 1024 edges (512
+                                       in tiles of more than 32768), and none at -1 */
     int32_t do_alpha;               /* direction-optimizing: go bottom-up when
                                        frontier edges * alpha > unexplored edges */
     int32_t do_beta;                /* direction-optimizing: back to top-down when
