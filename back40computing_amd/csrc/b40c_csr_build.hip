@@ -412,7 +412,7 @@ struct BuildSet {
         hipError_t e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking);
         if (e == hipSuccess) e = hipEventCreate(&ev0);
         if (e == hipSuccess) e = hipEventCreate(&ev1);
-        if (e == hipSuccess) e = chain.init(device, stream);
+        if (e == hipSuccess) e = chain.init(device);
         if (e != hipSuccess) drop();
         return e;
     }

@@ -331,19 +331,24 @@ void give_pinned_word(uint32_t *word)
 // ---------------------------------------------------------------------------
 // Chain state: the tile counter and the per-tile status words.
 // ---------------------------------------------------------------------------
-hipError_t ChainState::init(int dev, hipStream_t st)
+hipError_t ChainState::init(int dev)
 {
     device = dev;
     hipError_t e = device_malloc(&d_counter, sizeof(unsigned long long) + 4 * sizeof(uint32_t));
     if (e != hipSuccess) return e;
     d_word = reinterpret_cast<uint32_t *>(d_counter + 1);
-    // on the launches' own stream: non-blocking streams do not wait for the
-    // null stream, whose fill may still run when hipMemset returns
-    return hipMemsetAsync(d_counter, 0, sizeof(unsigned long long) + 4 * sizeof(uint32_t), st);
+    return hipSuccess;
 }
 
 hipError_t ChainState::prepare(long long items, int tile_items, ChainArgs *c, hipStream_t st)
 {
+    if (epoch == 0) {
+        // The first launch: its tile counter starts at zero.  Cleared on the
+        // launches' own stream: non-blocking streams do not wait for the null
+        // stream, whose fill may still run when hipMemset returns.
+        hipError_t e = hipMemsetAsync(d_counter, 0, sizeof(unsigned long long), st);
+        if (e != hipSuccess) return e;
+    }
     const long long tiles = std::max(1LL, (items + tile_items - 1) / tile_items);
     if (tiles > capacity) {
         // earlier launches on the stream may still read the old words
@@ -427,7 +432,7 @@ bfs_status b40c_scan_enactor_create(int32_t device, b40c_scan_enactor **out)
     en->device = device;
     if ((e = hipStreamCreateWithFlags(&en->stream, hipStreamNonBlocking)) != hipSuccess ||
         (e = hipEventCreate(&en->ev0)) != hipSuccess || (e = hipEventCreate(&en->ev1)) != hipSuccess ||
-        (e = en->chain.init(device, en->stream)) != hipSuccess ||
+        (e = en->chain.init(device)) != hipSuccess ||
         (e = take_pinned_word(&en->h_word)) != hipSuccess ||
         (e = hipHostGetDevicePointer(reinterpret_cast<void **>(&en->h_word_dev), en->h_word, 0)) != hipSuccess) {
         b40c_scan_enactor_destroy(en);

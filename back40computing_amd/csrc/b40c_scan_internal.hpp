@@ -34,11 +34,11 @@ struct ChainState {
     long long capacity = 0;                   // status words allocated
     unsigned epoch = 0;
 
-    // The launches that follow are all on st.
-    hipError_t init(int dev, hipStream_t st);
+    hipError_t init(int dev);
     // Status words and a fresh epoch for a launch over `items` in tiles of
-    // tile_items.  (The tile counter needs no clearing: the workgroup that
-    // takes a launch's last tile sets it back to zero, prim::take_tile.)
+    // tile_items; every launch of a state is on the same stream.  (The tile
+    // counter is cleared before the first one alone: the workgroup that takes
+    // a launch's last tile sets it back to zero, prim::take_tile.)
     hipError_t prepare(long long items, int tile_items, ChainArgs *c, hipStream_t st);
     void release();
 };
