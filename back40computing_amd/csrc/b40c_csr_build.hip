@@ -389,21 +389,27 @@ int bits_for(int nodes)
 }
 
 // What a build needs besides its result -- a stream, events, chain state and
-// one block of device memory -- is kept per device between builds: allocating
-// and freeing 260 MB took longer than transposing 16 M edges (1.3 ms of 2.7,
-// on some boxes 8 of 9.5).  One build at a time has the kept set; others at
-// the same time make their own.  The block stays below kKeepBytes, and goes
-// back to the device when the last device CSR built here is freed, or when
-// an allocation of the library finds no room (device_malloc, run_build).
+// its buffers -- is kept per device between builds: allocating and freeing 260
+// MB took longer than transposing 16 M edges (1.3 ms of 2.7, on some boxes 8
+// of 9.5).  One build at a time has the kept set; others at the same time make
+// their own.  The buffers stay below kKeepBytes in all, and go back to the
+// device when the last device CSR built here is freed, or when an allocation
+// of the library finds no room (device_malloc, run_build).  They are separate
+// allocations: the runtime hands small ones that were freed out again at once,
+// where one block of all of them left it to map new memory for the problem
+// that is usually made next (R-MAT scale 13: 765 instead of 470 us).
 constexpr size_t kKeepBytes = (size_t) 512 << 20;
 constexpr int kKeepDevices = 64;
+
+// (the keys twice, the digit counts, the vertex permutation, the pairs)
+enum Buffer { kKeys0, kKeys1, kCounts, kPerm, kSrc, kDst, kBuffers };
 
 struct BuildSet {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     ChainState chain;
-    char *block = nullptr;
-    size_t bytes = 0;
+    void *buffer[kBuffers] = {};
+    size_t bytes[kBuffers] = {};
     bool busy = false;
 
     hipError_t make(int device)
@@ -416,28 +422,38 @@ struct BuildSet {
         if (e != hipSuccess) drop();
         return e;
     }
-    hipError_t reserve(size_t need)
+    size_t held() const
     {
-        if (need <= bytes) return hipSuccess;
-        release_block();
-        hipError_t e = device_malloc(&block, need);
+        size_t sum = 0;
+        for (size_t b : bytes) sum += b;
+        return sum;
+    }
+    hipError_t reserve(int k, size_t need)
+    {
+        if (need <= bytes[k]) return hipSuccess;
+        release(k);
+        hipError_t e = device_malloc(&buffer[k], need);
         if (e != hipSuccess) {
-            block = nullptr;
+            buffer[k] = nullptr;
             return e;
         }
-        bytes = need;
+        bytes[k] = need;
         return hipSuccess;
     }
-    void release_block()
+    void release(int k)
     {
-        if (block) (void) hipFree(block);
-        block = nullptr;
-        bytes = 0;
+        if (buffer[k]) (void) hipFree(buffer[k]);
+        buffer[k] = nullptr;
+        bytes[k] = 0;
+    }
+    void release_all()
+    {
+        for (int k = 0; k < kBuffers; k++) release(k);
     }
     void drop()
     {
         if (stream) (void) hipStreamSynchronize(stream);
-        release_block();
+        release_all();
         chain.release();
         if (ev0) (void) hipEventDestroy(ev0);
         if (ev1) (void) hipEventDestroy(ev1);
@@ -461,7 +477,7 @@ struct Builder {
     int *perm = nullptr;
     int *src = nullptr, *dst = nullptr;
     int status = 0;  // first failure: 1 invalid, 2 out of memory, 4 device error
-    size_t need = 0; // bytes of the block that the build uses
+    size_t need = 0; // bytes of buffers that the build uses
 
     ~Builder()
     {
@@ -472,17 +488,17 @@ struct Builder {
             return;
         }
         std::lock_guard<std::mutex> lock(g_keep_mu);
-        if (set->bytes > kKeepBytes || g_live[device] == 0) set->release_block();
+        if (set->held() > kKeepBytes || g_live[device] == 0) set->release_all();
         set->busy = false;
     }
 
-    // After a build that ran out of memory: whether the kept block held more
-    // than it needed; the block is released.
+    // After a build that ran out of memory: whether the kept buffers held more
+    // than it needed; they are released.
     bool gives_room()
     {
-        if (!set || set == &own || set->bytes <= need) return false;
+        if (!set || set == &own || set->held() <= need) return false;
         (void) hipStreamSynchronize(stream);
-        set->release_block();
+        set->release_all();
         (void) hipGetLastError();
         return true;
     }
@@ -511,24 +527,23 @@ struct Builder {
         return ok(hipEventRecord(set->ev0, stream));
     }
 
-    // Device memory of a build over n keys: the keys twice, the digit counts,
-    // the vertex permutation (perm_n) and the pairs (pairs_n), 256-byte aligned.
+    // Device memory of a build over n keys, with a vertex permutation (perm_n
+    // entries) and pairs (pairs_n), either of which may be none.
     bool alloc(long long n, long long perm_n, long long pairs_n)
     {
-        auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-        const size_t kb = up(sizeof(unsigned long long) * (size_t) std::max(1LL, n));
-        const size_t tiles = ((size_t) std::max(1LL, n) + kTile - 1) / kTile;
-        const size_t cb = up(sizeof(unsigned) * tiles * kDigits);
-        const size_t pb = up(sizeof(int) * (size_t) perm_n), qb = up(sizeof(int) * (size_t) pairs_n);
-        need = 2 * kb + cb + pb + 2 * qb;
-        if (!ok(set->reserve(need))) return false;
-        char *at = set->block;
-        keys[0] = reinterpret_cast<unsigned long long *>(at);
-        keys[1] = reinterpret_cast<unsigned long long *>(at + kb);
-        counts = reinterpret_cast<unsigned *>(at + 2 * kb);
-        perm = reinterpret_cast<int *>(at + 2 * kb + cb);
-        src = reinterpret_cast<int *>(at + 2 * kb + cb + pb);
-        dst = reinterpret_cast<int *>(at + 2 * kb + cb + pb + qb);
+        const size_t keys_n = (size_t) std::max(1LL, n), tiles = (keys_n + kTile - 1) / kTile;
+        const size_t want[kBuffers] = {sizeof(unsigned long long) * keys_n, sizeof(unsigned long long) * keys_n,
+                                       sizeof(unsigned) * tiles * kDigits, sizeof(int) * (size_t) perm_n,
+                                       sizeof(int) * (size_t) pairs_n, sizeof(int) * (size_t) pairs_n};
+        for (size_t w : want) need += w;
+        for (int k = 0; k < kBuffers; k++)
+            if (!ok(set->reserve(k, want[k]))) return false;
+        keys[0] = static_cast<unsigned long long *>(set->buffer[kKeys0]);
+        keys[1] = static_cast<unsigned long long *>(set->buffer[kKeys1]);
+        counts = static_cast<unsigned *>(set->buffer[kCounts]);
+        perm = static_cast<int *>(set->buffer[kPerm]);
+        src = static_cast<int *>(set->buffer[kSrc]);
+        dst = static_cast<int *>(set->buffer[kDst]);
         return true;
     }
 
@@ -629,7 +644,7 @@ struct Builder {
     }
 };
 
-// Runs one build, and once more if it ran out of memory beside a kept block
+// Runs one build, and once more if it ran out of memory beside kept buffers
 // larger than its own.
 template <typename Build>
 int run_build(int device, Build &&build)
@@ -665,8 +680,8 @@ hipError_t device_malloc(void **p, size_t bytes)
         std::lock_guard<std::mutex> lock(g_keep_mu);
         bool room = false;
         for (BuildSet &k : g_keep) {
-            if (k.busy || !k.block) continue;
-            k.release_block();
+            if (k.busy || !k.held()) continue;
+            k.release_all();
             room = true;
         }
         if (!room) return e;
@@ -679,7 +694,7 @@ void device_csr_gone(int device)
 {
     if (device < 0 || device >= kKeepDevices) return;
     std::lock_guard<std::mutex> lock(g_keep_mu);
-    if (g_live[device] > 0 && --g_live[device] == 0 && !g_keep[device].busy) g_keep[device].release_block();
+    if (g_live[device] > 0 && --g_live[device] == 0 && !g_keep[device].busy) g_keep[device].release_all();
 }
 
 }  // namespace b40c_hip
