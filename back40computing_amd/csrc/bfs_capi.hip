@@ -593,6 +593,7 @@ bfs_status bfs_problem_reset(bfs_problem *p, bfs_frontier_type ft, double queue_
     size_t cap = (size_t) want;
     if (cap > p->q_cap) {
         free_queues(p);
+        p->frontier_type = -1;  // not reset until it has queues again
         const size_t words = cap / kBlock + 2;
         hipError_t e = allocate_queues(p, cap, words);
         if (e == hipErrorOutOfMemory && drop_optional(p)) e = allocate_queues(p, cap, words);

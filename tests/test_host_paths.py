@@ -140,3 +140,23 @@ def test_idle_build_memory_is_given_back_to_other_allocations(stub, use, room):
         keep = [%s]
         assert hip.stub_used() <= used + %d
     """ % (room, use, room))
+
+
+def test_a_search_after_a_failed_reset_is_refused(stub):
+    run(stub, """
+        import back40computing_amd as b40c
+        p = CsrProblem().from_host_problem(CsrGraph.grid2d(100))
+        p.reset(b40c.EDGE_FRONTIERS, 1.3)
+        hip.stub_budget(hip.stub_used())
+        try:
+            p.reset(b40c.EDGE_FRONTIERS, 100.0)
+            raise SystemExit("queues larger than the device")
+        except BfsError:
+            pass
+        before = hip.stub_launches()
+        try:
+            p.enact(b40c.CONTRACT_EXPAND, 0)
+        except BfsError:
+            pass
+        assert hip.stub_launches() == before  # (the old queues are gone)
+    """)
