@@ -558,7 +558,7 @@ struct Builder {
     }
 
     // LSD radix sort of keys[0][0, n) over bits [low_bit, key_bits); the result
-    // is in keys[0].  Every pass takes the same number of bits, at most 8.
+    // is in keys[0].
     bool sort(long long n, int key_bits, int low_bit = 0)
     {
         if (n <= 1) return true;

@@ -1,8 +1,7 @@
 // b40c_primitives.hpp -- device building blocks of the single-pass scan,
 // stream compaction and radix sort kernels (b40c_scan.hip,
-// b40c_csr_build.hip): wave64 and workgroup sums over uint32, and the
-// decoupled look-back that chains tile prefixes through one status word
-// per tile.
+// b40c_csr_build.hip): wave64 sums over uint32, and the decoupled look-back
+// that chains tile prefixes through one status word per tile.
 //
 // Status word of a tile (64 bits, written and read whole, so the value needs
 // no fence of its own): bits 63..34 the launch epoch, bits 33..32 the state
@@ -48,28 +47,6 @@ __device__ __forceinline__ unsigned wave_inclusive_sum_u32(unsigned x)
 __device__ __forceinline__ unsigned wave_total_u32(unsigned x)
 {
     return (unsigned) __builtin_amdgcn_readlane((int) wave_inclusive_sum_u32(x), kWave - 1);
-}
-
-// Exclusive sum over a workgroup of THREADS threads (one value each); the
-// workgroup total goes to *total.  Uses wave_tot[THREADS / 64] of LDS.
-template <int THREADS>
-__device__ __forceinline__ unsigned block_exclusive_sum_u32(unsigned x, unsigned *wave_tot, unsigned *total)
-{
-    constexpr int kWaves = THREADS / kWave;
-    const int w = threadIdx.x / kWave;
-    const unsigned incl = wave_inclusive_sum_u32(x);
-    if (lane() == kWave - 1) wave_tot[w] = incl;
-    __syncthreads();
-    unsigned off = 0, tot = 0;
-#pragma unroll
-    for (int k = 0; k < kWaves; k++) {
-        const unsigned t = wave_tot[k];
-        if (k < w) off += t;
-        tot += t;
-    }
-    *total = tot;
-    __syncthreads();
-    return off + incl - x;
 }
 
 __device__ __forceinline__ unsigned long long status_word(unsigned epoch, unsigned state, unsigned value)

@@ -34,7 +34,6 @@ struct alignas(128) BatchSlot {
     unsigned cap;             // queue capacity (elements)
     unsigned qlen[3];
     unsigned long long fedges[3];
-    unsigned long long pad;
     unsigned long long t_begin, t_end;  // wall clock at seeding / completion
     unsigned ovf[3];          // per-step overflow of the output queue, by step % 3
     int bits;                 // fbm[iteration & 1] holds exactly the current frontier
@@ -42,14 +41,13 @@ struct alignas(128) BatchSlot {
 };
 
 struct alignas(256) BatchControl {
-    unsigned pad2[2];
     int level;                // levels completed by the batch
     int pad0;
     unsigned long long t_start;
-    unsigned bar_pad[26];
+    unsigned bar_pad[28];
     unsigned long long hub_alloc[2];  // grid tier: (entries << 32) | chunks, by level & 1
     unsigned hub_steal[2];            // grid tier: chunk counter, by level & 1
-    unsigned pad1[28];
+    unsigned pad1[26];
     // tile counters by level parity and group of workgroups, a 128-byte line each
     unsigned group_steal[2 * kTileGroups * 32];
     // grid barrier state (same layout discipline as Control)
@@ -60,6 +58,9 @@ struct alignas(256) BatchControl {
     unsigned level_td_tiles[kLevelLog];
     unsigned level_bu_tiles[kLevelLog];
 };
+
+static_assert(offsetof(BatchControl, hub_alloc) % 128 == 0 && offsetof(BatchControl, group_steal) % 128 == 0,
+              "counters on lines of their own");
 
 struct BatchArgs {
     const BatchGraph *graphs;

@@ -285,7 +285,7 @@ __device__ void batch_td_tile(const BatchArgs &a, BatchLds &L, int q, unsigned l
     const BatchGraph g = a.graphs[sl.graph];
     const int step = L.step[q];
     const unsigned n = (unsigned) L.n[q];
-    HubList hub{a.hubs[level & 1], a.hub_cap, &a.ctl->hub_alloc[level & 1], L.grid_t, q, kHubChunk, nullptr, kHeavyTile, kHeavyRow};
+    HubList hub{a.hubs[level & 1], a.hub_cap, &a.ctl->hub_alloc[level & 1], L.grid_t, q, nullptr, kHeavyTile, kHeavyRow};
     const unsigned width = (unsigned) L.width[q];
     const unsigned i = local * width + threadIdx.x;
     int v[1] = {-1}, beg[1] = {0}, end[1] = {0};

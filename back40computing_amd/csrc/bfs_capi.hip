@@ -51,7 +51,7 @@ const bfs_config kDefaults = {
     /*wave_gather_threshold*/ 64,
     /*cta_gather_threshold*/ 512,
     /*fast_path_threshold*/ 1024,
-    /*saturation_threshold*/ 0,   // 0: persistent grid size * 256
+    /*saturation_threshold*/ 0,   // 0: persistent grid size * kBlock * 4
     /*blocks_per_cu*/ 1,
     /*cull_mode*/ BFS_CULL_EXACT,
     /*instrument*/ 0,

@@ -71,8 +71,7 @@ constexpr size_t kControlHead = 256;
 static_assert(offsetof(Control, bar_root) == kControlHead, "status head ends where the barrier lines begin");
 
 // Grid-tier work item: a row too long for one workgroup, split into
-// chunk-edge chunks [first_chunk, first_chunk + ceil(len / chunk)); the
-// chunk is kHubChunk, or kBlock for steps with fewer tiles than workgroups.
+// kHubChunk-edge chunks [first_chunk, first_chunk + ceil(len / kHubChunk)).
 struct HubEntry {
     int beg, end, par;
     unsigned first_chunk;
@@ -372,7 +371,6 @@ struct HubList {
     unsigned long long *alloc;
     int grid_t;        // rows at least this long go to the grid tier
     int tag;           // stored with every published row
-    int chunk;         // edges per chunk
     unsigned *out_len; // expansions: length of the output queue (null: none reserved)
     int heavy, heavy_row;  // edges from which a tile publishes its rows of heavy_row and more (gather_tile)
 };
@@ -416,7 +414,7 @@ __device__ __forceinline__ bool publish_hub_row(int beg, int end, int par, const
     const bool pub = len >= hub.grid_t;
     const uint64_t pm = ballot(pub);
     if (!pm) return false;
-    const int nch = pub ? (len + hub.chunk - 1) / hub.chunk : 0;
+    const int nch = pub ? (len + kHubChunk - 1) / kHubChunk : 0;
     const int incl = wave_inclusive_sum(nch);
     const unsigned total = (unsigned) readlane(incl, kWave - 1);
     unsigned lo = 0, hi = 0;

@@ -174,7 +174,6 @@ __device__ __forceinline__ HubList hub_list(const SearchArgs &s, int step, bool 
     h.grid_t = enabled ? s.grid_t : 0x7fffffff;
     if (enabled && narrow_step(n)) h.grid_t = min(h.grid_t, kHubChunk);
     h.tag = 0;
-    h.chunk = kHubChunk;
     h.out_len = nullptr;
     h.heavy = narrow_step(n) ? kHeavyTileNarrow : kHeavyTile;
     h.heavy_row = narrow_step(n) ? kHeavyRowNarrow : kHeavyRow;
