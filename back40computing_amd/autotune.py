@@ -9,10 +9,11 @@ fastest one whose output is identical to the starting configuration's:
 
   * tile shape: workgroups per CU, tiles per counter grab, bottom-up tile
     size and grab layout (batched);
-  * gather tiers: wave / workgroup / grid row-length thresholds
-    (ExpandByWarp / ExpandByCta, two_phase/expand_atomic/cta.cuh:215-393),
-    and whether few-member top-down levels spread their edges evenly over
-    the grid instead;
+  * gathering: the row length from which the grid shares a row (a tile's
+    other rows are spread over its workgroup whatever their lengths, where
+    the reference has ExpandByWarp / ExpandByCta thresholds,
+    two_phase/expand_atomic/cta.cuh:215-393), and whether few-member
+    top-down levels spread their edges evenly over the grid instead;
   * direction switch points: alpha (top-down -> bottom-up) and beta
     (bottom-up -> top-down) of the direction-optimizing search.
 
@@ -32,6 +33,9 @@ import time
 import zlib
 
 from . import _native
+
+# bfs_config fields that select nothing: left out of the table.
+UNUSED = ("wave_gather_threshold", "cta_gather_threshold")
 
 TABLE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned.json")
 
@@ -189,7 +193,10 @@ def tune_batch(batch, graph_ids, sources, mode=0, reps=3, space=None, passes=3, 
             sig = zlib.crc32(batch.depths(q).tobytes(), sig)
         return _median(runs), sig
 
-    return coordinate_descent(measure, default_config("batch"), space, passes, log)
+    # (a batch shares no rows below half a grid-tier chunk)
+    start = default_config("batch")
+    start["grid_gather_threshold"] = max(start["grid_gather_threshold"], 1024)
+    return coordinate_descent(measure, start, space, passes, log)
 
 
 def load_table(path=TABLE_PATH):
@@ -204,7 +211,7 @@ def save_entry(kind, cfg, ms, workload, path=TABLE_PATH, device=None):
     table = load_table(path)
     dev = device or device_name()
     table.setdefault(dev, {})[kind] = {
-        "config": cfg,
+        "config": {k: v for k, v in cfg.items() if k not in UNUSED},
         "ms": round(ms, 4),
         "workload": workload,
         "tuned_at": time.strftime("%Y-%m-%dT%H:%M:%SZ", time.gmtime()),

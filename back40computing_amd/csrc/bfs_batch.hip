@@ -266,8 +266,8 @@ bfs_status bfs_batch_config_default(bfs_config *cfg)
     // Autotuned on the 256-query R-MAT pool (64 graphs, scale 14..20):
     // bottom-up tiles of up to 64 blocks (16384 consecutive vertices per
     // workgroup; levels with few blocks use smaller ones), two workgroups
-    // per CU, large consecutive grabs, an early grid tier (rows of 256
-    // neighbours and more) and a later turn to bottom-up than one search
+    // per CU, large grabs, an early grid tier (below half a chunk, 1024
+    // edges, no row is shared) and a later turn to bottom-up than one search
     // alone takes (alpha 12).
     cfg->blocks_per_cu = 2;
     cfg->bu_tile_blocks = 64;
