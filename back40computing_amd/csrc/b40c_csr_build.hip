@@ -393,12 +393,11 @@ int bits_for(int nodes)
 // MB took longer than transposing 16 M edges (1.3 ms of 2.7, on some boxes 8
 // of 9.5).  One build at a time has the kept set; others at the same time make
 // their own.  The buffers stay below kKeepBytes in all, and go back to the
-// device when an allocation of the library finds no room (device_malloc,
-// run_build); the whole set goes when the last device CSR built here is freed.
-// The problem that is usually made next takes over what the runtime recycles:
-// small allocations, which is why the buffers are not one block (R-MAT scale
-// 13: 765 instead of 470 us for it), and the stream (a new one takes 340 us
-// right after large buffers were unmapped, a recycled one 35).
+// device when the last device CSR built here is freed, or when an allocation
+// of the library finds no room (device_malloc, run_build).  They are separate
+// allocations: the runtime hands small ones that were freed out again at once,
+// where one block of all of them left it to map new memory for the problem
+// that is usually made next (R-MAT scale 13: 765 instead of 470 us).
 constexpr size_t kKeepBytes = (size_t) 512 << 20;
 constexpr int kKeepDevices = 64;
 
@@ -489,8 +488,7 @@ struct Builder {
             return;
         }
         std::lock_guard<std::mutex> lock(g_keep_mu);
-        if (g_live[device] == 0) set->drop();
-        else if (set->held() > kKeepBytes) set->release_all();
+        if (set->held() > kKeepBytes || g_live[device] == 0) set->release_all();
         set->busy = false;
     }
 
@@ -696,7 +694,7 @@ void device_csr_gone(int device)
 {
     if (device < 0 || device >= kKeepDevices) return;
     std::lock_guard<std::mutex> lock(g_keep_mu);
-    if (g_live[device] > 0 && --g_live[device] == 0 && !g_keep[device].busy) g_keep[device].drop();
+    if (g_live[device] > 0 && --g_live[device] == 0 && !g_keep[device].busy) g_keep[device].release_all();
 }
 
 }  // namespace b40c_hip

@@ -337,7 +337,6 @@ hipError_t ChainState::init(int dev)
     hipError_t e = device_malloc(&d_counter, sizeof(unsigned long long) + 4 * sizeof(uint32_t));
     if (e != hipSuccess) return e;
     d_word = reinterpret_cast<uint32_t *>(d_counter + 1);
-    epoch = 0;  // (a state that was released starts anew)
     return hipSuccess;
 }
 
