@@ -303,11 +303,11 @@ __device__ __forceinline__ int row_of_edge(const int *row, int nodes, long long 
 // maximum hands every edge its row.  (A search per edge, 20 dependent loads,
 // made 16 M edges 249 us; 55 now.)
 // A tile of more than kWalkRows rows an edge searches all the same, a thread's
-// sixteen edges together: its empty rows have no bound, and one workgroup
-// walked all of them (whole transposes of 1000 edges over 2^21 vertices
-// 3051 us walked, 680 searched; of 5000 over 20 M 19360 and 1250; 300 k over
-// 2^21, seven rows an edge, 83 to 109 us either way, as from 1 to 16).
+// edges kSearches at a time (sixteen at a time took 104 registers and half the
+// waves from the tiles that walk: 16 M edges 85 us instead of 55): its empty
+// rows have no bound, and one workgroup walked all of them.
 constexpr int kWalkRows = 4;
+constexpr int kSearches = 4;
 
 __global__ __launch_bounds__(kThreads) void transpose_keys_kernel(const int *row, const int *col, int nodes,
                                                                   long long edges, int bits,
@@ -323,24 +323,29 @@ __global__ __launch_bounds__(kThreads) void transpose_keys_kernel(const int *row
     __syncthreads();
     const int first = s_first, last = s_last;
     if (last - first > kWalkRows * kTile) {  // workgroup-uniform
-        int r[kRounds], top = 1;
+        int top = 1;  // (last - first < 2^31)
+        while (top <= (last - first) / 2) top *= 2;
+#pragma unroll 1
+        for (int k0 = 0; k0 * kThreads < count; k0 += kSearches) {
+            int r[kSearches], e[kSearches];
 #pragma unroll
-        for (int k = 0; k < kRounds; k++) r[k] = first;
-        while (2 * (long long) top <= last - first) top *= 2;
-        for (int st = top; st > 0; st >>= 1) {
-            int at[kRounds];
-#pragma unroll
-            for (int k = 0; k < kRounds; k++) at[k] = row[min((long long) r[k] + st, (long long) last)];
-#pragma unroll
-            for (int k = 0; k < kRounds; k++) {
-                const int i = min(k * kThreads + (int) threadIdx.x, count - 1);
-                if ((long long) r[k] + st <= last && at[k] <= e0 + i) r[k] += st;
+            for (int k = 0; k < kSearches; k++) {
+                r[k] = first;
+                e[k] = (int) e0 + min((k0 + k) * kThreads + (int) threadIdx.x, count - 1);
             }
-        }
+            for (int st = top; st > 0; st >>= 1) {
+                int at[kSearches];
 #pragma unroll
-        for (int k = 0; k < kRounds; k++) {
-            const int i = k * kThreads + (int) threadIdx.x;
-            if (i < count) keys[e0 + i] = ((unsigned long long) (unsigned) col[e0 + i] << bits) | (unsigned) r[k];
+                for (int k = 0; k < kSearches; k++) at[k] = row[r[k] + min(st, last - r[k])];
+#pragma unroll
+                for (int k = 0; k < kSearches; k++)
+                    if (st <= last - r[k] && at[k] <= e[k]) r[k] += st;
+            }
+#pragma unroll
+            for (int k = 0; k < kSearches; k++) {
+                const int i = (k0 + k) * kThreads + (int) threadIdx.x;
+                if (i < count) keys[e0 + i] = ((unsigned long long) (unsigned) col[e0 + i] << bits) | (unsigned) r[k];
+            }
         }
         return;
     }
