@@ -206,8 +206,9 @@ bfs_status bfs_problem_device_arrays(const bfs_problem *p, const int32_t **d_row
                                     const int32_t **d_in_column_indices, int32_t **d_depths);
 
 /* addition: per-step record of the last enact (first 64 steps): input
- * frontier length and start time in microseconds relative to step 0.
- * Returns the number of steps recorded in *steps. */
+ * frontier length and start time in microseconds relative to step 0.  A
+ * two-phase level is two steps (its expand step filters too), or three with
+ * compaction = 2.  Returns the number of steps recorded in *steps. */
 bfs_status bfs_get_level_log(const bfs_problem *p, int32_t max_steps, uint32_t *lengths, double *start_us,
                              int32_t *steps);
 
